@@ -11,6 +11,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -20,7 +21,7 @@ FSRC = os.path.join(HERE, "fortran")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 # packed FP32 instructions are kept out of the device code
-HIP_FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC", "-shared",
+HIP_FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wall", "-Wno-unused-function", "-Wno-unused-variable"]
 
@@ -34,10 +35,21 @@ def _run(cmd, cwd=None):
 
 def build_hip(verbose=False):
     out = os.path.join(HERE, "libbiefhip.so")
-    srcs = [os.path.join(CSRC, f) for f in ("bief_hip.hip", "layout.cpp")]
+    obj_dir = os.path.join(HERE, "_build")
+    os.makedirs(obj_dir, exist_ok=True)
+
+    def compile_one(f):
+        obj = os.path.join(obj_dir, os.path.splitext(f)[0] + ".o")
+        return obj, _run([HIPCC, *HIP_FLAGS, "-c", "-I", os.path.join(ROOT, "include"),
+                          os.path.join(CSRC, f), "-o", obj])
+
+    srcs = ("bief_hip.hip", "rows.hip", "layout.cpp", "rows_layout.cpp")
+    with ThreadPoolExecutor(len(srcs)) as ex:
+        done = list(ex.map(compile_one, srcs))
     tmp = out + ".tmp"
-    log = _run([HIPCC, *HIP_FLAGS, "-I", os.path.join(ROOT, "include"), *srcs, "-o", tmp])
+    _run([HIPCC, "-shared", f"--offload-arch={ARCH}", *(o for o, _ in done), "-o", tmp])
     os.replace(tmp, out)
+    log = "".join(text for _, text in done)
     if verbose:
         print(log)
     return out
@@ -85,7 +97,7 @@ def build_dropin():
     os.makedirs(mod, exist_ok=True)
     srcs = [os.path.join(FSRC, "bief_hip_capi.f90"), os.path.join(FSRC, "bief_hip_shim.F90"),
             os.path.join(ROOT, "oracle", "ref_driver.f90")]
-    _run([_fc(), "-O2", "-cpp", "-ffixed-line-length-132", "-fPIC", "-shared",
+    _run([_fc(), "-O2", "-cpp", "-ffixed-line-length-132", "-fPIC",
           "-I", os.path.join(ref, "mod"), "-module-dir", mod, *srcs,
           os.path.join(ref, "libbief_ref.a"), "-L", HERE, "-lbiefhip",
           "-Wl,-rpath,$ORIGIN/../../opentelemac_amd", "-o", out])

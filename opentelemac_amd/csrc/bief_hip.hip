@@ -32,155 +32,11 @@
 #include <vector>
 
 #include "../../include/bief_hip.h"
+#include "device_common.h"
 #include "layout.h"
+#include "rows_dev.h"
 
 namespace bhip {
-
-constexpr int kThreads = 256;
-static_assert(kThreads == kPhaseSlots, "colour phases are balanced for this workgroup size");
-constexpr int kWaves = kThreads / 64;
-
-#define HIP_OK(expr)                                              \
-  do {                                                            \
-    hipError_t e_ = (expr);                                       \
-    if (e_ != hipSuccess) {                                       \
-      fprintf(stderr, "libbiefhip: %s failed: %s (%s:%d)\n", #expr, \
-              hipGetErrorString(e_), __FILE__, __LINE__);         \
-      return BHIP_EDEVICE;                                        \
-    }                                                             \
-  } while (0)
-
-// ---------------------------------------------------------------------------
-// solver state (device resident)
-// ---------------------------------------------------------------------------
-enum : int { ST_RUNNING = 0, ST_CONVERGED = 1, ST_FINAL = 2, ST_MAXITER = 3 };
-
-// Iteration m of a CG solve runs U_m (vector update, parity p = m & 1) then
-// E_m (direction + EBE mat-vec). Slot [p] is written by iteration m and read
-// by iteration m + 1.
-struct SolveState {
-  double xl;        // max(||b'||^2, 1) (gracjg.F:189-209)
-  double eps2xl;    // stop threshold on ||r||^2 (inner solves: relative)
-  double rr0;       // ||r_0||^2 of the solve (inner solves scale eps2xl by it)
-  double dot;       // result of k_reduce_into
-  double rr[2];     // RMRM of iteration m, by parity
-  double rho[2];    // RO of iteration m (informational)
-  int m[2];         // iteration number M, by parity
-  int status[2];    // ST_RUNNING or ST_FINAL (NITMAX reached), by parity
-  int done;         // sticky: 0, ST_CONVERGED or ST_MAXITER
-  int nitmax;
-  int final_m;      // M at exit
-  int use_rr0;      // threshold = eps2xl * rr0
-  double final_rr;  // RMRM at exit
-  int final_flag;   // set by the update kernel that applied the last X update
-  int zero_rhs;     // ||b'|| < 1e-15 (gracjg.F:194-202)
-  double xl_raw;    // ||b'||^2
-  // mixed precision outer loop (device-side control)
-  double eps2_outer;   // outer stop threshold on the FP64 ||r'||^2
-  double rr_outer;     // last FP64 ||r'||^2
-  double inner_eps2;   // inner relative threshold
-  int inner_nitmax;    // iteration cap of one inner solve
-  int nitmax_total;    // NITMAX of the whole mixed solve (inner iterations)
-  int outer_done;      // the outer loop has stopped (outer_status says why)
-  int outer_status;    // ST_CONVERGED or ST_MAXITER once outer_done
-  int outer_count;     // inner solves started
-  int inner_total;     // inner iterations of finished inner solves
-  int done1;           // inner solve finished: (M << 2) | status, set by a kernel
-                       // after the one that applied the last update
-  int fresh;           // an outer test started an inner solve whose first
-                       // kernel has not run yet (set by k_outer_check,
-                       // cleared by the first update kernel of that solve)
-  int xpar;            // which of the two FP64 solution buffers holds x
-  int dpar;            // reliable updates: parity of the direction the next inner
-                       // start continues from, -1 for a fresh start
-  int reliable;        // mixed path: inner CG continued across outer steps
-  int inner_pairs[8];  // CG iterations (update + direction launches) of the
-                       // first inner solves, the next solve's launch plan
-  int stop;            // CG kernels of this solve return at once. Set by the
-                       // kernel after the one that set done, so that no
-                       // workgroup of a direction kernel skips its work on a
-                       // flag another workgroup of the same launch has set
-  long long t_start;   // device clock at the set-up of the solve
-  long long t_done;    // device clock when this system stopped
-};
-
-// ---------------------------------------------------------------------------
-// deterministic reductions
-// ---------------------------------------------------------------------------
-__device__ inline double wave_sum(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  return v;
-}
-
-// fixed-order block sum; result valid in thread 0
-__device__ inline double block_sum(double v, double* sh) {
-  v = wave_sum(v);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (lane == 0) sh[w] = v;
-  __syncthreads();
-  double s = 0.0;
-  if (threadIdx.x == 0) {
-    for (int i = 0; i < (int)(blockDim.x >> 6); ++i) s += sh[i];
-  }
-  __syncthreads();
-  return s;
-}
-
-// Fixed-order sum of n partials computed by every workgroup that calls it
-// (identical result in all of them); valid in all threads.
-__device__ inline double reduce_partials(const double* __restrict__ partial, int n,
-                                         double* sh, double* bcast) {
-  double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) s += partial[i];
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) *bcast = s;
-  __syncthreads();
-  s = *bcast;
-  __syncthreads();
-  return s;
-}
-
-// reduce_partials in two steps, for kernels that want other loads in
-// flight meanwhile: load_partials issues this thread's share of the partial
-// sums first (indices clamped, no branches around the loads); sum_partials
-// adds them in reduce_partials' order, so the result is the same to the bit.
-template <int P>
-__device__ inline void load_partials(double (&pv)[P], const double* __restrict__ partial,
-                                     int n) {
-#pragma unroll
-  for (int k = 0; k < P; ++k) pv[k] = partial[min((int)threadIdx.x + k * kThreads, n - 1)];
-}
-template <int P>
-__device__ inline double sum_partials(const double (&pv)[P], const double* __restrict__ partial,
-                                      int n, double* sh, double* bcast) {
-  double s = 0.0;
-#pragma unroll
-  for (int k = 0; k < P; ++k)
-    if ((int)threadIdx.x + k * kThreads < n) s += pv[k];
-  for (int i = threadIdx.x + P * kThreads; i < n; i += blockDim.x) s += partial[i];
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) *bcast = s;
-  __syncthreads();
-  s = *bcast;
-  __syncthreads();
-  return s;
-}
-
-// XCD-aware block order: workgroup g is dispatched to XCD g % 8; each XCD
-// gets a contiguous range of node blocks so that blocks sharing halo nodes
-// share an L2. Bijective for any block count.
-__device__ inline int xcd_block(int g, int nb) {
-  const int q = nb >> 3, r = nb & 7;
-  const int xcd = g & 7, k = g >> 3;
-  return xcd * q + (xcd < r ? xcd : r) + k;
-}
-
-__device__ inline int load_relaxed(const int* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void store_relaxed(int* p, int v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // ---------------------------------------------------------------------------
 // EBE kernel
@@ -794,6 +650,7 @@ __global__ void k_cg_setup(const double* __restrict__ partial, int nblocks,
   st->rr_outer = 0.0;
   st->dpar = -1;
   st->fresh = 0;
+  st->gave_up = 0;
   st->xpar = 0;
   st->reliable = mixed && reliable;
   for (int k = 0; k < 8; ++k) st->inner_pairs[k] = 0;
@@ -870,6 +727,7 @@ __global__ void k_outer_check(const double* __restrict__ partial, int nblocks,
     st->outer_done = 1;
     st->done = ST_CONVERGED;
     st->stop = 1;
+    st->fresh = 0;
     st->t_done = wall_clock64();
     return;
   }
@@ -1177,6 +1035,8 @@ struct bhip_ctx {
   };
   std::vector<SolveGraph> solve_graphs;
   bool use_graphs = true;
+  bhip::RowsDev* rows = nullptr;  // assembled rows for the persistent CG, or none
+  bool rows_off = false;          // it gave up once: the two-kernel CG from then on
   int prefetch_j = 0;  // register prefetch depth of the element kernels
   int iter_hint[4] = {0, 0, 0, 0};  // FP64 CG, inner CG, inner solves, CGSTAB
   int inner_hint[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // iterations of inner solve k (mixed CG)
@@ -1459,6 +1319,12 @@ static int ctx_setup(std::unique_ptr<bhip_ctx>& c, bhip_ctx** out) {
                      c->vdz.p, 0.0, (long)n);
   HIP_OK(hipGetLastError());
   HIP_OK(hipStreamSynchronize(c->stream));
+  {
+    const int64_t whole[2] = {0, n};
+    hipError_t e;
+    c->rows = rows_create(L, c->nsys, c->nsys > 1 ? c->sys_node_off.data() : whole, c->stream, &e);
+    HIP_OK(e);
+  }
   *out = c.release();
   return BHIP_OK;
 }
@@ -1538,6 +1404,7 @@ int bhip_ctx_destroy(bhip_ctx* c) {
     if (gr.exec) (void)hipGraphExecDestroy(gr.exec);
   for (auto& sg : c->solve_graphs)
     if (sg.exec) (void)hipGraphExecDestroy(sg.exec);
+  if (c->rows) rows_destroy(c->rows);
   if (c->st_host) (void)hipHostFree(c->st_host);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -2116,6 +1983,34 @@ static int cg_fp64(bhip_ctx* c, double* x, const double* b, double eps, int nitm
 }
 
 
+// Outer step of a mixed solve: x - delta into the other solution buffer, r =
+// A x - b with its partial sums, the inner right-hand side -r; then the test
+// (the first one of a solve, first = true: r = A x - b with x as given, no
+// delta to apply and no buffer switch)
+static int mixed_outer_step(bhip_ctx* c, double* x, const double* b, const float* delta,
+                            bool first) {
+  EbeArgs<double, double> a = base_args<double, double>(c, c->xa.p, c->da.p);
+  a.b = b;
+  a.r32 = c->fr.p;
+  a.partial = part_u(c, 0);
+  a.skip_if_outer_done = 1;
+  if (first) {
+    a.y = x;
+    HIP_OK((launch_ebe<double, double, STAGE_PLAIN, EPI_RESID_MIXED, FIN_PARTIAL>(
+        c, a, false, c->typdia, c->typext)));
+  } else {
+    a.xb0 = x;
+    a.xb1 = c->vx2.p;
+    a.delta = delta;
+    HIP_OK((launch_ebe<double, double, STAGE_XUPD, EPI_RESID_MIXED, FIN_PARTIAL>(
+        c, a, false, c->typdia, c->typext)));
+  }
+  hipLaunchKernelGGL(k_outer_check, dim3(c->nsys), dim3(kThreads), 0, c->stream, part_u(c, 0),
+                     c->L.nblocks, sys_ptr(c->sys_blocks), c->st_p, first ? 0 : 1);
+  HIP_OK(hipGetLastError());
+  return BHIP_OK;
+}
+
 // Mixed precision CG: FP64 true residual r = A'x - b' and FP64 update
 // x <- x - delta, with delta from an FP32 EBE CG on the FP32 copy of A'
 // (inner stop ||R||^2 <= inner_eps^2 ||r||^2). Same stop rule as GRACJG on the
@@ -2150,32 +2045,8 @@ static int cg_mixed(bhip_ctx* c, double* x, const double* b, double eps, int nit
                                                 c->fd0.p, c->fd1.p, c->fad.p, c->xa32.p,
                                                 c->da32.p);
   };
-  // outer step: x - delta into the other solution buffer, r = A x - b with
-  // its partial sums, the inner right-hand side -r; then the test
-  // (the first one of a solve, first = true: r = A x - b with x as given,
-  // no delta to apply and no buffer switch)
   auto outer_step = [&](bool first = false) -> int {
-    EbeArgs<double, double> a = base_args<double, double>(c, c->xa.p, c->da.p);
-    a.b = b;
-    a.r32 = c->fr.p;
-    a.partial = part_u(c, 0);
-    a.skip_if_outer_done = 1;
-    if (first) {
-      a.y = x;
-      HIP_OK((launch_ebe<double, double, STAGE_PLAIN, EPI_RESID_MIXED, FIN_PARTIAL>(
-          c, a, false, c->typdia, c->typext)));
-    } else {
-      a.xb0 = x;
-      a.xb1 = c->vx2.p;
-      a.delta = delta;
-      HIP_OK((launch_ebe<double, double, STAGE_XUPD, EPI_RESID_MIXED, FIN_PARTIAL>(
-          c, a, false, c->typdia, c->typext)));
-    }
-    hipLaunchKernelGGL(k_outer_check, dim3(c->nsys), dim3(kThreads), 0, c->stream,
-                       part_u(c, 0), L.nblocks, sys_ptr(c->sys_blocks), c->st_p,
-                       first ? 0 : 1);
-    HIP_OK(hipGetLastError());
-    return BHIP_OK;
+    return mixed_outer_step(c, x, b, delta, first);
   };
   const bool reliable = c->reliable;
   // the first kernel of the inner solves an outer test has just started
@@ -2270,6 +2141,100 @@ static int cg_mixed(bhip_ctx* c, double* x, const double* b, double eps, int nit
   return collect_infos(c, x, true, info);
 }
 
+// ---------------------------------------------------------------------------
+// CG on assembled rows: one persistent launch per (inner) solve
+// ---------------------------------------------------------------------------
+constexpr int kGaveUp = -1;  // the launch gave up: use the two-kernel CG
+
+// At most one persistent launch per GPU at a time: its workgroups wait for
+// each other, so two launches that share the CUs could each hold what the
+// other needs.
+static std::mutex& rows_mutex(int dev) {
+  static std::mutex mu[64];
+  return mu[dev & 63];
+}
+
+// GRACJG as in cg_fp64; the solution is left in xout (x stays the initial one)
+static int cg_rows_fp64(bhip_ctx* c, double* x, double* xout, const double* b, double eps,
+                        int nitmax, bhip_solve_info* info, const std::function<int()>& tail) {
+  std::lock_guard<std::mutex> one(rows_mutex(c->device));
+  HIP_OK(enqueue_bb_setup(c, b, eps, nitmax, 0, 0.0, 0));
+  EbeArgs<double, double> a = base_args<double, double>(c, c->xa.p, c->da.p);
+  a.y = x;
+  a.b = b;
+  a.out = c->vr.p;
+  a.partial = part_u(c, 0);
+  HIP_OK((launch_ebe<double, double, STAGE_PLAIN, EPI_RESID, FIN_PARTIAL>(c, a, false, c->typdia,
+                                                                          c->typext)));
+  RowsCg<double> q = {};
+  q.r0 = c->vr.p;
+  q.x0 = x;
+  q.x = xout;
+  q.diag = c->typdia == 'Q' ? c->da.p : nullptr;
+  q.part_rr = part_u(c, 0);
+  q.nblocks = c->L.nblocks;
+  q.sys_blocks = sys_ptr(c->sys_blocks);
+  q.st = c->st_p;
+  HIP_OK(rows_cg<double>(c->rows, q, c->stream));
+  int rc;
+  if ((rc = tail())) return rc;
+  if (read_state(c)) return BHIP_EDEVICE;
+  for (int sy = 0; sy < c->nsys; ++sy)
+    if (c->st_host[sy].gave_up) return kGaveUp;
+  return collect_infos(c, xout, false, info);
+}
+
+// mixed precision as in cg_mixed, each inner solve one persistent FP32 launch
+static int cg_rows_mixed(bhip_ctx* c, double* x, const double* b, double eps, int nitmax,
+                         double inner_eps, int inner_nitmax, bhip_solve_info* info,
+                         const std::function<int()>& tail) {
+  const Layout& L = c->L;
+  SolveState* sh = c->st_host;
+  HIP_OK(c->vx2.alloc(L.npoin));
+  float* delta = c->fx0.p;
+  std::lock_guard<std::mutex> one(rows_mutex(c->device));
+  if (c->typdia == 'Q') {
+    hipLaunchKernelGGL(k_to_f32, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream, c->da32.p,
+                       c->da.p, (long)L.npoin);
+    HIP_OK(hipGetLastError());
+  }
+  HIP_OK(enqueue_bb_setup(c, b, eps, nitmax, 1, inner_eps, inner_nitmax, c->reliable ? 1 : 0));
+  auto inner = [&]() -> int {
+    RowsCg<float> q = {};
+    q.r0 = c->fr.p;
+    q.x = delta;
+    q.diag = c->typdia == 'Q' ? c->da32.p : nullptr;
+    q.dlast = c->fdz.p;
+    q.st = c->st_p;
+    q.inner = 1;
+    HIP_OK(rows_cg<float>(c->rows, q, c->stream));
+    return BHIP_OK;
+  };
+  int rc = mixed_outer_step(c, x, b, delta, true);
+  int& hint_out = c->iter_hint[2];  // inner solves of one mixed solve
+  int nout = std::min(std::max(hint_out, 1), 8);
+  for (int rounds = 0;; ++rounds) {
+    for (int k = 0; k < nout && !rc; ++k) {
+      rc = inner();
+      if (!rc) rc = mixed_outer_step(c, x, b, delta, false);
+    }
+    if (rc || (rc = tail())) return rc;
+    if (read_state(c)) return BHIP_EDEVICE;
+    bool all = true;
+    for (int sy = 0; sy < c->nsys; ++sy) {
+      if (sh[sy].gave_up) return kGaveUp;
+      all = all && sh[sy].outer_done != 0;
+    }
+    if (all) break;
+    if (rounds > 2 * kMaxOuter) return BHIP_EDEVICE;
+    nout = 1;
+  }
+  int maxout = 0;
+  for (int sy = 0; sy < c->nsys; ++sy) maxout = std::max(maxout, sh[sy].outer_count);
+  hint_out = maxout;
+  return collect_infos(c, x, true, info);
+}
+
 }  // namespace bhip
 
 extern "C" {
@@ -2349,6 +2314,9 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   const bool mixed = cfg->precision == BHIP_PREC_MIXED;
   if (mixed && ensure_f32(c)) return BHIP_EDEVICE;
   bool xa32_ready = false;
+  // CG on assembled rows where the context has them (the state of the
+  // diagonal after the preconditioning below decides with it)
+  const bool want_rows = cfg->slv == 1 && c->rows && !c->rows_off;
   if (diag) {
     // PRECD1 (precd1.f:90-149), X and B taken from the caller's vectors
     hipLaunchKernelGGL(k_precd1_nodes, dim3(g), dim3(kThreads), 0, c->stream, c->vx.p, c->vb.p,
@@ -2358,13 +2326,22 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
     if (c->typdia == 'I') c->typdia = 'Q';
     if (c->ncoef > 0) {
       // the mixed path takes its FP32 copy of D A D in the same pass
-      float* x32 = mixed ? c->xa32.p : nullptr;
+      float* x32 = mixed && !want_rows ? c->xa32.p : nullptr;
       HIP_OK(launch_dmd(c, x32, c->vdinv.p, xa_src));
-      xa32_ready = mixed;
+      xa32_ready = x32 != nullptr;
     }
     if (precon % 2 == 0 || precon % 3 == 0) c->typdia = 'I';
   }
+  const bool use_rows = want_rows && c->typdia != '0';
+  if (use_rows) {
+    const int bytes = mixed ? 4 : 8, npair = L.ndp * (L.ndp - 1) / 2;
+    HIP_OK(rows_reserve(c->rows, bytes));
+    HIP_OK(rows_assemble(c->rows, bytes, c->xa.p, L.nslot_pad, npair, c->typext == 'Q',
+                         c->stream));
+  }
   int rc;
+  // where the solution is left (the persistent FP64 CG keeps the initial one)
+  double* xsrc = use_rows && !mixed ? c->vd1.p : c->vx.p;
   // X <- X*D (solve.f:637-641) and B <- D*B (as the reference leaves it),
   // back to the caller's order or copied as they are (internal). A mixed
   // solve of one system reads X from the solution buffer its state names;
@@ -2379,7 +2356,7 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
       hipLaunchKernelGGL(k_xpar_gather, dim3(L.nblocks), dim3(kThreads), 0, c->stream, c->vx.p,
                          c->vx2.p, c->node_start.p, sys_ptr(c->block_sys), c->st_p);
     }
-    hipLaunchKernelGGL(k_x_out, dim3(g), dim3(kThreads), 0, c->stream, x_dev, c->vx.p,
+    hipLaunchKernelGGL(k_x_out, dim3(g), dim3(kThreads), 0, c->stream, x_dev, xsrc,
                        c->vx2.p, stx, diag ? c->vdinv.p : nullptr, idx, n);
     hipLaunchKernelGGL(k_x_out, dim3(g), dim3(kThreads), 0, c->stream, b_dev, c->vb.p,
                        nullptr, nullptr, nullptr, idx, n);
@@ -2396,10 +2373,30 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   } else if (cfg->precision == BHIP_PREC_MIXED) {
     double ie = cfg->inner_eps > 0 ? cfg->inner_eps : 1e-4;
     int inn = cfg->inner_nitmax > 0 ? cfg->inner_nitmax : std::max(cfg->nitmax, 1);
-    rc = cg_mixed(c, c->vx.p, c->vb.p, cfg->eps, std::max(cfg->nitmax, 1), ie, inn, xa32_ready,
-                  info, tail);
+    const int nit = std::max(cfg->nitmax, 1);
+    rc = kGaveUp;
+    if (use_rows) {
+      rc = cg_rows_mixed(c, c->vx.p, c->vb.p, cfg->eps, nit, ie, inn, info, tail);
+      if (rc == kGaveUp) {
+        // from the solution its finished inner solves have left
+        c->rows_off = true;
+        hipLaunchKernelGGL(k_xpar_gather, dim3(L.nblocks), dim3(kThreads), 0, c->stream, c->vx.p,
+                           c->vx2.p, c->node_start.p, sys_ptr(c->block_sys), c->st_p);
+      }
+    }
+    if (rc == kGaveUp)
+      rc = cg_mixed(c, c->vx.p, c->vb.p, cfg->eps, nit, ie, inn, xa32_ready, info, tail);
   } else {
-    rc = cg_fp64(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, info, tail);
+    rc = kGaveUp;
+    if (use_rows) {
+      rc = cg_rows_fp64(c, c->vx.p, xsrc, c->vb.p, cfg->eps, cfg->nitmax, info, tail);
+      if (rc == kGaveUp) {
+        c->rows_off = true;
+        xsrc = c->vx.p;
+      }
+    }
+    if (rc == kGaveUp)
+      rc = cg_fp64(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, info, tail);
   }
   if (rc != BHIP_OK && rc != BHIP_MAXITER && rc != BHIP_ZERO_RHS) return rc;
   // the CG drivers wrote the results before their last wait, unless a

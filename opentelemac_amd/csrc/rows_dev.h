@@ -1,0 +1,47 @@
+// Device side of the assembled row storage: the matrix in row form and the
+// persistent CG on it (rows.hip).
+#pragma once
+
+#include "device_common.h"
+#include "rows.h"
+
+namespace bhip {
+
+struct RowsDev;
+
+// The rows of a layout on the current device, or nullptr when they cannot be
+// used (build_rows; *err stays hipSuccess then). Work is queued on stream;
+// the host arrays are read before it returns.
+RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStream_t stream,
+                     hipError_t* err);
+void rows_destroy(RowsDev* r);
+
+// Row values of precision 8 or 4 bytes: allocated here when first asked for.
+hipError_t rows_reserve(RowsDev* r, int bytes);
+
+// Assembles the rows of the precision from the slot coefficients xa (upper
+// npair columns, and the lower ones when nonsym), nslot_pad apart.
+hipError_t rows_assemble(RowsDev* r, int bytes, const double* xa, int nslot_pad, int npair,
+                         bool nonsym, hipStream_t stream);
+
+// One CG solve per system of the context (gracjg.F:248-409), from the
+// residual r0 to the stop, in one launch. Vectors in internal node order.
+template <typename T>
+struct RowsCg {
+  const T* r0;             // A x - b (FP64), or b - A x of an inner solve (its sign)
+  const T* x0;             // initial solution, or nullptr for zero
+  T* x;                    // solution (not x0: a launch that gives up leaves x0 as it is)
+  const T* diag;           // diagonal, or nullptr for a unit diagonal
+  T* dlast;                // the previous direction of a continued solve (read), and the
+                           // last direction of this one (written); nullptr: neither
+  const double* part_rr;   // partial sums of ||r0||^2 per node block, or nullptr: the
+                           // state's rr0
+  int nblocks;
+  const int32_t* sys_blocks;
+  SolveState* st;
+  int inner;               // an inner solve: only systems with a fresh start
+};
+template <typename T>
+hipError_t rows_cg(RowsDev* r, const RowsCg<T>& a, hipStream_t stream);
+
+}  // namespace bhip

@@ -1,0 +1,91 @@
+"""CG on assembled rows (one persistent launch per solve): the sizes where its
+partition changes, against the oracle, and the path it falls back to.
+
+Tolerances: FP64 solves to eps 1e-10 differ from the oracle's by rounding that
+CG amplifies, 1e-10 of the solution as in the other solve tests; a mixed solve
+and the oracle both stop at a relative residual of eps 1e-9, so their
+solutions agree within the condition number of the scaled system (under 100
+for these time steps) times that, 1e-7."""
+import numpy as np
+import pytest
+
+from opentelemac_amd import bief, mesh as M, system as S
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(m):
+    return S.wave_system(m, 2.0 + m.x / m.x.max(), dt=1.0)
+
+
+def _check(m, sysd, precon=2, block_nodes=0, typext="S", seed=0):
+    rng = np.random.default_rng(seed)
+    b = sysd["b"] + 1e-2 * rng.normal(size=m.npoin)
+    xa = sysd["xa"] if typext == "S" else np.concatenate([sysd["xa"], sysd["xa"]])
+    A = O.Matrix(sysd["da"], xa, "Q", typext)
+    out = []
+    for prec, eps, tol in ((bief.PREC_FP64, 1e-10, 1e-10), (bief.PREC_MIXED, 1e-9, 1e-7)):
+        xr, ir, _, _ = O.solve(A, m.ikle, b, sysd["x0"], slv=1, precon=precon, eps=eps,
+                               nitmax=2000)
+        ctx = bief.Context(m, block_nodes=block_nodes)
+        ctx.set_matrix("Q", typext, sysd["da"], xa)
+        x, info = ctx.solve(sysd["x0"].copy(), b.copy(), slv=1, precon=precon, eps=eps,
+                            nitmax=2000, precision=prec)
+        assert info["converged"], info
+        if prec == bief.PREC_FP64:
+            assert abs(info["niter"] - ir.niter) <= 1, (info, ir.niter)
+        assert np.linalg.norm(x - xr) <= tol * np.linalg.norm(xr), (prec, info)
+        out.append(x)
+        ctx.close()
+    return out
+
+
+# nodes around one slab of 1024 rows, and the first sizes of 2, 4 and 8 slabs
+# per workgroup
+@pytest.mark.parametrize("nx,ny", [(1, 1), (30, 32), (31, 31), (24, 40), (682, 2), (514, 510),
+                                   (730, 719), (1030, 1020)])
+def test_rows_cg_at_partition_edges(gpu, nx, ny):
+    m = M.channel_mesh(nx, ny, 10.0 * nx, 10.0 * ny)
+    _check(m, _system(m))
+
+
+@pytest.mark.parametrize("precon", [0, 5])
+@pytest.mark.parametrize("typext", ["S", "Q"])
+def test_rows_cg_with_a_diagonal(gpu, precon, typext):
+    """No unit diagonal (PRECON 5, none) and coefficients stored in both
+    halves; node blocks that do not match the slabs."""
+    m = M.random_small_mesh(70, 61, seed=3)
+    _check(m, S.wave_system(m, 2.0 + m.x / 10.0, dt=0.3), precon=precon, block_nodes=300,
+           typext=typext)
+
+
+def test_more_workgroups_than_the_gpu_holds(gpu):
+    """300 systems of one workgroup each: workgroups numbered as they start."""
+    meshes = [M.random_small_mesh(4 + k % 5, 5 + k % 3, seed=k) for k in range(300)]
+    systems = [S.wave_system(m, 2.0 + m.x / 10.0, dt=1.0 + 0.01 * k)
+               for k, m in enumerate(meshes)]
+    cat = lambda key: np.concatenate([s[key] for s in systems], axis=-1)  # noqa: E731
+    ens = bief.Ensemble(meshes)
+    for prec, eps, tol in ((bief.PREC_FP64, 1e-10, 1e-10), (bief.PREC_MIXED, 1e-9, 1e-7)):
+        ens.set_matrix("Q", "S", cat("da"), cat("xa"))
+        x, info = ens.solve(cat("x0"), cat("b"), slv=1, precon=2, eps=eps, nitmax=500,
+                            precision=prec)
+        assert info["converged"]
+        for m, sd, xs, si in zip(meshes, systems, ens.split(x), ens.infos()):
+            xr, ir, _, _ = O.solve(O.Matrix(sd["da"], sd["xa"], "Q", "S"), m.ikle, sd["b"],
+                                   sd["x0"], slv=1, precon=2, eps=eps, nitmax=500)
+            assert np.linalg.norm(xs - xr) <= tol * np.linalg.norm(xr)
+            if prec == bief.PREC_FP64:
+                assert abs(si["niter"] - ir.niter) <= 1
+
+
+def test_a_launch_that_gives_up_falls_back(gpu, monkeypatch):
+    """A limit of zero on the workgroups' waits: the persistent launch gives up
+    at its first meeting and the two-kernel CG solves the system."""
+    m = M.channel_mesh(120, 90, 1200.0, 900.0)
+    sysd = _system(m)
+    want = _check(m, sysd)
+    monkeypatch.setenv("BHIP_ROWS_WAIT", "0")
+    got = _check(m, sysd)
+    assert np.linalg.norm(got[0] - want[0]) <= 1e-10 * np.linalg.norm(want[0])
