@@ -2,19 +2,30 @@
 // the workgroups of the persistent Krylov kernels (rows.hip).
 //
 // Rows (nodes, internal order) are cut into slabs of kSlab consecutive rows of
-// one system. Inside a slab rows are sorted by their number of off-diagonal
-// entries, so that the 64 rows of a wave (a slice) have nearly the same count
-// and padding stays at a few per cent. A slice stores its entries entry by
-// entry, 64 lanes wide (coalesced): entry j of lane l of slice q is
-// (slice_off[q] + j) * 64 + l.
+// one system; a workgroup owns `group` consecutive slabs (a power of two, the
+// same for the whole context), `group` rows per thread. Every row has a leaf
+// number in its slab that does not depend on the group, and thread t of a
+// workgroup owns the leaves t * group ... t * group + group - 1 of its slabs:
+// sums over rows are binary trees over leaves, first within a thread, so they
+// do not depend on the group either.
 //
-// A workgroup owns `group` consecutive slabs (a power of two, the same for
-// the whole context). It holds the multiplied vector of its own rows and of
-// its halo (rows of other workgroups that its entries name) in LDS; ids[] are
-// indices into that array: own row at position p of the workgroup's k-th slab
-// is k * kSlab + p, halo entry h is group * kSlab + h. Between products each
-// workgroup hands the rows that others need (exp_loc) to them through global
-// memory.
+// Leaves are given out so that the 64 rows a wave works on at once (a slice:
+// the k-th rows of its lanes) have nearly the same number of entries. Each
+// half of a slab is sorted by it; rank g * 64 + v becomes leaf 8 v + j(g), j =
+// 0, 4, 1, 5, 2, 6, 3, 7: groups of 8 take one run of 64 ranks per slice,
+// groups of 4 two neighbouring ones. (Groups of 1 and 2 keep their rows'
+// first entries in registers, where padding costs nothing.)
+//
+// A slice stores its coefficients entry by entry, 64 lanes wide (coalesced):
+// entry j of lane l of slice q is (slice_off[q] + j) * 64 + l. Its column ids
+// are stored two entries to a 32-bit word: ids[((pair_off[q] + j / 2) * 64 + l) * 2
+// + (j & 1)]. Slice k * kSlices + w of workgroup g is q = g * group * kSlices + that.
+//
+// A workgroup holds the multiplied vector of its own rows and of its halo (rows
+// of other workgroups that its entries name) in LDS; ids[] are indices into that
+// array: thread t's k-th row is k * kSlab + t, halo entry h is group * kSlab + h.
+// With each product the workgroups hand the rows that others need (exp_loc) to
+// them through global memory.
 #pragma once
 
 #include <cstdint>
@@ -26,29 +37,28 @@
 namespace bhip {
 
 constexpr int kSlab = 1024;          // rows of a slab, threads of a workgroup
-constexpr int kSlices = kSlab / 64;  // slices (waves) of a slab
+constexpr int kSlices = kSlab / 64;  // waves of a workgroup, slices of one row per thread
 constexpr int kMaxGroup = 8;         // slabs of one workgroup
 constexpr int kMaxGang = 256;        // workgroups of one system
 
 struct RowLayout {
-  int nslab = 0, group = 1, nwg = 0;
+  int group = 1, nwg = 0, nslice = 0;
   int max_halo = 0, max_gang = 0;
   int64_t nent = 0;                  // entries, 64 per unit of slice_off
   int64_t nref = 0;
-  std::vector<int32_t> slab_row0;    // [nslab] first row (internal node id)
-  std::vector<int32_t> slab_rows;    // [nslab] rows of the slab
-  std::vector<uint16_t> rowpos;      // [nslab * kSlab] row - slab_row0 at position p, 0xffff: none
-  std::vector<int32_t> slice_off;    // [nslab * kSlices + 1]
-  std::vector<uint16_t> ids;         // [nent] LDS index of the entry's column
+  std::vector<int32_t> wg_row0;      // [nwg] first row (internal node id)
+  std::vector<uint16_t> rowpos;      // [nwg * group * kSlab] row - wg_row0 at LDS index, 0xffff: none
+  std::vector<int32_t> slice_off;    // [nslice + 1]
+  std::vector<int32_t> pair_off;     // [nslice + 1]
+  std::vector<uint16_t> ids;         // LDS index of the entry's column
   // assembly: entry column j of slice q sums cnt[slice_off[q] + j] coefficients,
   // whose references start at ref_off[q] * 64, 64 lanes wide, column by column.
   // A reference is pair * nslot_pad + slot, its top bit set for a term below
   // the element's diagonal (the second half of a non-symmetric matrix), or -1
   std::vector<uint8_t> cnt;
-  std::vector<int64_t> ref_off;      // [nslab * kSlices]
+  std::vector<int64_t> ref_off;      // [nslice]
   std::vector<int32_t> refs;
   // workgroups
-  std::vector<int32_t> wg_slab0;     // [nwg + 1]
   std::vector<int32_t> wg_sys;       // [nwg]
   std::vector<int32_t> sys_wg;       // [nsys + 1]
   std::vector<int32_t> halo_off;     // [nwg + 1]

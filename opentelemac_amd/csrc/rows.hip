@@ -1,25 +1,35 @@
 // Persistent Krylov kernels on assembled rows (rows.h), MI355X.
 //
 // One launch runs a whole CG solve. Each workgroup (one per CU, 1024 threads)
-// keeps the residual, the solution and A D of its rows in registers, one row
-// of each of its slabs per thread, and the direction D of its rows and halo in
-// LDS; only the matrix is read again each iteration, and at most 2M rows of it
-// (120 MB in FP64) stay in the last-level cache.
+// keeps the residual and the solution of its rows in registers, `group` rows
+// per thread, and D and A D in LDS; the first kFront coefficients of each row
+// stay in registers too where they fit (FP64 groups of 1 and 2, FP32 up to 4).
+// Larger groups read the matrix again each iteration, out of the last-level
+// cache (120 MB for 2M rows in FP64).
 //
-// Workgroups meet twice per iteration (D.AD; ||R||^2 together with the
-// exchange of halo residuals). There are no fences: every word that crosses
-// workgroups is written and read with 64-bit relaxed atomics at agent scope
-// and carries the number of the meeting in its low half (a double travels as
-// two such words), so reading the right number is the synchronisation. Each
-// workgroup writes its sum to kReplicas places and reads all sums of its
-// system from one of them, which spreads the readers over the memory
-// channels. Measured per meeting on 8 XCDs: 1.35 us for 16 workgroups, 1.6
-// for 64, 2.0 for 128, 2.8 for 256 (one place instead of 8: 4.0 for 256; two
-// levels of 16: 3.5).
+// Workgroups meet once per iteration: D.AD, AD.AD, R.AD and R.R together, with
+// the exchange of A D of the halo rows. RO is R.R / D.AD; the next ||R||^2 is
+// R.R - 2 RO R.AD + RO^2 AD.AD, which is what a second meeting would add up
+// to the last digits (see kTrust); R and D of the halo follow locally. There
+// are no fences: every word that crosses workgroups is written and read with
+// 64-bit relaxed atomics at agent scope and carries the number of the meeting
+// in its low half (a double travels as two such words), so reading the right
+// number is the synchronisation. Each workgroup writes its sums to kReplicas
+// places and reads all sums of its system from one of them, which spreads the
+// readers over the memory channels. Measured for one sum: 1.35 us for 16
+// workgroups, 1.6 for 64, 2.0 for 128, 2.8 for 256 (one place instead of 8:
+// 4.0 for 256; two levels of 16: 3.5).
 //
-// Sums are binary trees over rows aligned on powers of two, so they do not
-// depend on how many slabs a workgroup holds: a system gives the same bits
-// alone and in an ensemble.
+// us per iteration, FP64 / FP32 rows: 1.4 / 1.7 (1,000 nodes, one workgroup),
+// 3.2 / 3.1 (20k), 3.9 / 3.7 (100k), 4.7 / 4.7 (260k), 5.8 / 5.5 (500k), 14.0 /
+// 7.9 (1M), 24.4 / 16.7 (2M). The two-kernel CG takes 15 at 20k, 50 (FP64) at
+// 2M and 22 (FP32) at 1M. What bounds it: below 500k the meeting (two trips
+// through memory, 1.7 us for 20 workgroups, 3.5 for 245), then the matrix
+// (8.0 TB/s in FP64 and 8.7 in FP32 at 2M rows).
+//
+// Sums are binary trees over the rows' leaf numbers (rows.h) and do not depend
+// on how many rows a workgroup holds: a system gives the same bits alone and
+// in an ensemble.
 //
 // Every wait ends: on the number it waits for, or after kWaitTicks of the
 // device clock, when the launch gives up (abort in the sync words), leaves the
@@ -33,6 +43,7 @@
 #include "rows_dev.h"
 
 #include <cstdlib>
+#include <type_traits>
 #include <memory>
 #include <vector>
 
@@ -41,6 +52,10 @@ namespace bhip {
 typedef unsigned long long u64;
 
 constexpr int kReplicas = 8;
+constexpr int kSums = 4;  // sums of one meeting
+// ||R||^2 of the next iteration is taken from this one's sums while it is at
+// least this part of ||R||^2: its relative error is then below 4e-16 / kTrust
+constexpr double kTrust = 1e-3;
 constexpr int kRowWaves = kSlab / 64;
 constexpr u64 kWaitTicks = 400000000ull;  // 4 s of the 100 MHz clock, unless the
                                           // environment says otherwise (rows_create)
@@ -56,17 +71,26 @@ __device__ inline double ld_f64(const double* p) {
 }
 
 // a value in numbered words: two for a double, one for a float
-template <typename T>
-constexpr int kWords = sizeof(T) / 4;
-__device__ inline void post(u64* p, unsigned e, double v) {
+// (the words of a double are `stride` apart)
+__device__ inline void post(u64* p, size_t stride, unsigned e, double v) {
   const u64 b = __double_as_longlong(v);
   st_word(p, (b & 0xffffffff00000000ull) | e);
-  st_word(p + 1, (b << 32) | e);
+  st_word(p + stride, (b << 32) | e);
 }
-__device__ inline void post(u64* p, unsigned e, float v) {
+__device__ inline void post(u64* p, size_t, unsigned e, float v) {
   st_word(p, ((u64)__float_as_uint(v) << 32) | e);
 }
-// waits for the value numbered e; false after the deadline
+// one look: the value, if it is the one numbered e
+__device__ inline bool look(const u64* p, size_t stride, unsigned e, double& v) {
+  const u64 a = ld_word(p), b = ld_word(p + stride);
+  v = __longlong_as_double((a & 0xffffffff00000000ull) | (b >> 32));
+  return (unsigned)a == e && (unsigned)b == e;
+}
+__device__ inline bool look(const u64* p, size_t, unsigned e, float& v) {
+  const u64 a = ld_word(p);
+  v = __uint_as_float((unsigned)(a >> 32));
+  return (unsigned)a == e;
+}
 struct Deadline {
   u64 t0, ticks;
   const int* abort;
@@ -75,32 +99,12 @@ struct Deadline {
            ((u64)wall_clock64() - t0 >= ticks || load_relaxed(abort));
   }
 };
-__device__ inline bool await(const u64* p, unsigned e, double& v, const Deadline& dl) {
-  u64 a, b;
-  for (int n = 0;;) {
-    a = ld_word(p);
-    b = ld_word(p + 1);
-    if ((unsigned)a == e && (unsigned)b == e) break;
-    if (dl.past(n)) return false;
-  }
-  v = __longlong_as_double((a & 0xffffffff00000000ull) | (b >> 32));
-  return true;
-}
-__device__ inline bool await(const u64* p, unsigned e, float& v, const Deadline& dl) {
-  u64 a;
-  for (int n = 0;;) {
-    a = ld_word(p);
-    if ((unsigned)a == e) break;
-    if (dl.past(n)) return false;
-  }
-  v = __uint_as_float((unsigned)(a >> 32));
-  return true;
-}
 
 // the sync words of one precision
 struct SyncWords {
-  u64* slots;       // [2][kReplicas][nwg][2] sums, by parity of the meeting
-  u64* xch;         // [exported rows][kWords]
+  u64* slots;       // [2][kReplicas][kSums][nwg][2] sums, by parity of the meeting
+  u64* xch;         // [2][2][exported rows], by parity of the meeting (a float has one
+                    // word only)
   unsigned* epoch;  // [2][nsys] number of the last meeting, by parity of the launch
   int* abort;       // a launch has given up
   unsigned* ticket; // workgroups started (launches larger than the GPU)
@@ -109,10 +113,10 @@ struct SyncWords {
 
 struct RowArgs {
   const int32_t* slice_off;
-  const uint16_t* ids;
+  const int32_t* pair_off;
+  const unsigned* ids;
   const uint16_t* rowpos;
-  const int32_t* slab_row0;
-  const int32_t* wg_slab0;
+  const int32_t* wg_row0;
   const int32_t* wg_sys;
   const int32_t* sys_wg;
   const int32_t* halo_off;
@@ -120,7 +124,7 @@ struct RowArgs {
   const int32_t* halo_src;
   const int32_t* exp_off;
   const uint16_t* exp_loc;
-  int nwg, nsys, nslab;
+  int nwg, nsys, nexp;
   SyncWords sy;
   int ep;        // parity of the launch
   int ticketed;  // workgroup numbers by order of start
@@ -129,100 +133,191 @@ struct RowArgs {
 // ---------------------------------------------------------------------------
 // sums
 // ---------------------------------------------------------------------------
-__device__ inline double lane_tree(double v, int from) {
-  for (int m = from; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);
-  return v;
+// Lane exchanges by DPP within rows of 16 lanes and the permlane swaps across
+// them. fold<M>(x, y): x + x of lane ^ M where bit M of the lane is 0, y + y of
+// lane ^ M where it is 1; one step of sums over lanes that halves the values
+// a lane carries. (fold<M>(x, x): x + x of lane ^ M.)
+template <int CTRL>
+__device__ inline double dpp(double v) {
+  const u64 b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((u64)hi << 32) | lo);
+}
+constexpr int kXor1 = 0xb1, kXor2 = 0x4e, kHalfMirror = 0x141, kMirror = 0x140, kRor8 = 0x128;
+__device__ inline double xor4(double v) {
+  const u64 b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_ds_swizzle((int)(unsigned)b, 0x101f);
+  const unsigned hi = __builtin_amdgcn_ds_swizzle((int)(unsigned)(b >> 32), 0x101f);
+  return __longlong_as_double(((u64)hi << 32) | lo);
+}
+template <int M>
+__device__ inline double fold(double x, double y) {
+  if constexpr (M >= 16) {
+    const u64 a = __double_as_longlong(x), b = __double_as_longlong(y);
+    auto swap = [](unsigned p, unsigned q) {
+      if constexpr (M == 16)
+        return __builtin_amdgcn_permlane16_swap(p, q, false, false);
+      else
+        return __builtin_amdgcn_permlane32_swap(p, q, false, false);
+    };
+    const auto lo = swap((unsigned)a, (unsigned)b);
+    const auto hi = swap((unsigned)(a >> 32), (unsigned)(b >> 32));
+    return __longlong_as_double(((u64)hi[0] << 32) | lo[0]) +
+           __longlong_as_double(((u64)hi[1] << 32) | lo[1]);
+  } else {
+    const bool up = threadIdx.x & M;
+    const double keep = up ? y : x, give = up ? x : y;
+    if constexpr (M == 8)
+      return keep + dpp<kRor8>(give);
+    else if constexpr (M == 2)
+      return keep + dpp<kXor2>(give);
+    else
+      return keep + dpp<kXor1>(give);
+  }
+}
+// sum over 16 lanes, over 64 (in all of them)
+__device__ inline double sum16(double v) {
+  v += dpp<kXor1>(v);
+  v += dpp<kXor2>(v);
+  v += dpp<kHalfMirror>(v);
+  return v + dpp<kMirror>(v);
+}
+__device__ inline double sum64(double v) {
+  v = sum16(v);
+  v = fold<16>(v, v);
+  return fold<32>(v, v);
 }
 
-// the workgroup's sum of v[k] over threads and slabs, as an aligned binary
-// tree over rows (slab k, thread t). Valid in wave 0. sh: [R * kRowWaves].
-// Ends with nothing pending on sh that the next call's first barrier does not
-// cover (one barrier between two calls is enough).
-template <int R>
-__device__ inline double tree_sum(const double (&v)[R], double* sh) {
+template <int V>
+struct Sums {
+  double v[V];
+};
+
+// The workgroup's V (1 or 4) sums of val(k) over threads and their rows k, as
+// aligned binary trees over leaves (thread t's k-th row is leaf t * R + k).
+// Sum i is valid in wave i. sh: [V * kRowWaves]. One barrier between two calls
+// is enough for sh. Four sums over the lanes of a wave: the first two steps
+// halve the sums a lane carries, 7 additions in all.
+template <int R, int V, typename F>
+__device__ inline double tree_sum(F&& val, double* sh) {
+#pragma clang fp contract(off)
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // lanes halve the slabs they carry while summing over lane pairs
-  double a[R];
+  static_assert(V == 1 || V == 4, "sums");
+  Sums<V> a[R];
 #pragma unroll
-  for (int k = 0; k < R; ++k) a[k] = v[k];
-  int slab = 0, mask = 1;
+  for (int k = 0; k < R; ++k) {
+    a[k] = val(k);
+    // pairs, pairs of pairs, ... as soon as they are complete
 #pragma unroll
-  for (int h = R / 2; h >= 1; h >>= 1) {
-    const bool up = lane & mask;
+    for (int h = 1; h < R && ((k + 1) & (2 * h - 1)) == 0; h *= 2) {
 #pragma unroll
-    for (int k = 0; k < h; ++k) {
-      const double keep = up ? a[k + h] : a[k];
-      const double give = up ? a[k] : a[k + h];
-      a[k] = keep + __shfl_xor(give, mask, 64);
+      for (int i = 0; i < V; ++i) a[k + 1 - 2 * h].v[i] = a[k + 1 - 2 * h].v[i] + a[k + 1 - h].v[i];
     }
-    slab += up ? h : 0;
-    mask <<= 1;
+    if constexpr (R >= 4)
+      if (k & 1) __builtin_amdgcn_sched_barrier(0);
   }
-  const double s = lane_tree(a[0], R);
-  if (lane < R) sh[slab * kRowWaves + w] = s;
+  double s;
+  int which = 0;
+  if constexpr (V == 4) {
+    const double p = fold<1>(a[0].v[0], a[0].v[2]), q = fold<1>(a[0].v[1], a[0].v[3]);
+    s = fold<2>(p, q);
+    which = (lane & 1 ? 2 : 0) + (lane & 2 ? 1 : 0);
+    s += xor4(s);
+  } else {
+    s = a[0].v[0];
+    s += dpp<kXor1>(s);
+    s += dpp<kXor2>(s);
+    s += dpp<kHalfMirror>(s);
+  }
+  s += dpp<kRor8>(s);
+  s = fold<16>(s, s);
+  s = fold<32>(s, s);
+  if (lane < V) sh[which * kRowWaves + w] = s;
   __syncthreads();
   double t = 0.0;
-  if (w == 0) {
-    const int wl = lane & 15, g = lane >> 4;
-    if constexpr (R == 8) {
-      double p = sh[(2 * g) * kRowWaves + wl], q = sh[(2 * g + 1) * kRowWaves + wl];
-      for (int m = 1; m < 16; m <<= 1) {
-        p += __shfl_xor(p, m, 64);
-        q += __shfl_xor(q, m, 64);
-      }
-      t = p + q;
-    } else {
-      t = g < R ? sh[g * kRowWaves + wl] : 0.0;
-      for (int m = 1; m < 16; m <<= 1) t += __shfl_xor(t, m, 64);
-    }
-    t += __shfl_xor(t, 16, 64);
-    t += __shfl_xor(t, 32, 64);
-  }
+  if (w < V) t = sum16(sh[w * kRowWaves + (lane & 15)]);
   return t;
 }
 
 // ---------------------------------------------------------------------------
 // row products
 // ---------------------------------------------------------------------------
-// sum of W entries of this lane's row of a slice whose entries start at v, id
-// (the same in the whole wave: scalar bases, one 32-bit offset per lane)
+// sum of W entries of this lane's row of a slice (v, id: the slice's
+// coefficients and id words, the same in the whole wave), W / 2 more loads
+// for the ids, all in flight at once
 template <typename T, int W>
-__device__ inline T row_dot(const T* __restrict__ v, const uint16_t* __restrict__ id,
+__device__ inline T row_dot(const T* __restrict__ v, const unsigned* __restrict__ id,
                             unsigned lane, const T* ys) {
   T c[W];
-  int i[W];
+  unsigned i[(W + 1) / 2];
 #pragma unroll
-  for (int j = 0; j < W; ++j) {
-    c[j] = v[j * 64 + lane];
-    i[j] = id[j * 64 + lane];
-  }
-  T s = c[0] * ys[i[0]];
+  for (int j = 0; j < (W + 1) / 2; ++j) i[j] = id[j * 64 + lane];
 #pragma unroll
-  for (int j = 1; j < W; ++j) s += c[j] * ys[i[j]];
+  for (int j = 0; j < W; ++j) c[j] = v[j * 64 + lane];
+  T s = (T)0;
+#pragma unroll
+  for (int j = 0; j < W; ++j) s += c[j] * ys[j & 1 ? i[j / 2] >> 16 : i[j / 2] & 0xffffu];
   return s;
 }
-
-// sum over the w entries (w the same in the whole wave), eight in flight
-template <typename T>
-__device__ inline T slice_dot(const T* __restrict__ v, const uint16_t* __restrict__ id,
-                              unsigned lane, int w, const T* ys) {
+// sum over the w entries of the slice's rows from entry `from` (even) on, C
+// (4 or 8) at a time
+template <int C, typename T>
+__device__ inline T slice_dot(const T* __restrict__ v, const unsigned* __restrict__ id,
+                              unsigned lane, int from, int w, const T* ys) {
+  v += from * 64;
+  id += from * 32;
+  w -= from;
   T s = (T)0;
-  while (w >= 8) {
-    s += row_dot<T, 8>(v, id, lane, ys);
-    v += 8 * 64;
-    id += 8 * 64;
-    w -= 8;
+  while (w >= C) {
+    s += row_dot<T, C>(v, id, lane, ys);
+    v += C * 64;
+    id += C * 32;
+    w -= C;
+  }
+  if constexpr (C > 4) {
+    switch (w) {
+      case 7: return s + row_dot<T, 7>(v, id, lane, ys);
+      case 6: return s + row_dot<T, 6>(v, id, lane, ys);
+      case 5: return s + row_dot<T, 5>(v, id, lane, ys);
+      case 4: return s + row_dot<T, 4>(v, id, lane, ys);
+      default: break;
+    }
   }
   switch (w) {
-    case 7: s += row_dot<T, 7>(v, id, lane, ys); break;
-    case 6: s += row_dot<T, 6>(v, id, lane, ys); break;
-    case 5: s += row_dot<T, 5>(v, id, lane, ys); break;
-    case 4: s += row_dot<T, 4>(v, id, lane, ys); break;
-    case 3: s += row_dot<T, 3>(v, id, lane, ys); break;
-    case 2: s += row_dot<T, 2>(v, id, lane, ys); break;
-    case 1: s += row_dot<T, 1>(v, id, lane, ys); break;
-    default: break;
+    case 3: return s + row_dot<T, 3>(v, id, lane, ys);
+    case 2: return s + row_dot<T, 2>(v, id, lane, ys);
+    case 1: return s + row_dot<T, 1>(v, id, lane, ys);
+    default: return s;
   }
+}
+
+// The first kFront entries of one row, kept in registers for a whole solve.
+// Slices with fewer read their last one again and multiply it by zero.
+constexpr int kFront = 8;
+template <typename T>
+struct RowFront {
+  T c[kFront];
+  unsigned i[kFront / 2];  // two ids each
+};
+template <typename T>
+__device__ inline void load_front(RowFront<T>& f, const T* __restrict__ v,
+                                  const unsigned* __restrict__ id, unsigned lane, int w) {
+  const int last = max(w - 1, 0);
+#pragma unroll
+  for (int j = 0; j < kFront / 2; ++j) f.i[j] = (id + min(j, last / 2) * 64)[lane];
+#pragma unroll
+  for (int j = 0; j < kFront; ++j) {
+    const T c = (v + min(j, last) * 64)[lane];
+    f.c[j] = j < w ? c : (T)0;
+  }
+}
+template <typename T>
+__device__ inline T front_dot(const RowFront<T>& f, const T* ys) {
+  T s = (T)0;
+#pragma unroll
+  for (int j = 0; j < kFront; ++j)
+    s += f.c[j] * ys[j & 1 ? f.i[j / 2] >> 16 : f.i[j / 2] & 0xffffu];
   return s;
 }
 
@@ -233,8 +328,8 @@ template <typename T, int R, bool DQ>
 __global__ void __launch_bounds__(kSlab)
 k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ double sh_sum[R * kRowWaves];
-  __shared__ double sh_in[4];
+  __shared__ double sh_sum[kSums * kRowWaves];
+  __shared__ double sh_in[kRowWaves];
   __shared__ int sh_bad, sh_wg;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   if (t == 0) {
@@ -261,24 +356,24 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
     return;
   }
   const Deadline dl = {(u64)wall_clock64(), ra.sy.ticks, ra.sy.abort};
-  const int k0 = ra.wg_slab0[wg], nk = ra.wg_slab0[wg + 1] - k0;
+  const int r0 = ra.wg_row0[wg];
+  const uint16_t* rowpos = ra.rowpos + (size_t)wg * R * kSlab;
   const int h0 = ra.halo_off[wg], nh = ra.halo_off[wg + 1] - h0;
   const int x0 = ra.exp_off[wg], nx = ra.exp_off[wg + 1] - x0;
   T* ds = reinterpret_cast<T*>(smem_raw);  // D: own rows, then halo
   T* dh = ds + R * kSlab;
-  T* hr = dh + nh;                         // halo residuals as they arrive
-  // also holds the exported residuals of the workgroup (by LDS index) while
-  // they are posted: the residuals themselves live in registers
-  T* rs = hr + nh;
+  T* ah = dh + nh;                         // A D of the halo as it arrives
+  T* rh = ah + nh;                         // R of the halo
+  T* as = rh + nh;                         // A D of own rows
 
   // ||r0||^2: the state's, or the partial sums per node block
   double rr;
   if (a.part_rr) {
     const int pb0 = a.sys_blocks ? a.sys_blocks[sys] : 0;
     const int pb1 = a.sys_blocks ? a.sys_blocks[sys + 1] : a.nblocks;
-    double p[1] = {0.0};
-    for (int i = pb0 + t; i < pb1; i += kSlab) p[0] += a.part_rr[i];
-    const double s = tree_sum<1>(p, sh_sum);
+    double p = 0.0;
+    for (int i = pb0 + t; i < pb1; i += kSlab) p += a.part_rr[i];
+    const double s = tree_sum<1, 1>([&](int) { return Sums<1>{{p}}; }, sh_sum);
     if (t == 0) sh_in[0] = s;
     __syncthreads();
     rr = sh_in[0];
@@ -291,80 +386,116 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
   const double thr = ld_f64(&st->eps2xl) * (load_relaxed(&st->use_rr0) ? ld_f64(&st->rr0) : 1.0);
   const int nitmax = load_relaxed(&st->nitmax);
 
-  int off[R];         // slices of this wave: first entries and widths (scalars)
-  int wid[R];
-  unsigned have = 0;  // bit k: this thread has a row in slab k
-  T rv[R], xv[R], ad[R], dq[DQ ? R : 1];
+  // the coefficients of small partitions stay in registers for the whole solve
+  constexpr bool kKeep = R * sizeof(T) <= 16;
+  RowFront<T> front[kKeep ? R : 1];
+  int wid[kKeep ? R : 1];
+  // the slice of this wave's k-th rows: its coefficients, id words and width
+  auto slice = [&](int k, const T*& v, const unsigned*& id) -> int {
+    const int q = __builtin_amdgcn_readfirstlane((wg * R + k) * kSlices + wave);
+    const int o = ra.slice_off[q];
+    v = val + (size_t)o * 64;
+    id = ra.ids + (size_t)ra.pair_off[q] * 64;
+    return ra.slice_off[q + 1] - o;
+  };
+  unsigned have = 0;  // bit k: this thread has a k-th row
+  T rv[R], xv[R], dq[DQ ? R : 1];
   const double beta0 = m == 0 ? 0.0 : rr / rr_prev;
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    off[k] = wid[k] = 0;
-    rv[k] = xv[k] = ad[k] = (T)0;
+    // (a few rows' addresses at a time)
+    if constexpr (R >= 4) __builtin_amdgcn_sched_barrier(0);
+    rv[k] = xv[k] = (T)0;
     if constexpr (DQ) dq[k] = (T)0;
     T d = (T)0;
-    if (k < nk) {
-      const int q = (k0 + k) * kSlices + wave;
-      off[k] = __builtin_amdgcn_readfirstlane(ra.slice_off[q]);
-      wid[k] = __builtin_amdgcn_readfirstlane(ra.slice_off[q + 1]) - off[k];
-      const int p = ra.rowpos[(size_t)(k0 + k) * kSlab + t];
-      if (p != 0xffff) {
-        const int row = ra.slab_row0[k0 + k] + p;
-        have |= 1u << k;
-        rv[k] = a.r0[row];
-        if (a.x0) xv[k] = a.x0[row];
-        if constexpr (DQ) dq[k] = a.diag[row];
-        d = rv[k];
-        if (m > 0) d += (T)beta0 * a.dlast[row];
-      }
+    const int p = rowpos[k * kSlab + t];
+    if (p != 0xffff) {
+      const int row = r0 + p;
+      have |= 1u << k;
+      rv[k] = a.r0[row];
+      if (a.x0) xv[k] = a.x0[row];
+      if constexpr (DQ) dq[k] = a.diag[row];
+      d = rv[k];
+      if (m > 0) d += (T)beta0 * a.dlast[row];
     }
     ds[k * kSlab + t] = d;
+    if constexpr (kKeep) {
+      const T* v;
+      const unsigned* id;
+      wid[k] = slice(k, v, id);
+      load_front(front[k], v, id, lane, wid[k]);
+    }
   }
   for (int h = t; h < nh; h += kSlab) {
     const int g = ra.halo_row[h0 + h];
     T d = a.r0[g];
+    rh[h] = d;
     if (m > 0) d += (T)beta0 * a.dlast[g];
     dh[h] = d;
   }
   __syncthreads();
 
-  // a meeting: the system's sum of v (and, in `halo`, the halo residuals of
-  // rv into hr); false when it gave up
-  auto meet = [&](const double (&v)[R], bool halo, double& sum) -> bool {
+  // the thread's first exported row and first halo value
+  const int my_exp = t < nx ? ra.exp_loc[x0 + t] : 0;
+  const int my_src = t < nh ? ra.halo_src[h0 + t] : 0;
+
+  // a meeting: the system's V sums of val(k) and, with `halo`, the exchange
+  // of A D (into ah); false when it gave up
+  auto meet = [&](auto val, auto sums, auto halo, double* sum) -> bool {
+    constexpr int V = sums.value;
     ++e;
-    if (gang > 1 && halo) {
-#pragma unroll
-      for (int k = 0; k < R; ++k) rs[k * kSlab + t] = rv[k];
-    }
-    const double s = tree_sum<R>(v, sh_sum);
+    const double s = tree_sum<R, V>(val, sh_sum);
     if (gang == 1) {
-      if (t == 0) sh_in[0] = s;
+      if (lane == 0 && wave < V) sh_in[wave] = s;
       __syncthreads();
-      sum = sh_in[0];
+#pragma unroll
+      for (int i = 0; i < V; ++i) sum[i] = sh_in[i];
       return true;
     }
-    u64* slots = ra.sy.slots + (size_t)(e & 1) * kReplicas * ra.nwg * 2;
-    if (t < kReplicas) post(slots + ((size_t)t * ra.nwg + wg) * 2, e, s);
-    if (halo) {
-      // (rs is complete: tree_sum's barrier)
-      for (int i = t; i < nx; i += kSlab)
-        post(ra.sy.xch + (size_t)(x0 + i) * kWords<T>, e, rs[ra.exp_loc[x0 + i]]);
+    // (opaque: the addresses below are made anew instead of kept over the loop)
+    int tt = t;
+    asm volatile("" : "+v"(tt));
+    u64* slots = ra.sy.slots + (size_t)(e & 1) * kReplicas * kSums * ra.nwg * 2;
+    u64* xch = ra.sy.xch + (size_t)(e & 1) * 2 * ra.nexp;
+    if (wave < V && lane < kReplicas)
+      post(slots + ((size_t)(lane * kSums + wave) * ra.nwg + wg) * 2, 1, e, s);
+    if constexpr (halo.value) {
+      // (A D is complete: tree_sum's barrier)
+      if (tt < nx) post(xch + x0 + tt, ra.nexp, e, as[my_exp]);
+      for (int i = tt + kSlab; i < nx; i += kSlab)
+        post(xch + x0 + i, ra.nexp, e, as[ra.exp_loc[x0 + i]]);
     }
-    bool ok = true;
-    if (wave < 4) {
-      double p = 0.0;
-      if (t < gang)
-        ok = await(slots + ((size_t)(wg & (kReplicas - 1)) * ra.nwg + g0 + t) * 2, e, p, dl);
-      p = lane_tree(p, 1);
-      if (lane == 0) sh_in[wave] = p;
+    // 256 threads per sum, one workgroup each; every thread looks for its sum
+    // and its first halo value together
+    const int sw = tt & 255, sv = tt >> 8;
+    const u64* sp =
+        slots + ((size_t)((wg & (kReplicas - 1)) * kSums + sv) * ra.nwg + g0 + sw) * 2;
+    bool need_s = sv < V && sw < gang, need_h = halo.value && tt < nh;
+    const u64* hp = xch + my_src;
+    double p = 0.0;
+    T hv = (T)0;
+    int n = 0;
+    while (need_s || need_h) {
+      if (need_s) need_s = !look(sp, 1, e, p);
+      if constexpr (halo.value)
+        if (need_h) need_h = !look(hp, ra.nexp, e, hv);
+      if ((need_s || need_h) && dl.past(n)) break;
     }
-    if (halo) {
-      // waves 4 and up first, so that the sums and most halos are read at once
-      for (int h = (t + kSlab - 256) & (kSlab - 1); h < nh && ok; h += kSlab) {
+    bool ok = !(need_s || need_h);
+    if constexpr (halo.value) {
+      if (tt < nh) ah[tt] = hv;
+      for (int h = tt + kSlab; h < nh && ok; h += kSlab) {
         T v2;
-        ok = await(ra.sy.xch + (size_t)ra.halo_src[h0 + h] * kWords<T>, e, v2, dl);
-        if (ok) hr[h] = v2;
+        while (!look(xch + ra.halo_src[h0 + h], ra.nexp, e, v2))
+          if (dl.past(n)) {
+            ok = false;
+            break;
+          }
+        ah[h] = v2;
       }
     }
+    p = sum64(sv < V && sw < gang ? p : 0.0);
+    if (lane == 0) sh_in[wave] = p;
     if (!ok) sh_bad = 1;
     __syncthreads();
     if (sh_bad) {
@@ -374,35 +505,61 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
       }
       return false;
     }
-    sum = (sh_in[0] + sh_in[1]) + (sh_in[2] + sh_in[3]);
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      sum[i] = (sh_in[4 * i] + sh_in[4 * i + 1]) + (sh_in[4 * i + 2] + sh_in[4 * i + 3]);
     return true;
   };
 
-  int status;
-  for (;;) {
-    // stop test (gracjg.F:306-324; strict for the initial residual, :219)
-    if (m == 0 ? rr < thr : rr <= thr) {
-      status = ST_CONVERGED;
-      break;
-    }
-    // AD, D.AD
-    double part[R];
+  // stop test (gracjg.F:306-324; strict for the initial residual, :219)
+  bool stop = m == 0 ? rr < thr : rr <= thr;
+  int status = ST_CONVERGED;
+  while (!stop) {
+    // AD
+    if constexpr (kKeep) {
 #pragma unroll
-    for (int k = 0; k < R; ++k) {
-      // (opaque, or the base addresses of all slabs are kept over the loop)
-      int o = off[k];
-      asm volatile("" : "+s"(o));
-      const T s = slice_dot<T>(val + (size_t)o * 64, ra.ids + (size_t)o * 64, lane, wid[k], ds);
-      const T d = ds[k * kSlab + t];
-      ad[k] = s + (DQ ? dq[k] * d : d);
+      for (int k = 0; k < R; ++k) {
+        T s = front_dot(front[k], ds);
+        if (wid[k] > kFront) {
+          const T* v;
+          const unsigned* id;
+          slice(k, v, id);
+          s += slice_dot<4>(v, id, lane, kFront, wid[k], ds);
+        }
+        as[k * kSlab + t] = s;
+        // (one slab's gathers at a time, as above)
+        if constexpr (R >= 2) __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma nounroll
+      for (int k = 0; k < R; ++k) {
+        const T* v;
+        const unsigned* id;
+        const int w = slice(k, v, id);
+        as[k * kSlab + t] = slice_dot<8>(v, id, lane, 0, w, ds);
+      }
     }
+    if constexpr (DQ) {
 #pragma unroll
-    for (int k = 0; k < R; ++k)
-      part[k] = (have >> k & 1) ? (double)ds[k * kSlab + t] * (double)ad[k] : 0.0;
-    double dad;
-    if (!meet(part, false, dad)) return;
+      for (int k = 0; k < R; ++k)
+        as[k * kSlab + t] += dq[k] * ds[k * kSlab + t];
+    } else {
+#pragma unroll
+      for (int k = 0; k < R; ++k)
+        as[k * kSlab + t] += ds[k * kSlab + t];
+    }
+    // D.AD, AD.AD, R.AD, R.R
+    auto dots = [&](int k) -> Sums<kSums> {
+      if (!(have >> k & 1)) return {};
+      const double d = (double)ds[k * kSlab + t], s = (double)as[k * kSlab + t];
+      const double r = (double)rv[k];
+      return {{d * s, s * s, r * s, r * r}};
+    };
+    double sum[kSums];
+    if (!meet(dots, std::integral_constant<int, kSums>(), std::true_type(), sum)) return;
+    rr = sum[3];
     // RO, X -= RO D (gracjg.F:380-388); after iteration NITMAX no more
-    const double rho = rr / dad;
+    const double rho = rr / sum[0];
     const T rhot = (T)rho;
 #pragma unroll
     for (int k = 0; k < R; ++k) xv[k] -= rhot * ds[k * kSlab + t];
@@ -411,27 +568,41 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
       break;
     }
 #pragma unroll
-    for (int k = 0; k < R; ++k) {
-      rv[k] -= rhot * ad[k];
-      part[k] = (have >> k & 1) ? (double)rv[k] * (double)rv[k] : 0.0;
-    }
+    for (int k = 0; k < R; ++k)
+      if (have >> k & 1) rv[k] -= rhot * as[k * kSlab + t];
+    // ||R||^2 after this update, from the sums before it (no second meeting).
+    // It loses digits where it falls far in one step, and the stop test wants
+    // the sum itself: both are summed anew
     rr_prev = rr;
-    if (!meet(part, true, rr)) return;
+    rr = rr - 2.0 * rho * sum[2] + rho * rho * sum[1];
+    if (!(rr > kTrust * rr_prev && rr > 1.001 * thr)) {
+      auto own = [&](int k) -> Sums<1> {
+        return {{(have >> k & 1) ? (double)rv[k] * (double)rv[k] : 0.0}};
+      };
+      if (!meet(own, std::integral_constant<int, 1>(), std::false_type(), &rr)) return;
+    }
     ++m;
+    stop = rr <= thr;
+    if (stop) break;
     // D = R + BETA D, halo included
     const T beta = (T)(rr / rr_prev);
-    if (!(rr <= thr)) {
 #pragma unroll
-      for (int k = 0; k < R; ++k) ds[k * kSlab + t] = rv[k] + beta * ds[k * kSlab + t];
-      for (int h = (t + kSlab - 256) & (kSlab - 1); h < nh; h += kSlab)
-        dh[h] = hr[h] + beta * dh[h];
+    for (int k = 0; k < R; ++k) ds[k * kSlab + t] = rv[k] + beta * ds[k * kSlab + t];
+    if (gang > 1) {
+      int h = t;
+      asm volatile("" : "+v"(h));
+      for (; h < nh; h += kSlab) {
+        const T r = rh[h] - rhot * ah[h];
+        rh[h] = r;
+        dh[h] = r + beta * dh[h];
+      }
     }
     __syncthreads();
   }
 #pragma unroll
   for (int k = 0; k < R; ++k)
     if (have >> k & 1) {
-      const int row = ra.slab_row0[k0 + k] + ra.rowpos[(size_t)(k0 + k) * kSlab + t];
+      const int row = r0 + rowpos[k * kSlab + t];
       a.x[row] = xv[k];
       if (a.dlast) a.dlast[row] = ds[k * kSlab + t];
     }
@@ -506,10 +677,10 @@ struct Buf {
 };
 
 struct RowsDev {
-  int nslab = 0, group = 1, nwg = 0, nsys = 1, max_halo = 0;
+  int nslice = 0, group = 1, nwg = 0, nsys = 1, max_halo = 0;
   int64_t nent = 0;
-  int ncu = 0;
-  Buf<int32_t> slab_row0, slice_off, refs, wg_slab0, wg_sys, sys_wg, halo_off, halo_row, halo_src,
+  int ncu = 0, nexp = 0;
+  Buf<int32_t> wg_row0, slice_off, pair_off, refs, wg_sys, sys_wg, halo_off, halo_row, halo_src,
       exp_off;
   Buf<uint16_t> rowpos, ids, exp_loc;
   Buf<uint8_t> cnt;
@@ -522,8 +693,8 @@ struct RowsDev {
 };
 
 static size_t cg_lds(const RowsDev& r, int bytes) {
-  // D of own rows and halo, halo residuals, own residuals for the exchange
-  return ((size_t)2 * r.group * kSlab + (size_t)2 * r.max_halo) * bytes;
+  // D and A D of own rows; D, A D and R of the halo
+  return ((size_t)2 * r.group * kSlab + (size_t)3 * r.max_halo) * bytes;
 }
 
 template <typename T, typename F>
@@ -570,15 +741,18 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
     return nullptr;
   RowLayout R;
   if (!build_rows(L, nsys, node_off, ncu, R)) return nullptr;
+  // the kernels may read one entry column past the last slice (load_front)
+  R.ids.resize(R.ids.size() + 128, 0);
   std::unique_ptr<RowsDev> r(new RowsDev());
-  r->nslab = R.nslab;
+  r->nslice = R.nslice;
   r->group = R.group;
   r->nwg = R.nwg;
   r->nsys = nsys;
   r->max_halo = R.max_halo;
-  r->nent = R.nent;
+  r->nent = R.nent + 64;
   r->ncu = ncu;
-  lds_max -= 4096;  // the kernels' static LDS: their sums
+  r->nexp = (int)R.exp_loc.size();
+  lds_max -= 2048;  // the kernels' static LDS: their sums
   if (cg_lds(*r, sizeof(double)) > (size_t)lds_max) return nullptr;
   bool fits = true;
   if ((*err = cg_fits<double>(*r, lds_max, &fits)) != hipSuccess) return nullptr;
@@ -588,19 +762,20 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
     if (e != hipSuccess) *err = e;
     return e == hipSuccess;
   };
-  if (!ok(r->slab_row0.put(R.slab_row0, stream)) || !ok(r->slice_off.put(R.slice_off, stream)) ||
-      !ok(r->refs.put(R.refs, stream)) || !ok(r->wg_slab0.put(R.wg_slab0, stream)) ||
+  if (!ok(r->wg_row0.put(R.wg_row0, stream)) || !ok(r->slice_off.put(R.slice_off, stream)) ||
+      !ok(r->pair_off.put(R.pair_off, stream)) ||
+      !ok(r->refs.put(R.refs, stream)) ||
       !ok(r->wg_sys.put(R.wg_sys, stream)) || !ok(r->sys_wg.put(R.sys_wg, stream)) ||
       !ok(r->halo_off.put(R.halo_off, stream)) || !ok(r->halo_row.put(R.halo_row, stream)) ||
       !ok(r->halo_src.put(R.halo_src, stream)) || !ok(r->exp_off.put(R.exp_off, stream)) ||
       !ok(r->rowpos.put(R.rowpos, stream)) || !ok(r->ids.put(R.ids, stream)) ||
       !ok(r->exp_loc.put(R.exp_loc, stream)) || !ok(r->cnt.put(R.cnt, stream)) ||
-      !ok(r->ref_off.put(R.ref_off, stream)) || !ok(r->v64.alloc(R.nent)))
+      !ok(r->ref_off.put(R.ref_off, stream)) || !ok(r->v64.alloc(r->nent)))
     return nullptr;
   // sync words: per precision sums and exchange, then the counters
-  const size_t nslot = (size_t)2 * kReplicas * R.nwg * 2, nexp = R.exp_loc.size();
+  const size_t nslot = (size_t)2 * kReplicas * kSums * R.nwg * 2, nexp = R.exp_loc.size();
   const size_t nepoch = (2 * (size_t)nsys + 1) / 2 + 1;  // in 64-bit words
-  const size_t one = nslot + 2 * nexp + nepoch + 2;
+  const size_t one = nslot + 4 * nexp + nepoch + 2;
   if (!ok(r->words.alloc(2 * one))) return nullptr;
   u64 ticks = kWaitTicks;
   if (const char* ev = getenv("BHIP_ROWS_WAIT")) ticks = strtoull(ev, nullptr, 10);
@@ -608,7 +783,7 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
     u64* p = r->words.p + k * one;
     r->sy[k].slots = p;
     r->sy[k].xch = p + nslot;
-    r->sy[k].epoch = reinterpret_cast<unsigned*>(p + nslot + 2 * nexp);
+    r->sy[k].epoch = reinterpret_cast<unsigned*>(p + nslot + 4 * nexp);
     r->sy[k].abort = reinterpret_cast<int*>(p + one - 2);
     r->sy[k].ticket = reinterpret_cast<unsigned*>(p + one - 1);
     r->sy[k].ticks = ticks;
@@ -627,7 +802,7 @@ hipError_t rows_reserve(RowsDev* r, int bytes) {
 
 hipError_t rows_assemble(RowsDev* r, int bytes, const double* xa, int nslot_pad, int npair,
                          bool nonsym, hipStream_t stream) {
-  const int nslice = r->nslab * kSlices;
+  const int nslice = r->nslice;
   const unsigned lower = nonsym ? (unsigned)npair * (unsigned)nslot_pad : 0u;
   const dim3 grid((nslice + 3) / 4), block(256);
   if (bytes == 8)
@@ -642,10 +817,10 @@ hipError_t rows_assemble(RowsDev* r, int bytes, const double* xa, int nslot_pad,
 static RowArgs row_args(const RowsDev* r, int k) {
   RowArgs a;
   a.slice_off = r->slice_off.p;
-  a.ids = r->ids.p;
+  a.pair_off = r->pair_off.p;
+  a.ids = reinterpret_cast<const unsigned*>(r->ids.p);
   a.rowpos = r->rowpos.p;
-  a.slab_row0 = r->slab_row0.p;
-  a.wg_slab0 = r->wg_slab0.p;
+  a.wg_row0 = r->wg_row0.p;
   a.wg_sys = r->wg_sys.p;
   a.sys_wg = r->sys_wg.p;
   a.halo_off = r->halo_off.p;
@@ -655,7 +830,7 @@ static RowArgs row_args(const RowsDev* r, int k) {
   a.exp_loc = r->exp_loc.p;
   a.nwg = r->nwg;
   a.nsys = r->nsys;
-  a.nslab = r->nslab;
+  a.nexp = r->nexp;
   a.sy = r->sy[k];
   a.ep = r->ep[k];
   a.ticketed = r->nwg > r->ncu;

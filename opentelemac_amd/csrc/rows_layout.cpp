@@ -3,7 +3,6 @@
 
 #include <algorithm>
 #include <atomic>
-#include <functional>
 #include <thread>
 
 namespace bhip {
@@ -33,18 +32,19 @@ struct Contribution {
 struct Entry {
   int32_t col, first, count;
 };
-struct SlabScratch {
-  std::vector<int32_t> off, fill;
+struct Scratch {
+  std::vector<int32_t> off, fill, order, row_at;
   std::vector<Contribution> con;
   std::vector<std::vector<Entry>> rows;
-  std::vector<int> order;
+  std::vector<int32_t> mark;  // per row: the last workgroup that saw it
 };
-// one slab's slices before they are joined
-struct SlabOut {
+// one workgroup's slices before they are joined
+struct WgOut {
   std::vector<int32_t> width;  // per slice
-  std::vector<int32_t> cols;   // per entry (internal node id)
+  std::vector<int32_t> cols;   // per entry (internal node id, -1: none)
   std::vector<uint8_t> cnt;
   std::vector<int32_t> refs, ref_units;  // per slice: 64-wide reference columns
+  std::vector<int32_t> halo;
 };
 
 }  // namespace
@@ -56,49 +56,48 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
   if (cap < 1) return false;
   // references hold pair * nslot_pad + slot in 31 bits
   if ((int64_t)ndp * (ndp - 1) / 2 * L.nslot_pad >= INT32_MAX) return false;
-  // slabs
-  std::vector<int32_t> sys_slab(nsys + 1, 0);
+  std::vector<int64_t> slabs(nsys);
   for (int s = 0; s < nsys; ++s) {
-    const int64_t n = node_off[s + 1] - node_off[s];
-    const int64_t ns = (n + kSlab - 1) / kSlab;
-    if (ns > (int64_t)cap * kMaxGroup) return false;
-    for (int64_t k = 0; k < ns; ++k) {
-      R.slab_row0.push_back((int32_t)(node_off[s] + k * kSlab));
-      R.slab_rows.push_back((int32_t)std::min<int64_t>(kSlab, n - k * kSlab));
-    }
-    sys_slab[s + 1] = (int32_t)R.slab_row0.size();
+    slabs[s] = (node_off[s + 1] - node_off[s] + kSlab - 1) / kSlab;
+    if (slabs[s] > (int64_t)cap * kMaxGroup) return false;
   }
-  R.nslab = (int)R.slab_row0.size();
   // slabs per workgroup: the fewest that let every system be resident at
-  // once, or (many systems) as many as a workgroup can hold
+  // once, or (many systems) as many as a workgroup can hold. Two instead of one
+  // already past half of the workgroups: a meeting of 256 workgroups takes 1 us
+  // longer than one of 128, a second slab kept in registers less
   auto wgs = [&](int g) {
     int64_t t = 0;
-    for (int s = 0; s < nsys; ++s) t += (sys_slab[s + 1] - sys_slab[s] + g - 1) / g;
+    for (int s = 0; s < nsys; ++s) t += (slabs[s] + g - 1) / g;
     return t;
   };
-  R.group = 1;
+  R.group = wgs(1) <= cap / 2 ? 1 : 2;
   while (R.group < kMaxGroup && wgs(R.group) > cap) R.group *= 2;
+  const int G = R.group, wrows = G * kSlab;
   R.sys_wg.assign(1, 0);
+  std::vector<int32_t> nrows;  // of each workgroup
   for (int s = 0; s < nsys; ++s) {
-    for (int k = sys_slab[s]; k < sys_slab[s + 1]; k += R.group) {
-      R.wg_slab0.push_back(k);
+    for (int64_t k = 0; k < slabs[s]; k += G) {
+      const int64_t r0 = node_off[s] + k * kSlab;
+      R.wg_row0.push_back((int32_t)r0);
+      nrows.push_back((int32_t)std::min<int64_t>(wrows, node_off[s + 1] - r0));
       R.wg_sys.push_back(s);
     }
     R.sys_wg.push_back((int32_t)R.wg_sys.size());
     R.max_gang = std::max(R.max_gang, R.sys_wg[s + 1] - R.sys_wg[s]);
   }
   R.nwg = (int)R.wg_sys.size();
-  R.wg_slab0.push_back(R.nslab);
+  const int wslices = G * kSlices;  // slices of a workgroup
+  R.nslice = R.nwg * wslices;
 
-  // ---- rows of each slab ---------------------------------------------------
-  std::vector<SlabOut> out(R.nslab);
-  R.rowpos.assign((size_t)R.nslab * kSlab, 0xffff);
-  std::vector<uint16_t> pos_of((size_t)L.npoin);  // position of a row in its slab
+  // ---- rows of each workgroup ------------------------------------------------
+  std::vector<WgOut> out(R.nwg);
+  R.rowpos.assign((size_t)R.nwg * wrows, 0xffff);
+  std::vector<uint16_t> lid_of((size_t)L.npoin);  // LDS index of a row in its workgroup
   int pair_idx[6][6];
   for (int i = 0, q = 0; i < ndp; ++i)
     for (int j = i + 1; j < ndp; ++j, ++q) pair_idx[i][j] = pair_idx[j][i] = q;
-  parallel_for(R.nslab, [] { return SlabScratch(); }, [&](int k, SlabScratch& w) {
-    const int r0 = R.slab_row0[k], nr = R.slab_rows[k], r1 = r0 + nr;
+  parallel_for(R.nwg, [] { return Scratch(); }, [&](int wg, Scratch& w) {
+    const int r0 = R.wg_row0[wg], nr = nrows[wg], r1 = r0 + nr;
     const int b0 = (int)(std::upper_bound(L.node_start.begin(), L.node_start.end(), r0) -
                          L.node_start.begin()) - 1;
     // every (row, column, coefficient) of the blocks that own these rows, in
@@ -133,8 +132,7 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
         w.con[w.fill[g[a] - r0]++] = {g[j], (int32_t)(ref | (a > j ? 0x80000000u : 0u))};
       }
     });
-    w.rows.resize(kSlab);
-    w.order.resize(nr);
+    w.rows.resize(wrows);
     for (int i = 0; i < nr; ++i) {
       auto first = w.con.begin() + w.off[i], last = w.con.begin() + w.off[i + 1];
       std::stable_sort(first, last,
@@ -150,126 +148,128 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
       // agree on the count of each entry column
       std::stable_sort(e.begin(), e.end(),
                        [](const Entry& p, const Entry& q) { return p.count > q.count; });
-      w.order[i] = i;
     }
-    std::stable_sort(w.order.begin(), w.order.end(),
-                     [&](int p, int q) { return w.rows[p].size() > w.rows[q].size(); });
-    SlabOut& o = out[k];
-    o.width.assign(kSlices, 0);
-    o.ref_units.assign(kSlices, 0);
-    for (int p = 0; p < nr; ++p) {
-      R.rowpos[(size_t)k * kSlab + p] = (uint16_t)w.order[p];
-      pos_of[r0 + w.order[p]] = (uint16_t)p;
+    // leaves, half a slab at a time; row_at[LDS index]
+    w.row_at.assign(wrows, -1);
+    static const int kRun[8] = {0, 4, 1, 5, 2, 6, 3, 7};
+    constexpr int kHalf = kSlab / 2;
+    static_assert(kHalf == 8 * 64, "eight runs of 64 ranks");
+    for (int h = 0; h < nr; h += kHalf) {
+      const int n = std::min(kHalf, nr - h);
+      w.order.resize(n);
+      for (int i = 0; i < n; ++i) w.order[i] = h + i;
+      std::stable_sort(w.order.begin(), w.order.end(),
+                       [&](int p, int q) { return w.rows[p].size() > w.rows[q].size(); });
+      for (int i = 0; i < n; ++i) {
+        const int leaf = h + 8 * (i % 64) + kRun[i / 64];
+        const int id = leaf % G * kSlab + leaf / G;
+        w.row_at[id] = w.order[i];
+        lid_of[r0 + w.order[i]] = (uint16_t)id;
+      }
     }
-    for (int q = 0; q < kSlices; ++q) {
-      const int p0 = q * 64, p1 = std::min(nr, p0 + 64);
+    for (int id = 0; id < wrows; ++id)
+      if (w.row_at[id] >= 0) R.rowpos[(size_t)wg * wrows + id] = (uint16_t)w.row_at[id];
+    WgOut& o = out[wg];
+    o.width.assign(wslices, 0);
+    o.ref_units.assign(wslices, 0);
+    for (int q = 0; q < wslices; ++q) {
+      const int32_t* at = &w.row_at[(size_t)q * 64];  // (k * kSlab + wave * 64)
       int width = 0;
-      for (int p = p0; p < p1; ++p) width = std::max(width, (int)w.rows[w.order[p]].size());
+      for (int l = 0; l < 64; ++l)
+        if (at[l] >= 0) width = std::max(width, (int)w.rows[at[l]].size());
       o.width[q] = width;
       for (int j = 0; j < width; ++j) {
         int c = 0;
-        for (int p = p0; p < p1; ++p) {
-          const auto& e = w.rows[w.order[p]];
-          if (j < (int)e.size()) c = std::max(c, e[j].count);
-        }
+        for (int l = 0; l < 64; ++l)
+          if (at[l] >= 0 && j < (int)w.rows[at[l]].size())
+            c = std::max(c, w.rows[at[l]][j].count);
         o.cnt.push_back((uint8_t)std::min(c, 255));
         o.ref_units[q] += c;
         const size_t base = o.refs.size(), cb = o.cols.size();
         o.refs.resize(base + (size_t)c * 64, -1);
         o.cols.resize(cb + 64, -1);
-        for (int p = p0; p < p1; ++p) {
-          const auto& e = w.rows[w.order[p]];
+        for (int l = 0; l < 64; ++l) {
+          if (at[l] < 0) continue;
+          const auto& e = w.rows[at[l]];
           // padding names the row itself (its coefficient stays 0)
-          o.cols[cb + p - p0] = j < (int)e.size() ? e[j].col : r0 + w.order[p];
+          o.cols[cb + l] = j < (int)e.size() ? e[j].col : r0 + at[l];
           for (int t = 0; j < (int)e.size() && t < e[j].count; ++t)
-            o.refs[base + (size_t)t * 64 + p - p0] = w.con[e[j].first + t].ref;
+            o.refs[base + (size_t)t * 64 + l] = w.con[e[j].first + t].ref;
         }
       }
     }
+    // halo: the other workgroups' rows these entries name, by row
+    if (w.mark.empty()) w.mark.assign(L.npoin, -1);
+    for (int c : o.cols)
+      if (c >= 0 && (c < r0 || c >= r1) && w.mark[c] != wg) {
+        w.mark[c] = wg;
+        o.halo.push_back(c);
+      }
+    std::sort(o.halo.begin(), o.halo.end());
   });
   // ---- joined --------------------------------------------------------------
-  R.slice_off.assign((size_t)R.nslab * kSlices + 1, 0);
-  R.ref_off.assign((size_t)R.nslab * kSlices, 0);
+  R.slice_off.assign(R.nslice + 1, 0);
+  R.pair_off.assign(R.nslice + 1, 0);
+  R.ref_off.assign(R.nslice, 0);
   int64_t units = 0, runits = 0;
-  for (int k = 0; k < R.nslab; ++k)
-    for (int q = 0; q < kSlices; ++q) {
-      const size_t i = (size_t)k * kSlices + q;
+  for (int g = 0; g < R.nwg; ++g)
+    for (int q = 0; q < wslices; ++q) {
+      const size_t i = (size_t)g * wslices + q;
       R.ref_off[i] = runits;
-      units += out[k].width[q];
-      runits += out[k].ref_units[q];
+      units += out[g].width[q];
+      runits += out[g].ref_units[q];
       R.slice_off[i + 1] = (int32_t)units;
-      for (int j = 0; j < out[k].width[q]; ++j)
-        if (units > INT32_MAX / 64) {
-          R = RowLayout();
-          return false;
-        }
+      R.pair_off[i + 1] = R.pair_off[i] + (out[g].width[q] + 1) / 2;
     }
-  R.nent = units * 64;
-  R.nref = runits * 64;
-  for (const auto& o : out)
-    for (uint8_t c : o.cnt)
-      if (c == 255) {  // a pair shared by 255 elements: not a mesh this storage is for
-        R = RowLayout();
-        return false;
-      }
-  R.ids.resize(R.nent);
-  R.refs.resize(R.nref);
-  R.cnt.resize(units);
-  // ---- workgroups: halo, then local ids ---------------------------------------
-  struct Marks {
-    std::vector<int32_t> wg, idx;
-  };
-  std::vector<std::vector<int32_t>> halo(R.nwg);
-  std::atomic<bool> fits{true};
-  parallel_for(R.nwg, [&] { return Marks{std::vector<int32_t>(L.npoin, -1),
-                                         std::vector<int32_t>(L.npoin, 0)}; },
-               [&](int g, Marks& m) {
-    const int k0 = R.wg_slab0[g], k1 = R.wg_slab0[g + 1];
-    const int r0 = R.slab_row0[k0], r1 = R.slab_row0[k1 - 1] + R.slab_rows[k1 - 1];
-    auto& h = halo[g];
-    for (int k = k0; k < k1; ++k)
-      for (int c : out[k].cols)
-        if (c >= 0 && (c < r0 || c >= r1) && m.wg[c] != g) {
-          m.wg[c] = g;
-          h.push_back(c);
-        }
-    std::sort(h.begin(), h.end());
-    for (size_t i = 0; i < h.size(); ++i) m.idx[h[i]] = (int32_t)i;
-    if (R.group * kSlab + h.size() > 65535) fits = false;
-    for (int k = k0; k < k1; ++k) {
-      const int64_t e0 = (int64_t)R.slice_off[(size_t)k * kSlices] * 64;
-      const auto& cols = out[k].cols;
-      for (size_t i = 0; i < cols.size(); ++i) {
-        const int c = cols[i];
-        int id = 0;  // a lane without a row: any index, its coefficient is 0
-        if (c >= r0 && c < r1)
-          id = (c - r0) / kSlab * kSlab + pos_of[c];
-        else if (c >= 0)
-          id = R.group * kSlab + m.idx[c];
-        R.ids[e0 + i] = (uint16_t)id;
-      }
-      std::copy(out[k].refs.begin(), out[k].refs.end(),
-                R.refs.begin() + R.ref_off[(size_t)k * kSlices] * 64);
-      std::copy(out[k].cnt.begin(), out[k].cnt.end(), R.cnt.begin() + e0 / 64);
-    }
-  });
+  bool fits = units <= INT32_MAX / 128;
+  for (const auto& o : out) {
+    fits = fits && wrows + o.halo.size() <= 65535;
+    for (uint8_t c : o.cnt) fits = fits && c < 255;  // (a pair shared by 255 elements)
+  }
   if (!fits) {
     R = RowLayout();
     return false;
   }
+  R.nent = units * 64;
+  R.nref = runits * 64;
+  R.ids.assign((size_t)R.pair_off.back() * 128, 0);
+  R.refs.resize(R.nref);
+  R.cnt.resize(units);
+  parallel_for(R.nwg, [] { return 0; }, [&](int g, int&) {
+    const int r0 = R.wg_row0[g], r1 = r0 + nrows[g];
+    const WgOut& o = out[g];
+    const size_t q0 = (size_t)g * wslices;
+    size_t i = 0;
+    for (int q = 0; q < wslices; ++q) {
+      uint16_t* id = R.ids.data() + (size_t)R.pair_off[q0 + q] * 128;
+      for (int j = 0; j < o.width[q]; ++j)
+        for (int l = 0; l < 64; ++l, ++i) {
+          const int c = o.cols[i];
+          int v = 0;  // a lane without a row: any index, its coefficient is 0
+          if (c >= r0 && c < r1)
+            v = lid_of[c];
+          else if (c >= 0)
+            v = wrows + (int)(std::lower_bound(o.halo.begin(), o.halo.end(), c) - o.halo.begin());
+          id[((size_t)(j / 2) * 64 + l) * 2 + (j & 1)] = (uint16_t)v;
+        }
+    }
+    std::copy(o.refs.begin(), o.refs.end(), R.refs.begin() + R.ref_off[q0] * 64);
+    std::copy(o.cnt.begin(), o.cnt.end(), R.cnt.begin() + R.slice_off[q0]);
+  });
+  std::vector<std::vector<int32_t>> halo(R.nwg);
+  for (int g = 0; g < R.nwg; ++g) halo[g] = std::move(out[g].halo);
   // ---- exported rows ---------------------------------------------------------
   std::vector<int32_t> rank(L.npoin, -1);
   for (const auto& h : halo)
     for (int c : h) rank[c] = 0;
   R.exp_off.assign(1, 0);
   for (int g = 0; g < R.nwg; ++g) {
-    for (int k = R.wg_slab0[g]; k < R.wg_slab0[g + 1]; ++k)
-      for (int p = 0; p < R.slab_rows[k]; ++p) {
-        const int row = R.slab_row0[k] + R.rowpos[(size_t)k * kSlab + p];
-        if (rank[row] < 0) continue;
-        rank[row] = (int32_t)R.exp_loc.size();
-        R.exp_loc.push_back((uint16_t)((k - R.wg_slab0[g]) * kSlab + p));
-      }
+    for (int id = 0; id < wrows; ++id) {
+      const int at = R.rowpos[(size_t)g * wrows + id];
+      if (at == 0xffff || rank[R.wg_row0[g] + at] < 0) continue;
+      rank[R.wg_row0[g] + at] = (int32_t)R.exp_loc.size();
+      R.exp_loc.push_back((uint16_t)id);
+    }
     R.exp_off.push_back((int32_t)R.exp_loc.size());
   }
   R.halo_off.assign(1, 0);

@@ -80,6 +80,29 @@ def test_more_workgroups_than_the_gpu_holds(gpu):
                 assert abs(si["niter"] - ir.niter) <= 1
 
 
+@pytest.mark.parametrize("filler", [270000, 600000, 1100000])
+def test_a_member_gives_the_same_bits_in_any_partition(gpu, filler):
+    """Sums are trees over rows: a system solved alone (one slab per
+    workgroup) and beside a mesh that makes the context use 2, 4 or 8."""
+    meshes = [M.channel_mesh_n(n, seed=k, length=20.0 * n ** 0.5, width=15.0 * n ** 0.5)
+              for k, n in enumerate((2500, 21000, filler))]
+    systems = [S.wave_system(m, 2.0 + m.x / m.x.max(), dt=1.0) for m in meshes]
+    cat = lambda key: np.concatenate([s[key] for s in systems], axis=-1)  # noqa: E731
+    ens = bief.Ensemble(meshes)
+    for prec in (bief.PREC_FP64, bief.PREC_MIXED):
+        kw = dict(slv=1, precon=2, eps=1e-9, nitmax=500, precision=prec)
+        ens.set_matrix("Q", "S", cat("da"), cat("xa"))
+        x, _ = ens.solve(cat("x0"), cat("b"), **kw)
+        for m, sd, xs, si in zip(meshes[:2], systems, ens.split(x), ens.infos()):
+            ctx = bief.Context(m)
+            ctx.set_matrix("Q", "S", sd["da"], sd["xa"])
+            xa, ia = ctx.solve(sd["x0"].copy(), sd["b"].copy(), **kw)
+            assert si["niter"] == ia["niter"] and si["relres"] == ia["relres"]
+            assert np.array_equal(xs, xa)
+            ctx.close()
+    ens.close()
+
+
 def test_a_launch_that_gives_up_falls_back(gpu, monkeypatch):
     """A limit of zero on the workgroups' waits: the persistent launch gives up
     at its first meeting and the two-kernel CG solves the system."""
