@@ -1382,7 +1382,10 @@ int bhip_batch_latency(const bhip_ctx* c, int nsys, double* ms) {
 
 int bhip_ctx_destroy(bhip_ctx* c) {
   if (!c) return BHIP_OK;
-  if (c->stream) (void)hipStreamSynchronize(c->stream);
+  if (c->stream) {
+    (void)hipStreamSynchronize(c->stream);
+    HostCopier::get().forget(c->stream);
+  }
   for (auto* v : {&c->node_start, &c->halo_start, &c->halo, &c->color_off, &c->slot_elem,
                   &c->perm, &c->first_slot})
     v->release();

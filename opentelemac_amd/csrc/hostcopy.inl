@@ -44,14 +44,25 @@ class HostCopier {
       const int slot = (int)(k % kSlots);
       const size_t off = k * kChunk, len = std::min(kChunk, bytes - off);
       // the slot's previous DMA (of this call or an earlier one) has read it
-      if ((e = hipEventSynchronize(ev[slot])) != hipSuccess) return e;
+      if ((e = ring_[dev].wait(slot)) != hipSuccess) return e;
       pcopy(pin[slot], in + off, len);
       if ((e = hipMemcpyAsync(out + off, pin[slot], len, hipMemcpyHostToDevice, s)) !=
           hipSuccess)
         return e;
       if ((e = hipEventRecord(ev[slot], s)) != hipSuccess) return e;
+      ring_[dev].on[slot] = s;
     }
     return hipSuccess;
+  }
+
+  // stream s is about to be destroyed, its work done: its slots' events are
+  // not waited for any more (an event must not outlive the stream it was
+  // recorded on)
+  void forget(hipStream_t s) {
+    std::lock_guard<std::mutex> use(use_mu_);
+    for (Ring& r : ring_)
+      for (hipStream_t& on : r.on)
+        if (on == s) on = nullptr;
   }
 
   hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t s, int dev) {
@@ -70,10 +81,11 @@ class HostCopier {
     auto issue = [&](size_t k) {
       const int slot = (int)(k % kSlots);
       const size_t off = k * kChunk, len = std::min(kChunk, bytes - off);
-      hipError_t r = hipEventSynchronize(ev[slot]);
+      hipError_t r = ring_[dev].wait(slot);
       if (r == hipSuccess)
         r = hipMemcpyAsync(pin[slot], in + off, len, hipMemcpyDeviceToHost, s);
       if (r == hipSuccess) r = hipEventRecord(ev[slot], s);
+      if (r == hipSuccess) ring_[dev].on[slot] = s;
       return r;
     };
     for (size_t k = 0; k < std::min(nch, (size_t)kSlots); ++k)
@@ -81,7 +93,7 @@ class HostCopier {
     for (size_t k = 0; k < nch; ++k) {
       const int slot = (int)(k % kSlots);
       const size_t off = k * kChunk, len = std::min(kChunk, bytes - off);
-      if ((e = hipEventSynchronize(ev[slot])) != hipSuccess) return e;
+      if ((e = ring_[dev].wait(slot)) != hipSuccess) return e;
       pcopy(out + off, pin[slot], len);
       if (k + kSlots < nch && (e = issue(k + kSlots)) != hipSuccess) return e;
     }
@@ -164,6 +176,14 @@ class HostCopier {
   struct Ring {
     char* pin[kSlots] = {nullptr, nullptr, nullptr};
     hipEvent_t ev[kSlots] = {nullptr, nullptr, nullptr};
+    hipStream_t on[kSlots] = {nullptr, nullptr, nullptr};  // stream of the last DMA, if it
+                                                           // has not been waited for
+    hipError_t wait(int k) {
+      if (!on[k]) return hipSuccess;
+      const hipError_t e = hipEventSynchronize(ev[k]);
+      if (e == hipSuccess) on[k] = nullptr;
+      return e;
+    }
   };
   std::mutex use_mu_;  // one transfer at a time (the thread pool is shared)
   Ring ring_[kMaxDevices];
