@@ -2317,29 +2317,36 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   const bool mixed = cfg->precision == BHIP_PREC_MIXED;
   if (mixed && ensure_f32(c)) return BHIP_EDEVICE;
   bool xa32_ready = false;
-  // CG on assembled rows where the context has them (the state of the
-  // diagonal after the preconditioning below decides with it)
-  const bool want_rows = cfg->slv == 1 && c->rows && !c->rows_off;
+  // CG on assembled rows where the context has them; the diagonal as the
+  // preconditioning will leave it
+  char td = c->typdia;
+  if (diag && td == 'I') td = 'Q';
+  if (diag && precon % 2 == 0) td = 'I';
+  const bool use_rows = cfg->slv == 1 && c->rows && !c->rows_off && td != '0';
+  const int row_bytes = mixed ? 4 : 8, npair = L.ndp * (L.ndp - 1) / 2;
+  const bool by_block = use_rows && rows_by_block(c->rows);
+  if (use_rows) HIP_OK(rows_reserve(c->rows, row_bytes));
   if (diag) {
     // PRECD1 (precd1.f:90-149), X and B taken from the caller's vectors
     hipLaunchKernelGGL(k_precd1_nodes, dim3(g), dim3(kThreads), 0, c->stream, c->vx.p, c->vb.p,
                        x_dev, b_dev, internal ? nullptr : c->perm.p, da_src, c->da.p, c->vdinv.p,
                        n, precon, c->typdia == 'Q', c->typdia == 'I');
     HIP_OK(hipGetLastError());
-    if (c->typdia == 'I') c->typdia = 'Q';
-    if (c->ncoef > 0) {
+    if (c->ncoef > 0 && !by_block) {
       // the mixed path takes its FP32 copy of D A D in the same pass
-      float* x32 = mixed && !want_rows ? c->xa32.p : nullptr;
+      float* x32 = mixed && !use_rows ? c->xa32.p : nullptr;
       HIP_OK(launch_dmd(c, x32, c->vdinv.p, xa_src));
       xa32_ready = x32 != nullptr;
     }
-    if (precon % 2 == 0 || precon % 3 == 0) c->typdia = 'I';
+    c->typdia = td;
   }
-  const bool use_rows = want_rows && c->typdia != '0';
-  if (use_rows) {
-    const int bytes = mixed ? 4 : 8, npair = L.ndp * (L.ndp - 1) / 2;
-    HIP_OK(rows_reserve(c->rows, bytes));
-    HIP_OK(rows_assemble(c->rows, bytes, c->xa.p, L.nslot_pad, npair, c->typext == 'Q',
+  if (by_block) {
+    RowsDmd a = {xa_src, c->xa.p, diag && c->ncoef > 0 ? c->vdinv.p : nullptr, L.ndp, L.nslot_pad, L.nblocks,
+                 L.max_local, c->typext == 'Q', c->lid.p, c->node_start.p, c->halo_start.p,
+                 c->halo.p, c->color_off.p};
+    HIP_OK(rows_dmd(c->rows, row_bytes, a, c->stream));
+  } else if (use_rows) {
+    HIP_OK(rows_assemble(c->rows, row_bytes, c->xa.p, L.nslot_pad, npair, c->typext == 'Q',
                          c->stream));
   }
   int rc;

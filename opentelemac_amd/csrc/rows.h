@@ -38,6 +38,8 @@ namespace bhip {
 
 constexpr int kSlab = 1024;          // rows of a slab, threads of a workgroup
 constexpr int kSlices = kSlab / 64;  // waves of a workgroup, slices of one row per thread
+constexpr int kRefChunk = 4;
+constexpr size_t kSlabLds = 152 << 10;  // LDS of the fused D A D and assembly (by_block)
 constexpr int kMaxGroup = 8;         // slabs of one workgroup
 constexpr int kMaxGang = 256;        // workgroups of one system
 
@@ -51,13 +53,22 @@ struct RowLayout {
   std::vector<int32_t> slice_off;    // [nslice + 1]
   std::vector<int32_t> pair_off;     // [nslice + 1]
   std::vector<uint16_t> ids;         // LDS index of the entry's column
-  // assembly: entry column j of slice q sums cnt[slice_off[q] + j] coefficients,
-  // whose references start at ref_off[q] * 64, 64 lanes wide, column by column.
-  // A reference is pair * nslot_pad + slot, its top bit set for a term below
-  // the element's diagonal (the second half of a non-symmetric matrix), or -1
-  std::vector<uint8_t> cnt;
-  std::vector<int64_t> ref_off;      // [nslice]
+  // assembly: the coefficients a slice's entries sum, reference column by
+  // reference column, 64 lanes wide, entry after entry: column c of slice q is
+  // refs[(ref_off[q] + c) * 64 + lane]. A reference is pair * nslot_pad + slot,
+  // its top bit set for a term below the element's diagonal (the second half
+  // of a non-symmetric matrix), or -1. Columns come in chunks of kRefChunk
+  // (filled up with -1); bit c of a chunk's byte in ref_end says that column c
+  // is the last one of its entry.
+  std::vector<int32_t> ref_off;      // [nslice + 1], multiples of kRefChunk
+  std::vector<uint8_t> ref_end;      // [ref_off / kRefChunk]
   std::vector<int32_t> refs;
+  // node blocks that are the slabs (triangles and segments, blocks of kSlab
+  // nodes): the references within a block instead, pair * slots of the block +
+  // slot - its first slot, top bit as above, 0xffff: none
+  bool by_block = false;
+  int max_slots = 0;                 // slots of one block
+  std::vector<uint16_t> refs16;
   // workgroups
   std::vector<int32_t> wg_sys;       // [nwg]
   std::vector<int32_t> sys_wg;       // [nsys + 1]

@@ -42,6 +42,7 @@
 // so the system with the lowest numbers always has all of its own running.
 #include "rows_dev.h"
 
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 #include <memory>
@@ -622,31 +623,153 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
 }
 
 // ---------------------------------------------------------------------------
-// assembly: one wave per slice
+// D A D and assembly of one node block: its coefficients are scaled, written
+// back and kept in LDS, where the block's 16 slices sum them. A gather from
+// memory instead takes a cache line per coefficient (k_rows_assemble: 138 us
+// for 2M nodes in FP64, after 49 us for the scaling alone). Bound by memory:
+// 105 us for 2M nodes in FP64 (450 MB, 4.3 TB/s), 48 us for 1M in FP32. 512
+// threads: two blocks per CU, one gathers while the other loads.
+// ---------------------------------------------------------------------------
+constexpr int kDmdThreads = 512;
+template <int NDP, bool Q, typename T>
+__global__ void __launch_bounds__(kDmdThreads)
+k_dmd_rows(RowsDmd a, T* __restrict__ val, const int32_t* __restrict__ slice_off,
+           const int32_t* __restrict__ ref_off, const uint8_t* __restrict__ ref_end,
+           const uint16_t* __restrict__ refs, const int32_t* __restrict__ slab_slice, int group) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  constexpr int npair = NDP * (NDP - 1) / 2, nc = Q ? 2 * npair : npair;
+  const int b = xcd_block(blockIdx.x, a.nblocks);
+  const int t = threadIdx.x, wave = t >> 6;
+  const unsigned lane = t & 63;
+  const int s0 = a.color_off[(size_t)b * (kMaxColors + 1)];
+  const int ns = a.color_off[(size_t)b * (kMaxColors + 1) + kMaxColors] - s0;
+  const size_t np = a.nslot_pad;
+  double* cs = reinterpret_cast<double*>(smem_raw);  // [nc][ns]
+  double* ds = cs + (size_t)nc * ns;
+  if (a.d) {
+    const int n0 = a.node_start[b], nown = a.node_start[b + 1] - n0;
+    const int h0 = a.halo_start[b], nloc = nown + a.halo_start[b + 1] - h0;
+    for (int l = t; l < nloc; l += kDmdThreads)
+      ds[l] = a.d[l < nown ? n0 + l : a.halo[h0 + l - nown]];
+    __syncthreads();
+  }
+  for (int i = t; i < ns; i += kDmdThreads) {
+    const int s = s0 + i;
+    double c[nc], dv[NDP];
+#pragma unroll
+    for (int q = 0; q < nc; ++q) c[q] = a.src[q * np + s];
+    if (a.d) {
+#pragma unroll
+      for (int k = 0; k < NDP; ++k) dv[k] = ds[a.lid[k * np + s]];
+      int q = 0;
+#pragma unroll
+      for (int p = 0; p < NDP; ++p)
+#pragma unroll
+        for (int j = p + 1; j < NDP; ++j, ++q) {
+          // elements: XM * D(j) * D(i) (om1111.f:583-600); segments (NDP 2):
+          // XM * D(GLOSEG1) * D(GLOSEG2) (omseg.f:524-536)
+#pragma unroll
+          for (int h = 0; h < nc / npair; ++h) {
+            double& v = c[h * npair + q];
+            v = NDP == 2 ? v * dv[p] * dv[j] : v * dv[j] * dv[p];
+            a.xa[(h * npair + q) * np + s] = v;
+          }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < nc; ++q) cs[q * ns + i] = c[q];
+  }
+  __syncthreads();
+  // the block's slices: for each of its 16 / group waves, one per row of a thread
+  const int q0 = slab_slice[b];
+  constexpr int U = kRefChunk;
+  for (int i = wave; i < kSlices; i += kDmdThreads / 64) {
+    const int q = __builtin_amdgcn_readfirstlane(q0 + i % group * kSlices + i / group);
+    const int c1 = ref_off[q + 1];
+    T* out = val + (size_t)slice_off[q] * 64;
+    double s = 0.0;
+    for (int c = ref_off[q]; c < c1; c += U) {
+      const uint16_t* p = refs + (size_t)c * 64;
+      int f[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) f[u] = p[u * 64 + lane];
+      const int ends = ref_end[c / U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = (f[u] & 0x7fff) + (Q && (f[u] & 0x8000) ? npair * ns : 0);
+        s += f[u] == 0xffff ? 0.0 : cs[k];
+        if (ends >> u & 1) {
+          out[lane] = (T)s;
+          out += 64;
+          s = 0.0;
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// assembly from memory: one wave per slice, two chunks of references in
+// flight. Bound by the cache line each gathered coefficient takes (600k-node
+// prisms: 34M references, 146 us).
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ void __launch_bounds__(256)
 k_rows_assemble(T* __restrict__ val, const double* __restrict__ xa,
-                const int32_t* __restrict__ slice_off, const uint8_t* __restrict__ cnt,
-                const int64_t* __restrict__ ref_off, const int32_t* __restrict__ refs,
-                int nslice, unsigned lower) {
+                const int32_t* __restrict__ slice_off, const int32_t* __restrict__ ref_off,
+                const uint8_t* __restrict__ ref_end, const int32_t* __restrict__ refs, int nslice,
+                unsigned lower) {
   // each XCD takes a contiguous range of slices: a block's coefficients are
   // read by the slices of its rows
-  const int nb = gridDim.x;
-  const int b = xcd_block(blockIdx.x, nb);
-  const int q = b * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int b = xcd_block(blockIdx.x, gridDim.x);
+  const int q = __builtin_amdgcn_readfirstlane(b * 4 + (int)(threadIdx.x >> 6));
+  const unsigned lane = threadIdx.x & 63;
   if (q >= nslice) return;
-  const int o0 = __builtin_amdgcn_readfirstlane(slice_off[q]);
-  const int o1 = __builtin_amdgcn_readfirstlane(slice_off[q + 1]);
-  const int32_t* r = refs + ref_off[q] * 64 + lane;
-  for (int j = o0; j < o1; ++j) {
-    const int c = __builtin_amdgcn_readfirstlane(cnt[j]);
-    double s = 0.0;
-    for (int i = 0; i < c; ++i, r += 64) {
-      const int f = *r;
-      if (f != -1) s += xa[(size_t)(f & 0x7fffffff) + (f < 0 ? lower : 0u)];
+  const int c0 = ref_off[q], c1 = ref_off[q + 1];
+  T* out = val + (size_t)slice_off[q] * 64;
+  double s = 0.0;
+  constexpr int U = kRefChunk;
+  auto load = [&](int c, int (&r)[U]) {
+    const int32_t* p = refs + (size_t)c * 64;
+#pragma unroll
+    for (int u = 0; u < U; ++u) r[u] = p[u * 64 + lane];
+  };
+  auto gather = [&](const int (&r)[U], double (&v)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int f = r[u];
+      // (no branch around the load: reference 0 stands in for none)
+      const size_t i = f == -1 ? 0 : (size_t)(f & 0x7fffffff) + (f < 0 ? lower : 0u);
+      const double x = xa[i];
+      v[u] = f == -1 ? 0.0 : x;
     }
-    val[(size_t)j * 64 + lane] = (T)s;
+  };
+  auto add = [&](int c, const double (&v)[U]) {
+    const int ends = ref_end[c / U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      s += v[u];
+      if (ends >> u & 1) {
+        out[lane] = (T)s;
+        out += 64;
+        s = 0.0;
+      }
+    }
+  };
+  for (int c = c0; c < c1; c += 2 * U) {
+    int ra[U], rb[U];
+    double va[U], vb[U];
+    load(c, ra);
+    if (c + U < c1) {
+      load(c + U, rb);
+      gather(ra, va);
+      gather(rb, vb);
+      add(c, va);
+      add(c + U, vb);
+    } else {
+      gather(ra, va);
+      add(c, va);
+    }
   }
 }
 
@@ -680,11 +803,13 @@ struct RowsDev {
   int nslice = 0, group = 1, nwg = 0, nsys = 1, max_halo = 0;
   int64_t nent = 0;
   int ncu = 0, nexp = 0;
-  Buf<int32_t> wg_row0, slice_off, pair_off, refs, wg_sys, sys_wg, halo_off, halo_row, halo_src,
+  Buf<int32_t> wg_row0, slice_off, pair_off, ref_off, refs, wg_sys, sys_wg, halo_off, halo_row, halo_src,
       exp_off;
-  Buf<uint16_t> rowpos, ids, exp_loc;
-  Buf<uint8_t> cnt;
-  Buf<int64_t> ref_off;
+  Buf<uint16_t> rowpos, ids, exp_loc, refs16;
+  Buf<int32_t> slab_slice;  // by_block: first slice of each block's slab
+  bool by_block = false;
+  int max_slots = 0, lds_max = 0;
+  Buf<uint8_t> ref_end;
   Buf<double> v64;
   Buf<float> v32;
   Buf<u64> words;
@@ -749,6 +874,9 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
   r->nwg = R.nwg;
   r->nsys = nsys;
   r->max_halo = R.max_halo;
+  r->by_block = R.by_block;
+  r->max_slots = R.max_slots;
+  r->lds_max = lds_max;
   r->nent = R.nent + 64;
   r->ncu = ncu;
   r->nexp = (int)R.exp_loc.size();
@@ -762,14 +890,24 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
     if (e != hipSuccess) *err = e;
     return e == hipSuccess;
   };
-  if (!ok(r->wg_row0.put(R.wg_row0, stream)) || !ok(r->slice_off.put(R.slice_off, stream)) ||
+  std::vector<int32_t> slab_slice;
+  if (R.by_block)
+    for (int b = 0; b < L.nblocks; ++b) {
+      // the workgroup that holds the block's rows, and the first of its waves that do
+      const int row = L.node_start[b];
+      const int g = (int)(std::upper_bound(R.wg_row0.begin(), R.wg_row0.end(), row) -
+                          R.wg_row0.begin()) - 1;
+      slab_slice.push_back(g * R.group * kSlices + (row - R.wg_row0[g]) / kSlab * (kSlices / R.group));
+    }
+  if (!ok(r->wg_row0.put(R.wg_row0, stream)) || !ok(r->refs16.put(R.refs16, stream)) ||
+      !ok(r->slab_slice.put(slab_slice, stream)) || !ok(r->slice_off.put(R.slice_off, stream)) ||
       !ok(r->pair_off.put(R.pair_off, stream)) ||
       !ok(r->refs.put(R.refs, stream)) ||
       !ok(r->wg_sys.put(R.wg_sys, stream)) || !ok(r->sys_wg.put(R.sys_wg, stream)) ||
       !ok(r->halo_off.put(R.halo_off, stream)) || !ok(r->halo_row.put(R.halo_row, stream)) ||
       !ok(r->halo_src.put(R.halo_src, stream)) || !ok(r->exp_off.put(R.exp_off, stream)) ||
       !ok(r->rowpos.put(R.rowpos, stream)) || !ok(r->ids.put(R.ids, stream)) ||
-      !ok(r->exp_loc.put(R.exp_loc, stream)) || !ok(r->cnt.put(R.cnt, stream)) ||
+      !ok(r->exp_loc.put(R.exp_loc, stream)) || !ok(r->ref_end.put(R.ref_end, stream)) ||
       !ok(r->ref_off.put(R.ref_off, stream)) || !ok(r->v64.alloc(r->nent)))
     return nullptr;
   // sync words: per precision sums and exchange, then the counters
@@ -807,11 +945,37 @@ hipError_t rows_assemble(RowsDev* r, int bytes, const double* xa, int nslot_pad,
   const dim3 grid((nslice + 3) / 4), block(256);
   if (bytes == 8)
     hipLaunchKernelGGL(k_rows_assemble<double>, grid, block, 0, stream, r->v64.p, xa,
-                       r->slice_off.p, r->cnt.p, r->ref_off.p, r->refs.p, nslice, lower);
+                       r->slice_off.p, r->ref_off.p, r->ref_end.p, r->refs.p, nslice, lower);
   else
     hipLaunchKernelGGL(k_rows_assemble<float>, grid, block, 0, stream, r->v32.p, xa,
-                       r->slice_off.p, r->cnt.p, r->ref_off.p, r->refs.p, nslice, lower);
+                       r->slice_off.p, r->ref_off.p, r->ref_end.p, r->refs.p, nslice, lower);
   return hipGetLastError();
+}
+
+bool rows_by_block(const RowsDev* r) { return r->by_block; }
+
+hipError_t rows_dmd(RowsDev* r, int bytes, const RowsDmd& a, hipStream_t stream) {
+  const int nc = a.ndp * (a.ndp - 1) / 2 * (a.nonsym ? 2 : 1);
+  const size_t lds = ((size_t)nc * r->max_slots + a.max_local + 1) * sizeof(double);
+  auto go = [&](auto kern, auto* val) -> hipError_t {
+    if (lds > (size_t)r->lds_max) return hipErrorInvalidValue;
+    if (lds > 65536) {
+      const hipError_t e =
+          hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, r->lds_max);
+      if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(kern, dim3(a.nblocks), dim3(kDmdThreads), lds, stream, a, val,
+                       r->slice_off.p, r->ref_off.p, r->ref_end.p, r->refs16.p, r->slab_slice.p,
+                       r->group);
+    return hipGetLastError();
+  };
+#define BHIP_DMD_ROWS(NDP, Q)                                        \
+  (bytes == 8 ? go(&k_dmd_rows<NDP, Q, double>, r->v64.p)            \
+              : go(&k_dmd_rows<NDP, Q, float>, r->v32.p))
+  if (a.ndp == 2) return a.nonsym ? BHIP_DMD_ROWS(2, true) : BHIP_DMD_ROWS(2, false);
+  return a.nonsym ? BHIP_DMD_ROWS(3, true) : BHIP_DMD_ROWS(3, false);
+#undef BHIP_DMD_ROWS
 }
 
 static RowArgs row_args(const RowsDev* r, int k) {

@@ -24,6 +24,24 @@ hipError_t rows_reserve(RowsDev* r, int bytes);
 hipError_t rows_assemble(RowsDev* r, int bytes, const double* xa, int nslot_pad, int npair,
                          bool nonsym, hipStream_t stream);
 
+// OM 'M=DMD' and the assembly in one pass, where node blocks are slabs
+// (rows_by_block): the coefficients src times D(i) D(j), written to xa and
+// summed into the rows. d nullptr: src as it is, xa not written.
+bool rows_by_block(const RowsDev* r);
+struct RowsDmd {
+  const double* src;
+  double* xa;
+  const double* d;
+  int ndp, nslot_pad, nblocks, max_local;
+  bool nonsym;
+  const uint16_t* lid;
+  const int32_t* node_start;
+  const int32_t* halo_start;
+  const int32_t* halo;
+  const int32_t* color_off;
+};
+hipError_t rows_dmd(RowsDev* r, int bytes, const RowsDmd& a, hipStream_t stream);
+
 // One CG solve per system of the context (gracjg.F:248-409), from the
 // residual r0 to the stop, in one launch. Vectors in internal node order.
 template <typename T>

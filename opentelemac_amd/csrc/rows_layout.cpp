@@ -42,8 +42,8 @@ struct Scratch {
 struct WgOut {
   std::vector<int32_t> width;  // per slice
   std::vector<int32_t> cols;   // per entry (internal node id, -1: none)
-  std::vector<uint8_t> cnt;
-  std::vector<int32_t> refs, ref_units;  // per slice: 64-wide reference columns
+  std::vector<uint8_t> ref_end;
+  std::vector<int32_t> refs, ref_cols;  // per slice: reference columns
   std::vector<int32_t> halo;
 };
 
@@ -73,6 +73,17 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
   R.group = wgs(1) <= cap / 2 ? 1 : 2;
   while (R.group < kMaxGroup && wgs(R.group) > cap) R.group *= 2;
   const int G = R.group, wrows = G * kSlab;
+  // slabs and node blocks are the same rows when both start anew with each
+  // system and hold kSlab of them
+  auto block_slots = [&](int b) {
+    const int32_t* co = &L.color_off[(size_t)b * (kMaxColors + 1)];
+    return co[kMaxColors] - co[0];
+  };
+  for (int b = 0; b < L.nblocks; ++b) R.max_slots = std::max(R.max_slots, block_slots(b));
+  R.by_block = ndp <= 3 && L.block_nodes == kSlab &&
+               R.max_slots * (ndp * (ndp - 1) / 2) < 0x7fff &&
+               // k_dmd_rows keeps a block's coefficients and D in LDS
+               ((size_t)ndp * (ndp - 1) * R.max_slots + L.max_local + 1) * 8 <= kSlabLds;
   R.sys_wg.assign(1, 0);
   std::vector<int32_t> nrows;  // of each workgroup
   for (int s = 0; s < nsys; ++s) {
@@ -171,7 +182,7 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
       if (w.row_at[id] >= 0) R.rowpos[(size_t)wg * wrows + id] = (uint16_t)w.row_at[id];
     WgOut& o = out[wg];
     o.width.assign(wslices, 0);
-    o.ref_units.assign(wslices, 0);
+    o.ref_cols.assign(wslices, 0);
     for (int q = 0; q < wslices; ++q) {
       const int32_t* at = &w.row_at[(size_t)q * 64];  // (k * kSlab + wave * 64)
       int width = 0;
@@ -183,8 +194,11 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
         for (int l = 0; l < 64; ++l)
           if (at[l] >= 0 && j < (int)w.rows[at[l]].size())
             c = std::max(c, w.rows[at[l]][j].count);
-        o.cnt.push_back((uint8_t)std::min(c, 255));
-        o.ref_units[q] += c;
+        for (int t = 0; t < c; ++t) {
+          const int col = o.ref_cols[q]++;
+          if (col % kRefChunk == 0) o.ref_end.push_back(0);
+          if (t == c - 1) o.ref_end.back() |= (uint8_t)(1 << col % kRefChunk);
+        }
         const size_t base = o.refs.size(), cb = o.cols.size();
         o.refs.resize(base + (size_t)c * 64, -1);
         o.cols.resize(cb + 64, -1);
@@ -197,6 +211,10 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
             o.refs[base + (size_t)t * 64 + l] = w.con[e[j].first + t].ref;
         }
       }
+      o.ref_cols[q] = (o.ref_cols[q] + kRefChunk - 1) / kRefChunk * kRefChunk;
+      size_t total = 0;
+      for (int i = 0; i <= q; ++i) total += o.ref_cols[i];
+      o.refs.resize(total * 64, -1);
     }
     // halo: the other workgroups' rows these entries name, by row
     if (w.mark.empty()) w.mark.assign(L.npoin, -1);
@@ -210,22 +228,23 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
   // ---- joined --------------------------------------------------------------
   R.slice_off.assign(R.nslice + 1, 0);
   R.pair_off.assign(R.nslice + 1, 0);
-  R.ref_off.assign(R.nslice, 0);
+  R.ref_off.assign(R.nslice + 1, 0);
   int64_t units = 0, runits = 0;
   for (int g = 0; g < R.nwg; ++g)
     for (int q = 0; q < wslices; ++q) {
       const size_t i = (size_t)g * wslices + q;
-      R.ref_off[i] = runits;
       units += out[g].width[q];
-      runits += out[g].ref_units[q];
+      runits += out[g].ref_cols[q];
+      if (runits > INT32_MAX || units > INT32_MAX / 128) {
+        R = RowLayout();
+        return false;
+      }
+      R.ref_off[i + 1] = (int32_t)runits;
       R.slice_off[i + 1] = (int32_t)units;
       R.pair_off[i + 1] = R.pair_off[i] + (out[g].width[q] + 1) / 2;
     }
-  bool fits = units <= INT32_MAX / 128;
-  for (const auto& o : out) {
-    fits = fits && wrows + o.halo.size() <= 65535;
-    for (uint8_t c : o.cnt) fits = fits && c < 255;  // (a pair shared by 255 elements)
-  }
+  bool fits = true;
+  for (const auto& o : out) fits = fits && wrows + o.halo.size() <= 65535;
   if (!fits) {
     R = RowLayout();
     return false;
@@ -233,8 +252,9 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
   R.nent = units * 64;
   R.nref = runits * 64;
   R.ids.assign((size_t)R.pair_off.back() * 128, 0);
-  R.refs.resize(R.nref);
-  R.cnt.resize(units);
+  if (!R.by_block) R.refs.resize(R.nref);
+  R.ref_end.resize(runits / kRefChunk);
+  if (R.by_block) R.refs16.resize(R.nref);
   parallel_for(R.nwg, [] { return 0; }, [&](int g, int&) {
     const int r0 = R.wg_row0[g], r1 = r0 + nrows[g];
     const WgOut& o = out[g];
@@ -253,8 +273,28 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
           id[((size_t)(j / 2) * 64 + l) * 2 + (j & 1)] = (uint16_t)v;
         }
     }
-    std::copy(o.refs.begin(), o.refs.end(), R.refs.begin() + R.ref_off[q0] * 64);
-    std::copy(o.cnt.begin(), o.cnt.end(), R.cnt.begin() + R.slice_off[q0]);
+    if (R.by_block) {
+      // slice by slice: its rows lie in one slab, so in one block
+      size_t i = 0;
+      for (int q = 0; q < wslices; ++q) {
+        const int leaf = q % kSlices * 64 * G;  // first leaf of the slice's first lane
+        const int row = r0 + leaf / kSlab * kSlab;
+        const int b = (int)(std::upper_bound(L.node_start.begin(), L.node_start.end(), row) -
+                            L.node_start.begin()) - 1;
+        const int s0 = b < L.nblocks ? L.color_off[(size_t)b * (kMaxColors + 1)] : 0;
+        const int ns = b < L.nblocks ? block_slots(b) : 1;
+        uint16_t* to = R.refs16.data() + (size_t)R.ref_off[q0 + q] * 64;
+        for (int c = 0; c < o.ref_cols[q] * 64; ++c, ++i) {
+          const uint32_t f = (uint32_t)o.refs[i], low = f & 0x7fffffffu;
+          to[c] = o.refs[i] == -1 ? 0xffff
+                                  : (uint16_t)((f >> 31 << 15) | (low / L.nslot_pad * ns +
+                                                                  low % L.nslot_pad - s0));
+        }
+      }
+    } else {
+      std::copy(o.refs.begin(), o.refs.end(), R.refs.begin() + (size_t)R.ref_off[q0] * 64);
+    }
+    std::copy(o.ref_end.begin(), o.ref_end.end(), R.ref_end.begin() + R.ref_off[q0] / kRefChunk);
   });
   std::vector<std::vector<int32_t>> halo(R.nwg);
   for (int g = 0; g < R.nwg; ++g) halo[g] = std::move(out[g].halo);

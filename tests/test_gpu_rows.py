@@ -8,6 +8,7 @@ solutions agree within the condition number of the scaled system (under 100
 for these time steps) times that, 1e-7."""
 import numpy as np
 import pytest
+import torch
 
 from opentelemac_amd import bief, mesh as M, system as S
 from oracle import oracle as O
@@ -58,6 +59,45 @@ def test_rows_cg_with_a_diagonal(gpu, precon, typext):
     m = M.random_small_mesh(70, 61, seed=3)
     _check(m, S.wave_system(m, 2.0 + m.x / 10.0, dt=0.3), precon=precon, block_nodes=300,
            typext=typext)
+
+
+@pytest.mark.parametrize("precon", [0, 2, 5])
+@pytest.mark.parametrize("typext", ["S", "Q"])
+def test_rows_summed_with_the_scaling(gpu, precon, typext):
+    """Node blocks that are the slabs (1024 rows, the last one ragged): rows
+    summed in the pass that scales the coefficients, or that only reads them;
+    from the context's matrix and from the saved copy."""
+    m = M.random_small_mesh(70, 61, seed=4)
+    sysd = S.wave_system(m, 2.0 + m.x / 10.0, dt=0.3)
+    want = _check(m, sysd, precon=precon, block_nodes=1024, typext=typext)[0]
+    rng = np.random.default_rng(0)
+    b = sysd["b"] + 1e-2 * rng.normal(size=m.npoin)
+    ctx = bief.Context(m, block_nodes=1024)
+    xa = sysd["xa"] if typext == "S" else np.concatenate([sysd["xa"], sysd["xa"]])
+    ctx.set_matrix("Q", typext, sysd["da"], xa)
+    ctx.save_matrix()
+    for _ in range(2):
+        dx, db = torch.tensor(sysd["x0"], device="cuda"), torch.tensor(b, device="cuda")
+        ctx.solve(dx, db, slv=1, precon=precon, eps=1e-10, nitmax=2000, restore=True)
+        assert np.array_equal(dx.cpu().numpy(), want)
+    ctx.close()
+
+
+def test_rows_of_a_diagonal_matrix(gpu):
+    """No off-diagonal terms (TYPEXT '0'): the rows hold zeros."""
+    m = M.random_small_mesh(40, 31, seed=5)
+    sysd = S.wave_system(m, 2.0 + m.x / 10.0, dt=0.3)
+    ctx = bief.Context(m, block_nodes=1024)
+    ctx.set_matrix("Q", "S", sysd["da"], sysd["xa"])
+    ctx.solve(sysd["x0"].copy(), sysd["b"].copy(), slv=1, precon=2, eps=1e-8, nitmax=100)
+    for precon in (0, 2):
+        ctx.set_matrix("Q", "0", sysd["da"], None)
+        x, info = ctx.solve(sysd["x0"].copy(), sysd["b"].copy(), slv=1, precon=precon, eps=1e-12,
+                            nitmax=4000)
+        assert info["converged"]
+        np.testing.assert_allclose(x, sysd["b"] / sysd["da"],
+                                   atol=1e-10 * np.abs(sysd["b"] / sysd["da"]).max())
+    ctx.close()
 
 
 def test_more_workgroups_than_the_gpu_holds(gpu):
