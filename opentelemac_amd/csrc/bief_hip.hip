@@ -1038,7 +1038,8 @@ struct bhip_ctx {
   bhip::RowsDev* rows = nullptr;  // assembled rows for the persistent CG, or none
   bool rows_off = false;          // it gave up once: the two-kernel CG from then on
   int prefetch_j = 0;  // register prefetch depth of the element kernels
-  int iter_hint[4] = {0, 0, 0, 0};  // FP64 CG, inner CG, inner solves, CGSTAB
+  int iter_hint[5] = {0, 0, 0, 0, 0};  // FP64 CG, inner CG, inner solves, CGSTAB, cycles
+                                       // of mixed GMRES
   int inner_hint[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // iterations of inner solve k (mixed CG)
   // BiCGSTAB scalars and extra partial sums; GMRES basis and scalars
   bhip::DevBuf<double> bicg_sc, bicg_part, gm, gm_scal;
@@ -2317,13 +2318,14 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   const bool mixed = cfg->precision == BHIP_PREC_MIXED;
   if (mixed && ensure_f32(c)) return BHIP_EDEVICE;
   bool xa32_ready = false;
-  // CG on assembled rows where the context has them; the diagonal as the
-  // preconditioning will leave it
+  // CG and GMRES on assembled rows where the context has them; the diagonal
+  // as the preconditioning will leave it
   char td = c->typdia;
   if (diag && td == 'I') td = 'Q';
   if (diag && precon % 2 == 0) td = 'I';
-  const bool use_rows = cfg->slv == 1 && c->rows && !c->rows_off && td != '0';
   const int row_bytes = mixed ? 4 : 8, npair = L.ndp * (L.ndp - 1) / 2;
+  const bool use_rows = c->rows && !c->rows_off && td != '0' &&
+                        (cfg->slv == 1 || (cfg->slv == 7 && rows_gmres_fits(c->rows, row_bytes)));
   const bool by_block = use_rows && rows_by_block(c->rows);
   if (use_rows) HIP_OK(rows_reserve(c->rows, row_bytes));
   if (diag) {
@@ -2351,7 +2353,7 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   }
   int rc;
   // where the solution is left (the persistent FP64 CG keeps the initial one)
-  double* xsrc = use_rows && !mixed ? c->vd1.p : c->vx.p;
+  double* xsrc = use_rows && !mixed && cfg->slv == 1 ? c->vd1.p : c->vx.p;
   // X <- X*D (solve.f:637-641) and B <- D*B (as the reference leaves it),
   // back to the caller's order or copied as they are (internal). A mixed
   // solve of one system reads X from the solution buffer its state names;
@@ -2375,11 +2377,22 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   };
   if (cfg->slv == 6) {
     rc = bhip::cgstab_fp64(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, info);
-  } else if (cfg->slv == 7 && mixed) {
-    rc = bhip::gmres_mixed(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, cfg->krylov, xa32_ready,
-                           info);
   } else if (cfg->slv == 7) {
-    rc = bhip::gmres_fp64(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, cfg->krylov, info);
+    rc = kGaveUp;
+    if (use_rows) {
+      bool moved = false;
+      rc = mixed ? gmres_rows<float>(c, c->vx.p, c->vd1.p, &moved, c->vb.p, cfg->eps, cfg->nitmax,
+                                     cfg->krylov, info)
+                 : gmres_rows<double>(c, c->vx.p, c->vd1.p, &moved, c->vb.p, cfg->eps,
+                                      cfg->nitmax, cfg->krylov, info);
+      if (moved) xsrc = c->vd1.p;
+      if (rc == kGaveUp) c->rows_off = true;
+    }
+    if (rc == kGaveUp && mixed)
+      rc = bhip::gmres_mixed(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, cfg->krylov, xa32_ready,
+                             info);
+    else if (rc == kGaveUp)
+      rc = bhip::gmres_fp64(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, cfg->krylov, info);
   } else if (cfg->precision == BHIP_PREC_MIXED) {
     double ie = cfg->inner_eps > 0 ? cfg->inner_eps : 1e-4;
     int inn = cfg->inner_nitmax > 0 ? cfg->inner_nitmax : std::max(cfg->nitmax, 1);

@@ -1,4 +1,5 @@
-// Persistent Krylov kernels on assembled rows (rows.h), MI355X.
+// Persistent Krylov kernels on assembled rows (rows.h), MI355X. What follows is
+// CG's; GMRES is built alike and described at its kernel.
 //
 // One launch runs a whole CG solve. Each workgroup (one per CU, 1024 threads)
 // keeps the residual and the solution of its rows in registers, `group` rows
@@ -53,7 +54,8 @@ namespace bhip {
 typedef unsigned long long u64;
 
 constexpr int kReplicas = 8;
-constexpr int kSums = 4;  // sums of one meeting
+constexpr int kSums = 4;  // sums of one meeting of CG
+constexpr int kGmMaxK = 20, kGmSums = 2 * kGmMaxK + 4;  // of GMRES
 // ||R||^2 of the next iteration is taken from this one's sums while it is at
 // least this part of ||R||^2: its relative error is then below 4e-16 / kTrust
 constexpr double kTrust = 1e-3;
@@ -92,12 +94,17 @@ __device__ inline bool look(const u64* p, size_t, unsigned e, float& v) {
   v = __uint_as_float((unsigned)(a >> 32));
   return (unsigned)a == e;
 }
+// one wait's limit: from its 256th look on
 struct Deadline {
-  u64 t0, ticks;
+  u64 ticks;
   const int* abort;
-  __device__ bool past(int& n) const {
-    return ((++n & 255) == 0 || ticks == 0) &&
-           ((u64)wall_clock64() - t0 >= ticks || load_relaxed(abort));
+  u64 t0 = 0;
+  int n = 0;
+  __device__ bool past() {
+    if ((++n & 255) != 0 && ticks != 0) return false;
+    const u64 now = wall_clock64();
+    if (!t0) t0 = now;
+    return now - t0 >= ticks || load_relaxed(abort);
   }
 };
 
@@ -125,7 +132,7 @@ struct RowArgs {
   const int32_t* halo_src;
   const int32_t* exp_off;
   const uint16_t* exp_loc;
-  int nwg, nsys, nexp;
+  int nwg, nsys, nexp, nhalo;
   SyncWords sy;
   int ep;        // parity of the launch
   int ticketed;  // workgroup numbers by order of start
@@ -322,6 +329,59 @@ __device__ inline T front_dot(const RowFront<T>& f, const T* ys) {
   return s;
 }
 
+// as = A ds of the workgroup's rows, without the diagonal: thread t's k-th row
+// at k * kSlab + t. The coefficients of small partitions stay in registers
+// for the whole solve.
+template <typename T, int R>
+struct RowProduct {
+  static constexpr bool kKeep = R * sizeof(T) <= 16;
+  RowFront<T> front[kKeep ? R : 1];
+  int wid[kKeep ? R : 1];
+  // the slice of this wave's k-th rows: its coefficients, id words and width
+  static __device__ inline int slice(const RowArgs& ra, const T* val, int wg, int k, const T*& v,
+                                     const unsigned*& id) {
+    const int q = __builtin_amdgcn_readfirstlane((wg * R + k) * kSlices + (int)(threadIdx.x >> 6));
+    const int o = ra.slice_off[q];
+    v = val + (size_t)o * 64;
+    id = ra.ids + (size_t)ra.pair_off[q] * 64;
+    return ra.slice_off[q + 1] - o;
+  }
+  __device__ inline void load(const RowArgs& ra, const T* val, int wg, int k) {
+    if constexpr (kKeep) {
+      const T* v;
+      const unsigned* id;
+      wid[k] = slice(ra, val, wg, k, v, id);
+      load_front(front[k], v, id, threadIdx.x & 63, wid[k]);
+    }
+  }
+  __device__ inline void apply(const RowArgs& ra, const T* val, int wg, const T* ds, T* as) const {
+    const int t = threadIdx.x, lane = t & 63;
+    if constexpr (kKeep) {
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        T s = front_dot(front[k], ds);
+        if (wid[k] > kFront) {
+          const T* v;
+          const unsigned* id;
+          slice(ra, val, wg, k, v, id);
+          s += slice_dot<4>(v, id, lane, kFront, wid[k], ds);
+        }
+        as[k * kSlab + t] = s;
+        // (one slab's gathers at a time)
+        if constexpr (R >= 2) __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma nounroll
+      for (int k = 0; k < R; ++k) {
+        const T* v;
+        const unsigned* id;
+        const int w = slice(ra, val, wg, k, v, id);
+        as[k * kSlab + t] = slice_dot<8>(v, id, lane, 0, w, ds);
+      }
+    }
+  }
+};
+
 // ---------------------------------------------------------------------------
 // CG
 // ---------------------------------------------------------------------------
@@ -356,7 +416,6 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
                          __HIP_MEMORY_SCOPE_AGENT);
     return;
   }
-  const Deadline dl = {(u64)wall_clock64(), ra.sy.ticks, ra.sy.abort};
   const int r0 = ra.wg_row0[wg];
   const uint16_t* rowpos = ra.rowpos + (size_t)wg * R * kSlab;
   const int h0 = ra.halo_off[wg], nh = ra.halo_off[wg + 1] - h0;
@@ -387,18 +446,7 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
   const double thr = ld_f64(&st->eps2xl) * (load_relaxed(&st->use_rr0) ? ld_f64(&st->rr0) : 1.0);
   const int nitmax = load_relaxed(&st->nitmax);
 
-  // the coefficients of small partitions stay in registers for the whole solve
-  constexpr bool kKeep = R * sizeof(T) <= 16;
-  RowFront<T> front[kKeep ? R : 1];
-  int wid[kKeep ? R : 1];
-  // the slice of this wave's k-th rows: its coefficients, id words and width
-  auto slice = [&](int k, const T*& v, const unsigned*& id) -> int {
-    const int q = __builtin_amdgcn_readfirstlane((wg * R + k) * kSlices + wave);
-    const int o = ra.slice_off[q];
-    v = val + (size_t)o * 64;
-    id = ra.ids + (size_t)ra.pair_off[q] * 64;
-    return ra.slice_off[q + 1] - o;
-  };
+  RowProduct<T, R> prod;
   unsigned have = 0;  // bit k: this thread has a k-th row
   T rv[R], xv[R], dq[DQ ? R : 1];
   const double beta0 = m == 0 ? 0.0 : rr / rr_prev;
@@ -420,12 +468,7 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
       if (m > 0) d += (T)beta0 * a.dlast[row];
     }
     ds[k * kSlab + t] = d;
-    if constexpr (kKeep) {
-      const T* v;
-      const unsigned* id;
-      wid[k] = slice(k, v, id);
-      load_front(front[k], v, id, lane, wid[k]);
-    }
+    prod.load(ra, val, wg, k);
   }
   for (int h = t; h < nh; h += kSlab) {
     const int g = ra.halo_row[h0 + h];
@@ -475,12 +518,12 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
     const u64* hp = xch + my_src;
     double p = 0.0;
     T hv = (T)0;
-    int n = 0;
+    Deadline dl = {ra.sy.ticks, ra.sy.abort};
     while (need_s || need_h) {
       if (need_s) need_s = !look(sp, 1, e, p);
       if constexpr (halo.value)
         if (need_h) need_h = !look(hp, ra.nexp, e, hv);
-      if ((need_s || need_h) && dl.past(n)) break;
+      if ((need_s || need_h) && dl.past()) break;
     }
     bool ok = !(need_s || need_h);
     if constexpr (halo.value) {
@@ -488,7 +531,7 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
       for (int h = tt + kSlab; h < nh && ok; h += kSlab) {
         T v2;
         while (!look(xch + ra.halo_src[h0 + h], ra.nexp, e, v2))
-          if (dl.past(n)) {
+          if (dl.past()) {
             ok = false;
             break;
           }
@@ -517,29 +560,7 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
   int status = ST_CONVERGED;
   while (!stop) {
     // AD
-    if constexpr (kKeep) {
-#pragma unroll
-      for (int k = 0; k < R; ++k) {
-        T s = front_dot(front[k], ds);
-        if (wid[k] > kFront) {
-          const T* v;
-          const unsigned* id;
-          slice(k, v, id);
-          s += slice_dot<4>(v, id, lane, kFront, wid[k], ds);
-        }
-        as[k * kSlab + t] = s;
-        // (one slab's gathers at a time, as above)
-        if constexpr (R >= 2) __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-#pragma nounroll
-      for (int k = 0; k < R; ++k) {
-        const T* v;
-        const unsigned* id;
-        const int w = slice(k, v, id);
-        as[k * kSlab + t] = slice_dot<8>(v, id, lane, 0, w, ds);
-      }
-    }
+    prod.apply(ra, val, wg, ds, as);
     if constexpr (DQ) {
 #pragma unroll
       for (int k = 0; k < R; ++k)
@@ -620,6 +641,450 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
     __hip_atomic_store(ra.sy.epoch + (1 - ra.ep) * ra.nsys + sys, e, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+// ---------------------------------------------------------------------------
+// GMRES(K): FP64, a whole solve; FP32 (mixed precision), one cycle from an
+// FP64 residual
+// ---------------------------------------------------------------------------
+// One meeting per Arnoldi step: w = A V_j with w.V_i and V_j.V_i (i <= j), w.w
+// and the exchange of w of the halo rows. From these every workgroup has the
+// coefficients of modified Gram-Schmidt, h_i = w.V_i - sum over l < i of h_l
+// V_l.V_i (the dot of V_i with what the earlier steps leave of w), and ||w -
+// sum h_i V_i||^2, summed anew where it falls below kTrust w.w. The halo's V
+// follow from the exchanged w. The basis lies in memory, each thread's rows
+// together, and mostly in L2; V_j and w are in LDS, R0 in registers.
+//
+// us per solve at K = 5, FP64 / mixed (the same from the host, one kernel per
+// orthogonalisation step: 11 launches, 9 of them with a sum over all
+// workgroups, for a cycle of K = 3): 20k nodes 531 / 746 (2361 / 2760), 500k
+// 889 / 1072 (2896 / 3120), 2M 3303 / 2528 (5275 / 4711); 11 cycles each. A step
+// takes 7 us at 20k, most of it the meeting, 60 at 2M, where the basis (170 MB)
+// and the matrix come from the last-level cache.
+struct GmLds {
+  double part[kGmSums * kRowWaves];
+  double tot[kGmSums * 4];
+  double h[kGmMaxK + 1][kGmMaxK];
+  double g[kGmMaxK][kGmMaxK];  // V_i.V_l
+  double coef[kGmMaxK + 1];
+  double cs[kGmMaxK], sn[kGmMaxK], y[kGmMaxK + 1];
+  int bad, exit_now;
+};
+
+// v: 8 sums over the 64 lanes; the lane's sum is that of v[sum8_index()]
+__device__ inline int sum8_index() {
+  const int l = threadIdx.x;
+  return (l & 32 ? 4 : 0) + (l & 16 ? 2 : 0) + (l & 8 ? 1 : 0);
+}
+__device__ inline double sum8(const double (&v)[8]) {
+  const double a0 = fold<32>(v[0], v[4]), a1 = fold<32>(v[1], v[5]);
+  const double a2 = fold<32>(v[2], v[6]), a3 = fold<32>(v[3], v[7]);
+  double s = fold<8>(fold<16>(a0, a2), fold<16>(a1, a3));
+  s += dpp<kXor1>(s);
+  s += dpp<kXor2>(s);
+  return s + dpp<kHalfMirror>(s);
+}
+__device__ inline double lane_value(double v, int lane) {
+  const u64 b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)b, lane);
+  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+  return __longlong_as_double(((u64)hi << 32) | lo);
+}
+
+template <typename T, int R>
+__global__ void __launch_bounds__(kSlab)
+k_gmres_rows(RowArgs ra, const T* __restrict__ val, RowsGmres a, T* basis, T* hbasis,
+             GmState* st) {
+  constexpr bool kMixed = sizeof(T) == 4;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ GmLds sh;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int wg = blockIdx.x, gang = ra.nwg;
+  const bool lead = wg == 0 && t == 0;
+  unsigned e = __hip_atomic_load(ra.sy.epoch + ra.ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  auto leave = [&]() {
+    if (lead)
+      __hip_atomic_store(ra.sy.epoch + 1 - ra.ep, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  // (the lead writes `done` without a meeting only where every workgroup
+  // finds by itself that the solve has ended)
+  if (load_relaxed(ra.sy.abort) || (!a.first && load_relaxed(&st->done))) {
+    leave();
+    return;
+  }
+  const int r0 = ra.wg_row0[wg];
+  const uint16_t* rowpos = ra.rowpos + (size_t)wg * R * kSlab;
+  const int h0 = ra.halo_off[wg], nh = ra.halo_off[wg + 1] - h0;
+  const int x0 = ra.exp_off[wg], nx = ra.exp_off[wg + 1] - x0;
+  T* ds = reinterpret_cast<T*>(smem_raw);  // V_j: own rows, then halo
+  T* dh = ds + R * kSlab;
+  T* ah = dh + nh;                         // A V_j of the halo
+  T* as = ah + nh;                         // A V_j of own rows
+  // this thread's part of the scratch: V, A V (FP64) and the diagonal
+  const size_t vstride = (size_t)ra.nwg * R * kSlab, hstride = ra.nhalo;
+  T* vb = basis + (size_t)wg * R * kSlab + t;
+  T* avb = vb + (size_t)a.krylov * vstride;
+  T* dq = vb + (size_t)(kMixed ? 1 : 2) * a.krylov * vstride;
+  T* vh = hbasis + h0;
+  if (t == 0) sh.bad = 0;
+  __syncthreads();
+
+  auto total = [&](int s) {
+    return (sh.tot[4 * s] + sh.tot[4 * s + 1]) + (sh.tot[4 * s + 2] + sh.tot[4 * s + 3]);
+  };
+  // a meeting: n sums from the waves' sh.part[sum][wave], and with `halo` the
+  // exchange of `as` (into ah); false when it gave up
+  auto meet = [&](int n, bool halo) -> bool {
+    ++e;
+    __syncthreads();
+    u64* slots = ra.sy.slots + (size_t)(e & 1) * kReplicas * kGmSums * ra.nwg * 2;
+    u64* xch = ra.sy.xch + (size_t)(e & 1) * 2 * ra.nexp;
+    for (int s = wave; s < n; s += kRowWaves) {
+      const double v = sum16(sh.part[s * kRowWaves + (lane & 15)]);
+      if (gang == 1) {
+        if (lane < 4) sh.tot[4 * s + lane] = lane ? 0.0 : v;
+      } else if (lane < kReplicas) {
+        post(slots + ((size_t)(lane * kGmSums + s) * ra.nwg + wg) * 2, 1, e, v);
+      }
+    }
+    if (gang == 1) {
+      __syncthreads();
+      return true;
+    }
+    if (halo)
+      for (int i = t; i < nx; i += kSlab) post(xch + x0 + i, ra.nexp, e, as[ra.exp_loc[x0 + i]]);
+    // 256 threads per sum, one workgroup each, up to 16 sums at a time
+    const int sw = t & 255, sv = t >> 8;
+    bool ok = true;
+    for (int s0 = 0; s0 < n; s0 += 16) {
+      const u64* sp =
+          slots + ((size_t)((wg & (kReplicas - 1)) * kGmSums + s0 + sv) * ra.nwg + sw) * 2;
+      unsigned need = 0;
+      double p[4] = {};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (s0 + sv + 4 * i < n && sw < gang) need |= 1u << i;
+      Deadline dl = {ra.sy.ticks, ra.sy.abort};
+      while (need) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (need >> i & 1)
+            if (look(sp + (size_t)8 * i * ra.nwg, 1, e, p[i])) need &= ~(1u << i);
+        if (need && dl.past()) break;
+      }
+      ok = ok && !need;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (s0 + 4 * i < n) {
+          const double q = sum64(p[i]);
+          // (sum s0 + sv + 4 i; its waves are 4 sv .. 4 sv + 3)
+          if (lane == 0 && s0 + sv + 4 * i < n) sh.tot[(s0 + sv + 4 * i) * 4 + (wave & 3)] = q;
+        }
+    }
+    if (halo)
+      for (int h = t; h < nh && ok; h += kSlab) {
+        T v = (T)0;
+        Deadline dl = {ra.sy.ticks, ra.sy.abort};
+        while (!look(xch + ra.halo_src[h0 + h], ra.nexp, e, v))
+          if (dl.past()) {
+            ok = false;
+            break;
+          }
+        ah[h] = v;
+      }
+    if (!ok) sh.bad = 1;
+    __syncthreads();
+    if (sh.bad) {
+      if (t == 0) store_relaxed(ra.sy.abort, 1);
+      return false;
+    }
+    return true;
+  };
+  // one sum of val(k) over rows, as sum `s` of the next meeting
+  auto sum_rows = [&](int s, auto val1) {
+    double p = 0.0;
+#pragma unroll
+    for (int k = 0; k < R; ++k) p += val1(k);
+    p = sum64(p);
+    if (lane == 0) sh.part[s * kRowWaves + wave] = p;
+  };
+
+  RowProduct<T, R> prod;
+  auto product = [&]() {
+    prod.apply(ra, val, wg, ds, as);
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const T d = ds[k * kSlab + t];
+      as[k * kSlab + t] += a.diag ? dq[(size_t)k * kSlab] * d : d;
+    }
+  };
+  T rv[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    if constexpr (R >= 4) __builtin_amdgcn_sched_barrier(0);
+    const int p = rowpos[k * kSlab + t];
+    rv[k] = (T)0;
+    T xv = (T)0, d = (T)0;
+    if (p != 0xffff) {
+      if constexpr (!kMixed) {
+        rv[k] = a.b[r0 + p];
+        xv = a.x0[r0 + p];
+      }
+      if (a.diag) d = (T)a.diag[r0 + p];
+    }
+    if constexpr (!kMixed) ds[k * kSlab + t] = xv;
+    if (a.diag) dq[(size_t)k * kSlab] = d;
+    prod.load(ra, val, wg, k);
+  }
+  double nr0, nb;
+  int m = 0;
+  if constexpr (kMixed) {
+    // the sums of the residual's kernel and of ||b||^2
+    double p = 0.0, q = 0.0;
+    for (int i = t; i < a.npart_rr; i += kSlab) p += a.part_rr[i];
+    for (int i = t; i < a.npart_bb; i += kSlab) q += a.part_bb[i];
+    p = sum64(p);
+    q = sum64(q);
+    if (lane == 0) {
+      sh.part[wave] = p;
+      sh.part[kRowWaves + wave] = q;
+    }
+    __syncthreads();
+    nr0 = sqrt(sum16(sh.part[lane & 15]));
+    nb = sqrt(sum16(sh.part[kRowWaves + (lane & 15)]));
+    __syncthreads();
+    m = a.first ? 0 : load_relaxed(&st->m);
+  } else {
+    // R0 = A X - B, ||R0||^2, ||B||^2 (gmres.f:188-207)
+    for (int h = t; h < nh; h += kSlab) dh[h] = a.x0[ra.halo_row[h0 + h]];
+    __syncthreads();
+    product();
+    sum_rows(0, [&](int k) { return (double)rv[k] * (double)rv[k]; });
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      rv[k] = as[k * kSlab + t] - rv[k];
+      as[k * kSlab + t] = rv[k];
+    }
+    sum_rows(1, [&](int k) { return (double)rv[k] * (double)rv[k]; });
+    if (!meet(2, true)) return;
+    nb = sqrt(total(0));
+    nr0 = sqrt(total(1));
+  }
+  const int relat = nb < 1.0 ? 0 : 1;
+  if (nb < 1.0) nb = 1.0;
+  double prec = nr0 / nb;
+  int products = 0;
+  bool updated = false;
+  // the stop tests (gmres.f:207, :367)
+  bool stop = m == 0 ? prec <= a.eps : !(prec >= a.eps && m < a.nitmax);
+  const bool ran = !stop;
+  while (!stop) {
+    ++m;
+    // V_0 = -R0 / ||R0|| (gmres.f:243), halo included
+    if constexpr (kMixed) {
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        const int p = rowpos[k * kSlab + t];
+        const T v = p != 0xffff ? (T)(-1.0 / nr0 * a.r0[r0 + p]) : (T)0;
+        ds[k * kSlab + t] = vb[(size_t)k * kSlab] = v;
+      }
+      for (int h = t; h < nh; h += kSlab)
+        dh[h] = vh[h] = (T)(-1.0 / nr0 * a.r0[ra.halo_row[h0 + h]]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < R; ++k)
+        ds[k * kSlab + t] = vb[(size_t)k * kSlab] = (T)(-1.0 / nr0) * rv[k];
+      for (int h = t; h < nh; h += kSlab) dh[h] = vh[h] = (T)(-1.0 / nr0) * ah[h];
+    }
+    __syncthreads();
+    int kk = a.krylov;
+    for (int j = 0; j < kk; ++j) {
+      product();
+      if constexpr (!kMixed) {
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+          avb[j * vstride + (size_t)k * kSlab] = as[k * kSlab + t];
+      }
+      // sums 2 q and 2 q + 1: w.V_q and V_j.V_q; w.w follows
+      for (int q0 = 0; q0 < j + 2; q0 += 4) {
+        double v[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int q = q0 + i;
+          double pw = 0.0, pd = 0.0;
+          if (q < j) {
+            T b[R];
+#pragma unroll
+            for (int k = 0; k < R; ++k) b[k] = vb[q * vstride + (size_t)k * kSlab];
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+              pw += (double)as[k * kSlab + t] * (double)b[k];
+              pd += (double)ds[k * kSlab + t] * (double)b[k];
+            }
+          } else if (q == j) {
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+              const double d = (double)ds[k * kSlab + t];
+              pw += (double)as[k * kSlab + t] * d;
+              pd += d * d;
+            }
+          } else if (q == j + 1) {
+#pragma unroll
+            for (int k = 0; k < R; ++k) {
+              const double w = (double)as[k * kSlab + t];
+              pw += w * w;
+            }
+          }
+          v[2 * i] = pw;
+          v[2 * i + 1] = pd;
+        }
+        const double s = sum8(v);
+        const int i = 2 * q0 + sum8_index();
+        if ((lane & 7) == 0 && i < 2 * j + 3) sh.part[i * kRowWaves + wave] = s;
+      }
+      const bool last = j == a.krylov - 1;
+      if (!meet(2 * j + 3, !last)) return;
+      // every wave for itself: lane q <= j has w.V_q and row q of V.V
+      const double c = lane <= j ? total(2 * lane) : 0.0;
+      const double ww = total(2 * j + 2);
+      double hq = c;
+      if (lane <= j) sh.g[j][lane] = sh.g[lane][j] = total(2 * lane + 1);
+      const double* grow = sh.g[min(lane, j)];
+      // K-th column (gmres.f:285-296): H(I,K) = w.V_I, H(K+1,K) by Pythagoras
+      bool reduced = last;
+      if (!last) {
+        for (int l = 0; l < j; ++l) {
+          const double hl = lane_value(hq, l);
+          if (lane > l && lane <= j) hq -= hl * grow[l];
+        }
+        double gh = 0.0;
+        for (int l = 0; l <= j; ++l) gh += lane_value(hq, l) * grow[l];
+        double n2 = ww + sum64(lane <= j ? hq * (gh - 2.0 * c) : 0.0);
+        if (lane <= j) sh.coef[lane] = hq;
+        T w[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) w[k] = as[k * kSlab + t] - (T)sh.coef[j] * ds[k * kSlab + t];
+        for (int q = 0; q < j; ++q) {
+          const T hc = (T)sh.coef[q];
+#pragma unroll
+          for (int k = 0; k < R; ++k) w[k] -= hc * vb[q * vstride + (size_t)k * kSlab];
+        }
+        if (!(n2 > kTrust * ww)) {
+          sum_rows(0, [&](int k) { return (double)w[k] * (double)w[k]; });
+          if (!meet(1, false)) return;
+          n2 = total(0);
+        }
+        const double r = sqrt(n2);
+        if (r < 1e-20) {
+          // reduction of the Krylov space (gmres.f:274-283)
+          reduced = true;
+          kk = j + 1;
+          ++products;
+        } else {
+          if (wave == 0 && lane <= j) sh.h[lane][j] = hq;
+          if (t == 0) sh.h[j + 1][j] = r;
+          const double s = 1.0 / r;
+#pragma unroll
+          for (int k = 0; k < R; ++k) {
+            const T v = (T)(s * (double)w[k]);
+            ds[k * kSlab + t] = vb[(j + 1) * vstride + (size_t)k * kSlab] = v;
+          }
+          for (int h = t; h < nh; h += kSlab) {
+            T v = ah[h] - (T)sh.coef[j] * dh[h];
+            for (int q = 0; q < j; ++q) v -= (T)sh.coef[q] * vh[q * hstride + h];
+            dh[h] = vh[(j + 1) * hstride + h] = (T)(s * (double)v);
+          }
+          __syncthreads();
+        }
+      }
+      if (reduced) {
+        if (wave == 0 && lane <= j) sh.h[lane][j] = c;
+        if (t == 0) {
+          double hk = ww;
+          for (int q = 0; q <= j; ++q) hk -= sh.h[q][j] * sh.h[q][j];
+          sh.h[j + 1][j] = sqrt(max(hk, 0.0));
+        }
+      }
+    }
+    // (steps past a reduction count: the host-driven solver runs them too)
+    products += a.krylov;
+    // Givens rotations and H y = e (gmres.f:304-350)
+    if (t == 0) {
+      auto& h = sh.h;
+      double* y = sh.y;
+      y[0] = nr0;
+      int ex = 0;
+      for (int i = 0; i < kk; ++i) {
+        for (int j = 0; j < i; ++j) {
+          const double zz = sh.cs[j] * h[j][i] + sh.sn[j] * h[j + 1][i];
+          h[j + 1][i] = -sh.sn[j] * h[j][i] + sh.cs[j] * h[j + 1][i];
+          h[j][i] = zz;
+        }
+        const double rr = sqrt(h[i][i] * h[i][i] + h[i + 1][i] * h[i + 1][i]);
+        if (fabs(rr) < 1e-6) {
+          ex = 1;
+          break;
+        }
+        sh.cs[i] = h[i][i] / rr;
+        sh.sn[i] = h[i + 1][i] / rr;
+        h[i][i] = rr;
+        y[i + 1] = -sh.sn[i] * y[i];
+        y[i] = sh.cs[i] * y[i];
+      }
+      if (!ex)
+        for (int j = kk - 1; j >= 0; --j) {
+          double v = y[j];
+          for (int l = j + 1; l < kk; ++l) v -= h[j][l] * y[l];
+          y[j] = v / h[j][j];
+        }
+      sh.exit_now = ex;
+    }
+    __syncthreads();
+    if (sh.exit_now) {
+      stop = true;
+      break;
+    }
+    // X += sum y_l V_l, R0 += sum y_l A V_l (gmres.f:354-359)
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const int p = rowpos[k * kSlab + t];
+      double xv = p == 0xffff ? 0.0 : a.first && !updated ? a.x0[r0 + p] : a.x[r0 + p];
+#pragma unroll 2
+      for (int l = 0; l < kk; ++l) {
+        const double yl = sh.y[l];
+        xv += yl * (double)vb[l * vstride + (size_t)k * kSlab];
+        if constexpr (!kMixed) rv[k] += yl * avb[l * vstride + (size_t)k * kSlab];
+      }
+      if (p != 0xffff) a.x[r0 + p] = xv;
+    }
+    updated = true;
+    if constexpr (kMixed) break;
+    nr0 = fabs(sh.y[kk]);
+    prec = nr0 / nb;
+    stop = !(prec >= a.eps && m < a.nitmax);
+    if (!stop) {
+      // R0 of the halo, and ||R0|| itself: |E(K+1)| is it up to rounding that
+      // grows by ||R0||^2 / |E(K+1)|^2 each cycle if V_0 is divided by it
+#pragma unroll
+      for (int k = 0; k < R; ++k) as[k * kSlab + t] = rv[k];
+      sum_rows(0, [&](int k) { return (double)rv[k] * (double)rv[k]; });
+      if (!meet(1, true)) return;
+      nr0 = sqrt(total(0));
+      prec = nr0 / nb;
+      stop = !(prec >= a.eps);
+    }
+  }
+  if (lead) {
+    st->prec = prec;
+    st->relat = relat;
+    if (ran || a.first) {
+      store_relaxed(&st->m, m);
+      st->products = (a.first ? 0 : st->products) + products;
+      st->updated = updated || (!a.first && st->updated);
+    }
+    store_relaxed(&st->done, stop ? 1 : 0);
+  }
+  leave();
 }
 
 // ---------------------------------------------------------------------------
@@ -813,8 +1278,14 @@ struct RowsDev {
   Buf<double> v64;
   Buf<float> v32;
   Buf<u64> words;
-  SyncWords sy[2];  // FP64, FP32
-  int ep[2] = {0, 0};
+  SyncWords sy[3];  // CG FP64, CG FP32, GMRES
+  int ep[3] = {0, 0, 0};
+  // GMRES: fits (FP64, FP32), scratch for a basis of gm_k vectors
+  bool gm_fits[2] = {false, false};
+  int nhalo = 0;
+  Buf<unsigned char> gm, gmh;
+  size_t gm_bytes = 0, gmh_bytes = 0;
+  GmState* gm_state = nullptr;
 };
 
 static size_t cg_lds(const RowsDev& r, int bytes) {
@@ -853,6 +1324,39 @@ static hipError_t cg_fits(const RowsDev& r, int lds_max, bool* fits) {
   return hipSuccess;
 }
 
+static size_t gm_lds(const RowsDev& r, int bytes) {
+  // V_j and A V_j of own rows and of the halo
+  return (size_t)2 * (r.group * kSlab + r.max_halo) * bytes;
+}
+
+template <typename T, typename F>
+static hipError_t with_gm_kernel(int group, F&& f) {
+  switch (group) {
+    case 1: return f(&k_gmres_rows<T, 1>);
+    case 2: return f(&k_gmres_rows<T, 2>);
+    case 4: return f(&k_gmres_rows<T, 4>);
+    default: return f(&k_gmres_rows<T, 8>);
+  }
+}
+
+template <typename T>
+static hipError_t gm_fits(const RowsDev& r, int lds_max, bool* fits) {
+  const size_t lds = gm_lds(r, sizeof(T));
+  lds_max -= (int)((sizeof(GmLds) + 1023) / 1024 * 1024);
+  *fits = lds_max > 0 && lds <= (size_t)lds_max && r.nsys == 1 && r.nwg <= r.ncu;
+  if (!*fits) return hipSuccess;
+  return with_gm_kernel<T>(r.group, [&](auto kern) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_max);
+    int nb = 0;
+    if (e == hipSuccess)
+      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(kern),
+                                                       kSlab, lds);
+    *fits = nb >= 1;
+    return e;
+  });
+}
+
 RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStream_t stream,
                      hipError_t* err) {
   *err = hipSuccess;
@@ -886,6 +1390,9 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
   if ((*err = cg_fits<double>(*r, lds_max, &fits)) != hipSuccess) return nullptr;
   if ((*err = cg_fits<float>(*r, lds_max, &fits)) != hipSuccess) return nullptr;
   if (!fits) return nullptr;
+  if ((*err = gm_fits<double>(*r, r->lds_max, &r->gm_fits[0])) != hipSuccess) return nullptr;
+  if ((*err = gm_fits<float>(*r, r->lds_max, &r->gm_fits[1])) != hipSuccess) return nullptr;
+  r->nhalo = (int)R.halo_row.size();
   auto ok = [&](hipError_t e) {
     if (e != hipSuccess) *err = e;
     return e == hipSuccess;
@@ -910,23 +1417,36 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
       !ok(r->exp_loc.put(R.exp_loc, stream)) || !ok(r->ref_end.put(R.ref_end, stream)) ||
       !ok(r->ref_off.put(R.ref_off, stream)) || !ok(r->v64.alloc(r->nent)))
     return nullptr;
-  // sync words: per precision sums and exchange, then the counters
-  const size_t nslot = (size_t)2 * kReplicas * kSums * R.nwg * 2, nexp = R.exp_loc.size();
+  // sync words of CG in both precisions and of GMRES: sums, exchange, then
+  // the counters
+  const bool gm = r->gm_fits[0] || r->gm_fits[1];
+  const size_t nexp = R.exp_loc.size();
   const size_t nepoch = (2 * (size_t)nsys + 1) / 2 + 1;  // in 64-bit words
-  const size_t one = nslot + 4 * nexp + nepoch + 2;
-  if (!ok(r->words.alloc(2 * one))) return nullptr;
+  const size_t tail = 4 * nexp + nepoch + 2 + (sizeof(GmState) + 7) / 8;
+  const size_t nslot[3] = {(size_t)2 * kReplicas * kSums * R.nwg * 2,
+                           (size_t)2 * kReplicas * kSums * R.nwg * 2,
+                           gm ? (size_t)2 * kReplicas * kGmSums * R.nwg * 2 : 0};
+  const size_t nwords = nslot[0] + nslot[1] + nslot[2] + 3 * tail;
+  if (!ok(r->words.alloc(nwords))) return nullptr;
   u64 ticks = kWaitTicks;
   if (const char* ev = getenv("BHIP_ROWS_WAIT")) ticks = strtoull(ev, nullptr, 10);
-  for (int k = 0; k < 2; ++k) {
-    u64* p = r->words.p + k * one;
-    r->sy[k].slots = p;
-    r->sy[k].xch = p + nslot;
-    r->sy[k].epoch = reinterpret_cast<unsigned*>(p + nslot + 4 * nexp);
-    r->sy[k].abort = reinterpret_cast<int*>(p + one - 2);
-    r->sy[k].ticket = reinterpret_cast<unsigned*>(p + one - 1);
-    r->sy[k].ticks = ticks;
+  u64* p = r->words.p;
+  for (int k = 0; k < 3; ++k) {
+    SyncWords& s = r->sy[k];
+    s.slots = p;
+    s.xch = (p += nslot[k]);
+    s.epoch = reinterpret_cast<unsigned*>(p += 4 * nexp);
+    s.ticket = reinterpret_cast<unsigned*>(p += nepoch);
+    s.abort = reinterpret_cast<int*>(p += 1);
+    s.ticks = ticks;
+    p += 1;
+    if (k == 2) {
+      r->gm_state = reinterpret_cast<GmState*>(p);
+      s.abort = &r->gm_state->gave_up;
+    }
+    p += (sizeof(GmState) + 7) / 8;
   }
-  hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, stream, r->words.p, (long)(2 * one));
+  hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, stream, r->words.p, (long)nwords);
   if (!ok(hipGetLastError()) || !ok(hipStreamSynchronize(stream))) return nullptr;
   return r.release();
 }
@@ -995,6 +1515,7 @@ static RowArgs row_args(const RowsDev* r, int k) {
   a.nwg = r->nwg;
   a.nsys = r->nsys;
   a.nexp = r->nexp;
+  a.nhalo = r->nhalo;
   a.sy = r->sy[k];
   a.ep = r->ep[k];
   a.ticketed = r->nwg > r->ncu;
@@ -1022,5 +1543,50 @@ hipError_t rows_cg(RowsDev* r, const RowsCg<T>& a, hipStream_t stream) {
 }
 template hipError_t rows_cg<double>(RowsDev*, const RowsCg<double>&, hipStream_t);
 template hipError_t rows_cg<float>(RowsDev*, const RowsCg<float>&, hipStream_t);
+
+bool rows_gmres_fits(const RowsDev* r, int bytes) { return r->gm_fits[bytes == 4]; }
+
+template <typename T>
+hipError_t rows_gmres(RowsDev* r, const RowsGmres& a, hipStream_t stream) {
+  if (a.krylov < 1 || a.krylov > kGmMaxK) return hipErrorInvalidValue;
+  // V, A V (FP64 only) and the diagonal of own rows; V of the halo
+  const size_t own = (size_t)r->nwg * r->group * kSlab * sizeof(T) *
+                     ((sizeof(T) == 8 ? 2 : 1) * a.krylov + 1);
+  const size_t halo = (size_t)std::max(r->nhalo, 1) * sizeof(T) * a.krylov;
+  auto grow = [&](Buf<unsigned char>& b, size_t& have, size_t want) -> hipError_t {
+    if (have >= want) return hipSuccess;
+    if (b.p) {
+      const hipError_t e = hipFree(b.p);
+      b.p = nullptr;
+      have = 0;
+      if (e != hipSuccess) return e;
+    }
+    const hipError_t e = b.alloc(want);
+    if (e == hipSuccess) have = want;
+    return e;
+  };
+  hipError_t e = grow(r->gm, r->gm_bytes, own);
+  if (e == hipSuccess) e = grow(r->gmh, r->gmh_bytes, halo);
+  if (e != hipSuccess) return e;
+  const RowArgs ra = row_args(r, 2);
+  r->ep[2] ^= 1;
+  const T* val;
+  if constexpr (sizeof(T) == 8)
+    val = r->v64.p;
+  else
+    val = r->v32.p;
+  return with_gm_kernel<T>(r->group, [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(r->nwg), dim3(kSlab), gm_lds(*r, sizeof(T)), stream, ra, val, a,
+                       reinterpret_cast<T*>(r->gm.p), reinterpret_cast<T*>(r->gmh.p),
+                       r->gm_state);
+    return hipGetLastError();
+  });
+}
+template hipError_t rows_gmres<double>(RowsDev*, const RowsGmres&, hipStream_t);
+template hipError_t rows_gmres<float>(RowsDev*, const RowsGmres&, hipStream_t);
+
+hipError_t rows_gmres_state(const RowsDev* r, GmState* host, hipStream_t stream) {
+  return hipMemcpyAsync(host, r->gm_state, sizeof(GmState), hipMemcpyDeviceToHost, stream);
+}
 
 }  // namespace bhip

@@ -62,4 +62,32 @@ struct RowsCg {
 template <typename T>
 hipError_t rows_cg(RowsDev* r, const RowsCg<T>& a, hipStream_t stream);
 
+// Restarted GMRES (gmres.f:171-372) of a context of one system: FP64, the
+// whole solve in one launch; FP32, one cycle of the mixed solve from the FP64
+// residual r0 (nothing where the stop test on it ends the solve). Vectors in
+// internal node order.
+struct GmState {  // on the device, written by a launch
+  double prec;    // ||R0|| / max(||B||, 1)
+  int m, products, done, relat;
+  int updated;    // x has been written
+  int gave_up;    // a launch gave up waiting for its workgroups (never reset)
+};
+struct RowsGmres {
+  const double* x0;  // initial solution
+  double* x;         // solution, if updated (not x0: see RowsCg)
+  const double* diag;  // diagonal, or nullptr for a unit diagonal
+  const double* b;     // FP64
+  const double* r0;    // FP32: A x - b, and the partial sums of r0.r0 and b.b
+  const double* part_rr;
+  const double* part_bb;
+  int npart_rr, npart_bb;
+  double eps;
+  int nitmax, krylov;
+  int first;           // first launch of the solve
+};
+bool rows_gmres_fits(const RowsDev* r, int bytes);
+template <typename T>
+hipError_t rows_gmres(RowsDev* r, const RowsGmres& a, hipStream_t stream);
+hipError_t rows_gmres_state(const RowsDev* r, GmState* host, hipStream_t stream);
+
 }  // namespace bhip

@@ -1,11 +1,12 @@
-"""CG on assembled rows (one persistent launch per solve): the sizes where its
+"""CG and GMRES on assembled rows (one persistent launch per solve): the sizes where its
 partition changes, against the oracle, and the path it falls back to.
 
 Tolerances: FP64 solves to eps 1e-10 differ from the oracle's by rounding that
 CG amplifies, 1e-10 of the solution as in the other solve tests; a mixed solve
 and the oracle both stop at a relative residual of eps 1e-9, so their
 solutions agree within the condition number of the scaled system (under 100
-for these time steps) times that, 1e-7."""
+for these time steps) times that, 1e-7. GMRES likewise: 2e-8 in FP64 (eps 1e-10
+on both sides), 2e-7 mixed (eps 1e-9)."""
 import numpy as np
 import pytest
 import torch
@@ -152,3 +153,68 @@ def test_a_launch_that_gives_up_falls_back(gpu, monkeypatch):
     monkeypatch.setenv("BHIP_ROWS_WAIT", "0")
     got = _check(m, sysd)
     assert np.linalg.norm(got[0] - want[0]) <= 1e-10 * np.linalg.norm(want[0])
+
+
+def _check_gmres(m, sysd, krylov, precon=2, typext="S", block_nodes=0, seed=1):
+    rng = np.random.default_rng(seed)
+    b = sysd["b"] + 1e-2 * rng.normal(size=m.npoin)
+    xa = sysd["xa"]
+    if typext == "Q":
+        # not symmetric, still diagonally dominant
+        xa = np.concatenate([sysd["xa"], 0.5 * sysd["xa"]])
+    A = O.Matrix(sysd["da"], None if typext == "0" else xa, "Q", typext)
+    for prec, eps, tol in ((bief.PREC_FP64, 1e-10, 2e-8), (bief.PREC_MIXED, 1e-9, 2e-7)):
+        if krylov == 1:
+            # the oracle's residual estimate ||A V||^2 - H^2 loses all its
+            # digits below 1e-9 here (its relres is then 0)
+            eps, tol = 1e-8, 2e-6
+        kw = dict(slv=7, precon=precon, eps=eps, nitmax=400, krylov=krylov)
+        xr, ir, _, _ = O.solve(A, m.ikle, b, sysd["x0"], **kw)
+        ctx = bief.Context(m, block_nodes=block_nodes)
+        ctx.set_matrix("Q", typext, sysd["da"], None if typext == "0" else xa)
+        x, info = ctx.solve(sysd["x0"].copy(), b.copy(), precision=prec, **kw)
+        assert info["converged"], (prec, info)
+        if prec == bief.PREC_FP64:
+            assert abs(info["niter"] - ir.niter) <= 1, (info, ir.niter)
+        assert np.linalg.norm(x - xr) <= tol * np.linalg.norm(xr), (prec, info)
+        ctx.close()
+
+
+# one workgroup; several; 2, 4 and 8 slabs each
+@pytest.mark.parametrize("nx,ny,krylov", [(1, 1, 2), (30, 32, 5), (120, 90, 1), (120, 90, 2),
+                                          (120, 90, 20), (514, 510, 5), (730, 719, 3),
+                                          (1030, 1020, 3)])
+def test_rows_gmres_at_partition_edges(gpu, nx, ny, krylov):
+    m = M.channel_mesh(nx, ny, 10.0 * nx, 10.0 * ny)
+    _check_gmres(m, _system(m), krylov)
+
+
+@pytest.mark.parametrize("block_nodes", [300, 1024])
+@pytest.mark.parametrize("precon", [0, 2, 5])
+@pytest.mark.parametrize("typext", ["S", "Q"])
+def test_rows_gmres_with_a_diagonal(gpu, precon, typext, block_nodes):
+    m = M.random_small_mesh(70, 61, seed=3)
+    _check_gmres(m, S.wave_system(m, 2.0 + m.x / 10.0, dt=0.3), 6, precon=precon, typext=typext,
+                 block_nodes=block_nodes)
+
+
+def test_rows_gmres_reduces_the_krylov_space(gpu):
+    """The unit matrix and a right-hand side whose norm is a power of two: A V_1
+    is V_1 to the bit, so the cycle stops at one vector."""
+    m = M.random_small_mesh(40, 31, seed=5)
+    b = np.zeros(m.npoin)
+    b[[3, 400, 800, 1200]] = 8.0
+    for prec in (bief.PREC_FP64, bief.PREC_MIXED):
+        ctx = bief.Context(m)
+        ctx.set_matrix("Q", "0", np.ones(m.npoin), None)
+        x, info = ctx.solve(np.zeros(m.npoin), b.copy(), slv=7, precon=0, eps=1e-10, nitmax=9,
+                            krylov=4, precision=prec)
+        assert info["converged"] and info["niter"] == 1 and info["relres"] == 0.0, info
+        assert np.array_equal(x, b)
+        ctx.close()
+
+
+def test_a_gmres_launch_that_gives_up_falls_back(gpu, monkeypatch):
+    monkeypatch.setenv("BHIP_ROWS_WAIT", "0")
+    m = M.channel_mesh(120, 90, 1200.0, 900.0)
+    _check_gmres(m, _system(m), 5)
