@@ -2761,14 +2761,70 @@ __global__ void k_geo_slots(double* __restrict__ geo, const double* __restrict__
   }
 }
 
+// Sums of NV terms per corner of the block's slots onto its owned nodes, in LDS
+// (acc: [NV][nown], zeroed; valid after the call): terms(s) gives slot s's.
+// Slots are taken a workgroup at a time, their terms computed side by side and
+// kept in registers; only the additions run colour by colour, a barrier after
+// each, so a node's terms are added in the order of its colours whatever the
+// workgroup's size. (With each colour's terms computed in its turn, 10 to 12
+// times per block, a chain of three loads stood alone before each barrier.)
+//
+// us before -> now: MT03AA/MT04AA/MT05AA (k_elem_supg) 57 -> 41 at 500k nodes, 41
+// -> 21 at 90k; MT01AA/MT02AA (k_elem_tri) 43 -> 27 and 36 -> 16; the wave step's
+// kernels at 100k nodes 26 -> 16 (k_wave_grad), 26 -> 20 (k_wave_assemble), 48 ->
+// 34 (its adjoint). Few blocks: bound by the chains of loads of two or three
+// rounds, so as many threads as there are; where the blocks fill the GPU, by
+// the gathers of node values, and two blocks of 512 per CU overlap one's
+// additions with the other's loads (500k nodes, k_elem_supg: 41, with 1024
+// threads 48, with 256 51).
+constexpr int kElemThreads = 1024;
+static dim3 elem_threads(const Layout& L) {
+  return dim3(L.nblocks <= 256 ? kElemThreads : kElemThreads / 2);
+}
+template <int NV>
+struct NodeTerms {
+  int l[3];  // local node ids; owned nodes come first
+  double c[NV][3];
+};
+template <int NV, typename F>
+__device__ inline void colour_sum(const int32_t* __restrict__ co, int nown, double* acc,
+                                  F&& terms) {
+  // lane c holds the colour boundary c
+  static_assert(kMaxColors < 64, "one lane per boundary");
+  const int lane = threadIdx.x & 63;
+  const int bound = co[min(lane, kMaxColors)];
+  const int send = __builtin_amdgcn_readlane(bound, kMaxColors);
+  int col = 0;
+  for (int w0 = __builtin_amdgcn_readlane(bound, 0); w0 < send; w0 += (int)blockDim.x) {
+    const int w1 = min(w0 + (int)blockDim.x, send), s = w0 + (int)threadIdx.x;
+    NodeTerms<NV> v;
+    if (s < w1) v = terms(s);
+    for (;;) {
+      const int c0 = __builtin_amdgcn_readlane(bound, col);
+      const int c1 = __builtin_amdgcn_readlane(bound, col + 1);
+      if (s < w1 && s >= c0 && s < c1) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          if (v.l[k] < nown) {
+#pragma unroll
+            for (int q = 0; q < NV; ++q) acc[q * nown + v.l[k]] += v.c[q][k];
+          }
+      }
+      __syncthreads();
+      if (c1 > w1) break;  // the rest of this colour is in the next window
+      ++col;
+      if (c1 == w1) break;
+    }
+  }
+}
+
 // Element matrices per slot (each element instance computes the same values)
-// and the assembly of their diagonal terms onto owned nodes in LDS, colour
-// by colour (same deterministic scheme as the mat-vec).
+// and the assembly of their diagonal terms onto owned nodes (colour_sum).
 //   kind 100: MT01AA mass (mt01aa.f:83-106)
 //   kind 1  : MT02AA P1 isotropic viscosity (mt02aa.f:247-290)
 //   kind 2  : MT02AA 'UV' (mt02aa.f:200-240)
 // accumulate: OM 'M=M+N' (else 'M=N').
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kElemThreads)
 k_elem_tri(int kind, double xmul, const double* __restrict__ surfac,
            const double* __restrict__ xel, const double* __restrict__ yel, int nelem,
            const double* __restrict__ u_int, const double* __restrict__ v_int,
@@ -2780,72 +2836,66 @@ k_elem_tri(int kind, double xmul, const double* __restrict__ surfac,
            const double* __restrict__ geo) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   double* acc = reinterpret_cast<double*>(smem_raw);
-  const int b = blockIdx.x;
-  if (b >= nblocks) return;
+  const int b = xcd_block(blockIdx.x, nblocks);
   const int n0 = node_start[b], nown = node_start[b + 1] - n0;
   const int h0 = halo_start[b];
   for (int l = threadIdx.x; l < nown; l += blockDim.x) acc[l] = 0.0;
   __syncthreads();
   const int32_t* co = color_off + (size_t)b * (kMaxColors + 1);
-  const int send = co[kMaxColors];
-  for (int c = 0; c < kMaxColors; ++c) {
-    const int s0 = co[c];
-    if (s0 >= send) break;
-    const int s1 = co[c + 1];
-    for (int s = s0 + threadIdx.x; s < s1; s += blockDim.x) {
-      const int e = slot_elem[s];
-      int l[3], g[3];
+  colour_sum<1>(co, nown, acc, [&](int s) {
+    const int e = slot_elem[s];
+    NodeTerms<1> nt;
+    int(&l)[3] = nt.l;
+    int g[3];
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        l[k] = lid[(size_t)k * nslot_pad + s];
-        g[k] = l[k] < nown ? n0 + l[k] : halo[h0 + l[k] - nown];
-      }
-      const SlotGeo G = load_geo(geo, nslot_pad, s, xel, yel, surfac, nelem, e, kind != 100);
-      double a12, a13, a23, t1, t2, t3;
-      if (kind == 100) {
-        const double det = G.s * (xmul / 12.0);
-        a12 = a13 = a23 = det;
-        t1 = t2 = t3 = det + det;
-      } else {
-        const double x2 = G.x2, x3 = G.x3;
-        const double y2 = G.y2, y3 = G.y3;
-        if (kind == 2) {
-          const double g1 = v_int[g[0]], g2 = v_int[g[1]], g3 = v_int[g[2]];
-          const double coef1 = (xmul / 48.0) / G.s;
-          const double g123 = g1 + g2 + g3;
-          const double coef2 = u_int[g[0]] * (g1 + g123) + u_int[g[1]] * (g2 + g123) +
-                               u_int[g[2]] * (g3 + g123);
-          a12 = (y3 * (y2 - y3) + x3 * (x2 - x3)) * coef2 * coef1;
-          a13 = -(y2 * (y2 - y3) + x2 * (x2 - x3)) * coef2 * coef1;
-          a23 = -(y2 * y3 + x2 * x3) * coef2 * coef1;
-        } else {
-          const double somvx = (u_int[g[0]] + u_int[g[1]] + u_int[g[2]]) * (xmul / 12.0) /
-                               G.s;
-          const double x2x3 = x2 * x3 + y2 * y3;
-          const double x2aux = x2 * (-x2 + x3) + y2 * (-y2 + y3);
-          const double x3aux = x3 * (-x2 + x3) + y3 * (-y2 + y3);
-          a12 = -somvx * x3aux;
-          a13 = somvx * x2aux;
-          a23 = -somvx * x2x3;
-        }
-        t1 = -a12 - a13;
-        t2 = -a12 - a23;
-        t3 = -a13 - a23;
-      }
-      // a symmetric element matrix; into a non-symmetric ('Q') target it
-      // goes to both halves (OM 'M=M+N' of an 'S' N into a 'Q' M)
-      const double av[3] = {a12, a13, a23};
-      for (int cc = 0; cc < (target_q ? 6 : 3); ++cc) {
-        double* p = xa + (size_t)cc * nslot_pad + s;
-        *p = accumulate ? *p + av[cc % 3] : av[cc % 3];
-      }
-      const double tk[3] = {t1, t2, t3};
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-        if (l[k] < nown) acc[l[k]] += tk[k];
+    for (int k = 0; k < 3; ++k) {
+      l[k] = lid[(size_t)k * nslot_pad + s];
+      g[k] = l[k] < nown ? n0 + l[k] : halo[h0 + l[k] - nown];
     }
-    __syncthreads();
-  }
+    const SlotGeo G = load_geo(geo, nslot_pad, s, xel, yel, surfac, nelem, e, kind != 100);
+    double a12, a13, a23, t1, t2, t3;
+    if (kind == 100) {
+      const double det = G.s * (xmul / 12.0);
+      a12 = a13 = a23 = det;
+      t1 = t2 = t3 = det + det;
+    } else {
+      const double x2 = G.x2, x3 = G.x3;
+      const double y2 = G.y2, y3 = G.y3;
+      if (kind == 2) {
+        const double g1 = v_int[g[0]], g2 = v_int[g[1]], g3 = v_int[g[2]];
+        const double coef1 = (xmul / 48.0) / G.s;
+        const double g123 = g1 + g2 + g3;
+        const double coef2 = u_int[g[0]] * (g1 + g123) + u_int[g[1]] * (g2 + g123) +
+                             u_int[g[2]] * (g3 + g123);
+        a12 = (y3 * (y2 - y3) + x3 * (x2 - x3)) * coef2 * coef1;
+        a13 = -(y2 * (y2 - y3) + x2 * (x2 - x3)) * coef2 * coef1;
+        a23 = -(y2 * y3 + x2 * x3) * coef2 * coef1;
+      } else {
+        const double somvx = (u_int[g[0]] + u_int[g[1]] + u_int[g[2]]) * (xmul / 12.0) /
+                             G.s;
+        const double x2x3 = x2 * x3 + y2 * y3;
+        const double x2aux = x2 * (-x2 + x3) + y2 * (-y2 + y3);
+        const double x3aux = x3 * (-x2 + x3) + y3 * (-y2 + y3);
+        a12 = -somvx * x3aux;
+        a13 = somvx * x2aux;
+        a23 = -somvx * x2x3;
+      }
+      t1 = -a12 - a13;
+      t2 = -a12 - a23;
+      t3 = -a13 - a23;
+    }
+    // a symmetric element matrix; into a non-symmetric ('Q') target it
+    // goes to both halves (OM 'M=M+N' of an 'S' N into a 'Q' M)
+    const double av[3] = {a12, a13, a23};
+    for (int cc = 0; cc < (target_q ? 6 : 3); ++cc) {
+      double* p = xa + (size_t)cc * nslot_pad + s;
+      *p = accumulate ? *p + av[cc % 3] : av[cc % 3];
+    }
+    nt.c[0][0] = t1;
+    nt.c[0][1] = t2;
+    nt.c[0][2] = t3;
+    return nt;
+  });
   for (int l = threadIdx.x; l < nown; l += blockDim.x) {
     if (accumulate)
       da[n0 + l] += acc[l];
@@ -3444,7 +3494,7 @@ static int elem_common(bhip_ctx* c, int kind, double xmul, const double* xel, co
     if (v && !(dV = node_in(c, 1, v))) return BHIP_EDEVICE;
   }
   const size_t lds = (size_t)L.max_owned * sizeof(double);
-  hipLaunchKernelGGL(k_elem_tri, dim3(L.nblocks), dim3(kThreads), lds, c->stream, kind, xmul,
+  hipLaunchKernelGGL(k_elem_tri, dim3(L.nblocks), elem_threads(L), lds, c->stream, kind, xmul,
                      dS.p, dX.p, dY.p, ne, dU, v ? dV : dU, c->slot_elem.p, c->lid.p,
                      L.nslot_pad, c->node_start.p, c->halo_start.p, c->halo.p, c->color_off.p,
                      L.nblocks, c->xa.p, c->da.p, accumulate, target_q,

@@ -11,9 +11,8 @@
 //
 // Each slot computes its element's 3x3 matrix (every instance of an element
 // computes the same values), writes the off-diagonal terms into the slot
-// matrix and assembles the diagonal onto owned nodes in LDS, colour by
-// colour (the deterministic scheme of the mat-vec). Element formulas keep
-// the reference's order of operations.
+// matrix and assembles the diagonal onto owned nodes in LDS in colour order
+// (colour_sum). Element formulas keep the reference's order of operations.
 
 namespace bhip {
 
@@ -79,7 +78,7 @@ struct SupgArgs {
   int target_q;  // the target matrix stores 6 columns
 };
 
-__global__ void __launch_bounds__(kThreads) k_elem_supg(SupgArgs a) {
+__global__ void __launch_bounds__(kElemThreads) k_elem_supg(SupgArgs a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   double* acc = reinterpret_cast<double*>(smem_raw);
   const int b = xcd_block(blockIdx.x, a.nblocks);
@@ -88,149 +87,144 @@ __global__ void __launch_bounds__(kThreads) k_elem_supg(SupgArgs a) {
   for (int l = threadIdx.x; l < nown; l += blockDim.x) acc[l] = 0.0;
   __syncthreads();
   const int32_t* co = a.color_off + (size_t)b * (kMaxColors + 1);
-  const int send = co[kMaxColors];
   const size_t np = a.nslot_pad, ne = a.nelem;
-  for (int col = 0; col < kMaxColors; ++col) {
-    const int s0 = co[col];
-    if (s0 >= send) break;
-    const int s1 = co[col + 1];
-    for (int s = s0 + threadIdx.x; s < s1; s += blockDim.x) {
-      const int e = a.slot_elem[s];
-      int l[3], g[3];
+  colour_sum<1>(co, nown, acc, [&](int s) {
+    const int e = a.slot_elem[s];
+    NodeTerms<1> nt;
+    int(&l)[3] = nt.l;
+    int g[3];
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        l[k] = a.lid[(size_t)k * np + s];
-        g[k] = l[k] < nown ? n0 + l[k] : a.halo[hb + l[k] - nown];
-      }
-      const SlotGeo G = load_geo(a.geo, np, s, a.xel, a.yel, a.surfac, ne, e, true);
-      const double x2e = G.x2, x3e = G.x3;
-      const double y2e = G.y2, y3e = G.y3;
-      const bool p0 = (a.flags & SUPG_U_P0) && !(a.flags & SUPG_KSUPG);
-      double u1 = 0, u2 = 0, u3 = 0, v1 = 0, v2 = 0, v3 = 0;
-      if (!p0) {
-        u1 = a.u[g[0]];
-        u2 = a.u[g[1]];
-        u3 = a.u[g[2]];
-        v1 = a.v[g[0]];
-        v2 = a.v[g[1]];
-        v3 = a.v[g[2]];
-      }
-      // m[i][j] = A(i, j) of the element
-      double m[3][3];
-      if (a.kind == 3) {
-        double ff, gg;
-        if (a.flags & SUPG_KSUPG)
-          kspg11_elem(x2e, x3e, y2e, y3e, u1, u2, u3, v1, v2, v3, 1.0, ff, gg);
-        else {
-          ff = a.f[e];
-          gg = a.g[e];
-        }
-        const double den = (a.xmul / 12.0) / G.s;
-        const double kkx = ff * den, kky = gg * den;
-        const double u123 = u1 + u2 + u3, v123 = v1 + v2 + v3;
-        const double p1 = x2e * v123 - y2e * u123;
-        const double p2 = x3e * v123 - y3e * u123;
-        const double q1 = x2e * kky - y2e * kkx;
-        const double q2 = x3e * kky - y3e * kkx;
-        m[0][0] = (p1 - p2) * (q1 - q2);
-        m[1][1] = p2 * q2;
-        m[0][1] = p2 * (q1 - q2);
-        m[1][0] = (p1 - p2) * q2;
-        m[0][2] = -m[0][0] - m[0][1];
-        m[1][2] = -m[1][1] - m[1][0];
-        m[2][0] = -m[0][0] - m[1][0];
-        m[2][1] = -m[1][1] - m[0][1];
-        m[2][2] = -m[0][2] - m[1][2];
-      } else if (a.kind == 4) {
-        const double c = (a.xmul / 48.0) / G.s;
-        const double u123 = u1 + u2 + u3, v123 = v1 + v2 + v3;
-        const double uu = u1 * u123 + u2 * u2 + u2 * u3 + u3 * u3;
-        const double uv = u1 * (v123 + v1) + u2 * (v123 + v2) + u3 * (v123 + v3);
-        const double vv = v1 * v123 + v2 * v2 + v2 * v3 + v3 * v3;
-        const double b12 = (2 * y3e * (y2e - y3e) * uu +
-                            (x3e * (y3e - y2e) + (x3e - x2e) * y3e) * uv +
-                            2 * x3e * (x2e - x3e) * vv) * c;
-        const double b13 = (2 * y2e * (y3e - y2e) * uu +
-                            (2 * x2e * y2e - x2e * y3e - x3e * y2e) * uv +
-                            2 * x2e * (x3e - x2e) * vv) * c;
-        const double b23 =
-            (-(2 * y2e * y3e * uu) + (x2e * y3e + x3e * y2e) * uv - 2 * x2e * x3e * vv) * c;
-        m[0][1] = m[1][0] = b12;
-        m[0][2] = m[2][0] = b13;
-        m[1][2] = m[2][1] = b23;
-        m[0][0] = -b12 - b13;
-        m[1][1] = -b23 - b12;
-        m[2][2] = -b13 - b23;
-      } else if (a.flags & (SUPG_U_P0 | SUPG_KSUPG)) {
-        // MT05AA with U, V per element (given, or the SUPG vectors)
-        double ue, ve;
-        if (a.flags & SUPG_KSUPG)
-          kspg11_elem(x2e, x3e, y2e, y3e, u1, u2, u3, v1, v2, v3, 1.0, ue, ve);
-        else {
-          ue = a.u[e];
-          ve = a.v[e];
-        }
-        const double sur24 = a.xmul / 24.0;
-        const double x2 = x2e * sur24, x3 = x3e * sur24, y2 = y2e * sur24, y3 = y3e * sur24;
-        const double qu = 4 * ue, qv = 4 * ve;
-        const double r1 = (x3 - x2) * qv + (y2 - y3) * qu;
-        const double r2 = -(x3 * qv) + y3 * qu;
-        const double r3 = x2 * qv - y2 * qu;
-        m[0][0] = m[1][0] = m[2][0] = r1;
-        m[1][1] = m[0][1] = m[2][1] = r2;
-        m[2][2] = m[0][2] = m[1][2] = r3;
-      } else if (a.flags & SUPG_UPWIND) {
-        const double sur6 = a.xmul / 6.0;
-        const double us = (u1 + u2 + u3) * sur6, vs = (v1 + v2 + v3) * sur6;
-        const double k1 = us * (y2e - y3e) - vs * (x2e - x3e);
-        const double k2 = us * y3e - vs * x3e;
-        const double k3 = us * (-y2e) - vs * (-x2e);
-        const double l12 = fmax(fmin(k1, -k2), 0.0), l13 = fmax(fmin(k1, -k3), 0.0);
-        const double l21 = fmax(fmin(k2, -k1), 0.0), l23 = fmax(fmin(k2, -k3), 0.0);
-        const double l31 = fmax(fmin(k3, -k1), 0.0), l32 = fmax(fmin(k3, -k2), 0.0);
-        m[0][0] = l12 + l13;
-        m[1][1] = l21 + l23;
-        m[2][2] = l31 + l32;
-        m[0][1] = -l12;
-        m[0][2] = -l13;
-        m[1][2] = -l23;
-        m[1][0] = -l21;
-        m[2][0] = -l31;
-        m[2][1] = -l32;
-      } else {
-        const double sur24 = a.xmul / 24.0;
-        const double x2 = x2e * sur24, x3 = x3e * sur24, y2 = y2e * sur24, y3 = y3e * sur24;
-        const double u123 = u1 + u2 + u3, v123 = v1 + v2 + v3;
-        const double w1u = u123 + u1, w1v = v123 + v1;
-        const double w2u = u123 + u2, w2v = v123 + v2;
-        const double w3u = u123 + u3, w3v = v123 + v3;
-        m[0][0] = (x3 - x2) * w1v + (y2 - y3) * w1u;
-        m[1][1] = -(x3 * w2v) + y3 * w2u;
-        m[2][2] = x2 * w3v - y2 * w3u;
-        m[0][1] = -(x3 * w1v) + y3 * w1u;
-        m[0][2] = x2 * w1v - y2 * w1u;
-        m[1][2] = x2 * w2v - y2 * w2u;
-        m[1][0] = (x3 - x2) * w2v + (y2 - y3) * w2u;
-        m[2][0] = (x3 - x2) * w3v + (y2 - y3) * w3u;
-        m[2][1] = -(x3 * w3v) + y3 * w3u;
-      }
-      // 'M=M+TN' adds the transpose
-      const bool tr = a.op == 2;
-      const double c12 = tr ? m[1][0] : m[0][1], c21 = tr ? m[0][1] : m[1][0];
-      const double c13 = tr ? m[2][0] : m[0][2], c31 = tr ? m[0][2] : m[2][0];
-      const double c23 = tr ? m[2][1] : m[1][2], c32 = tr ? m[1][2] : m[2][1];
-      const double cv[6] = {c12, c13, c23, c21, c31, c32};
-      const int ncol = a.target_q ? 6 : 3;
-      for (int c = 0; c < ncol; ++c) {
-        double* p = a.xa + (size_t)c * np + s;
-        *p = a.op == 0 ? cv[c] : *p + cv[c];
-      }
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-        if (l[k] < nown) acc[l[k]] += m[k][k];
+    for (int k = 0; k < 3; ++k) {
+      l[k] = a.lid[(size_t)k * np + s];
+      g[k] = l[k] < nown ? n0 + l[k] : a.halo[hb + l[k] - nown];
     }
-    __syncthreads();
-  }
+    const SlotGeo G = load_geo(a.geo, np, s, a.xel, a.yel, a.surfac, ne, e, true);
+    const double x2e = G.x2, x3e = G.x3;
+    const double y2e = G.y2, y3e = G.y3;
+    const bool p0 = (a.flags & SUPG_U_P0) && !(a.flags & SUPG_KSUPG);
+    double u1 = 0, u2 = 0, u3 = 0, v1 = 0, v2 = 0, v3 = 0;
+    if (!p0) {
+      u1 = a.u[g[0]];
+      u2 = a.u[g[1]];
+      u3 = a.u[g[2]];
+      v1 = a.v[g[0]];
+      v2 = a.v[g[1]];
+      v3 = a.v[g[2]];
+    }
+    // m[i][j] = A(i, j) of the element
+    double m[3][3];
+    if (a.kind == 3) {
+      double ff, gg;
+      if (a.flags & SUPG_KSUPG)
+        kspg11_elem(x2e, x3e, y2e, y3e, u1, u2, u3, v1, v2, v3, 1.0, ff, gg);
+      else {
+        ff = a.f[e];
+        gg = a.g[e];
+      }
+      const double den = (a.xmul / 12.0) / G.s;
+      const double kkx = ff * den, kky = gg * den;
+      const double u123 = u1 + u2 + u3, v123 = v1 + v2 + v3;
+      const double p1 = x2e * v123 - y2e * u123;
+      const double p2 = x3e * v123 - y3e * u123;
+      const double q1 = x2e * kky - y2e * kkx;
+      const double q2 = x3e * kky - y3e * kkx;
+      m[0][0] = (p1 - p2) * (q1 - q2);
+      m[1][1] = p2 * q2;
+      m[0][1] = p2 * (q1 - q2);
+      m[1][0] = (p1 - p2) * q2;
+      m[0][2] = -m[0][0] - m[0][1];
+      m[1][2] = -m[1][1] - m[1][0];
+      m[2][0] = -m[0][0] - m[1][0];
+      m[2][1] = -m[1][1] - m[0][1];
+      m[2][2] = -m[0][2] - m[1][2];
+    } else if (a.kind == 4) {
+      const double c = (a.xmul / 48.0) / G.s;
+      const double u123 = u1 + u2 + u3, v123 = v1 + v2 + v3;
+      const double uu = u1 * u123 + u2 * u2 + u2 * u3 + u3 * u3;
+      const double uv = u1 * (v123 + v1) + u2 * (v123 + v2) + u3 * (v123 + v3);
+      const double vv = v1 * v123 + v2 * v2 + v2 * v3 + v3 * v3;
+      const double b12 = (2 * y3e * (y2e - y3e) * uu +
+                          (x3e * (y3e - y2e) + (x3e - x2e) * y3e) * uv +
+                          2 * x3e * (x2e - x3e) * vv) * c;
+      const double b13 = (2 * y2e * (y3e - y2e) * uu +
+                          (2 * x2e * y2e - x2e * y3e - x3e * y2e) * uv +
+                          2 * x2e * (x3e - x2e) * vv) * c;
+      const double b23 =
+          (-(2 * y2e * y3e * uu) + (x2e * y3e + x3e * y2e) * uv - 2 * x2e * x3e * vv) * c;
+      m[0][1] = m[1][0] = b12;
+      m[0][2] = m[2][0] = b13;
+      m[1][2] = m[2][1] = b23;
+      m[0][0] = -b12 - b13;
+      m[1][1] = -b23 - b12;
+      m[2][2] = -b13 - b23;
+    } else if (a.flags & (SUPG_U_P0 | SUPG_KSUPG)) {
+      // MT05AA with U, V per element (given, or the SUPG vectors)
+      double ue, ve;
+      if (a.flags & SUPG_KSUPG)
+        kspg11_elem(x2e, x3e, y2e, y3e, u1, u2, u3, v1, v2, v3, 1.0, ue, ve);
+      else {
+        ue = a.u[e];
+        ve = a.v[e];
+      }
+      const double sur24 = a.xmul / 24.0;
+      const double x2 = x2e * sur24, x3 = x3e * sur24, y2 = y2e * sur24, y3 = y3e * sur24;
+      const double qu = 4 * ue, qv = 4 * ve;
+      const double r1 = (x3 - x2) * qv + (y2 - y3) * qu;
+      const double r2 = -(x3 * qv) + y3 * qu;
+      const double r3 = x2 * qv - y2 * qu;
+      m[0][0] = m[1][0] = m[2][0] = r1;
+      m[1][1] = m[0][1] = m[2][1] = r2;
+      m[2][2] = m[0][2] = m[1][2] = r3;
+    } else if (a.flags & SUPG_UPWIND) {
+      const double sur6 = a.xmul / 6.0;
+      const double us = (u1 + u2 + u3) * sur6, vs = (v1 + v2 + v3) * sur6;
+      const double k1 = us * (y2e - y3e) - vs * (x2e - x3e);
+      const double k2 = us * y3e - vs * x3e;
+      const double k3 = us * (-y2e) - vs * (-x2e);
+      const double l12 = fmax(fmin(k1, -k2), 0.0), l13 = fmax(fmin(k1, -k3), 0.0);
+      const double l21 = fmax(fmin(k2, -k1), 0.0), l23 = fmax(fmin(k2, -k3), 0.0);
+      const double l31 = fmax(fmin(k3, -k1), 0.0), l32 = fmax(fmin(k3, -k2), 0.0);
+      m[0][0] = l12 + l13;
+      m[1][1] = l21 + l23;
+      m[2][2] = l31 + l32;
+      m[0][1] = -l12;
+      m[0][2] = -l13;
+      m[1][2] = -l23;
+      m[1][0] = -l21;
+      m[2][0] = -l31;
+      m[2][1] = -l32;
+    } else {
+      const double sur24 = a.xmul / 24.0;
+      const double x2 = x2e * sur24, x3 = x3e * sur24, y2 = y2e * sur24, y3 = y3e * sur24;
+      const double u123 = u1 + u2 + u3, v123 = v1 + v2 + v3;
+      const double w1u = u123 + u1, w1v = v123 + v1;
+      const double w2u = u123 + u2, w2v = v123 + v2;
+      const double w3u = u123 + u3, w3v = v123 + v3;
+      m[0][0] = (x3 - x2) * w1v + (y2 - y3) * w1u;
+      m[1][1] = -(x3 * w2v) + y3 * w2u;
+      m[2][2] = x2 * w3v - y2 * w3u;
+      m[0][1] = -(x3 * w1v) + y3 * w1u;
+      m[0][2] = x2 * w1v - y2 * w1u;
+      m[1][2] = x2 * w2v - y2 * w2u;
+      m[1][0] = (x3 - x2) * w2v + (y2 - y3) * w2u;
+      m[2][0] = (x3 - x2) * w3v + (y2 - y3) * w3u;
+      m[2][1] = -(x3 * w3v) + y3 * w3u;
+    }
+    // 'M=M+TN' adds the transpose
+    const bool tr = a.op == 2;
+    const double c12 = tr ? m[1][0] : m[0][1], c21 = tr ? m[0][1] : m[1][0];
+    const double c13 = tr ? m[2][0] : m[0][2], c31 = tr ? m[0][2] : m[2][0];
+    const double c23 = tr ? m[2][1] : m[1][2], c32 = tr ? m[1][2] : m[2][1];
+    const double cv[6] = {c12, c13, c23, c21, c31, c32};
+    const int ncol = a.target_q ? 6 : 3;
+    for (int c = 0; c < ncol; ++c) {
+      double* p = a.xa + (size_t)c * np + s;
+      *p = a.op == 0 ? cv[c] : *p + cv[c];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) nt.c[0][k] = m[k][k];
+    return nt;
+  });
   for (int l = threadIdx.x; l < nown; l += blockDim.x)
     a.da[n0 + l] = a.op == 0 ? acc[l] : a.da[n0 + l] + acc[l];
 }
@@ -357,7 +351,7 @@ static int supg_impl(bhip_ctx* c, int kind, double xmul, const double* xel, cons
   a.da = c->da.p;
   a.op = op;
   a.target_q = target_q ? 1 : 0;
-  hipLaunchKernelGGL(k_elem_supg, dim3(L.nblocks), dim3(kThreads),
+  hipLaunchKernelGGL(k_elem_supg, dim3(L.nblocks), elem_threads(L),
                      (size_t)L.max_owned * sizeof(double), c->stream, a);
   HIP_OK(hipGetLastError());
   if (!use_geo) HIP_OK(hipStreamSynchronize(c->stream));

@@ -31,7 +31,7 @@
 // The adjoint kernels are the transposes of these, derived by hand: the
 // element terms of each kernel are differentiated with respect to the node
 // values they gather, and the results are assembled onto owned nodes with the
-// same colour-by-colour LDS scheme (deterministic, no atomics). The floors
+// same LDS sums in colour order (colour_sum; deterministic, no atomics). The floors
 // max(h, .) pass the derivative where h is above them and nothing below.
 
 namespace bhip {
@@ -81,21 +81,6 @@ __device__ inline void slot_nodes(const WaveArgs& a, int s, int n0, int nown, in
   for (int k = 0; k < 3; ++k) {
     l[k] = a.lid[(size_t)k * a.nslot_pad + s];
     g[k] = l[k] < nown ? n0 + l[k] : a.halo[hb + l[k] - nown];
-  }
-}
-
-// walks the colours of block b, calling f(s) for each slot, a barrier after
-// each colour
-template <typename F>
-__device__ inline void colour_walk(const WaveArgs& a, int b, F&& f) {
-  const int32_t* co = a.color_off + (size_t)b * (kMaxColors + 1);
-  const int send = co[kMaxColors];
-  for (int col = 0; col < kMaxColors; ++col) {
-    const int s0 = co[col];
-    if (s0 >= send) break;
-    const int s1 = co[col + 1];
-    for (int s = s0 + threadIdx.x; s < s1; s += blockDim.x) f(s);
-    __syncthreads();
   }
 }
 
@@ -174,21 +159,23 @@ __global__ void k_wave_nodes(WaveArgs a, int n, const double* __restrict__ eta,
 
 // GRADF(eta) and the slope-weighted basis integrals at owned nodes, then
 // c = VOL / (VOL/dt + f VS) and the velocity predictor u* = c (u/dt - g GX/VOL)
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kElemThreads)
 k_wave_grad(WaveArgs a, const double* __restrict__ eta, const double* __restrict__ u,
             const double* __restrict__ v) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int b = wave_block(a);
   const int n0 = a.node_start[b], nown = a.node_start[b + 1] - n0;
   const int hb = a.halo_start[b];
+  const int32_t* co = a.color_off + (size_t)b * (kMaxColors + 1);
   double* acc_x = reinterpret_cast<double*>(smem_raw);
   double* acc_y = acc_x + nown;
   double* acc_v = acc_y + nown;
   for (int l = threadIdx.x; l < nown; l += blockDim.x) acc_x[l] = acc_y[l] = acc_v[l] = 0.0;
   __syncthreads();
-  colour_walk(a, b, [&](int s) {
-    int l[3], g[3];
-    slot_nodes(a, s, n0, nown, hb, l, g);
+  colour_sum<3>(co, nown, acc_x, [&](int s) {
+    NodeTerms<3> v;
+    int g[3];
+    slot_nodes(a, s, n0, nown, hb, v.l, g);
     const ElemGeo e = elem_geo(a, s);
     double ek[3];
 #pragma unroll
@@ -197,12 +184,11 @@ k_wave_grad(WaveArgs a, const double* __restrict__ eta, const double* __restrict
     const double vs = e.s / 3.0 * elem_slope(e, a.zb[g[0]], a.zb[g[1]], a.zb[g[2]]);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      if (l[k] < nown) {
-        acc_x[l[k]] += gx;
-        acc_y[l[k]] += gy;
-        acc_v[l[k]] += vs;
-      }
+      v.c[0][k] = gx;
+      v.c[1][k] = gy;
+      v.c[2][k] = vs;
     }
+    return v;
   });
   for (int l = threadIdx.x; l < nown; l += blockDim.x) {
     const int i = n0 + l;
@@ -220,21 +206,23 @@ k_wave_grad(WaveArgs a, const double* __restrict__ eta, const double* __restrict
 // the system of the step: A (diagonal into da, internal order; off-diagonal
 // terms with the sea rows and columns cleared into xa, slot order) and its
 // right-hand side
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kElemThreads)
 k_wave_assemble(WaveArgs a, double* __restrict__ da, double* __restrict__ xa,
                 double* __restrict__ rhs) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int b = wave_block(a);
   const int n0 = a.node_start[b], nown = a.node_start[b + 1] - n0;
   const int hb = a.halo_start[b];
+  const int32_t* co = a.color_off + (size_t)b * (kMaxColors + 1);
   double* acc_d = reinterpret_cast<double*>(smem_raw);
   double* acc_r = acc_d + nown;
   for (int l = threadIdx.x; l < nown; l += blockDim.x) acc_d[l] = acc_r[l] = 0.0;
   __syncthreads();
   const double mdt = 1.0 / (12.0 * a.dt);
-  colour_walk(a, b, [&](int s) {
-    int l[3], g[3];
-    slot_nodes(a, s, n0, nown, hb, l, g);
+  colour_sum<2>(co, nown, acc_d, [&](int s) {
+    NodeTerms<2> v;
+    int g[3];
+    slot_nodes(a, s, n0, nown, hb, v.l, g);
     const ElemGeo e = elem_geo(a, s);
     double hp[3], uu[3], sx[3], sy[3], fb[3], wk[3];
 #pragma unroll
@@ -269,11 +257,10 @@ k_wave_assemble(WaveArgs a, double* __restrict__ da, double* __restrict__ xa,
     xa[2 * np + s] = x23 * (wk[1] * wk[2]);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      if (l[k] < nown) {
-        acc_d[l[k]] += t[k];
-        acc_r[l[k]] += e.bx[k] * qx + e.by[k] * qy - af[k];
-      }
+      v.c[0][k] = t[k];
+      v.c[1][k] = e.bx[k] * qx + e.by[k] * qy - af[k];
     }
+    return v;
   });
   for (int l = threadIdx.x; l < nown; l += blockDim.x) {
     const int i = n0 + l;
@@ -286,7 +273,7 @@ k_wave_assemble(WaveArgs a, double* __restrict__ da, double* __restrict__ xa,
 
 // the new state from the increment: eta' = eta + deta, GRADF(eta') and the
 // momentum update u' = c (u/dt - g GRADF(eta')/VOL)
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kElemThreads)
 k_wave_momentum(WaveArgs a, const double* __restrict__ eta, const double* __restrict__ deta,
                 const double* __restrict__ u, const double* __restrict__ v,
                 double* __restrict__ eta_n, double* __restrict__ u_n, double* __restrict__ v_n) {
@@ -294,13 +281,15 @@ k_wave_momentum(WaveArgs a, const double* __restrict__ eta, const double* __rest
   const int b = wave_block(a);
   const int n0 = a.node_start[b], nown = a.node_start[b + 1] - n0;
   const int hb = a.halo_start[b];
+  const int32_t* co = a.color_off + (size_t)b * (kMaxColors + 1);
   double* acc_x = reinterpret_cast<double*>(smem_raw);
   double* acc_y = acc_x + nown;
   for (int l = threadIdx.x; l < nown; l += blockDim.x) acc_x[l] = acc_y[l] = 0.0;
   __syncthreads();
-  colour_walk(a, b, [&](int s) {
-    int l[3], g[3];
-    slot_nodes(a, s, n0, nown, hb, l, g);
+  colour_sum<2>(co, nown, acc_x, [&](int s) {
+    NodeTerms<2> v;
+    int g[3];
+    slot_nodes(a, s, n0, nown, hb, v.l, g);
     const ElemGeo e = elem_geo(a, s);
     double en[3];
 #pragma unroll
@@ -308,11 +297,10 @@ k_wave_momentum(WaveArgs a, const double* __restrict__ eta, const double* __rest
     const double gx = gradf_x(e, en), gy = gradf_y(e, en);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      if (l[k] < nown) {
-        acc_x[l[k]] += gx;
-        acc_y[l[k]] += gy;
-      }
+      v.c[0][k] = gx;
+      v.c[1][k] = gy;
     }
+    return v;
   });
   for (int l = threadIdx.x; l < nown; l += blockDim.x) {
     const int i = n0 + l;
@@ -326,7 +314,7 @@ k_wave_momentum(WaveArgs a, const double* __restrict__ eta, const double* __rest
 // transpose of GRADF: etot = ebar + GRADF^T(-g c ubar / VOL, -g c vbar / VOL)
 // (the momentum update's dependence on eta'; the c and u parts are
 // node-local and taken in k_wave_assemble_adj)
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kElemThreads)
 k_wave_momentum_adj(WaveArgs a, const double* __restrict__ ubar_n,
                     const double* __restrict__ vbar_n, const double* __restrict__ ebar_n,
                     double* __restrict__ etot) {
@@ -334,12 +322,14 @@ k_wave_momentum_adj(WaveArgs a, const double* __restrict__ ubar_n,
   const int b = wave_block(a);
   const int n0 = a.node_start[b], nown = a.node_start[b + 1] - n0;
   const int hb = a.halo_start[b];
+  const int32_t* co = a.color_off + (size_t)b * (kMaxColors + 1);
   double* acc = reinterpret_cast<double*>(smem_raw);
   for (int l = threadIdx.x; l < nown; l += blockDim.x) acc[l] = 0.0;
   __syncthreads();
-  colour_walk(a, b, [&](int s) {
-    int l[3], g[3];
-    slot_nodes(a, s, n0, nown, hb, l, g);
+  colour_sum<1>(co, nown, acc, [&](int s) {
+    NodeTerms<1> v;
+    int g[3];
+    slot_nodes(a, s, n0, nown, hb, v.l, g);
     const ElemGeo e = elem_geo(a, s);
     double sx = 0.0, sy = 0.0;
 #pragma unroll
@@ -349,8 +339,8 @@ k_wave_momentum_adj(WaveArgs a, const double* __restrict__ ubar_n,
       sy += f * vbar_n[g[k]];
     }
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-      if (l[k] < nown) acc[l[k]] += (e.bx[k] * sx + e.by[k] * sy) / 6.0;
+    for (int k = 0; k < 3; ++k) v.c[0][k] = (e.bx[k] * sx + e.by[k] * sy) / 6.0;
+    return v;
   });
   for (int l = threadIdx.x; l < nown; l += blockDim.x) {
     const int i = n0 + l;
@@ -384,12 +374,13 @@ struct WaveAdjOut {
   double* zbbar;  // accumulated
 };
 
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kElemThreads)
 k_wave_assemble_adj(WaveArgs a, WaveAdjIn in, WaveAdjOut out) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int b = wave_block(a);
   const int n0 = a.node_start[b], nown = a.node_start[b + 1] - n0;
   const int hb = a.halo_start[b];
+  const int32_t* co = a.color_off + (size_t)b * (kMaxColors + 1);
   double* acc_c = reinterpret_cast<double*>(smem_raw);
   double* acc_h = acc_c + nown;
   double* acc_sx = acc_h + nown;
@@ -399,9 +390,10 @@ k_wave_assemble_adj(WaveArgs a, WaveAdjIn in, WaveAdjOut out) {
     acc_c[l] = acc_h[l] = acc_sx[l] = acc_sy[l] = acc_fb[l] = 0.0;
   __syncthreads();
   const double mdt = 1.0 / (12.0 * a.dt);
-  colour_walk(a, b, [&](int s) {
-    int l[3], g[3];
-    slot_nodes(a, s, n0, nown, hb, l, g);
+  colour_sum<5>(co, nown, acc_c, [&](int s) {
+    NodeTerms<5> v;
+    int g[3];
+    slot_nodes(a, s, n0, nown, hb, v.l, g);
     const ElemGeo e = elem_geo(a, s);
     double hp[3], uu[3], sx[3], sy[3], fb[3], wk[3], lam[3], de[3], rho[3], dabar[3];
 #pragma unroll
@@ -454,15 +446,13 @@ k_wave_assemble_adj(WaveArgs a, WaveAdjIn in, WaveAdjOut out) {
     const double Sx = sx[0] + sx[1] + sx[2], Sy = sy[0] + sy[1] + sy[2];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      if (l[k] < nown) {
-        const int q = l[k];
-        acc_c[q] += a.grav * cb2 * (hp[k] + g123);
-        acc_h[q] += cb2 * (uu[k] + u123) + (rx * (Sx + sx[k]) + ry * (Sy + sy[k])) / 24.0;
-        acc_sx[q] += rx * (F123 + F[k]);
-        acc_sy[q] += ry * (F123 + F[k]);
-        acc_fb[q] -= arho[k];
-      }
+      v.c[0][k] = a.grav * cb2 * (hp[k] + g123);
+      v.c[1][k] = cb2 * (uu[k] + u123) + (rx * (Sx + sx[k]) + ry * (Sy + sy[k])) / 24.0;
+      v.c[2][k] = rx * (F123 + F[k]);
+      v.c[3][k] = ry * (F123 + F[k]);
+      v.c[4][k] = -arho[k];
     }
+    return v;
   });
   for (int l = threadIdx.x; l < nown; l += blockDim.x) {
     const int i = n0 + l;
@@ -523,19 +513,21 @@ k_wave_assemble_adj(WaveArgs a, WaveAdjIn in, WaveAdjOut out) {
 // the transposes of GRADF (u* = c (u/dt - g GX/VOL): eta gets GRADF^T of
 // -g c u*bar / VOL) and of the slope factor of VS (zb), from the scratch
 // vectors k_wave_assemble_adj left; completes ebar and zbbar
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kElemThreads)
 k_wave_grad_adj(WaveArgs a, double* __restrict__ ebar, double* __restrict__ zbbar) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int b = wave_block(a);
   const int n0 = a.node_start[b], nown = a.node_start[b + 1] - n0;
   const int hb = a.halo_start[b];
+  const int32_t* co = a.color_off + (size_t)b * (kMaxColors + 1);
   double* acc_e = reinterpret_cast<double*>(smem_raw);
   double* acc_z = acc_e + nown;
   for (int l = threadIdx.x; l < nown; l += blockDim.x) acc_e[l] = acc_z[l] = 0.0;
   __syncthreads();
-  colour_walk(a, b, [&](int s) {
-    int l[3], g[3];
-    slot_nodes(a, s, n0, nown, hb, l, g);
+  colour_sum<2>(co, nown, acc_e, [&](int s) {
+    NodeTerms<2> v;
+    int g[3];
+    slot_nodes(a, s, n0, nown, hb, v.l, g);
     const ElemGeo e = elem_geo(a, s);
     double sx = 0.0, sy = 0.0, sv = 0.0;
 #pragma unroll
@@ -552,11 +544,10 @@ k_wave_grad_adj(WaveArgs a, double* __restrict__ ebar, double* __restrict__ zbba
     const double zb3[3] = {-(d2 + d3) * slb, d2 * slb, d3 * slb};
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      if (l[k] < nown) {
-        acc_e[l[k]] += (e.bx[k] * sx + e.by[k] * sy) / 6.0;
-        acc_z[l[k]] += zb3[k];
-      }
+      v.c[0][k] = (e.bx[k] * sx + e.by[k] * sy) / 6.0;
+      v.c[1][k] = zb3[k];
     }
+    return v;
   });
   for (int l = threadIdx.x; l < nown; l += blockDim.x) {
     const int i = n0 + l;
@@ -676,9 +667,9 @@ int bhip_wave_assemble(bhip_ctx* c, const bhip_wave_params* p, const double* eta
   WaveArgs a = wave_args(c, p);
   hipLaunchKernelGGL(k_wave_nodes, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream, a,
                      L.npoin, eta, u, v, kstr, zb);
-  hipLaunchKernelGGL(k_wave_grad, dim3(L.nblocks), dim3(kThreads),
+  hipLaunchKernelGGL(k_wave_grad, dim3(L.nblocks), elem_threads(L),
                      3 * (size_t)L.max_owned * sizeof(double), c->stream, a, eta, u, v);
-  hipLaunchKernelGGL(k_wave_assemble, dim3(L.nblocks), dim3(kThreads),
+  hipLaunchKernelGGL(k_wave_assemble, dim3(L.nblocks), elem_threads(L),
                      2 * (size_t)L.max_owned * sizeof(double), c->stream, a, c->da.p, c->xa.p,
                      rhs);
   HIP_OK(hipGetLastError());
@@ -697,7 +688,7 @@ int bhip_wave_momentum(bhip_ctx* c, const bhip_wave_params* p, const double* eta
       !v_n)
     return BHIP_EBADARG;
   const Layout& L = c->L;
-  hipLaunchKernelGGL(k_wave_momentum, dim3(L.nblocks), dim3(kThreads),
+  hipLaunchKernelGGL(k_wave_momentum, dim3(L.nblocks), elem_threads(L),
                      2 * (size_t)L.max_owned * sizeof(double), c->stream, wave_args(c, p), eta,
                      deta, u, v, eta_n, u_n, v_n);
   HIP_OK(hipGetLastError());
@@ -709,7 +700,7 @@ int bhip_wave_momentum_adj(bhip_ctx* c, const bhip_wave_params* p, const double*
   if (!c || !c->wv_ready || !wave_params_ok(p) || !ubar_n || !vbar_n || !ebar_n || !etot)
     return BHIP_EBADARG;
   const Layout& L = c->L;
-  hipLaunchKernelGGL(k_wave_momentum_adj, dim3(L.nblocks), dim3(kThreads),
+  hipLaunchKernelGGL(k_wave_momentum_adj, dim3(L.nblocks), elem_threads(L),
                      (size_t)L.max_owned * sizeof(double), c->stream, wave_args(c, p), ubar_n,
                      vbar_n, ebar_n, etot);
   HIP_OK(hipGetLastError());
@@ -730,9 +721,9 @@ int bhip_wave_assemble_adj(bhip_ctx* c, const bhip_wave_params* p, const double*
   WaveAdjIn in = {lam, deta, eta, u, v, u_n, v_n, ubar_n, vbar_n, etot, kstr};
   WaveAdjOut out = {ebar, ubar, vbar, kbar, zbbar};
   const WaveArgs a = wave_args(c, p);
-  hipLaunchKernelGGL(k_wave_assemble_adj, dim3(L.nblocks), dim3(kThreads),
+  hipLaunchKernelGGL(k_wave_assemble_adj, dim3(L.nblocks), elem_threads(L),
                      5 * (size_t)L.max_owned * sizeof(double), c->stream, a, in, out);
-  hipLaunchKernelGGL(k_wave_grad_adj, dim3(L.nblocks), dim3(kThreads),
+  hipLaunchKernelGGL(k_wave_grad_adj, dim3(L.nblocks), elem_threads(L),
                      2 * (size_t)L.max_owned * sizeof(double), c->stream, a, ebar, zbbar);
   HIP_OK(hipGetLastError());
   return BHIP_OK;
