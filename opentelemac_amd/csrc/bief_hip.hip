@@ -977,7 +977,8 @@ struct bhip_ctx {
   bhip::Layout L;
   hipStream_t stream = nullptr;
   int device = 0;
-  int grid_nodes = 0;  // grid of the node-wise kernels
+  int grid_nodes = 0;  // grid of the node-wise kernels that leave a partial sum per block
+  int grid_wide = 0;   // of the others
   // layout on device
   bhip::DevBuf<int32_t> node_start, halo_start, halo, color_off, slot_elem, perm, first_slot;
   bhip::DevBuf<uint16_t> lid;
@@ -1077,7 +1078,7 @@ static size_t lds_bytes(const Layout& L, size_t elt) {
 // LDS of the DMD kernel: D of a block's owned and halo nodes
 static size_t dmd_lds(const Layout& L) { return ((size_t)L.max_local + 1) * sizeof(double); }
 
-static int grid_for(int n);
+static int grid_for(long n);
 
 // OM 'M=DMD' on the context's coefficients with the node vector d (and the
 // FP32 copy of the result when xa32 is given); the coefficients come from src
@@ -1100,7 +1101,15 @@ static hipError_t launch_dmd(bhip_ctx* c, float* xa32, const double* d,
   return hipGetLastError();
 }
 
-static int grid_for(int n) {
+// Blocks of an elementwise kernel: one item per thread up to 8 blocks per CU.
+// With 8 items per thread from the start, 100k nodes ran on 49 CUs, a serial
+// chain of 8 items each: k_gather 7.8 -> 4.7 us at 700k nodes, k_gather_shift 5.7
+// -> 2.9 at 90k, k_wave_nodes 12.5 -> 5 at 100k, the largest sizes alike.
+static int grid_for(long n) {
+  return (int)std::max(1l, std::min((n + kThreads - 1) / kThreads, 2048l));
+}
+// and of one whose blocks each leave a partial sum for others to add up
+static int grid_sums(int n) {
   int g = (n + kThreads * 8 - 1) / (kThreads * 8);
   return std::max(1, std::min(g, 1024));
 }
@@ -1256,7 +1265,8 @@ static int ctx_setup(std::unique_ptr<bhip_ctx>& c, bhip_ctx** out) {
   // dynamic LDS (checked above); only the prism element kernels raise their
   // limit, per launch, for their node records
   const int n = L.npoin;
-  c->grid_nodes = grid_for(n);
+  c->grid_nodes = grid_sums(n);
+  c->grid_wide = grid_for(n);
   HIP_OK(c->node_start.alloc(L.node_start.size()));
   HIP_OK(c->halo_start.alloc(L.halo_start.size()));
   HIP_OK(c->halo.alloc(std::max<size_t>(1, L.halo.size())));
@@ -1316,7 +1326,7 @@ static int ctx_setup(std::unique_ptr<bhip_ctx>& c, bhip_ctx** out) {
     HIP_OK(up(c->block_sys.p, bs.data(), bs.size() * 4));
     HIP_OK(up(c->sys_blocks.p, c->sys_blocks_h.data(), c->sys_blocks_h.size() * 4));
   }
-  hipLaunchKernelGGL(k_fill<double>, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream,
+  hipLaunchKernelGGL(k_fill<double>, dim3(c->grid_wide), dim3(kThreads), 0, c->stream,
                      c->vdz.p, 0.0, (long)n);
   HIP_OK(hipGetLastError());
   HIP_OK(hipStreamSynchronize(c->stream));
@@ -1467,10 +1477,10 @@ static int matrix_set_common(bhip_ctx* c, char typdia, char typext, const double
       HIP_OK(to_device(c, tmp, da, sizeof(double) * L.npoin));
     else
       HIP_OK(hipMemcpyAsync(tmp, da, sizeof(double) * L.npoin, kind, c->stream));
-    hipLaunchKernelGGL(k_gather<double>, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream,
+    hipLaunchKernelGGL(k_gather<double>, dim3(c->grid_wide), dim3(kThreads), 0, c->stream,
                        c->da.p, tmp, c->perm.p, L.npoin);
   } else {
-    hipLaunchKernelGGL(k_fill<double>, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream,
+    hipLaunchKernelGGL(k_fill<double>, dim3(c->grid_wide), dim3(kThreads), 0, c->stream,
                        c->da.p, 0.0, (long)L.npoin);
   }
   HIP_OK(hipGetLastError());
@@ -1483,7 +1493,7 @@ static int matrix_set_common(bhip_ctx* c, char typdia, char typext, const double
     } else {
       src = const_cast<double*>(xa);
     }
-    hipLaunchKernelGGL(k_matrix_to_slots, dim3(grid_for(L.nslot * ncoef)), dim3(kThreads), 0,
+    hipLaunchKernelGGL(k_matrix_to_slots, dim3(grid_for((long)L.nslot * ncoef)), dim3(kThreads), 0,
                        c->stream, c->xa.p, src, c->slot_elem.p, L.nslot, L.nslot_pad, L.nelem,
                        ncoef);
     HIP_OK(hipGetLastError());
@@ -1559,14 +1569,14 @@ int bhip_matrix_get(bhip_ctx* c, char* typdia, double* da, double* xa) {
   const Layout& L = c->L;
   if (typdia) *typdia = c->typdia;
   if (da) {
-    hipLaunchKernelGGL(k_scatter<double>, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream,
+    hipLaunchKernelGGL(k_scatter<double>, dim3(c->grid_wide), dim3(kThreads), 0, c->stream,
                        c->vio0.p, c->da.p, c->perm.p, L.npoin);
     HIP_OK(hipGetLastError());
     HIP_OK(to_host(c, da, c->vio0.p, sizeof(double) * L.npoin));
   }
   if (xa && c->ncoef > 0) {
     HIP_OK(c->h_xa.alloc((size_t)c->ncoef * L.nelem));
-    hipLaunchKernelGGL(k_matrix_from_slots, dim3(grid_for(L.nelem * c->ncoef)), dim3(kThreads),
+    hipLaunchKernelGGL(k_matrix_from_slots, dim3(grid_for((long)L.nelem * c->ncoef)), dim3(kThreads),
                        0, c->stream, c->h_xa.p, c->xa.p, c->first_slot.p, L.nelem, L.nslot_pad,
                        c->ncoef);
     HIP_OK(hipGetLastError());
@@ -1595,7 +1605,7 @@ static int matvec_internal(bhip_ctx* c, int op, double cst, const double* y_in,
 int bhip_matvec_dev(bhip_ctx* c, int op, double cst, const double* y, double* x) {
   if (!c || !c->have_matrix || op < 0 || op > 10 || !y || !x) return BHIP_EBADARG;
   const Layout& L = c->L;
-  const int g = c->grid_nodes;
+  const int g = c->grid_wide;
   hipLaunchKernelGGL(k_gather<double>, dim3(g), dim3(kThreads), 0, c->stream, c->vio0.p, y,
                      c->perm.p, L.npoin);
   hipLaunchKernelGGL(k_gather<double>, dim3(g), dim3(kThreads), 0, c->stream, c->vio1.p, x,
@@ -1846,7 +1856,7 @@ static int ensure_f32(bhip_ctx* c) {
   // after k_inner_dir has written a direction there: it only ever needs to
   // hold finite values, so it is zeroed once, when allocated
   if (fresh) {
-    hipLaunchKernelGGL(k_fill<float>, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream,
+    hipLaunchKernelGGL(k_fill<float>, dim3(c->grid_wide), dim3(kThreads), 0, c->stream,
                        c->fdz.p, 0.0f, (long)n);
     HIP_OK(hipGetLastError());
   }
@@ -1866,7 +1876,7 @@ static double clock_khz(bhip_ctx* c) {
 // fills c->sys_info and the ensemble summary in *info
 static int collect_infos(bhip_ctx* c, double* x, bool mixed, bhip_solve_info* info) {
   SolveState* sh = c->st_host;
-  const int g = c->grid_nodes;
+  const int g = c->grid_wide;
   const double khz = clock_khz(c);
   c->sys_latency_ms.assign(c->nsys, 0.0);
   int maxm = 0, nconv = 0, nzero = 0, maxout = 0, maxin = 0;
@@ -1932,7 +1942,7 @@ static int collect_infos(bhip_ctx* c, double* x, bool mixed, bhip_solve_info* in
 static int cg_fp64(bhip_ctx* c, double* x, const double* b, double eps, int nitmax,
                    bhip_solve_info* info, const std::function<int()>& tail) {
   const int n = c->L.npoin;
-  const int g = c->grid_nodes;
+  const int g = c->grid_wide;
   SolveState* sh = c->st_host;
   hipGraphExec_t exec;
   int rc = cg_batch_exec<double, double, double>(c, BHIP_PREC_FP64, x, c->vr.p, c->vd0.p,
@@ -2031,7 +2041,7 @@ static int cg_mixed(bhip_ctx* c, double* x, const double* b, double eps, int nit
                     bhip_solve_info* info, const std::function<int()>& tail) {
   const Layout& L = c->L;
   const int n = L.npoin;
-  const int g = c->grid_nodes;
+  const int g = c->grid_wide;
   SolveState* sh = c->st_host;
   if (ensure_f32(c)) return BHIP_EDEVICE;
   HIP_OK(c->vx2.alloc(n));
@@ -2198,7 +2208,7 @@ static int cg_rows_mixed(bhip_ctx* c, double* x, const double* b, double eps, in
   float* delta = c->fx0.p;
   std::lock_guard<std::mutex> one(rows_mutex(c->device));
   if (c->typdia == 'Q') {
-    hipLaunchKernelGGL(k_to_f32, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream, c->da32.p,
+    hipLaunchKernelGGL(k_to_f32, dim3(c->grid_wide), dim3(kThreads), 0, c->stream, c->da32.p,
                        c->da.p, (long)L.npoin);
     HIP_OK(hipGetLastError());
   }
@@ -2281,7 +2291,7 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   if (c->nsys > 1 && cfg->slv != 1) return BHIP_EBADARG;
   const Layout& L = c->L;
   const int n = L.npoin;
-  const int g = c->grid_nodes;
+  const int g = c->grid_wide;
   const bool diag = (precon % 2 == 0) || (precon % 5 == 0);
   // OM 'M=N' from the saved copy first: with diagonal preconditioning and
   // off-diagonal terms, PRECD1 and D A D read the saved copy and write the
@@ -2486,7 +2496,7 @@ int bhip_solve_dev_noalloc(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_de
   // the scratch keeps the previous call's contents: clear what this call uses
   const long nd = (long)4 * c->max_part;
   const long ns = (long)(sizeof(SolveState) * c->nsys / sizeof(double));
-  hipLaunchKernelGGL(k_fill<double>, dim3(grid_for((int)nd)), dim3(kThreads), 0, c->stream,
+  hipLaunchKernelGGL(k_fill<double>, dim3(grid_for((long)nd)), dim3(kThreads), 0, c->stream,
                      c->part_p, 0.0, nd);
   hipLaunchKernelGGL(k_fill<double>, dim3(1), dim3(kThreads), 0, c->stream,
                      reinterpret_cast<double*>(c->st_p), 0.0, ns);
@@ -3281,7 +3291,7 @@ static double* node_in(bhip_ctx* c, int k, const double* src, int shift = 0) {
       return nullptr;
     from = stage;
   }
-  hipLaunchKernelGGL(k_gather_shift, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream, dst, from,
+  hipLaunchKernelGGL(k_gather_shift, dim3(c->grid_wide), dim3(kThreads), 0, c->stream, dst, from,
                      c->perm.p, shift, n);
   if (hipGetLastError() != hipSuccess) return nullptr;
   // the staging area is reused by the next host field
@@ -3335,7 +3345,7 @@ static double* node_in_prism4(bhip_ctx* c, const double* z, const double* f, con
       src[k] = stage;
     }
   }
-  hipLaunchKernelGGL(k_gather_prism4, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream,
+  hipLaunchKernelGGL(k_gather_prism4, dim3(c->grid_wide), dim3(kThreads), 0, c->stream,
                      c->nsc.p, src[0], src[1], src[2], src[3], c->perm.p, npou0, n);
   if (hipGetLastError() != hipSuccess) return nullptr;
   if (!c->in_dev && hipStreamSynchronize(c->stream) != hipSuccess) return nullptr;
@@ -3354,7 +3364,7 @@ static int dirich_impl(bhip_ctx* c, double* f, double* sm, const double* fbor,
                        const int32_t* limdir, int kdir) {
   const Layout& L = c->L;
   const int n = L.npoin;
-  const int g = c->grid_nodes;
+  const int g = c->grid_wide;
   const double* nb = node_in(c, 0, fbor);
   const double* ns = nb ? node_in(c, 1, sm) : nullptr;
   const double* nf = ns ? node_in(c, 2, f) : nullptr;
@@ -3407,7 +3417,7 @@ static int dirich_impl(bhip_ctx* c, double* f, double* sm, const double* fbor,
 // LUMP (lump.f): DIAG = A * XMUL, caller order
 static int lump_impl(bhip_ctx* c, double xmul, double* diag) {
   const int n = c->L.npoin;
-  const int g = c->grid_nodes;
+  const int g = c->grid_wide;
   hipLaunchKernelGGL(k_fill<double>, dim3(g), dim3(kThreads), 0, c->stream, c->vio0.p, xmul,
                      (long)n);
   HIP_OK(hipGetLastError());

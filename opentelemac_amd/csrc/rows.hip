@@ -1092,10 +1092,11 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, RowsGmres a, T* basis, T* hb
 // back and kept in LDS, where the block's 16 slices sum them. A gather from
 // memory instead takes a cache line per coefficient (k_rows_assemble: 138 us
 // for 2M nodes in FP64, after 49 us for the scaling alone). Bound by memory:
-// 105 us for 2M nodes in FP64 (450 MB, 4.3 TB/s), 48 us for 1M in FP32. 512
-// threads: two blocks per CU, one gathers while the other loads.
+// 105 us for 2M nodes in FP64 (450 MB, 4.3 TB/s), 48 us for 1M in FP32. More
+// blocks than CUs: 512 threads, so that one block gathers while another loads;
+// else 1024 (20k nodes 11.2 -> 8.5 us, 100k 14.7 -> 11.3).
 // ---------------------------------------------------------------------------
-constexpr int kDmdThreads = 512;
+constexpr int kDmdThreads = 1024;
 template <int NDP, bool Q, typename T>
 __global__ void __launch_bounds__(kDmdThreads)
 k_dmd_rows(RowsDmd a, T* __restrict__ val, const int32_t* __restrict__ slice_off,
@@ -1114,11 +1115,11 @@ k_dmd_rows(RowsDmd a, T* __restrict__ val, const int32_t* __restrict__ slice_off
   if (a.d) {
     const int n0 = a.node_start[b], nown = a.node_start[b + 1] - n0;
     const int h0 = a.halo_start[b], nloc = nown + a.halo_start[b + 1] - h0;
-    for (int l = t; l < nloc; l += kDmdThreads)
+    for (int l = t; l < nloc; l += (int)blockDim.x)
       ds[l] = a.d[l < nown ? n0 + l : a.halo[h0 + l - nown]];
     __syncthreads();
   }
-  for (int i = t; i < ns; i += kDmdThreads) {
+  for (int i = t; i < ns; i += (int)blockDim.x) {
     const int s = s0 + i;
     double c[nc], dv[NDP];
 #pragma unroll
@@ -1148,7 +1149,7 @@ k_dmd_rows(RowsDmd a, T* __restrict__ val, const int32_t* __restrict__ slice_off
   // the block's slices: for each of its 16 / group waves, one per row of a thread
   const int q0 = slab_slice[b];
   constexpr int U = kRefChunk;
-  for (int i = wave; i < kSlices; i += kDmdThreads / 64) {
+  for (int i = wave; i < kSlices; i += (int)(blockDim.x >> 6)) {
     const int q = __builtin_amdgcn_readfirstlane(q0 + i % group * kSlices + i / group);
     const int c1 = ref_off[q + 1];
     T* out = val + (size_t)slice_off[q] * 64;
@@ -1485,7 +1486,8 @@ hipError_t rows_dmd(RowsDev* r, int bytes, const RowsDmd& a, hipStream_t stream)
                               hipFuncAttributeMaxDynamicSharedMemorySize, r->lds_max);
       if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(kern, dim3(a.nblocks), dim3(kDmdThreads), lds, stream, a, val,
+    const int threads = a.nblocks <= r->ncu ? kDmdThreads : kDmdThreads / 2;
+    hipLaunchKernelGGL(kern, dim3(a.nblocks), dim3(threads), lds, stream, a, val,
                        r->slice_off.p, r->ref_off.p, r->ref_end.p, r->refs16.p, r->slab_slice.p,
                        r->group);
     return hipGetLastError();

@@ -301,7 +301,7 @@ static int supg_impl(bhip_ctx* c, int kind, double xmul, const double* xel, cons
   }
   if (op != 0 && target_q && c->typext == 'S') {
     // OM 'M=X(M)' first: the target becomes non-symmetric
-    hipLaunchKernelGGL(k_om_slots, dim3(grid_for((int)(6 * (long)L.nslot_pad))), dim3(kThreads), 0,
+    hipLaunchKernelGGL(k_om_slots, dim3(grid_for(6 * (long)L.nslot_pad)), dim3(kThreads), 0,
                        c->stream, 0, 0.0, c->xa.p, (const double*)nullptr, 1, 1, L.nslot_pad,
                        (long)6 * L.nslot_pad);
     HIP_OK(hipGetLastError());
@@ -411,16 +411,16 @@ int bhip_matrix_om(bhip_ctx* c, const char* op, double cc) {
   // the result is non-symmetric when either operand is, or for M + N^T of a 'Q' N
   const bool out_q = code == 0 || m_q || n_q;
   if (out_q && !m_q && code != 0) {
-    hipLaunchKernelGGL(k_om_slots, dim3(grid_for((int)(6 * (long)L.nslot_pad))), dim3(kThreads), 0,
+    hipLaunchKernelGGL(k_om_slots, dim3(grid_for(6 * (long)L.nslot_pad)), dim3(kThreads), 0,
                        c->stream, 0, 0.0, c->xa.p, (const double*)nullptr, 1, 1, L.nslot_pad,
                        (long)6 * L.nslot_pad);
   }
   const long ncol = out_q ? 6 : 3;
-  hipLaunchKernelGGL(k_om_slots, dim3(grid_for((int)(ncol * L.nslot_pad))), dim3(kThreads), 0,
+  hipLaunchKernelGGL(k_om_slots, dim3(grid_for(ncol * L.nslot_pad)), dim3(kThreads), 0,
                      c->stream, code, cc, c->xa.p, c->xa_saved.p, 1, n_q ? 1 : 0, L.nslot_pad,
                      ncol * L.nslot_pad);
   if (code != 0)
-    hipLaunchKernelGGL(k_om_diag, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream, code, cc,
+    hipLaunchKernelGGL(k_om_diag, dim3(c->grid_wide), dim3(kThreads), 0, c->stream, code, cc,
                        c->da.p, c->da_saved.p, L.npoin);
   HIP_OK(hipGetLastError());
   c->typext = out_q ? 'Q' : 'S';

@@ -665,7 +665,7 @@ int bhip_wave_assemble(bhip_ctx* c, const bhip_wave_params* p, const double* eta
     return BHIP_EBADARG;
   const Layout& L = c->L;
   WaveArgs a = wave_args(c, p);
-  hipLaunchKernelGGL(k_wave_nodes, dim3(c->grid_nodes), dim3(kThreads), 0, c->stream, a,
+  hipLaunchKernelGGL(k_wave_nodes, dim3(c->grid_wide), dim3(kThreads), 0, c->stream, a,
                      L.npoin, eta, u, v, kstr, zb);
   hipLaunchKernelGGL(k_wave_grad, dim3(L.nblocks), elem_threads(L),
                      3 * (size_t)L.max_owned * sizeof(double), c->stream, a, eta, u, v);
