@@ -102,6 +102,11 @@ int bhip_ctx_create(int npoin, int nelem, int ndp, const int32_t* ikle,
 int bhip_ctx_destroy(bhip_ctx* ctx);
 /* the HIP stream (hipStream_t) all work of the context runs on */
 void* bhip_ctx_stream(bhip_ctx* ctx);
+/* Order on the device, without waiting on the host: the context's stream after
+ * what is queued on `stream` (hipStream_t) so far, and `stream` after what the
+ * context has queued. Safe from several threads. */
+int bhip_ctx_after_stream(bhip_ctx* ctx, void* stream);
+int bhip_stream_after_ctx(bhip_ctx* ctx, void* stream);
 /* layout statistics: nblocks, max colours per block, element instances
  * (duplicated halo elements included), halo node count */
 int bhip_ctx_stats(const bhip_ctx* ctx, int* nblocks, int* max_colors,

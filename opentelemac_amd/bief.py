@@ -84,6 +84,8 @@ def lib():
         L.bhip_ctx_destroy.argtypes = [_P]
         L.bhip_ctx_stream.argtypes = [_P]
         L.bhip_ctx_stream.restype = _P
+        L.bhip_ctx_after_stream.argtypes = [_P, _P]
+        L.bhip_stream_after_ctx.argtypes = [_P, _P]
         L.bhip_ctx_stats.argtypes = [_P, ctypes.POINTER(_I), ctypes.POINTER(_I),
                                      ctypes.POINTER(ctypes.c_int64),
                                      ctypes.POINTER(ctypes.c_int64)]
@@ -272,7 +274,7 @@ class Context:
             _dev_n(da, self.npoin, "set_matrix: da")
             if ncoef:
                 _dev_n(xa, ncoef * self.nelem, "set_matrix: xa")
-            self._sync_torch()
+            caller = self._sync_torch()
             rc = lib().bhip_matrix_set_dev(self._h, typdia.encode(), typext.encode(),
                                            da.data_ptr(), xa.data_ptr() if xa is not None else None)
             # the copy runs later on the context stream: torch's stream waits
@@ -280,7 +282,7 @@ class Context:
             # the copy has read it. (Not record_stream: the context's stream
             # may be destroyed before the tensor is freed, and torch would
             # then record an event on a stream that no longer exists.)
-            self._join_torch()
+            self._join_torch(caller)
         else:
             da = _host_n_or_none(da, self.npoin, "set_matrix: da")
             npair = self.ndp * (self.ndp - 1) // 2
@@ -336,10 +338,10 @@ class Context:
                     limdir.is_contiguous() and limdir.numel() == n):
                 raise BiefError("dirich: limdir: expected a contiguous int32 CUDA tensor of "
                                 f"{n} values")
-            self._sync_torch()
+            caller = self._sync_torch()
             _check(lib().bhip_dirich_dev(self._h, f.data_ptr(), sm.data_ptr(), fbor.data_ptr(),
                                          limdir.data_ptr(), int(kdir)), "bhip_dirich_dev")
-            self._join_torch()
+            self._join_torch(caller)
             return f, sm
         f = _host_n(f, n, "dirich: f").copy()
         sm = _host_n(sm, n, "dirich: sm").copy()
@@ -356,9 +358,9 @@ class Context:
         receives it on the context stream."""
         if out is not None:
             _dev_n(out, self.npoin, "lump: out")
-            self._sync_torch()
+            caller = self._sync_torch()
             _check(lib().bhip_lump_dev(self._h, float(xmul), out.data_ptr()), "bhip_lump_dev")
-            self._join_torch()
+            self._join_torch(caller)
             return out
         d = np.empty(self.npoin)
         _check(lib().bhip_lump(self._h, float(xmul), d.ctypes.data), "bhip_lump")
@@ -380,10 +382,10 @@ class Context:
         surfac None: the geometry of set_geometry."""
         if surfac is None and getattr(self, "has_geometry", False):
             # no host array at all: queued on the context stream
-            self._sync_torch()
+            caller = self._sync_torch()
             _check(lib().bhip_matrix_mt01aa_dev(self._h, float(xmul), int(accumulate)),
                    "bhip_matrix_mt01aa_dev")
-            self._join_torch()
+            self._join_torch(caller)
         else:
             s = _host_n_or_none(surfac, self.nelem, "surfac")
             _check(lib().bhip_matrix_mt01aa(self._h, float(xmul), _ptr(s), int(accumulate)),
@@ -401,11 +403,11 @@ class Context:
             _dev_n(u, n, "u")
             if v is not None:
                 _dev_n(v, n, "v")
-            self._sync_torch()
+            caller = self._sync_torch()
             _check(lib().bhip_matrix_mt02aa_dev(self._h, int(kind), float(xmul), u.data_ptr(),
                                                 None if v is None else v.data_ptr(),
                                                 int(accumulate)), "bhip_matrix_mt02aa_dev")
-            self._join_torch()
+            self._join_torch(caller)
         else:
             xel, yel = _host_n_or_none(xel, 3 * ne, "xel"), _host_n_or_none(yel, 3 * ne, "yel")
             s = _host_n_or_none(surfac, ne, "surfac")
@@ -434,12 +436,12 @@ class Context:
             for a in (f, g):
                 if a is not None:
                     _dev_n(a, ne, "f, g")
-            self._sync_torch()
+            caller = self._sync_torch()
             _check(lib().bhip_matrix_supg_dev(
                 self._h, int(kind), float(xmul), None if f is None else f.data_ptr(),
                 None if g is None else g.data_ptr(), u.data_ptr(), v.data_ptr(), int(flags),
                 self._OM_OPS[op]), "bhip_matrix_supg_dev")
-            self._join_torch()
+            self._join_torch(caller)
         else:
             geo = [_host_n_or_none(xel, 3 * ne, "xel"), _host_n_or_none(yel, 3 * ne, "yel"),
                    _host_n_or_none(surfac, ne, "surfac")]
@@ -467,10 +469,10 @@ class Context:
             if surfac is not None:
                 raise BiefError("matrix_mt01pp: device fields take the context's geometry")
             _dev_n(z, self.npoin, "z")
-            self._sync_torch()
+            caller = self._sync_torch()
             _check(lib().bhip_matrix_mt01pp_dev(self._h, float(xmul), z.data_ptr(),
                                                 int(accumulate)), "bhip_matrix_mt01pp_dev")
-            self._join_torch()
+            self._join_torch(caller)
         else:
             s = _host_n_or_none(surfac, self.nelem, "surfac")
             z = _host_n(z, self.npoin, "z")
@@ -490,12 +492,12 @@ class Context:
                 raise BiefError("matrix_mt02pp: device fields take the context's geometry")
             for a in (z, f, g, h):
                 _dev_n(a, n, "z, f, g, h")
-            self._sync_torch()
+            caller = self._sync_torch()
             _check(lib().bhip_matrix_mt02pp_dev(self._h, float(xmul), z.data_ptr(), f.data_ptr(),
                                                 g.data_ptr(), h.data_ptr(), int(h_zero),
                                                 int(npou0), int(inchyd), int(mon),
                                                 int(accumulate)), "bhip_matrix_mt02pp_dev")
-            self._join_torch()
+            self._join_torch(caller)
         else:
             arrs = [_host_n_or_none(xel, 3 * ne, "xel"), _host_n_or_none(yel, 3 * ne, "yel"),
                     _host_n_or_none(surfac, ne, "surfac")] + \
@@ -506,29 +508,41 @@ class Context:
         self.typdia, self.typext = "Q", ("Q" if accumulate and self.typext == "Q" else "S")
 
     # ---- MATVEC ---------------------------------------------------------
-    def _on_own_stream(self):
-        import torch
-        return torch.cuda.current_stream().cuda_stream == self.stream_ptr()
-
+    # (ordered in the library: as two torch events each, the handshakes of a
+    # call took about 45 us of host time, now 20)
     def _sync_torch(self):
         """Orders the context stream after the work queued so far on torch's
-        current stream (an event wait on the device, no host round trip);
-        nothing to do when torch already runs on the context's stream."""
+        current stream (an event wait on the device, no host round trip; nothing
+        to do when torch already runs on the context's stream). Returns that
+        stream's handle, for _join_torch."""
         import torch
-        if self._on_own_stream():
-            return
-        ev = torch.cuda.Event()
-        ev.record(torch.cuda.current_stream())
-        self.torch_stream().wait_event(ev)
+        caller = torch.cuda.current_stream().cuda_stream
+        _check(lib().bhip_ctx_after_stream(self._h, caller), "bhip_ctx_after_stream")
+        return caller
 
-    def _join_torch(self):
-        """Orders torch's current stream after the context stream's work."""
+    def _join_torch(self, caller):
+        """Orders the caller's stream after the context stream's work."""
+        _check(lib().bhip_stream_after_ctx(self._h, caller), "bhip_stream_after_ctx")
+
+    def on_own_stream(self, fn, *args):
+        """fn(*args) with torch on the context's stream, ordered with the
+        caller's at both ends: several calls and the tensor operations between
+        them need no handshakes of their own. Tensors that fn returns are
+        marked as used by the caller's stream."""
         import torch
-        if self._on_own_stream():
-            return
-        ev = torch.cuda.Event()
-        ev.record(self.torch_stream())
-        torch.cuda.current_stream().wait_event(ev)
+        caller = torch.cuda.current_stream()
+        if caller.cuda_stream == self.stream_ptr():
+            return fn(*args)
+        self._sync_torch()
+        try:
+            with torch.cuda.stream(self.torch_stream()):
+                out = fn(*args)
+        finally:
+            self._join_torch(caller.cuda_stream)
+        for t in out if isinstance(out, (tuple, list)) else (out,):
+            if torch.is_tensor(t):
+                t.record_stream(caller)
+        return out
 
     def matvec(self, op: str, y, x=None, c: float = 0.0):
         """X = op(A, Y, C) as BIEF MATVEC. Host arrays: returns a new array.
@@ -540,10 +554,10 @@ class Context:
                 x = torch.zeros_like(y)
             _dev_n(y, self.npoin, "matvec: y")
             _dev_n(x, self.npoin, "matvec: x")
-            self._sync_torch()
+            caller = self._sync_torch()
             _check(lib().bhip_matvec_dev(self._h, code, float(c), y.data_ptr(), x.data_ptr()),
                    "bhip_matvec_dev")
-            self._join_torch()
+            self._join_torch(caller)
             return x
         y = _host_n(y, self.npoin, "matvec: y")
         x = np.zeros(self.npoin) if x is None else _host_n(x, self.npoin, "matvec: x").copy()
@@ -567,11 +581,11 @@ class Context:
         _dev_n(b, self.npoin, "solve: b")
         cfg = SolverCfg(slv, precon, krylov, nitmax, eps, precision, inner_eps, inner_nitmax)
         info = SolveInfo()
-        self._sync_torch()
+        caller = self._sync_torch()
         rc = lib().bhip_solve_dev_internal(self._h, ctypes.byref(cfg), x.data_ptr(),
                                            b.data_ptr(), ctypes.byref(info))
         _check(rc, "bhip_solve_dev_internal")
-        self._join_torch()
+        self._join_torch(caller)
         self.typdia = "I" if precon in (2,) else self.typdia
         d = info.as_dict()
         d["status"] = STATUS[rc]
@@ -595,7 +609,7 @@ class Context:
                 and flush.is_contiguous()):
             raise BiefError("time_cg_dir_cold: flush must be a contiguous float64 CUDA tensor")
         ms = ctypes.c_double()
-        self._sync_torch()
+        caller = self._sync_torch()
         _check(lib().bhip_time_cg_dir_cold(self._h, precision, reps,
                                            ctypes.c_void_p(flush.data_ptr()),
                                            flush.numel(), ctypes.byref(ms)),
@@ -624,11 +638,11 @@ class Context:
         if _is_torch(x):
             _dev_n(x, self.npoin, "solve: x")
             _dev_n(b, self.npoin, "solve: b")
-            self._sync_torch()
+            caller = self._sync_torch()
             fn = lib().bhip_solve_dev_restored if restore else lib().bhip_solve_dev
             rc = fn(self._h, ctypes.byref(cfg), x.data_ptr(), b.data_ptr(), ctypes.byref(info))
             _check(rc, "bhip_solve_dev_restored" if restore else "bhip_solve_dev")
-            self._join_torch()
+            self._join_torch(caller)
             if restore:
                 self.typext = getattr(self, "_saved_typext", self.typext)
         else:
@@ -686,10 +700,10 @@ class WaveStep:
                     t.element_size() == 8 and t.is_contiguous() and t.numel() == self.ctx.npoin):
                 raise BiefError(f"{name}: node vectors must be contiguous float64 CUDA tensors "
                                 f"of {self.ctx.npoin} entries")
-        self.ctx._sync_torch()
+        caller = self.ctx._sync_torch()
         _check(getattr(lib(), name)(self.ctx._h, ctypes.byref(p),
                                     *(t.data_ptr() for t in tensors)), name)
-        self.ctx._join_torch()
+        self.ctx._join_torch(caller)
 
     def assemble(self, p, eta, u, v, kstr, zb, rhs):
         self._run("bhip_wave_assemble", p, eta, u, v, kstr, zb, rhs)

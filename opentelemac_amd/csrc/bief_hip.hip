@@ -977,6 +977,8 @@ struct bhip_ctx {
   bhip::Layout L;
   hipStream_t stream = nullptr;
   int device = 0;
+  std::mutex order_mu;
+  hipEvent_t order_ev = nullptr;  // order_streams
   int grid_nodes = 0;  // grid of the node-wise kernels that leave a partial sum per block
   int grid_wide = 0;   // of the others
   // layout on device
@@ -1420,12 +1422,46 @@ int bhip_ctx_destroy(bhip_ctx* c) {
     if (sg.exec) (void)hipGraphExecDestroy(sg.exec);
   if (c->rows) rows_destroy(c->rows);
   if (c->st_host) (void)hipHostFree(c->st_host);
+  if (c->order_ev) (void)hipEventDestroy(c->order_ev);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return BHIP_OK;
 }
 
 void* bhip_ctx_stream(bhip_ctx* c) { return c ? (void*)c->stream : nullptr; }
+
+// `second` after what `first` holds now. One event of the context serves all
+// such calls (a wait keeps the recording it was given); streams of another
+// device than the context's take one of their own.
+static int order_streams(bhip_ctx* c, hipStream_t first, hipStream_t second) {
+  if (first == second) return BHIP_OK;
+  int dev = 0;
+  HIP_OK(hipGetDevice(&dev));
+  if (dev != c->device) {
+    hipEvent_t ev;
+    HIP_OK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    hipError_t e = hipEventRecord(ev, first);
+    if (e == hipSuccess) e = hipStreamWaitEvent(second, ev, 0);
+    (void)hipEventDestroy(ev);
+    HIP_OK(e);
+    return BHIP_OK;
+  }
+  std::lock_guard<std::mutex> one(c->order_mu);
+  if (!c->order_ev) HIP_OK(hipEventCreateWithFlags(&c->order_ev, hipEventDisableTiming));
+  HIP_OK(hipEventRecord(c->order_ev, first));
+  HIP_OK(hipStreamWaitEvent(second, c->order_ev, 0));
+  return BHIP_OK;
+}
+
+int bhip_ctx_after_stream(bhip_ctx* c, void* stream) {
+  if (!c) return BHIP_EBADARG;
+  return order_streams(c, (hipStream_t)stream, c->stream);
+}
+
+int bhip_stream_after_ctx(bhip_ctx* c, void* stream) {
+  if (!c) return BHIP_EBADARG;
+  return order_streams(c, c->stream, (hipStream_t)stream);
+}
 
 int bhip_layout_check(int npoin, int nelem, int ndp, const int32_t* ikle, const double* x,
                       const double* y, int nplan, int block_nodes, int64_t* stats) {

@@ -34,10 +34,15 @@ def supg_system(ctx: bief.Context, mesh, u, v, nu, dt, fn, tetat=1.0, sm0=None):
     if not getattr(ctx, "has_geometry", False):
         xe, ye = mesh.xel_yel()
         ctx.set_geometry(xe, ye, mesh.surfac())
+    if bief._is_torch(u):
+        return ctx.on_own_stream(_supg_system, ctx, u, v, nu, dt, fn, tetat, sm0)
+    if sm0 is not None:
+        sm0 = np.asarray(sm0, dtype=np.float64)
+    return _supg_system(ctx, u, v, nu, dt, np.ascontiguousarray(fn, dtype=np.float64), tetat, sm0)
+
+
+def _supg_system(ctx, u, v, nu, dt, fn, tetat, sm0):
     G = (None, None, None)  # the geometry kept on the device
-    dev = bief._is_torch(u)
-    if not dev:
-        fn = np.ascontiguousarray(fn, dtype=np.float64)
     K = bief.Context.SUPG_KSUPG
     # AM2: centred advection plus the SUPG term (cvdftr.F:398-409)
     ctx.matrix_supg(5, 1.0, *G, u, v, op="M=N")
@@ -49,7 +54,7 @@ def supg_system(ctx: bief.Context, mesh, u, v, nu, dt, fn, tetat=1.0, sm0=None):
     ctx.matrix_mt01aa(1.0 / dt, None)
     ctx.matrix_om("M=X(M)")
     ctx.matrix_supg(5, 1.0 / dt, *G, u, v, flags=K, op="M=M+TN")
-    rhs = fn if sm0 is None else dt * (sm0 if dev else np.asarray(sm0, dtype=np.float64)) + fn
+    rhs = fn if sm0 is None else dt * sm0 + fn
     sm = ctx.matvec("X=AY", rhs)
     sm = sm + (tetat - 1.0) * t2
     ctx.matrix_om("M=M+CN", tetat)
