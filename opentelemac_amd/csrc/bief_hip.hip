@@ -821,7 +821,8 @@ __global__ void k_to_f32(float* __restrict__ out, const double* __restrict__ in,
 // internal-order copies x and b, so SOLVE needs no separate gather.
 // da_in and da_out may be the same array (the context's diagonal in place),
 // or the saved copy and the context's diagonal (OM 'M=N' fused into SOLVE)
-__global__ void k_precd1_nodes(double* x, double* b, const double* xs, const double* bs,
+// B*D also replaces the caller's B, as the reference leaves it.
+__global__ void k_precd1_nodes(double* x, double* b, const double* xs, double* bs,
                                const int32_t* __restrict__ perm, const double* da_in,
                                double* da_out, double* __restrict__ dout, int n, int precon,
                                int typdia_q, int typdia_i) {
@@ -843,7 +844,7 @@ __global__ void k_precd1_nodes(double* x, double* b, const double* xs, const dou
     } else if (da_out != da_in) {
       da_out[i] = a;
     }
-    b[i] = bv * d;
+    b[i] = bs[j] = bv * d;
   }
 }
 
@@ -1909,7 +1910,8 @@ static double clock_khz(bhip_ctx* c) {
 }
 
 // per-system outcome of a CG solve (FP64 or mixed) from the device states;
-// fills c->sys_info and the ensemble summary in *info
+// fills c->sys_info and the ensemble summary in *info; x (unless nullptr) is
+// set to 0 for systems with a zero right-hand side
 static int collect_infos(bhip_ctx* c, double* x, bool mixed, bhip_solve_info* info) {
   SolveState* sh = c->st_host;
   const int g = c->grid_wide;
@@ -1924,6 +1926,10 @@ static int collect_infos(bhip_ctx* c, double* x, bool mixed, bhip_solve_info* in
     si.relat = q.xl_raw >= 1.0;
     if (khz > 0 && q.t_done >= q.t_start) c->sys_latency_ms[sy] = (q.t_done - q.t_start) / khz;
     if (q.zero_rhs) {
+      si.converged = 1;
+      ++nzero;
+      ++nconv;
+      if (!x) continue;
       // X = 0 (gracjg.F:194-202) on this system's nodes
       const int b0 = c->nsys > 1 ? c->sys_blocks_h[sy] : 0;
       const int b1 = c->nsys > 1 ? c->sys_blocks_h[sy + 1] : c->L.nblocks;
@@ -1931,9 +1937,6 @@ static int collect_infos(bhip_ctx* c, double* x, bool mixed, bhip_solve_info* in
       hipLaunchKernelGGL(k_fill<double>, dim3(g), dim3(kThreads), 0, c->stream, x + n0, 0.0,
                          (long)(n1 - n0));
       HIP_OK(hipGetLastError());
-      si.converged = 1;
-      ++nzero;
-      ++nconv;
       continue;
     }
     if (mixed) {
@@ -2204,34 +2207,27 @@ static std::mutex& rows_mutex(int dev) {
   return mu[dev & 63];
 }
 
-// GRACJG as in cg_fp64; the solution is left in xout (x stays the initial one)
-static int cg_rows_fp64(bhip_ctx* c, double* x, double* xout, const double* b, double eps,
-                        int nitmax, bhip_solve_info* info, const std::function<int()>& tail) {
+// GRACJG as in cg_fp64; the solution goes to xout (idx, scale: see RowsCg), X = 0
+// of a zero right-hand side included
+static int cg_rows_fp64(bhip_ctx* c, const double* x, double* xout, const int32_t* idx,
+                        const double* scale, const double* b, double eps, int nitmax,
+                        bhip_solve_info* info) {
   std::lock_guard<std::mutex> one(rows_mutex(c->device));
-  HIP_OK(enqueue_bb_setup(c, b, eps, nitmax, 0, 0.0, 0));
-  EbeArgs<double, double> a = base_args<double, double>(c, c->xa.p, c->da.p);
-  a.y = x;
-  a.b = b;
-  a.out = c->vr.p;
-  a.partial = part_u(c, 0);
-  HIP_OK((launch_ebe<double, double, STAGE_PLAIN, EPI_RESID, FIN_PARTIAL>(c, a, false, c->typdia,
-                                                                          c->typext)));
   RowsCg<double> q = {};
-  q.r0 = c->vr.p;
-  q.x0 = x;
-  q.x = xout;
+  q.b = b;
   q.diag = c->typdia == 'Q' ? c->da.p : nullptr;
-  q.part_rr = part_u(c, 0);
-  q.nblocks = c->L.nblocks;
-  q.sys_blocks = sys_ptr(c->sys_blocks);
+  q.x = xout;
   q.st = c->st_p;
+  q.x0 = x;
+  q.scale = scale;
+  q.idx = idx;
+  q.eps = eps;
+  q.nitmax = std::max(nitmax, 1);
   HIP_OK(rows_cg<double>(c->rows, q, c->stream));
-  int rc;
-  if ((rc = tail())) return rc;
   if (read_state(c)) return BHIP_EDEVICE;
   for (int sy = 0; sy < c->nsys; ++sy)
     if (c->st_host[sy].gave_up) return kGaveUp;
-  return collect_infos(c, xout, false, info);
+  return collect_infos(c, nullptr, false, info);
 }
 
 // mixed precision as in cg_mixed, each inner solve one persistent FP32 launch
@@ -2251,12 +2247,11 @@ static int cg_rows_mixed(bhip_ctx* c, double* x, const double* b, double eps, in
   HIP_OK(enqueue_bb_setup(c, b, eps, nitmax, 1, inner_eps, inner_nitmax, c->reliable ? 1 : 0));
   auto inner = [&]() -> int {
     RowsCg<float> q = {};
-    q.r0 = c->fr.p;
+    q.b = c->fr.p;
     q.x = delta;
     q.diag = c->typdia == 'Q' ? c->da32.p : nullptr;
     q.dlast = c->fdz.p;
     q.st = c->st_p;
-    q.inner = 1;
     HIP_OK(rows_cg<float>(c->rows, q, c->stream));
     return BHIP_OK;
   };
@@ -2398,10 +2393,10 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
                          c->stream));
   }
   int rc;
-  // where the solution is left (the persistent FP64 CG keeps the initial one)
-  double* xsrc = use_rows && !mixed && cfg->slv == 1 ? c->vd1.p : c->vx.p;
-  // X <- X*D (solve.f:637-641) and B <- D*B (as the reference leaves it),
-  // back to the caller's order or copied as they are (internal). A mixed
+  double* xsrc = c->vx.p;  // where the solution is left
+  bool written = false;    // it is in x_dev already
+  // X <- X*D (solve.f:637-641), back to the caller's order or copied as it is
+  // (internal); B <- D*B is in place since the preconditioning. A mixed
   // solve of one system reads X from the solution buffer its state names;
   // an ensemble's first gathers each system's into vx.
   const bool mixed_cg = cfg->slv == 1 && mixed;
@@ -2416,8 +2411,6 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
     }
     hipLaunchKernelGGL(k_x_out, dim3(g), dim3(kThreads), 0, c->stream, x_dev, xsrc,
                        c->vx2.p, stx, diag ? c->vdinv.p : nullptr, idx, n);
-    hipLaunchKernelGGL(k_x_out, dim3(g), dim3(kThreads), 0, c->stream, b_dev, c->vb.p,
-                       nullptr, nullptr, nullptr, idx, n);
     HIP_OK(hipGetLastError());
     return BHIP_OK;
   };
@@ -2458,11 +2451,10 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   } else {
     rc = kGaveUp;
     if (use_rows) {
-      rc = cg_rows_fp64(c, c->vx.p, xsrc, c->vb.p, cfg->eps, cfg->nitmax, info, tail);
-      if (rc == kGaveUp) {
-        c->rows_off = true;
-        xsrc = c->vx.p;
-      }
+      rc = cg_rows_fp64(c, c->vx.p, x_dev, internal ? nullptr : c->perm.p,
+                        diag ? c->vdinv.p : nullptr, c->vb.p, cfg->eps, cfg->nitmax, info);
+      written = rc != kGaveUp;
+      if (rc == kGaveUp) c->rows_off = true;
     }
     if (rc == kGaveUp)
       rc = cg_fp64(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, info, tail);
@@ -2473,7 +2465,7 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   const bool cg = cfg->slv == 1;
   bool zero_any = false;
   for (int sy = 0; cg && sy < c->nsys; ++sy) zero_any = zero_any || c->st_host[sy].zero_rhs;
-  if (!cg || zero_any) {
+  if (!written && (!cg || zero_any)) {
     const int rt = tail();
     if (rt) return rt;
   }

@@ -1,7 +1,8 @@
 // Persistent Krylov kernels on assembled rows (rows.h), MI355X. What follows is
 // CG's; GMRES is built alike and described at its kernel.
 //
-// One launch runs a whole CG solve. Each workgroup (one per CU, 1024 threads)
+// One launch runs a whole CG solve: in FP64 from X and B to X in the caller's
+// order, in FP32 an inner solve of the mixed path. Each workgroup (one per CU, 1024 threads)
 // keeps the residual and the solution of its rows in registers, `group` rows
 // per thread, and D and A D in LDS; the first kFront coefficients of each row
 // stay in registers too where they fit (FP64 groups of 1 and 2, FP32 up to 4).
@@ -405,10 +406,14 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
   SolveState* st = a.st + sys;
   unsigned e = __hip_atomic_load(ra.sy.epoch + ra.ep * ra.nsys + sys, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
-  // (no workgroup writes a field that another may still have to read here: a
+  // FP64: a whole solve; FP32: an inner solve, if the outer test has started one.
+  // (No workgroup writes a field that another may still have to read here: a
   // solve that stops without a meeting would race with a late workgroup)
-  const bool skip = load_relaxed(&st->zero_rhs) || (a.inner && !load_relaxed(&st->fresh)) ||
-                    load_relaxed(ra.sy.abort);
+  constexpr bool kWhole = sizeof(T) == 8;
+  const u64 t_start = wall_clock64();
+  const bool skip =
+      (!kWhole && (load_relaxed(&st->zero_rhs) || !load_relaxed(&st->fresh))) ||
+      load_relaxed(ra.sy.abort);
   if (skip) {
     if (load_relaxed(ra.sy.abort)) store_relaxed(&st->gave_up, 1);
     if (lead)
@@ -426,25 +431,15 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
   T* rh = ah + nh;                         // R of the halo
   T* as = rh + nh;                         // A D of own rows
 
-  // ||r0||^2: the state's, or the partial sums per node block
-  double rr;
-  if (a.part_rr) {
-    const int pb0 = a.sys_blocks ? a.sys_blocks[sys] : 0;
-    const int pb1 = a.sys_blocks ? a.sys_blocks[sys + 1] : a.nblocks;
-    double p = 0.0;
-    for (int i = pb0 + t; i < pb1; i += kSlab) p += a.part_rr[i];
-    const double s = tree_sum<1, 1>([&](int) { return Sums<1>{{p}}; }, sh_sum);
-    if (t == 0) sh_in[0] = s;
-    __syncthreads();
-    rr = sh_in[0];
-    __syncthreads();
-  } else {
+  double rr = 0.0, rr_prev = 1.0, thr = 0.0, xl_raw = 0.0;
+  int m = 0, nitmax = a.nitmax;
+  if constexpr (!kWhole) {
     rr = ld_f64(&st->rr0);
+    m = load_relaxed(&st->m[1]) + 1;
+    rr_prev = ld_f64(&st->rr[1]);
+    thr = ld_f64(&st->eps2xl) * (load_relaxed(&st->use_rr0) ? rr : 1.0);
+    nitmax = load_relaxed(&st->nitmax);
   }
-  int m = load_relaxed(&st->m[1]) + 1;
-  double rr_prev = ld_f64(&st->rr[1]);
-  const double thr = ld_f64(&st->eps2xl) * (load_relaxed(&st->use_rr0) ? ld_f64(&st->rr0) : 1.0);
-  const int nitmax = load_relaxed(&st->nitmax);
 
   RowProduct<T, R> prod;
   unsigned have = 0;  // bit k: this thread has a k-th row
@@ -461,21 +456,28 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
     if (p != 0xffff) {
       const int row = r0 + p;
       have |= 1u << k;
-      rv[k] = a.r0[row];
-      if (a.x0) xv[k] = a.x0[row];
+      rv[k] = a.b[row];
       if constexpr (DQ) dq[k] = a.diag[row];
-      d = rv[k];
-      if (m > 0) d += (T)beta0 * a.dlast[row];
+      if constexpr (kWhole) {
+        d = xv[k] = a.x0[row];
+      } else {
+        d = rv[k];
+        if (m > 0) d += (T)beta0 * a.dlast[row];
+      }
     }
     ds[k * kSlab + t] = d;
     prod.load(ra, val, wg, k);
   }
   for (int h = t; h < nh; h += kSlab) {
     const int g = ra.halo_row[h0 + h];
-    T d = a.r0[g];
-    rh[h] = d;
-    if (m > 0) d += (T)beta0 * a.dlast[g];
-    dh[h] = d;
+    if constexpr (kWhole) {
+      dh[h] = a.x0[g];
+    } else {
+      T d = a.b[g];
+      rh[h] = d;
+      if (m > 0) d += (T)beta0 * a.dlast[g];
+      dh[h] = d;
+    }
   }
   __syncthreads();
 
@@ -555,21 +557,42 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
     return true;
   };
 
-  // stop test (gracjg.F:306-324; strict for the initial residual, :219)
-  bool stop = m == 0 ? rr < thr : rr <= thr;
-  int status = ST_CONVERGED;
-  while (!stop) {
-    // AD
+  auto product = [&]() {
     prod.apply(ra, val, wg, ds, as);
     if constexpr (DQ) {
 #pragma unroll
-      for (int k = 0; k < R; ++k)
-        as[k * kSlab + t] += dq[k] * ds[k * kSlab + t];
+      for (int k = 0; k < R; ++k) as[k * kSlab + t] += dq[k] * ds[k * kSlab + t];
     } else {
 #pragma unroll
-      for (int k = 0; k < R; ++k)
-        as[k * kSlab + t] += ds[k * kSlab + t];
+      for (int k = 0; k < R; ++k) as[k * kSlab + t] += ds[k * kSlab + t];
     }
+  };
+  if constexpr (kWhole) {
+    // R = A X - B, with ||B||^2 (gracjg.F:189-219); D = R
+    product();
+    auto start = [&](int k) -> Sums<kSums> {
+      const double b = (double)rv[k], r = as[k * kSlab + t] - b;
+      rv[k] = as[k * kSlab + t] = r;
+      return {{b * b, r * r, 0.0, 0.0}};
+    };
+    double sum[kSums];
+    if (!meet(start, std::integral_constant<int, kSums>(), std::true_type(), sum)) return;
+    xl_raw = sum[0];
+    rr = sum[1];
+    thr = a.eps * a.eps * (xl_raw < 1.0 ? 1.0 : xl_raw);
+#pragma unroll
+    for (int k = 0; k < R; ++k) ds[k * kSlab + t] = rv[k];
+    if (gang > 1)
+      for (int h = t; h < nh; h += kSlab) rh[h] = dh[h] = ah[h];
+    __syncthreads();
+  }
+  const bool zero = kWhole && sqrt(xl_raw) < 1e-15;  // X = 0 then (gracjg.F:194-202)
+
+  // stop test (gracjg.F:306-324; strict for the initial residual, :219)
+  bool stop = zero || (m == 0 ? rr < thr : rr <= thr);
+  int status = ST_CONVERGED;
+  while (!stop) {
+    product();  // AD
     // D.AD, AD.AD, R.AD, R.R
     auto dots = [&](int k) -> Sums<kSums> {
       if (!(have >> k & 1)) return {};
@@ -625,12 +648,23 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
   for (int k = 0; k < R; ++k)
     if (have >> k & 1) {
       const int row = r0 + rowpos[k * kSlab + t];
-      a.x[row] = xv[k];
-      if (a.dlast) a.dlast[row] = ds[k * kSlab + t];
+      if constexpr (kWhole) {
+        const T x = zero ? (T)0 : a.scale ? xv[k] * a.scale[row] : xv[k];
+        a.x[a.idx ? a.idx[row] : row] = x;
+      } else {
+        a.x[row] = xv[k];
+        if (a.dlast) a.dlast[row] = ds[k * kSlab + t];
+      }
     }
   if (lead) {
-    st->final_m = m;
-    st->final_rr = rr;
+    st->final_m = zero ? 0 : m;
+    st->final_rr = zero ? 0.0 : rr;
+    if constexpr (kWhole) {
+      st->xl_raw = xl_raw;
+      st->xl = xl_raw < 1.0 ? 1.0 : xl_raw;
+      st->zero_rhs = zero;
+      st->t_start = t_start;
+    }
     // the ||R||^2 that built the last direction (continued solves)
     st->rr[0] = rr_prev;
     st->rr[1] = rr_prev;

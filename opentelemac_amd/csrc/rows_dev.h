@@ -42,22 +42,25 @@ struct RowsDmd {
 };
 hipError_t rows_dmd(RowsDev* r, int bytes, const RowsDmd& a, hipStream_t stream);
 
-// One CG solve per system of the context (gracjg.F:248-409), from the
-// residual r0 to the stop, in one launch. Vectors in internal node order.
+// One CG per system of the context (gracjg.F:189-409) in one launch. Vectors in
+// internal node order. FP64: a whole solve of A x = b, from the initial
+// solution to the outcome in the state (gave_up is only ever set). FP32: the
+// inner solve that the outer test has started, if it has, with its state.
 template <typename T>
 struct RowsCg {
-  const T* r0;             // A x - b (FP64), or b - A x of an inner solve (its sign)
-  const T* x0;             // initial solution, or nullptr for zero
-  T* x;                    // solution (not x0: a launch that gives up leaves x0 as it is)
+  const T* b;              // FP64: b; FP32: the residual b - A x the inner solve starts from
+                           // (its sign as the mixed solver keeps it)
   const T* diag;           // diagonal, or nullptr for a unit diagonal
-  T* dlast;                // the previous direction of a continued solve (read), and the
-                           // last direction of this one (written); nullptr: neither
-  const double* part_rr;   // partial sums of ||r0||^2 per node block, or nullptr: the
-                           // state's rr0
-  int nblocks;
-  const int32_t* sys_blocks;
+  T* x;                    // solution; FP64: at idx[i] (or i), times scale[i] if given (not
+                           // x0: a launch that gives up leaves that as it is)
   SolveState* st;
-  int inner;               // an inner solve: only systems with a fresh start
+  const T* x0;             // FP64: initial solution
+  const T* scale;
+  const int32_t* idx;
+  double eps;
+  int nitmax;
+  T* dlast;                // FP32: the previous direction of a continued solve (read), and
+                           // the last direction of this one (written)
 };
 template <typename T>
 hipError_t rows_cg(RowsDev* r, const RowsCg<T>& a, hipStream_t stream);

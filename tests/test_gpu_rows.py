@@ -101,6 +101,43 @@ def test_rows_of_a_diagonal_matrix(gpu):
     ctx.close()
 
 
+@pytest.mark.parametrize("nx,ny", [(20, 12), (120, 90), (514, 510)])
+@pytest.mark.parametrize("precon", [0, 2])
+def test_rows_cg_from_an_initial_solution(gpu, nx, ny, precon):
+    """R = A X0 - B and its exchange inside the launch; a solve that NITMAX ends,
+    one that X0 ends, and a zero right-hand side."""
+    m = M.channel_mesh(nx, ny, 10.0 * nx, 10.0 * ny)
+    sysd = _system(m)
+    rng = np.random.default_rng(7)
+    x0 = rng.normal(size=m.npoin)
+    b = sysd["b"] + 1e-2 * rng.normal(size=m.npoin)
+    A = O.Matrix(sysd["da"], sysd["xa"], "Q", "S")
+
+    def both(x0, b, **kw):
+        kw = dict(dict(slv=1, precon=precon, eps=1e-10, nitmax=3000), **kw)
+        xr, ir, br, _ = O.solve(A, m.ikle, b, x0, **kw)
+        ctx = bief.Context(m)
+        ctx.set_matrix("Q", "S", sysd["da"], sysd["xa"])
+        bh = b.copy()
+        x, info = ctx.solve(x0.copy(), bh, **kw)
+        ctx.close()
+        assert bool(info["converged"]) == bool(ir.converged)
+        return x, xr, info, ir
+
+    x, xr, info, ir = both(x0, b)
+    assert abs(info["niter"] - ir.niter) <= 1
+    assert np.linalg.norm(x - xr) <= 1e-10 * np.linalg.norm(xr)
+    # few iterations: no rounding has grown yet
+    x, xr, info, ir = both(x0, b, nitmax=3)
+    assert info["niter"] == ir.niter == 3
+    assert np.linalg.norm(x - xr) <= 1e-12 * np.linalg.norm(xr)
+    x, _, info, _ = both(xr, b, eps=1e30)
+    assert info["niter"] == 0
+    np.testing.assert_allclose(x, xr, rtol=1e-15)
+    x, _, info, _ = both(x0, np.zeros(m.npoin))
+    assert info["niter"] == 0 and not x.any()
+
+
 def test_more_workgroups_than_the_gpu_holds(gpu):
     """300 systems of one workgroup each: workgroups numbered as they start."""
     meshes = [M.random_small_mesh(4 + k % 5, 5 + k % 3, seed=k) for k in range(300)]
