@@ -684,7 +684,6 @@ __global__ void k_cg_setup(const double* __restrict__ partial, int nblocks,
 // (its state reset on the device, rr0 = ||r'||^2). A system whose inner
 // solve is still running had no residual this step and is left alone, as
 // the residual kernel left it (outer_blocked).
-constexpr int kMaxOuter = 100;  // refinement sweeps of one mixed solve
 __global__ void k_outer_check(const double* __restrict__ partial, int nblocks,
                               const int32_t* __restrict__ sys_blocks, SolveState* st0,
                               int flip) {
@@ -2207,77 +2206,15 @@ static std::mutex& rows_mutex(int dev) {
   return mu[dev & 63];
 }
 
-// GRACJG as in cg_fp64; the solution goes to xout (idx, scale: see RowsCg), X = 0
-// of a zero right-hand side included
-static int cg_rows_fp64(bhip_ctx* c, const double* x, double* xout, const int32_t* idx,
-                        const double* scale, const double* b, double eps, int nitmax,
-                        bhip_solve_info* info) {
+// CG as in cg_fp64 or cg_mixed; the solution goes to q.x, X = 0 of a zero
+// right-hand side included
+static int cg_rows(bhip_ctx* c, bool mixed, const RowsCg& q, bhip_solve_info* info) {
   std::lock_guard<std::mutex> one(rows_mutex(c->device));
-  RowsCg<double> q = {};
-  q.b = b;
-  q.diag = c->typdia == 'Q' ? c->da.p : nullptr;
-  q.x = xout;
-  q.st = c->st_p;
-  q.x0 = x;
-  q.scale = scale;
-  q.idx = idx;
-  q.eps = eps;
-  q.nitmax = std::max(nitmax, 1);
-  HIP_OK(rows_cg<double>(c->rows, q, c->stream));
+  HIP_OK(rows_cg(c->rows, mixed, q, c->stream));
   if (read_state(c)) return BHIP_EDEVICE;
   for (int sy = 0; sy < c->nsys; ++sy)
     if (c->st_host[sy].gave_up) return kGaveUp;
-  return collect_infos(c, nullptr, false, info);
-}
-
-// mixed precision as in cg_mixed, each inner solve one persistent FP32 launch
-static int cg_rows_mixed(bhip_ctx* c, double* x, const double* b, double eps, int nitmax,
-                         double inner_eps, int inner_nitmax, bhip_solve_info* info,
-                         const std::function<int()>& tail) {
-  const Layout& L = c->L;
-  SolveState* sh = c->st_host;
-  HIP_OK(c->vx2.alloc(L.npoin));
-  float* delta = c->fx0.p;
-  std::lock_guard<std::mutex> one(rows_mutex(c->device));
-  if (c->typdia == 'Q') {
-    hipLaunchKernelGGL(k_to_f32, dim3(c->grid_wide), dim3(kThreads), 0, c->stream, c->da32.p,
-                       c->da.p, (long)L.npoin);
-    HIP_OK(hipGetLastError());
-  }
-  HIP_OK(enqueue_bb_setup(c, b, eps, nitmax, 1, inner_eps, inner_nitmax, c->reliable ? 1 : 0));
-  auto inner = [&]() -> int {
-    RowsCg<float> q = {};
-    q.b = c->fr.p;
-    q.x = delta;
-    q.diag = c->typdia == 'Q' ? c->da32.p : nullptr;
-    q.dlast = c->fdz.p;
-    q.st = c->st_p;
-    HIP_OK(rows_cg<float>(c->rows, q, c->stream));
-    return BHIP_OK;
-  };
-  int rc = mixed_outer_step(c, x, b, delta, true);
-  int& hint_out = c->iter_hint[2];  // inner solves of one mixed solve
-  int nout = std::min(std::max(hint_out, 1), 8);
-  for (int rounds = 0;; ++rounds) {
-    for (int k = 0; k < nout && !rc; ++k) {
-      rc = inner();
-      if (!rc) rc = mixed_outer_step(c, x, b, delta, false);
-    }
-    if (rc || (rc = tail())) return rc;
-    if (read_state(c)) return BHIP_EDEVICE;
-    bool all = true;
-    for (int sy = 0; sy < c->nsys; ++sy) {
-      if (sh[sy].gave_up) return kGaveUp;
-      all = all && sh[sy].outer_done != 0;
-    }
-    if (all) break;
-    if (rounds > 2 * kMaxOuter) return BHIP_EDEVICE;
-    nout = 1;
-  }
-  int maxout = 0;
-  for (int sy = 0; sy < c->nsys; ++sy) maxout = std::max(maxout, sh[sy].outer_count);
-  hint_out = maxout;
-  return collect_infos(c, x, true, info);
+  return collect_infos(c, nullptr, mixed, info);
 }
 
 }  // namespace bhip
@@ -2368,6 +2305,8 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   const bool use_rows = c->rows && !c->rows_off && td != '0' &&
                         (cfg->slv == 1 || (cfg->slv == 7 && rows_gmres_fits(c->rows, row_bytes)));
   const bool by_block = use_rows && rows_by_block(c->rows);
+  // mixed CG takes its FP64 residuals from rows too
+  const bool both = mixed && cfg->slv == 1;
   if (use_rows) HIP_OK(rows_reserve(c->rows, row_bytes));
   if (diag) {
     // PRECD1 (precd1.f:90-149), X and B taken from the caller's vectors
@@ -2387,10 +2326,10 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
     RowsDmd a = {xa_src, c->xa.p, diag && c->ncoef > 0 ? c->vdinv.p : nullptr, L.ndp, L.nslot_pad, L.nblocks,
                  L.max_local, c->typext == 'Q', c->lid.p, c->node_start.p, c->halo_start.p,
                  c->halo.p, c->color_off.p};
-    HIP_OK(rows_dmd(c->rows, row_bytes, a, c->stream));
+    HIP_OK(rows_dmd(c->rows, row_bytes, both, a, c->stream));
   } else if (use_rows) {
-    HIP_OK(rows_assemble(c->rows, row_bytes, c->xa.p, L.nslot_pad, npair, c->typext == 'Q',
-                         c->stream));
+    HIP_OK(rows_assemble(c->rows, row_bytes, both, c->xa.p, L.nslot_pad, npair,
+                         c->typext == 'Q', c->stream));
   }
   int rc;
   double* xsrc = c->vx.p;  // where the solution is left
@@ -2414,6 +2353,25 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
     HIP_OK(hipGetLastError());
     return BHIP_OK;
   };
+  auto on_rows = [&](double inner_eps, int inner_nitmax) -> int {
+    RowsCg q = {};
+    q.b = c->vb.p;
+    q.diag = c->typdia == 'Q' ? c->da.p : nullptr;
+    q.x0 = c->vx.p;
+    q.x = x_dev;
+    q.scale = diag ? c->vdinv.p : nullptr;
+    q.idx = internal ? nullptr : c->perm.p;
+    q.st = c->st_p;
+    q.eps = cfg->eps;
+    q.nitmax = std::max(cfg->nitmax, 1);
+    q.inner_eps = inner_eps;
+    q.inner_nitmax = std::max(inner_nitmax, 1);
+    q.reliable = c->reliable ? 1 : 0;
+    const int r = cg_rows(c, mixed, q, info);
+    written = r != kGaveUp;
+    if (r == kGaveUp) c->rows_off = true;
+    return r;
+  };
   if (cfg->slv == 6) {
     rc = bhip::cgstab_fp64(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, info);
   } else if (cfg->slv == 7) {
@@ -2436,26 +2394,11 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
     double ie = cfg->inner_eps > 0 ? cfg->inner_eps : 1e-4;
     int inn = cfg->inner_nitmax > 0 ? cfg->inner_nitmax : std::max(cfg->nitmax, 1);
     const int nit = std::max(cfg->nitmax, 1);
-    rc = kGaveUp;
-    if (use_rows) {
-      rc = cg_rows_mixed(c, c->vx.p, c->vb.p, cfg->eps, nit, ie, inn, info, tail);
-      if (rc == kGaveUp) {
-        // from the solution its finished inner solves have left
-        c->rows_off = true;
-        hipLaunchKernelGGL(k_xpar_gather, dim3(L.nblocks), dim3(kThreads), 0, c->stream, c->vx.p,
-                           c->vx2.p, c->node_start.p, sys_ptr(c->block_sys), c->st_p);
-      }
-    }
+    rc = use_rows ? on_rows(ie, inn) : kGaveUp;
     if (rc == kGaveUp)
       rc = cg_mixed(c, c->vx.p, c->vb.p, cfg->eps, nit, ie, inn, xa32_ready, info, tail);
   } else {
-    rc = kGaveUp;
-    if (use_rows) {
-      rc = cg_rows_fp64(c, c->vx.p, x_dev, internal ? nullptr : c->perm.p,
-                        diag ? c->vdinv.p : nullptr, c->vb.p, cfg->eps, cfg->nitmax, info);
-      written = rc != kGaveUp;
-      if (rc == kGaveUp) c->rows_off = true;
-    }
+    rc = use_rows ? on_rows(0.0, 0) : kGaveUp;
     if (rc == kGaveUp)
       rc = cg_fp64(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, info, tail);
   }

@@ -1,13 +1,13 @@
 // Persistent Krylov kernels on assembled rows (rows.h), MI355X. What follows is
 // CG's; GMRES is built alike and described at its kernel.
 //
-// One launch runs a whole CG solve: in FP64 from X and B to X in the caller's
-// order, in FP32 an inner solve of the mixed path. Each workgroup (one per CU, 1024 threads)
-// keeps the residual and the solution of its rows in registers, `group` rows
-// per thread, and D and A D in LDS; the first kFront coefficients of each row
-// stay in registers too where they fit (FP64 groups of 1 and 2, FP32 up to 4).
-// Larger groups read the matrix again each iteration, out of the last-level
-// cache (120 MB for 2M rows in FP64).
+// One launch runs a whole CG solve, from X and B to X in the caller's order.
+// Mixed precision: FP64 residuals on FP64 rows with X in LDS, and between them
+// inner solves on FP32 rows. Each workgroup (one per CU, 1024 threads) keeps the
+// residual and the (inner) solution of its rows in registers, `group` rows per
+// thread, and D and A D in LDS; the first coefficients of each row stay in
+// registers too where they fit (RowProduct). Larger groups read the matrix again
+// each iteration, out of the last-level cache (120 MB for 2M rows in FP64).
 //
 // Workgroups meet once per iteration: D.AD, AD.AD, R.AD and R.R together, with
 // the exchange of A D of the halo rows. RO is R.R / D.AD; the next ||R||^2 is
@@ -22,12 +22,15 @@
 // workgroups, 1.6 for 64, 2.0 for 128, 2.8 for 256 (one place instead of 8:
 // 4.0 for 256; two levels of 16: 3.5).
 //
-// us per iteration, FP64 / FP32 rows: 1.4 / 1.7 (1,000 nodes, one workgroup),
-// 3.2 / 3.1 (20k), 3.9 / 3.7 (100k), 4.7 / 4.7 (260k), 5.8 / 5.5 (500k), 14.0 /
-// 7.9 (1M), 24.4 / 16.7 (2M). The two-kernel CG takes 15 at 20k, 50 (FP64) at
-// 2M and 22 (FP32) at 1M. What bounds it: below 500k the meeting (two trips
-// through memory, 1.7 us for 20 workgroups, 3.5 for 245), then the matrix
-// (8.0 TB/s in FP64 and 8.7 in FP32 at 2M rows).
+// us per iteration, FP64 / mixed: 1.4 / 1.6 (1,000 nodes, one workgroup), 3.2 /
+// 3.1 (20k), 3.9 / 3.7 (100k), 4.9 / 4.5 (260k), 5.8 / 5.4 (500k), 14.0 / 7.9 (1M),
+// 24.4 / 17.7 (2M). The two-kernel CG takes 15 at 20k, 50 (FP64) at 2M and 22 (FP32)
+// at 1M. Beside the iterations a solve takes 75 to 130 us up to 500k nodes (PRECD1,
+// the rows, this launch's start, the state back on the host) and 310 / 380 at 2M.
+// What bounds it: below 500k the meeting (two trips through memory, 1.7 us for 20
+// workgroups, 3.5 for 245), then the matrix (8.0 TB/s in FP64 at 2M rows) and, in
+// FP32 at 2M, registers (33 spilled: with one launch per inner solve 16.7, but the
+// launches take what that gains).
 //
 // Sums are binary trees over the rows' leaf numbers (rows.h) and do not depend
 // on how many rows a workgroup holds: a system gives the same bits alone and
@@ -257,14 +260,13 @@ __device__ inline double tree_sum(F&& val, double* sh) {
 // for the ids, all in flight at once
 template <typename T, int W>
 __device__ inline T row_dot(const T* __restrict__ v, const unsigned* __restrict__ id,
-                            unsigned lane, const T* ys) {
+                            unsigned lane, const T* ys, T s = (T)0) {
   T c[W];
   unsigned i[(W + 1) / 2];
 #pragma unroll
   for (int j = 0; j < (W + 1) / 2; ++j) i[j] = id[j * 64 + lane];
 #pragma unroll
   for (int j = 0; j < W; ++j) c[j] = v[j * 64 + lane];
-  T s = (T)0;
 #pragma unroll
   for (int j = 0; j < W; ++j) s += c[j] * ys[j & 1 ? i[j / 2] >> 16 : i[j / 2] & 0xffffu];
   return s;
@@ -278,6 +280,7 @@ __device__ inline T slice_dot(const T* __restrict__ v, const unsigned* __restric
   id += from * 32;
   w -= from;
   T s = (T)0;
+#pragma nounroll
   while (w >= C) {
     s += row_dot<T, C>(v, id, lane, ys);
     v += C * 64;
@@ -301,31 +304,30 @@ __device__ inline T slice_dot(const T* __restrict__ v, const unsigned* __restric
   }
 }
 
-// The first kFront entries of one row, kept in registers for a whole solve.
+// The first F entries of one row, kept in registers for a whole solve.
 // Slices with fewer read their last one again and multiply it by zero.
-constexpr int kFront = 8;
-template <typename T>
+template <typename T, int F>
 struct RowFront {
-  T c[kFront];
-  unsigned i[kFront / 2];  // two ids each
+  T c[F];
+  unsigned i[F / 2];  // two ids each
 };
-template <typename T>
-__device__ inline void load_front(RowFront<T>& f, const T* __restrict__ v,
+template <typename T, int F>
+__device__ inline void load_front(RowFront<T, F>& f, const T* __restrict__ v,
                                   const unsigned* __restrict__ id, unsigned lane, int w) {
   const int last = max(w - 1, 0);
 #pragma unroll
-  for (int j = 0; j < kFront / 2; ++j) f.i[j] = (id + min(j, last / 2) * 64)[lane];
+  for (int j = 0; j < F / 2; ++j) f.i[j] = (id + min(j, last / 2) * 64)[lane];
 #pragma unroll
-  for (int j = 0; j < kFront; ++j) {
+  for (int j = 0; j < F; ++j) {
     const T c = (v + min(j, last) * 64)[lane];
     f.c[j] = j < w ? c : (T)0;
   }
 }
-template <typename T>
-__device__ inline T front_dot(const RowFront<T>& f, const T* ys) {
+template <typename T, int F>
+__device__ inline T front_dot(const RowFront<T, F>& f, const T* ys) {
   T s = (T)0;
 #pragma unroll
-  for (int j = 0; j < kFront; ++j)
+  for (int j = 0; j < F; ++j)
     s += f.c[j] * ys[j & 1 ? f.i[j / 2] >> 16 : f.i[j / 2] & 0xffffu];
   return s;
 }
@@ -336,10 +338,14 @@ __device__ inline T front_dot(const RowFront<T>& f, const T* ys) {
 template <typename T, int R>
 struct RowProduct {
   static constexpr bool kKeep = R * sizeof(T) <= 16;
-  RowFront<T> front[kKeep ? R : 1];
+  // (FP32, 4 rows: 8 entries each would be 48 of the 128 registers; the spills
+  // take longer than reading 4 of them again, 1M nodes 10.8 us per iteration
+  // instead of 7.6)
+  static constexpr int kFront = sizeof(T) == 4 && R == 4 ? 4 : 8;
+  RowFront<T, kFront> front[kKeep ? R : 1];
   int wid[kKeep ? R : 1];
   // the slice of this wave's k-th rows: its coefficients, id words and width
-  static __device__ inline int slice(const RowArgs& ra, const T* val, int wg, int k, const T*& v,
+  static __device__ __forceinline__ int slice(const RowArgs& ra, const T* val, int wg, int k, const T*& v,
                                      const unsigned*& id) {
     const int q = __builtin_amdgcn_readfirstlane((wg * R + k) * kSlices + (int)(threadIdx.x >> 6));
     const int o = ra.slice_off[q];
@@ -347,7 +353,7 @@ struct RowProduct {
     id = ra.ids + (size_t)ra.pair_off[q] * 64;
     return ra.slice_off[q + 1] - o;
   }
-  __device__ inline void load(const RowArgs& ra, const T* val, int wg, int k) {
+  __device__ __forceinline__ void load(const RowArgs& ra, const T* val, int wg, int k) {
     if constexpr (kKeep) {
       const T* v;
       const unsigned* id;
@@ -355,7 +361,7 @@ struct RowProduct {
       load_front(front[k], v, id, threadIdx.x & 63, wid[k]);
     }
   }
-  __device__ inline void apply(const RowArgs& ra, const T* val, int wg, const T* ds, T* as) const {
+  __device__ __forceinline__ void apply(const RowArgs& ra, const T* val, int wg, const T* ds, T* as) const {
     const int t = threadIdx.x, lane = t & 63;
     if constexpr (kKeep) {
 #pragma unroll
@@ -364,8 +370,19 @@ struct RowProduct {
         if (wid[k] > kFront) {
           const T* v;
           const unsigned* id;
-          slice(ra, val, wg, k, v, id);
-          s += slice_dot<4>(v, id, lane, kFront, wid[k], ds);
+          const int w = slice(ra, val, wg, k, v, id);
+          // (a row's first 8 terms are one chain whatever the registers hold)
+          if constexpr (kFront == 4) {
+            const T* v4 = v + 4 * 64;
+            const unsigned* id4 = id + 2 * 64;
+            switch (w) {
+              case 5: s = row_dot<T, 1>(v4, id4, lane, ds, s); break;
+              case 6: s = row_dot<T, 2>(v4, id4, lane, ds, s); break;
+              case 7: s = row_dot<T, 3>(v4, id4, lane, ds, s); break;
+              default: s = row_dot<T, 4>(v4, id4, lane, ds, s);
+            }
+          }
+          if (kFront == 8 || w > 8) s += slice_dot<4>(v, id, lane, 8, w, ds);
         }
         as[k * kSlab + t] = s;
         // (one slab's gathers at a time)
@@ -388,7 +405,7 @@ struct RowProduct {
 // ---------------------------------------------------------------------------
 template <typename T, int R, bool DQ>
 __global__ void __launch_bounds__(kSlab)
-k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
+k_cg_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ val64, RowsCg a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ double sh_sum[kSums * kRowWaves];
   __shared__ double sh_in[kRowWaves];
@@ -406,16 +423,10 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
   SolveState* st = a.st + sys;
   unsigned e = __hip_atomic_load(ra.sy.epoch + ra.ep * ra.nsys + sys, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
-  // FP64: a whole solve; FP32: an inner solve, if the outer test has started one.
-  // (No workgroup writes a field that another may still have to read here: a
-  // solve that stops without a meeting would race with a late workgroup)
-  constexpr bool kWhole = sizeof(T) == 8;
+  constexpr bool kMixed = sizeof(T) == 4;
   const u64 t_start = wall_clock64();
-  const bool skip =
-      (!kWhole && (load_relaxed(&st->zero_rhs) || !load_relaxed(&st->fresh))) ||
-      load_relaxed(ra.sy.abort);
-  if (skip) {
-    if (load_relaxed(ra.sy.abort)) store_relaxed(&st->gave_up, 1);
+  if (load_relaxed(ra.sy.abort)) {
+    store_relaxed(&st->gave_up, 1);
     if (lead)
       __hip_atomic_store(ra.sy.epoch + (1 - ra.ep) * ra.nsys + sys, e, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
@@ -425,58 +436,56 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
   const uint16_t* rowpos = ra.rowpos + (size_t)wg * R * kSlab;
   const int h0 = ra.halo_off[wg], nh = ra.halo_off[wg + 1] - h0;
   const int x0 = ra.exp_off[wg], nx = ra.exp_off[wg + 1] - x0;
+  // (D first: its gathers' addresses then have a constant base)
   T* ds = reinterpret_cast<T*>(smem_raw);  // D: own rows, then halo
   T* dh = ds + R * kSlab;
   T* ah = dh + nh;                         // A D of the halo as it arrives
   T* rh = ah + nh;                         // R of the halo
   T* as = rh + nh;                         // A D of own rows
+  // mixed: X, own rows, then halo
+  double* xs = reinterpret_cast<double*>(smem_raw) + (2 * R * kSlab + 3 * nh + 1) / 2;
 
   double rr = 0.0, rr_prev = 1.0, thr = 0.0, xl_raw = 0.0;
   int m = 0, nitmax = a.nitmax;
-  if constexpr (!kWhole) {
-    rr = ld_f64(&st->rr0);
-    m = load_relaxed(&st->m[1]) + 1;
-    rr_prev = ld_f64(&st->rr[1]);
-    thr = ld_f64(&st->eps2xl) * (load_relaxed(&st->use_rr0) ? rr : 1.0);
-    nitmax = load_relaxed(&st->nitmax);
-  }
+  // mixed: inner solves started, their iterations so far, whether the last
+  // one's direction can be continued
+  int outer = 0, itot = 0;
+  bool cont = false;
 
   RowProduct<T, R> prod;
   unsigned have = 0;  // bit k: this thread has a k-th row
   T rv[R], xv[R], dq[DQ ? R : 1];
-  const double beta0 = m == 0 ? 0.0 : rr / rr_prev;
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     // (a few rows' addresses at a time)
     if constexpr (R >= 4) __builtin_amdgcn_sched_barrier(0);
     rv[k] = xv[k] = (T)0;
     if constexpr (DQ) dq[k] = (T)0;
-    T d = (T)0;
+    double x = 0.0;
     const int p = rowpos[k * kSlab + t];
     if (p != 0xffff) {
       const int row = r0 + p;
       have |= 1u << k;
-      rv[k] = a.b[row];
-      if constexpr (DQ) dq[k] = a.diag[row];
-      if constexpr (kWhole) {
-        d = xv[k] = a.x0[row];
-      } else {
-        d = rv[k];
-        if (m > 0) d += (T)beta0 * a.dlast[row];
-      }
+      x = a.x0[row];
+      if constexpr (!kMixed) rv[k] = a.b[row];
+      if constexpr (DQ) dq[k] = (T)a.diag[row];
     }
-    ds[k * kSlab + t] = d;
+    if constexpr (kMixed) {
+      xs[k * kSlab + t] = x;
+      ds[k * kSlab + t] = (T)0;
+    } else {
+      ds[k * kSlab + t] = xv[k] = x;
+    }
     prod.load(ra, val, wg, k);
   }
   for (int h = t; h < nh; h += kSlab) {
-    const int g = ra.halo_row[h0 + h];
-    if constexpr (kWhole) {
-      dh[h] = a.x0[g];
+    const int row = ra.halo_row[h0 + h];
+    const double x = a.x0[row];
+    if constexpr (kMixed) {
+      xs[R * kSlab + h] = x;
+      dh[h] = (T)0;
     } else {
-      T d = a.b[g];
-      rh[h] = d;
-      if (m > 0) d += (T)beta0 * a.dlast[g];
-      dh[h] = d;
+      dh[h] = x;
     }
   }
   __syncthreads();
@@ -567,7 +576,11 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
       for (int k = 0; k < R; ++k) as[k * kSlab + t] += ds[k * kSlab + t];
     }
   };
-  if constexpr (kWhole) {
+  bool zero = false;  // ||B|| is 0, so X = 0 (gracjg.F:194-202)
+  bool stop;
+  int status = ST_CONVERGED;
+  double rr_out = 0.0;  // mixed: ||R||^2 in FP64
+  if constexpr (!kMixed) {
     // R = A X - B, with ||B||^2 (gracjg.F:189-219); D = R
     product();
     auto start = [&](int k) -> Sums<kSums> {
@@ -585,12 +598,72 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
     if (gang > 1)
       for (int h = t; h < nh; h += kSlab) rh[h] = dh[h] = ah[h];
     __syncthreads();
+    zero = sqrt(xl_raw) < 1e-15;
+    // stop test (gracjg.F:306-324; strict for the initial residual, :219)
+    stop = zero || rr < thr;
   }
-  const bool zero = kWhole && sqrt(xl_raw) < 1e-15;  // X = 0 then (gracjg.F:194-202)
-
-  // stop test (gracjg.F:306-324; strict for the initial residual, :219)
-  bool stop = zero || (m == 0 ? rr < thr : rr <= thr);
-  int status = ST_CONVERGED;
+  for (;;) {
+  if constexpr (kMixed) {
+    // R = B - A X in FP64 with its norm, and ||B||^2; FP32 from here on
+    // (through memory, so that the product can be a rolled loop)
+    // (opaque: addresses made here, not kept over the inner solves)
+    int tt = t;
+    asm volatile("" : "+v"(tt));
+    double* res = a.res + (size_t)wg * R * kSlab;
+#pragma nounroll
+    for (int k = 0; k < R; ++k) {
+      const double* v;
+      const unsigned* id;
+      const int w = RowProduct<double, R>::slice(ra, val64, wg, k, v, id);
+      double s = slice_dot<8>(v, id, lane, 0, w, xs);
+      const int p = rowpos[k * kSlab + tt];
+      double q = 0.0;
+      if (p != 0xffff) {
+        const double x = xs[k * kSlab + tt];
+        if constexpr (DQ) s += a.diag[r0 + p] * x; else s += x;
+        q = a.b[r0 + p] - s;
+      }
+      res[k * kSlab + tt] = q;
+    }
+    auto start = [&](int k) -> Sums<kSums> {
+      const int p = rowpos[k * kSlab + tt];
+      const double q = res[k * kSlab + tt], b = p != 0xffff ? a.b[r0 + p] : 0.0;
+      as[k * kSlab + t] = rv[k] = (T)q;
+      return {{b * b, q * q, 0.0, 0.0}};
+    };
+    double sum[kSums];
+    if (!meet(start, std::integral_constant<int, kSums>(), std::true_type(), sum)) return;
+    xl_raw = sum[0];
+    rr_out = sum[1];
+    const double eps2 = a.eps * a.eps * (xl_raw < 1.0 ? 1.0 : xl_raw);
+    zero = sqrt(xl_raw) < 1e-15;
+    const int left = a.nitmax - itot;
+    if (zero || rr_out <= eps2 || left <= 0 || outer >= kMaxOuter) {
+      status = zero || rr_out <= eps2 ? ST_CONVERGED : ST_MAXITER;
+      break;
+    }
+    ++outer;
+    // the inner solve: D = R, or continued R + BETA D
+    rr = rr_out;
+    thr = a.inner_eps * a.inner_eps * rr;
+    nitmax = min(a.inner_nitmax, left) + (cont ? 1 : 0);
+    m = cont ? 1 : 0;
+    const T beta = (T)(cont ? rr / rr_prev : 0.0);
+    if (!cont) rr_prev = 1.0;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      xv[k] = (T)0;
+      ds[k * kSlab + t] = cont ? rv[k] + beta * ds[k * kSlab + t] : rv[k];
+    }
+    if (gang > 1)
+      for (int h = tt; h < nh; h += kSlab) {
+        rh[h] = ah[h];
+        dh[h] = cont ? ah[h] + beta * dh[h] : ah[h];
+      }
+    __syncthreads();
+    status = ST_CONVERGED;
+    stop = m == 0 ? rr < thr : rr <= thr;
+  }
   while (!stop) {
     product();  // AD
     // D.AD, AD.AD, R.AD, R.R
@@ -644,34 +717,52 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, RowsCg<T> a) {
     }
     __syncthreads();
   }
+  if constexpr (!kMixed) break;
+  const int used = m - (cont ? 1 : 0);
+  itot += used;
+  cont = a.reliable && used >= 1 && status == ST_CONVERGED;
+  int tx = t;
+  asm volatile("" : "+v"(tx));
+  // X -= what the inner solve has found, halo included. (One sum, although
+  // nobody wants it: no workgroup may be two meetings ahead of another.)
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    if constexpr (kMixed) xs[k * kSlab + tx] -= (double)xv[k];
+    as[k * kSlab + tx] = xv[k];
+  }
+  auto none = [&](int) -> Sums<1> { return {{0.0}}; };
+  double sum0;
+  if (!meet(none, std::integral_constant<int, 1>(), std::true_type(), &sum0)) return;
+  if (gang > 1)
+    for (int h = tx; h < nh; h += kSlab) xs[R * kSlab + h] -= (double)ah[h];
+  __syncthreads();
+  }
 #pragma unroll
   for (int k = 0; k < R; ++k)
     if (have >> k & 1) {
       const int row = r0 + rowpos[k * kSlab + t];
-      if constexpr (kWhole) {
-        const T x = zero ? (T)0 : a.scale ? xv[k] * a.scale[row] : xv[k];
-        a.x[a.idx ? a.idx[row] : row] = x;
-      } else {
-        a.x[row] = xv[k];
-        if (a.dlast) a.dlast[row] = ds[k * kSlab + t];
-      }
+      double x = (double)xv[k];
+      if constexpr (kMixed) x = xs[k * kSlab + t];
+      if (a.scale) x *= a.scale[row];
+      a.x[a.idx ? a.idx[row] : row] = zero ? 0.0 : x;
     }
   if (lead) {
-    st->final_m = zero ? 0 : m;
-    st->final_rr = zero ? 0.0 : rr;
-    if constexpr (kWhole) {
-      st->xl_raw = xl_raw;
-      st->xl = xl_raw < 1.0 ? 1.0 : xl_raw;
-      st->zero_rhs = zero;
-      st->t_start = t_start;
+    st->xl_raw = xl_raw;
+    st->xl = xl_raw < 1.0 ? 1.0 : xl_raw;
+    st->zero_rhs = zero;
+    st->t_start = t_start;
+    if constexpr (kMixed) {
+      st->rr_outer = zero ? 0.0 : rr_out;
+      st->outer_count = outer;
+      st->inner_total = itot;
+      st->outer_status = status;
+      st->outer_done = 1;
+    } else {
+      st->final_m = zero ? 0 : m;
+      st->final_rr = zero ? 0.0 : rr;
     }
-    // the ||R||^2 that built the last direction (continued solves)
-    st->rr[0] = rr_prev;
-    st->rr[1] = rr_prev;
     st->t_done = wall_clock64();
-    store_relaxed(&st->done1, (m << 2) | status);
-    store_relaxed(&st->done, status);
-    store_relaxed(&st->stop, 1);
+    st->done = status;
     __hip_atomic_store(ra.sy.epoch + (1 - ra.ep) * ra.nsys + sys, e, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -1133,7 +1224,7 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, RowsGmres a, T* basis, T* hb
 constexpr int kDmdThreads = 1024;
 template <int NDP, bool Q, typename T>
 __global__ void __launch_bounds__(kDmdThreads)
-k_dmd_rows(RowsDmd a, T* __restrict__ val, const int32_t* __restrict__ slice_off,
+k_dmd_rows(RowsDmd a, T* __restrict__ val, double* __restrict__ val64, const int32_t* __restrict__ slice_off,
            const int32_t* __restrict__ ref_off, const uint8_t* __restrict__ ref_end,
            const uint16_t* __restrict__ refs, const int32_t* __restrict__ slab_slice, int group) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -1187,6 +1278,7 @@ k_dmd_rows(RowsDmd a, T* __restrict__ val, const int32_t* __restrict__ slice_off
     const int q = __builtin_amdgcn_readfirstlane(q0 + i % group * kSlices + i / group);
     const int c1 = ref_off[q + 1];
     T* out = val + (size_t)slice_off[q] * 64;
+    double* out64 = val64 + (size_t)slice_off[q] * 64;
     double s = 0.0;
     for (int c = ref_off[q]; c < c1; c += U) {
       const uint16_t* p = refs + (size_t)c * 64;
@@ -1201,6 +1293,10 @@ k_dmd_rows(RowsDmd a, T* __restrict__ val, const int32_t* __restrict__ slice_off
         if (ends >> u & 1) {
           out[lane] = (T)s;
           out += 64;
+          if constexpr (sizeof(T) == 4) {
+            if (val64) out64[lane] = s;
+            out64 += 64;
+          }
           s = 0.0;
         }
       }
@@ -1215,7 +1311,7 @@ k_dmd_rows(RowsDmd a, T* __restrict__ val, const int32_t* __restrict__ slice_off
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ void __launch_bounds__(256)
-k_rows_assemble(T* __restrict__ val, const double* __restrict__ xa,
+k_rows_assemble(T* __restrict__ val, double* __restrict__ val64, const double* __restrict__ xa,
                 const int32_t* __restrict__ slice_off, const int32_t* __restrict__ ref_off,
                 const uint8_t* __restrict__ ref_end, const int32_t* __restrict__ refs, int nslice,
                 unsigned lower) {
@@ -1227,6 +1323,7 @@ k_rows_assemble(T* __restrict__ val, const double* __restrict__ xa,
   if (q >= nslice) return;
   const int c0 = ref_off[q], c1 = ref_off[q + 1];
   T* out = val + (size_t)slice_off[q] * 64;
+  double* out64 = val64 + (size_t)slice_off[q] * 64;
   double s = 0.0;
   constexpr int U = kRefChunk;
   auto load = [&](int c, int (&r)[U]) {
@@ -1252,6 +1349,10 @@ k_rows_assemble(T* __restrict__ val, const double* __restrict__ xa,
       if (ends >> u & 1) {
         out[lane] = (T)s;
         out += 64;
+        if constexpr (sizeof(T) == 4) {
+          if (val64) out64[lane] = s;
+          out64 += 64;
+        }
         s = 0.0;
       }
     }
@@ -1312,6 +1413,7 @@ struct RowsDev {
   Buf<uint8_t> ref_end;
   Buf<double> v64;
   Buf<float> v32;
+  Buf<double> res;  // mixed CG: FP64 residual of each row
   Buf<u64> words;
   SyncWords sy[3];  // CG FP64, CG FP32, GMRES
   int ep[3] = {0, 0, 0};
@@ -1324,8 +1426,9 @@ struct RowsDev {
 };
 
 static size_t cg_lds(const RowsDev& r, int bytes) {
-  // D and A D of own rows; D, A D and R of the halo
-  return ((size_t)2 * r.group * kSlab + (size_t)3 * r.max_halo) * bytes;
+  // D and A D of own rows; D, A D and R of the halo; mixed: X of both in FP64
+  return ((size_t)2 * r.group * kSlab + (size_t)3 * r.max_halo) * bytes +
+         (bytes == 4 ? ((size_t)r.group * kSlab + r.max_halo + 1) * sizeof(double) : 0);
 }
 
 template <typename T, typename F>
@@ -1420,7 +1523,8 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
   r->ncu = ncu;
   r->nexp = (int)R.exp_loc.size();
   lds_max -= 2048;  // the kernels' static LDS: their sums
-  if (cg_lds(*r, sizeof(double)) > (size_t)lds_max) return nullptr;
+  if (cg_lds(*r, sizeof(double)) > (size_t)lds_max || cg_lds(*r, sizeof(float)) > (size_t)lds_max)
+    return nullptr;
   bool fits = true;
   if ((*err = cg_fits<double>(*r, lds_max, &fits)) != hipSuccess) return nullptr;
   if ((*err = cg_fits<float>(*r, lds_max, &fits)) != hipSuccess) return nullptr;
@@ -1490,26 +1594,32 @@ void rows_destroy(RowsDev* r) { delete r; }
 
 hipError_t rows_reserve(RowsDev* r, int bytes) {
   if (bytes == 8) return r->v64.p ? hipSuccess : r->v64.alloc(r->nent);
+  if (!r->res.p) {
+    const hipError_t e = r->res.alloc((size_t)r->nwg * r->group * kSlab);
+    if (e != hipSuccess) return e;
+  }
   return r->v32.p ? hipSuccess : r->v32.alloc(r->nent);
 }
 
-hipError_t rows_assemble(RowsDev* r, int bytes, const double* xa, int nslot_pad, int npair,
-                         bool nonsym, hipStream_t stream) {
+hipError_t rows_assemble(RowsDev* r, int bytes, bool both, const double* xa, int nslot_pad,
+                         int npair, bool nonsym, hipStream_t stream) {
   const int nslice = r->nslice;
   const unsigned lower = nonsym ? (unsigned)npair * (unsigned)nslot_pad : 0u;
   const dim3 grid((nslice + 3) / 4), block(256);
+  double* none = nullptr;
   if (bytes == 8)
-    hipLaunchKernelGGL(k_rows_assemble<double>, grid, block, 0, stream, r->v64.p, xa,
+    hipLaunchKernelGGL(k_rows_assemble<double>, grid, block, 0, stream, r->v64.p, none, xa,
                        r->slice_off.p, r->ref_off.p, r->ref_end.p, r->refs.p, nslice, lower);
   else
-    hipLaunchKernelGGL(k_rows_assemble<float>, grid, block, 0, stream, r->v32.p, xa,
-                       r->slice_off.p, r->ref_off.p, r->ref_end.p, r->refs.p, nslice, lower);
+    hipLaunchKernelGGL(k_rows_assemble<float>, grid, block, 0, stream, r->v32.p,
+                       both ? r->v64.p : none, xa, r->slice_off.p, r->ref_off.p, r->ref_end.p,
+                       r->refs.p, nslice, lower);
   return hipGetLastError();
 }
 
 bool rows_by_block(const RowsDev* r) { return r->by_block; }
 
-hipError_t rows_dmd(RowsDev* r, int bytes, const RowsDmd& a, hipStream_t stream) {
+hipError_t rows_dmd(RowsDev* r, int bytes, bool both, const RowsDmd& a, hipStream_t stream) {
   const int nc = a.ndp * (a.ndp - 1) / 2 * (a.nonsym ? 2 : 1);
   const size_t lds = ((size_t)nc * r->max_slots + a.max_local + 1) * sizeof(double);
   auto go = [&](auto kern, auto* val) -> hipError_t {
@@ -1522,7 +1632,7 @@ hipError_t rows_dmd(RowsDev* r, int bytes, const RowsDmd& a, hipStream_t stream)
     }
     const int threads = a.nblocks <= r->ncu ? kDmdThreads : kDmdThreads / 2;
     hipLaunchKernelGGL(kern, dim3(a.nblocks), dim3(threads), lds, stream, a, val,
-                       r->slice_off.p, r->ref_off.p, r->ref_end.p, r->refs16.p, r->slab_slice.p,
+                       both ? r->v64.p : (double*)nullptr, r->slice_off.p, r->ref_off.p, r->ref_end.p, r->refs16.p, r->slab_slice.p,
                        r->group);
     return hipGetLastError();
   };
@@ -1558,27 +1668,26 @@ static RowArgs row_args(const RowsDev* r, int k) {
   return a;
 }
 
-template <typename T>
-hipError_t rows_cg(RowsDev* r, const RowsCg<T>& a, hipStream_t stream) {
-  const int k = sizeof(T) == 4;
-  const RowArgs ra = row_args(r, k);
-  r->ep[k] ^= 1;
-  const T* val;
-  if constexpr (sizeof(T) == 8)
-    val = r->v64.p;
-  else
-    val = r->v32.p;
+hipError_t rows_cg(RowsDev* r, bool mixed, RowsCg a, hipStream_t stream) {
+  a.res = r->res.p;
+  const RowArgs ra = row_args(r, mixed);
+  r->ep[mixed] ^= 1;
   if (ra.ticketed) {
     hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, stream,
                        reinterpret_cast<u64*>(ra.sy.ticket), 1L);
   }
-  return with_cg_kernel<T>(r->group, a.diag != nullptr, [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(r->nwg), dim3(kSlab), cg_lds(*r, sizeof(T)), stream, ra, val, a);
+  const dim3 grid(r->nwg), block(kSlab);
+  const size_t lds = cg_lds(*r, mixed ? 4 : 8);
+  if (mixed)
+    return with_cg_kernel<float>(r->group, a.diag != nullptr, [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, block, lds, stream, ra, r->v32.p, r->v64.p, a);
+      return hipGetLastError();
+    });
+  return with_cg_kernel<double>(r->group, a.diag != nullptr, [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, block, lds, stream, ra, r->v64.p, r->v64.p, a);
     return hipGetLastError();
   });
 }
-template hipError_t rows_cg<double>(RowsDev*, const RowsCg<double>&, hipStream_t);
-template hipError_t rows_cg<float>(RowsDev*, const RowsCg<float>&, hipStream_t);
 
 bool rows_gmres_fits(const RowsDev* r, int bytes) { return r->gm_fits[bytes == 4]; }
 

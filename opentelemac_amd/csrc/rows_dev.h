@@ -20,9 +20,10 @@ void rows_destroy(RowsDev* r);
 hipError_t rows_reserve(RowsDev* r, int bytes);
 
 // Assembles the rows of the precision from the slot coefficients xa (upper
-// npair columns, and the lower ones when nonsym), nslot_pad apart.
-hipError_t rows_assemble(RowsDev* r, int bytes, const double* xa, int nslot_pad, int npair,
-                         bool nonsym, hipStream_t stream);
+// npair columns, and the lower ones when nonsym), nslot_pad apart. both: in
+// FP64 too (of 4 bytes).
+hipError_t rows_assemble(RowsDev* r, int bytes, bool both, const double* xa, int nslot_pad,
+                         int npair, bool nonsym, hipStream_t stream);
 
 // OM 'M=DMD' and the assembly in one pass, where node blocks are slabs
 // (rows_by_block): the coefficients src times D(i) D(j), written to xa and
@@ -40,30 +41,31 @@ struct RowsDmd {
   const int32_t* halo;
   const int32_t* color_off;
 };
-hipError_t rows_dmd(RowsDev* r, int bytes, const RowsDmd& a, hipStream_t stream);
+hipError_t rows_dmd(RowsDev* r, int bytes, bool both, const RowsDmd& a, hipStream_t stream);
 
-// One CG per system of the context (gracjg.F:189-409) in one launch. Vectors in
-// internal node order. FP64: a whole solve of A x = b, from the initial
-// solution to the outcome in the state (gave_up is only ever set). FP32: the
-// inner solve that the outer test has started, if it has, with its state.
-template <typename T>
+constexpr int kMaxOuter = 100;  // refinement sweeps of one mixed solve
+
+// SOLVE's CG, one per system of the context, in one launch: from the initial
+// solution to the outcome in the state (gave_up is only ever set). FP64
+// (gracjg.F:189-409), or mixed: FP64 residuals, each reduced by inner_eps by an
+// FP32 CG (the rows in both precisions). Vectors in internal node order.
 struct RowsCg {
-  const T* b;              // FP64: b; FP32: the residual b - A x the inner solve starts from
-                           // (its sign as the mixed solver keeps it)
-  const T* diag;           // diagonal, or nullptr for a unit diagonal
-  T* x;                    // solution; FP64: at idx[i] (or i), times scale[i] if given (not
-                           // x0: a launch that gives up leaves that as it is)
-  SolveState* st;
-  const T* x0;             // FP64: initial solution
-  const T* scale;
+  const double* b;
+  const double* diag;   // diagonal, or nullptr for a unit diagonal
+  const double* x0;     // initial solution
+  double* x;            // solution, at idx[i] (or i), times scale[i] if given (not x0: a
+                        // launch that gives up leaves that as it is)
+  const double* scale;
   const int32_t* idx;
+  SolveState* st;
   double eps;
-  int nitmax;
-  T* dlast;                // FP32: the previous direction of a continued solve (read), and
-                           // the last direction of this one (written)
+  int nitmax;           // iterations (mixed: of all inner solves)
+  double inner_eps;
+  int inner_nitmax;
+  int reliable;         // an inner solve continues the direction of the one before
+  double* res;          // (scratch, set by rows_cg)
 };
-template <typename T>
-hipError_t rows_cg(RowsDev* r, const RowsCg<T>& a, hipStream_t stream);
+hipError_t rows_cg(RowsDev* r, bool mixed, RowsCg a, hipStream_t stream);
 
 // Restarted GMRES (gmres.f:171-372) of a context of one system: FP64, the
 // whole solve in one launch; FP32, one cycle of the mixed solve from the FP64
