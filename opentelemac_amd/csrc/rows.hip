@@ -23,7 +23,7 @@
 // 4.0 for 256; two levels of 16: 3.5).
 //
 // us per iteration, FP64 / mixed: 1.4 / 1.6 (1,000 nodes, one workgroup), 3.2 /
-// 3.1 (20k), 3.9 / 3.7 (100k), 4.9 / 4.5 (260k), 5.8 / 5.4 (500k), 14.0 / 7.9 (1M),
+// 3.1 (20k), 3.9 / 3.7 (100k), 4.9 / 4.5 (260k), 5.8 / 5.4 (500k), 11.2 / 7.9 (1M),
 // 24.4 / 17.7 (2M). The two-kernel CG takes 15 at 20k, 50 (FP64) at 2M and 22 (FP32)
 // at 1M. Beside the iterations a solve takes 75 to 130 us up to 500k nodes (PRECD1,
 // the rows, this launch's start, the state back on the host) and 310 / 380 at 2M.
@@ -337,11 +337,11 @@ __device__ inline T front_dot(const RowFront<T, F>& f, const T* ys) {
 // for the whole solve.
 template <typename T, int R>
 struct RowProduct {
-  static constexpr bool kKeep = R * sizeof(T) <= 16;
-  // (FP32, 4 rows: 8 entries each would be 48 of the 128 registers; the spills
-  // take longer than reading 4 of them again, 1M nodes 10.8 us per iteration
-  // instead of 7.6)
-  static constexpr int kFront = sizeof(T) == 4 && R == 4 ? 4 : 8;
+  static constexpr bool kKeep = R * sizeof(T) <= 16 || R == 4;
+  // 4 rows per thread: 4 entries each. 8 would be 48 of the 128 registers in
+  // FP32 and spill (1M nodes 10.8 us per iteration instead of 7.6); FP64 without
+  // any takes 11.3 instead of 9.4 at 700k nodes, 14.0 instead of 11.2 at 1M
+  static constexpr int kFront = R == 4 ? 4 : 8;
   RowFront<T, kFront> front[kKeep ? R : 1];
   int wid[kKeep ? R : 1];
   // the slice of this wave's k-th rows: its coefficients, id words and width
