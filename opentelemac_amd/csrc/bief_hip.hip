@@ -1053,6 +1053,7 @@ struct bhip_ctx {
   int ncoef_saved = 0;
   bool have_saved = false;
   bhip::SolveState* st_host = nullptr;  // pinned
+  bhip::SolveState* st_host_dev = nullptr;  // and its address on the device
   size_t lds_f64 = 0, lds_f32 = 0;
   // the time-stepped wave equation on the device (wave.inl): slot geometry
   // [5][nslot_pad] (x2, x3, y2, y3, S of the slot's element) and node fields
@@ -1312,6 +1313,7 @@ static int ctx_setup(std::unique_ptr<bhip_ctx>& c, bhip_ctx** out) {
   }
   HIP_OK(c->st.alloc(c->nsys));
   HIP_OK(hipHostMalloc((void**)&c->st_host, sizeof(SolveState) * c->nsys, hipHostMallocDefault));
+  HIP_OK(hipHostGetDevicePointer((void**)&c->st_host_dev, c->st_host, 0));
   std::memset(c->st_host, 0, sizeof(SolveState) * c->nsys);
   HIP_OK(up(c->st.p, c->st_host, sizeof(SolveState) * c->nsys));
   c->part_p = c->partial.p;
@@ -2208,10 +2210,14 @@ static std::mutex& rows_mutex(int dev) {
 
 // CG as in cg_fp64 or cg_mixed; the solution goes to q.x, X = 0 of a zero
 // right-hand side included
-static int cg_rows(bhip_ctx* c, bool mixed, const RowsCg& q, bhip_solve_info* info) {
+static int cg_rows(bhip_ctx* c, bool mixed, RowsCg q, bhip_solve_info* info) {
   std::lock_guard<std::mutex> one(rows_mutex(c->device));
+  // the launch writes the states into the pinned host copies (a copy on the
+  // stream after it takes 4 us and a gap before it)
+  for (int sy = 0; sy < c->nsys; ++sy) c->st_host[sy].gave_up = 0;
+  q.st = c->st_host_dev;
   HIP_OK(rows_cg(c->rows, mixed, q, c->stream));
-  if (read_state(c)) return BHIP_EDEVICE;
+  HIP_OK(hipStreamSynchronize(c->stream));
   for (int sy = 0; sy < c->nsys; ++sy)
     if (c->st_host[sy].gave_up) return kGaveUp;
   return collect_infos(c, nullptr, mixed, info);
@@ -2361,7 +2367,6 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
     q.x = x_dev;
     q.scale = diag ? c->vdinv.p : nullptr;
     q.idx = internal ? nullptr : c->perm.p;
-    q.st = c->st_p;
     q.eps = cfg->eps;
     q.nitmax = std::max(cfg->nitmax, 1);
     q.inner_eps = inner_eps;

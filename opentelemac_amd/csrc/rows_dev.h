@@ -57,7 +57,8 @@ struct RowsCg {
                         // launch that gives up leaves that as it is)
   const double* scale;
   const int32_t* idx;
-  SolveState* st;
+  SolveState* st;       // the outcome, one per system; host memory will do: nothing is
+                        // read back
   double eps;
   int nitmax;           // iterations (mixed: of all inner solves)
   double inner_eps;
