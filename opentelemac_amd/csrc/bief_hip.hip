@@ -97,6 +97,7 @@ struct EbeArgs {
                               // or whose inner solve is still running
   // ensembles: system of each block and block range of each system (NULL
   // for one system: all blocks, partials [0, n_part_in))
+  const int32_t* idx;       // EPI_OP: y, xin and out in another order, or nullptr
   const int32_t* block_sys;
   const int32_t* sys_blocks;
 };
@@ -368,7 +369,27 @@ k_ebe(EbeArgs<T, TA> a) {
       xcur = xp ? a.xb1 : a.xb0;
       xnxt = xp ? a.xb0 : a.xb1;
     }
-    for (int l = threadIdx.x; l < nloc; l += blockDim.x) {
+    int l0 = threadIdx.x;
+    if constexpr (EPI == EPI_OP) {
+      // kStageUnroll nodes in flight: in the caller's order two loads each
+      for (; l0 < nloc; l0 += kStageUnroll * kThreads) {
+        int g[kStageUnroll];
+        T v[kStageUnroll];
+#pragma unroll
+        for (int u = 0; u < kStageUnroll; ++u) {
+          const int l = min(l0 + u * kThreads, nloc - 1);
+          g[u] = l < nown ? n0 + l : a.halo[h0 + l - nown];
+        }
+#pragma unroll
+        for (int u = 0; u < kStageUnroll; ++u) v[u] = a.y[a.idx ? a.idx[g[u]] : g[u]];
+#pragma unroll
+        for (int u = 0; u < kStageUnroll; ++u) {
+          const int l = l0 + u * kThreads;
+          if (l < nloc) put(l, g[u], v[u]);
+        }
+      }
+    }
+    for (int l = l0; l < nloc; l += blockDim.x) {
       const bool owned = l < nown;
       const int g = owned ? n0 + l : a.halo[h0 + l - nown];
       T v;
@@ -430,16 +451,17 @@ k_ebe(EbeArgs<T, TA> a) {
     const int g = n0 + l;
     const T v = acc[l];
     if constexpr (EPI == EPI_OP) {
+      const int i = a.idx ? a.idx[g] : g;
       T o;
       switch (a.op) {
         case BHIP_OP_AY: case BHIP_OP_TAY: o = v; break;
         case BHIP_OP_CAY: o = (T)a.c * v; break;
         case BHIP_OP_NAY: case BHIP_OP_NTAY: o = -v; break;
-        case BHIP_OP_XPAY: case BHIP_OP_XPTAY: o = a.xin[g] + v; break;
-        case BHIP_OP_XMAY: case BHIP_OP_XMTAY: o = a.xin[g] - v; break;
-        default: o = a.xin[g] + (T)a.c * v; break;  // X+CAY, X+CTAY
+        case BHIP_OP_XPAY: case BHIP_OP_XPTAY: o = a.xin[i] + v; break;
+        case BHIP_OP_XMAY: case BHIP_OP_XMTAY: o = a.xin[i] - v; break;
+        default: o = a.xin[i] + (T)a.c * v; break;  // X+CAY, X+CTAY
       }
-      a.out[g] = o;
+      a.out[i] = o;
     } else if constexpr (EPI == EPI_RESID) {
       const double rv = (double)v - a.b[g];
       a.out[g] = (T)rv;
@@ -1626,12 +1648,15 @@ int bhip_matrix_get(bhip_ctx* c, char* typdia, double* da, double* xa) {
 
 // y (caller order, device) -> vio0 (internal); result vio1 (internal) ->
 // x (caller order, device)
+// idx: y, x_in and x_out in another order than the context's (idx[i]: where
+// node i is); x_out may be x_in, but not overlap y
 static int matvec_internal(bhip_ctx* c, int op, double cst, const double* y_in,
-                           const double* x_in, double* x_out) {
+                           const double* x_in, double* x_out, const int32_t* idx = nullptr) {
   EbeArgs<double, double> a = base_args<double, double>(c, c->xa.p, c->da.p);
   a.y = y_in;
   a.xin = x_in;
   a.out = x_out;
+  a.idx = idx;
   a.op = op;
   a.c = cst;
   const bool trans = op >= BHIP_OP_TAY;
@@ -1644,6 +1669,11 @@ int bhip_matvec_dev(bhip_ctx* c, int op, double cst, const double* y, double* x)
   if (!c || !c->have_matrix || op < 0 || op > 10 || !y || !x) return BHIP_EBADARG;
   const Layout& L = c->L;
   const int g = c->grid_wide;
+  // in the caller's order directly (700k nodes: 23.5 us instead of 37 with two
+  // gathers and a scatter as kernels of their own), unless the product would
+  // write what other blocks still read
+  const bool apart = x + L.npoin <= y || y + L.npoin <= x;
+  if (apart) return matvec_internal(c, op, cst, y, x, x, c->perm.p);
   hipLaunchKernelGGL(k_gather<double>, dim3(g), dim3(kThreads), 0, c->stream, c->vio0.p, y,
                      c->perm.p, L.npoin);
   hipLaunchKernelGGL(k_gather<double>, dim3(g), dim3(kThreads), 0, c->stream, c->vio1.p, x,

@@ -92,3 +92,18 @@ def test_supg_system_is_ordered_with_the_caller(gpu):
         assert np.abs(got - want).max() <= 1e-12 * np.abs(want).max()
     host.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+def test_product_onto_its_operand(gpu, shift):
+    """x is y, or overlaps it: the same bits as with vectors of their own."""
+    m, ctx = _case(4)
+    n = m.npoin
+    buf = torch.rand(n + 1, dtype=torch.float64, device="cuda")
+    for op in bief.OPS:
+        b = buf.clone()
+        y, x = b[:n], b[shift:shift + n]
+        want = ctx.matvec(op, y.clone(), x.clone(), c=0.75)
+        got = ctx.matvec(op, y, x, c=0.75)
+        assert torch.equal(got, want), op
+    ctx.close()
