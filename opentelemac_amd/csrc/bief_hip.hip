@@ -2797,12 +2797,12 @@ constexpr int kElemThreads = 1024;
 static dim3 elem_threads(const Layout& L) {
   return dim3(L.nblocks <= 256 ? kElemThreads : kElemThreads / 2);
 }
-template <int NV>
+template <int NV, int NC = 3>
 struct NodeTerms {
-  int l[3];  // local node ids; owned nodes come first
-  double c[NV][3];
+  int l[NC];  // local node ids; owned nodes come first
+  double c[NV][NC];
 };
-template <int NV, typename F>
+template <int NV, int NC = 3, typename F>
 __device__ inline void colour_sum(const int32_t* __restrict__ co, int nown, double* acc,
                                   F&& terms) {
   // lane c holds the colour boundary c
@@ -2813,14 +2813,14 @@ __device__ inline void colour_sum(const int32_t* __restrict__ co, int nown, doub
   int col = 0;
   for (int w0 = __builtin_amdgcn_readlane(bound, 0); w0 < send; w0 += (int)blockDim.x) {
     const int w1 = min(w0 + (int)blockDim.x, send), s = w0 + (int)threadIdx.x;
-    NodeTerms<NV> v;
+    NodeTerms<NV, NC> v;
     if (s < w1) v = terms(s);
     for (;;) {
       const int c0 = __builtin_amdgcn_readlane(bound, col);
       const int c1 = __builtin_amdgcn_readlane(bound, col + 1);
       if (s < w1 && s >= c0 && s < c1) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
+        for (int k = 0; k < NC; ++k)
           if (v.l[k] < nown) {
 #pragma unroll
             for (int q = 0; q < NV; ++q) acc[q * nown + v.l[k]] += v.c[q][k];
@@ -2989,13 +2989,13 @@ __constant__ int kPrismRowPairs[6][5] = {{0, 1, 2, 3, 4},   {0, 5, 6, 7, 8},
 
 // inputs of one prism slot: ids, geometry, current coefficients for M=M+N
 struct PrismIn {
-  int s;           // slot; -1 when the thread has none in the phase
+  int s;           // slot
   int l[6];
   SlotGeo G;
   double old[15];  // target coefficients before 'M=M+N' (the first 15)
 };
 
-// Prism element matrices per slot, diagonal assembled in LDS colour by colour.
+// Prism element matrices per slot, diagonal assembled in LDS (colour_sum).
 //   KIND 200: MT01PP mass (mt01pp.f: XMUL*SURFAC/360 combinations of the
 //             column heights floored at 1e-3); nd holds Z per node
 //   KIND 201: MT02PP diffusion (mt02pp.f), P1 coefficients F, G, H; nd holds
@@ -3007,13 +3007,15 @@ struct PrismIn {
 // LDS once, after the diagonal accumulator (rec_off doubles in), and the
 // slots read them there; ST 0 gathers each slot's six records from global
 // memory. Both give the same bits. A workgroup of the staged MT02PP holds up
-// to 160 KB of LDS, so it may be alone on its CU: the staged form therefore
-// runs 2 * kThreads threads in two groups, each computing the slots of its
-// own colour, and adds their diagonal terms in colour order. ACC 0 writes the
+// to 160 KB of LDS, so it may be alone on its CU and runs more threads, as many
+// as the registers of MT02PP's terms allow (us, MT02PP at 600k nodes: two colours
+// of 256 slots at once 166, 512 slots of any colour 120, 1024 with spills 273;
+// MT01PP 59 -> 48; at 200k nodes 61 -> 39 and 26 -> 20). ACC 0 writes the
 // element matrices, 1 adds them to a symmetric target ('M=M+N'), 2 to both
 // halves of a non-symmetric one.
+constexpr int prism_threads(int st) { return st == 2 ? 2 * kThreads : kThreads; }
 template <int KIND, int ST, int ACC>
-__global__ void __launch_bounds__(ST == 2 ? 2 * kThreads : kThreads)
+__global__ void __launch_bounds__(prism_threads(ST))
 k_elem_prism(double xmul, const double* __restrict__ surfac,
              const double* __restrict__ xel, const double* __restrict__ yel, int nelem,
              const double* __restrict__ nd, int h_zero, int inchyd, int mon,
@@ -3027,21 +3029,15 @@ k_elem_prism(double xmul, const double* __restrict__ surfac,
   double* acc = reinterpret_cast<double*>(smem_raw);
   double* rec = acc + rec_off;
   constexpr int W = KIND == 200 ? 1 : 4;  // doubles per node record
-  const int b = blockIdx.x;
-  if (b >= nblocks) return;
+  const int b = xcd_block(blockIdx.x, nblocks);
   const int n0 = node_start[b], nown = node_start[b + 1] - n0;
   const int h0 = halo_start[b];
   const int32_t* co = color_off + (size_t)b * (kMaxColors + 1);
-  const int send = co[kMaxColors];
   const size_t np = nslot_pad;
-  // ST 2: two groups of kThreads threads, each on its own colour
-  constexpr int NT = ST == 2 ? 2 * kThreads : kThreads;
-  const int tg = (int)threadIdx.x % kThreads;
-  const int grp = (int)threadIdx.x / kThreads;
+  constexpr int NT = prism_threads(ST);
 
   auto load_slot = [&](PrismIn& in, int s) {
     in.s = s;
-    if (s < 0) return;
     // MT01PP reads all six ids: its three-id form measured slower (445 against
     // 382 us on 10.5 M slots), MT02PP's the same either way
     load_ids<6>(in.l, lid, np, s, KIND == 201 ? col_ids : 0);
@@ -3052,13 +3048,6 @@ k_elem_prism(double xmul, const double* __restrict__ surfac,
       for (int q = 0; q < 15; ++q) in.old[q] = xa[(size_t)q * np + s];
     }
   };
-  // the thread's first slot of colour c, or -1
-  auto first_slot = [&](int c) {
-    if (c >= kMaxColors || co[c] >= send) return -1;
-    const int s = co[c] + tg;
-    return s < co[c + 1] ? s : -1;
-  };
-
   // the element matrix of a slot into XA, its diagonal terms into t
   auto compute_slot = [&](const PrismIn& in, double (&t)[6]) {
     const int s = in.s;
@@ -3159,17 +3148,6 @@ k_elem_prism(double xmul, const double* __restrict__ surfac,
       for (int q = 0; q < 15; ++q) xa[(size_t)q * np + s] = cf[q];
     }
   };
-  auto add_slot = [&](const PrismIn& in, const double (&t)[6]) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k)
-      if (in.l[k] < nown) acc[in.l[k]] += t[k];
-  };
-  auto do_slot = [&](const PrismIn& in) {
-    double t[6];
-    compute_slot(in, t);
-    add_slot(in, t);
-  };
-
   for (int l = threadIdx.x; l < nown; l += blockDim.x) acc[l] = 0.0;
   if constexpr (ST) {
     // records of the local nodes, kStage per thread in flight at once
@@ -3206,48 +3184,15 @@ k_elem_prism(double xmul, const double* __restrict__ surfac,
     }
   }
   __syncthreads();
-  if constexpr (ST == 2) {
-    // colours c0 and c0 + 1 computed at once by the two groups; their
-    // diagonal terms go into the accumulator in colour order, one group
-    // after the other, so the sums are those of the one-group form
-    for (int c0 = 0; c0 < kMaxColors; c0 += 2) {
-      if (co[c0] >= send) break;
-      const int c = c0 + grp;
-      const bool has = c < kMaxColors && co[c] < send;
-      PrismIn cur;
-      double t[6];
-      load_slot(cur, first_slot(c));
-      if (cur.s >= 0) compute_slot(cur, t);
-      for (int k = 0; k < 2; ++k) {
-        if (grp == k && has) {
-          if (cur.s >= 0) add_slot(cur, t);
-          // slots beyond the first kThreads of a large colour
-          for (int s = co[c] + tg + kThreads; s < co[c + 1]; s += kThreads) {
-            PrismIn in;
-            load_slot(in, s);
-            do_slot(in);
-          }
-        }
-        __syncthreads();
-      }
-    }
-  } else {
-    for (int c = 0; c < kMaxColors; ++c) {
-      const int s0 = co[c];
-      if (s0 >= send) break;
-      const int s1 = co[c + 1];
-      PrismIn cur;
-      load_slot(cur, first_slot(c));
-      if (cur.s >= 0) do_slot(cur);
-      // slots beyond the first kThreads of a large colour
-      for (int s = s0 + tg + kThreads; s < s1; s += kThreads) {
-        PrismIn in;
-        load_slot(in, s);
-        do_slot(in);
-      }
-      __syncthreads();
-    }
-  }
+  colour_sum<1, 6>(co, nown, acc, [&](int s) {
+    PrismIn in;
+    load_slot(in, s);
+    NodeTerms<1, 6> nt;
+    compute_slot(in, nt.c[0]);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) nt.l[k] = in.l[k];
+    return nt;
+  });
   for (int l = threadIdx.x; l < nown; l += blockDim.x) {
     if constexpr (ACC > 0)
       da[n0 + l] += acc[l];
@@ -3591,8 +3536,8 @@ static int elem_prism(bhip_ctx* c, int kind, double xmul, const double* xel, con
   };
   const int acc_kind = !accumulate ? 0 : target_q ? 2 : 1;
 #define BHIP_PRISM_PICK(ST, ACC)                                                             \
-  (ST ? pick(k_elem_prism<200, 2, ACC>, k_elem_prism<201, 2, ACC>, lds_rec, 2 * kThreads) \
-      : pick(k_elem_prism<200, 0, ACC>, k_elem_prism<201, 0, ACC>, lds_acc, kThreads))
+  (ST ? pick(k_elem_prism<200, 2, ACC>, k_elem_prism<201, 2, ACC>, lds_rec, prism_threads(2)) \
+      : pick(k_elem_prism<200, 0, ACC>, k_elem_prism<201, 0, ACC>, lds_acc, prism_threads(0)))
   const int ls = staged ? (acc_kind == 0   ? BHIP_PRISM_PICK(1, 0)
                            : acc_kind == 1 ? BHIP_PRISM_PICK(1, 1)
                                            : BHIP_PRISM_PICK(1, 2))
