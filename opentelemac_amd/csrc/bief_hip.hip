@@ -1063,8 +1063,7 @@ struct bhip_ctx {
   bhip::RowsDev* rows = nullptr;  // assembled rows for the persistent CG, or none
   bool rows_off = false;          // it gave up once: the two-kernel CG from then on
   int prefetch_j = 0;  // register prefetch depth of the element kernels
-  int iter_hint[5] = {0, 0, 0, 0, 0};  // FP64 CG, inner CG, inner solves, CGSTAB, cycles
-                                       // of mixed GMRES
+  int iter_hint[4] = {0, 0, 0, 0};  // FP64 CG, inner CG, inner solves, CGSTAB
   int inner_hint[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // iterations of inner solve k (mixed CG)
   // BiCGSTAB scalars and extra partial sums; GMRES basis and scalars
   bhip::DevBuf<double> bicg_sc, bicg_part, gm, gm_scal;
@@ -2341,8 +2340,7 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   const bool use_rows = c->rows && !c->rows_off && td != '0' &&
                         (cfg->slv == 1 || (cfg->slv == 7 && rows_gmres_fits(c->rows, row_bytes)));
   const bool by_block = use_rows && rows_by_block(c->rows);
-  // mixed CG takes its FP64 residuals from rows too
-  const bool both = mixed && cfg->slv == 1;
+  const bool both = mixed;  // the FP64 residuals are taken from rows too
   if (use_rows) HIP_OK(rows_reserve(c->rows, row_bytes));
   if (diag) {
     // PRECD1 (precd1.f:90-149), X and B taken from the caller's vectors

@@ -607,15 +607,16 @@ static int gmres_mixed(bhip_ctx* c, double* x, const double* b, double eps, int 
   return gmres_impl<float>(c, x, b, eps, nitmax, krylov, xa32_ready, info);
 }
 
-// GMRES on assembled rows: FP64 in one persistent launch; mixed, one launch
-// per cycle with the FP64 residual between. The solution is left in xout when
-// *moved, else it is x (unchanged).
+// GMRES on assembled rows in one persistent launch. The solution is left in
+// xout when *moved, else it is x (unchanged).
 template <typename T>
 static int gmres_rows(bhip_ctx* c, double* x, double* xout, bool* moved, const double* b,
                       double eps, int nitmax, int krylov, bhip_solve_info* info) {
-  constexpr bool kMixed = sizeof(T) == 4;
-  const Layout& L = c->L;
   std::lock_guard<std::mutex> one(rows_mutex(c->device));
+  // the state lies in the pinned memory of the solver states
+  static_assert(sizeof(GmState) <= sizeof(SolveState), "one fits");
+  GmState* s = reinterpret_cast<GmState*>(c->st_host);
+  *s = GmState();
   RowsGmres q = {};
   q.x0 = x;
   q.x = xout;
@@ -624,62 +625,20 @@ static int gmres_rows(bhip_ctx* c, double* x, double* xout, bool* moved, const d
   q.eps = eps;
   q.nitmax = nitmax;
   q.krylov = krylov;
-  q.first = 1;
-  GmState s = {};
-  if constexpr (kMixed) {
-    const int g = c->grid_nodes;
-    hipLaunchKernelGGL(k_dot_partials<double>, dim3(g), dim3(kThreads), 0, c->stream, b, b,
-                       L.npoin, part_u(c, 0));
-    HIP_OK(hipGetLastError());
-    q.r0 = c->vr.p;
-    q.part_rr = part_u(c, 1);
-    q.npart_rr = L.nblocks;
-    q.part_bb = part_u(c, 0);
-    q.npart_bb = g;
-    // R0 = A X - B (FP64)
-    auto residual = [&](const double* y) -> int {
-      EbeArgs<double, double> a = base_args<double, double>(c, c->xa.p, c->da.p);
-      a.y = y;
-      a.b = b;
-      a.out = c->vr.p;
-      a.partial = part_u(c, 1);
-      HIP_OK((launch_ebe<double, double, STAGE_PLAIN, EPI_RESID, FIN_PARTIAL>(
-          c, a, false, c->typdia, c->typext)));
-      return BHIP_OK;
-    };
-    // the cycles the previous solve took, then one by one; a launch that
-    // finds its residual small enough ends the solve
-    int& hint = c->iter_hint[4];
-    if (residual(x)) return BHIP_EDEVICE;
-    for (int n = std::min(std::max(hint, 1), 8);; n = 1) {
-      for (int k = 0; k < n; ++k) {
-        HIP_OK(rows_gmres<T>(c->rows, q, c->stream));
-        q.first = 0;
-        if (residual(xout)) return BHIP_EDEVICE;
-      }
-      // (the stop test on the last residual)
-      HIP_OK(rows_gmres<T>(c->rows, q, c->stream));
-      HIP_OK(rows_gmres_state(c->rows, &s, c->stream));
-      HIP_OK(hipStreamSynchronize(c->stream));
-      if (s.gave_up) return kGaveUp;
-      if (s.done) break;
-      if (residual(xout)) return BHIP_EDEVICE;
-    }
-    hint = s.m;
-    info->inner_iters = s.products;
-    info->outer_iters = s.m;
-  } else {
-    HIP_OK(rows_gmres<T>(c->rows, q, c->stream));
-    HIP_OK(rows_gmres_state(c->rows, &s, c->stream));
-    HIP_OK(hipStreamSynchronize(c->stream));
-    if (s.gave_up) return kGaveUp;
+  q.st = reinterpret_cast<GmState*>(c->st_host_dev);
+  HIP_OK(rows_gmres<T>(c->rows, q, c->stream));
+  HIP_OK(hipStreamSynchronize(c->stream));
+  if (s->gave_up) return kGaveUp;
+  *moved = s->updated != 0;
+  info->niter = s->m;
+  info->relat = s->relat;
+  info->relres = s->prec;
+  info->converged = s->prec < eps;
+  if (sizeof(T) == 4) {
+    info->inner_iters = s->products;
+    info->outer_iters = s->m;
   }
-  *moved = s.updated != 0;
-  info->niter = s.m;
-  info->relat = s.relat;
-  info->relres = s.prec;
-  info->converged = s.prec < eps;
-  return s.prec < eps ? BHIP_OK : BHIP_MAXITER;
+  return s->prec < eps ? BHIP_OK : BHIP_MAXITER;
 }
 
 }  // namespace bhip

@@ -769,8 +769,7 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ val6
 }
 
 // ---------------------------------------------------------------------------
-// GMRES(K): FP64, a whole solve; FP32 (mixed precision), one cycle from an
-// FP64 residual
+// GMRES(K), a whole solve; mixed: FP32 cycles, each from the FP64 residual
 // ---------------------------------------------------------------------------
 // One meeting per Arnoldi step: w = A V_j with w.V_i and V_j.V_i (i <= j), w.w
 // and the exchange of w of the halo rows. From these every workgroup has the
@@ -780,12 +779,12 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ val6
 // follow from the exchanged w. The basis lies in memory, each thread's rows
 // together, and mostly in L2; V_j and w are in LDS, R0 in registers.
 //
-// us per solve at K = 5, FP64 / mixed (the same from the host, one kernel per
-// orthogonalisation step: 11 launches, 9 of them with a sum over all
-// workgroups, for a cycle of K = 3): 20k nodes 531 / 746 (2361 / 2760), 500k
-// 889 / 1072 (2896 / 3120), 2M 3303 / 2528 (5275 / 4711); 11 cycles each. A step
-// takes 7 us at 20k, most of it the meeting, 60 at 2M, where the basis (170 MB)
-// and the matrix come from the last-level cache.
+// us per solve at K = 5, FP64 / mixed (in brackets: from the host, one kernel per
+// orthogonalisation step, 11 launches for a cycle of K = 3, 9 of them with a sum
+// over all workgroups): 90k nodes 522 / 531 (2310 / 2661), 500k 854 / 838 (2896 /
+// 3120), 2M 3238 / 2088 (5275 / 4711); 11 cycles each. A step takes 7 us at 90k,
+// most of it the meeting, 55 at 2M, where the basis (170 MB in FP64) and the
+// matrix come from the last-level cache.
 struct GmLds {
   double part[kGmSums * kRowWaves];
   double tot[kGmSums * 4];
@@ -818,8 +817,8 @@ __device__ inline double lane_value(double v, int lane) {
 
 template <typename T, int R>
 __global__ void __launch_bounds__(kSlab)
-k_gmres_rows(RowArgs ra, const T* __restrict__ val, RowsGmres a, T* basis, T* hbasis,
-             GmState* st) {
+k_gmres_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ val64,
+             RowsGmres a, T* basis, T* hbasis) {
   constexpr bool kMixed = sizeof(T) == 4;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ GmLds sh;
@@ -827,14 +826,8 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, RowsGmres a, T* basis, T* hb
   const int wg = blockIdx.x, gang = ra.nwg;
   const bool lead = wg == 0 && t == 0;
   unsigned e = __hip_atomic_load(ra.sy.epoch + ra.ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  auto leave = [&]() {
-    if (lead)
-      __hip_atomic_store(ra.sy.epoch + 1 - ra.ep, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  // (the lead writes `done` without a meeting only where every workgroup
-  // finds by itself that the solve has ended)
-  if (load_relaxed(ra.sy.abort) || (!a.first && load_relaxed(&st->done))) {
-    leave();
+  if (load_relaxed(ra.sy.abort)) {
+    store_relaxed(&a.st->gave_up, 1);
     return;
   }
   const int r0 = ra.wg_row0[wg];
@@ -845,6 +838,8 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, RowsGmres a, T* basis, T* hb
   T* dh = ds + R * kSlab;
   T* ah = dh + nh;                         // A V_j of the halo
   T* as = ah + nh;                         // A V_j of own rows
+  // mixed: X, own rows, then halo
+  double* xs = reinterpret_cast<double*>(smem_raw) + (2 * R * kSlab + 2 * nh + 1) / 2;
   // this thread's part of the scratch: V, A V (FP64) and the diagonal
   const size_t vstride = (size_t)ra.nwg * R * kSlab, hstride = ra.nhalo;
   T* vb = basis + (size_t)wg * R * kSlab + t;
@@ -920,7 +915,10 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, RowsGmres a, T* basis, T* hb
     if (!ok) sh.bad = 1;
     __syncthreads();
     if (sh.bad) {
-      if (t == 0) store_relaxed(ra.sy.abort, 1);
+      if (t == 0) {
+        store_relaxed(ra.sy.abort, 1);
+        store_relaxed(&a.st->gave_up, 1);
+      }
       return false;
     }
     return true;
@@ -948,79 +946,90 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, RowsGmres a, T* basis, T* hb
   for (int k = 0; k < R; ++k) {
     if constexpr (R >= 4) __builtin_amdgcn_sched_barrier(0);
     const int p = rowpos[k * kSlab + t];
+    double x = 0.0;
+    T d = (T)0;
     rv[k] = (T)0;
-    T xv = (T)0, d = (T)0;
     if (p != 0xffff) {
-      if constexpr (!kMixed) {
-        rv[k] = a.b[r0 + p];
-        xv = a.x0[r0 + p];
-      }
+      x = a.x0[r0 + p];
+      if constexpr (!kMixed) rv[k] = a.b[r0 + p];
       if (a.diag) d = (T)a.diag[r0 + p];
     }
-    if constexpr (!kMixed) ds[k * kSlab + t] = xv;
+    if constexpr (kMixed)
+      xs[k * kSlab + t] = x;
+    else
+      ds[k * kSlab + t] = x;
     if (a.diag) dq[(size_t)k * kSlab] = d;
     prod.load(ra, val, wg, k);
   }
-  double nr0, nb;
-  int m = 0;
-  if constexpr (kMixed) {
-    // the sums of the residual's kernel and of ||b||^2
-    double p = 0.0, q = 0.0;
-    for (int i = t; i < a.npart_rr; i += kSlab) p += a.part_rr[i];
-    for (int i = t; i < a.npart_bb; i += kSlab) q += a.part_bb[i];
-    p = sum64(p);
-    q = sum64(q);
-    if (lane == 0) {
-      sh.part[wave] = p;
-      sh.part[kRowWaves + wave] = q;
-    }
-    __syncthreads();
-    nr0 = sqrt(sum16(sh.part[lane & 15]));
-    nb = sqrt(sum16(sh.part[kRowWaves + (lane & 15)]));
-    __syncthreads();
-    m = a.first ? 0 : load_relaxed(&st->m);
-  } else {
-    // R0 = A X - B, ||R0||^2, ||B||^2 (gmres.f:188-207)
-    for (int h = t; h < nh; h += kSlab) dh[h] = a.x0[ra.halo_row[h0 + h]];
-    __syncthreads();
-    product();
-    sum_rows(0, [&](int k) { return (double)rv[k] * (double)rv[k]; });
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-      rv[k] = as[k * kSlab + t] - rv[k];
-      as[k * kSlab + t] = rv[k];
-    }
-    sum_rows(1, [&](int k) { return (double)rv[k] * (double)rv[k]; });
-    if (!meet(2, true)) return;
-    nb = sqrt(total(0));
-    nr0 = sqrt(total(1));
+  for (int h = t; h < nh; h += kSlab) {
+    const double x = a.x0[ra.halo_row[h0 + h]];
+    if constexpr (kMixed)
+      xs[R * kSlab + h] = x;
+    else
+      dh[h] = x;
   }
+  __syncthreads();
+  // R0 = A X - B with its norm, and ||B||^2 (gmres.f:188-207), as the sums 0 and
+  // 1 of a meeting that brings the halo of R0; mixed: in FP64, FP32 in rv
+  auto residual = [&]() -> bool {
+    if constexpr (kMixed) {
+      int tt = t;
+      asm volatile("" : "+v"(tt));
+      double bb = 0.0, rr = 0.0;
+#pragma nounroll
+      for (int k = 0; k < R; ++k) {
+        const double* v;
+        const unsigned* id;
+        const int w = RowProduct<double, R>::slice(ra, val64, wg, k, v, id);
+        double s = slice_dot<8>(v, id, lane, 0, w, xs);
+        const int p = rowpos[k * kSlab + tt];
+        double q = 0.0, b = 0.0;
+        if (p != 0xffff) {
+          const double x = xs[k * kSlab + tt];
+          b = a.b[r0 + p];
+          s += a.diag ? a.diag[r0 + p] * x : x;
+          q = s - b;
+        }
+        bb += b * b;
+        rr += q * q;
+        as[k * kSlab + tt] = (T)q;
+      }
+      bb = sum64(bb);
+      rr = sum64(rr);
+      if (lane == 0) {
+        sh.part[wave] = bb;
+        sh.part[kRowWaves + wave] = rr;
+      }
+    } else {
+      product();
+      sum_rows(0, [&](int k) { return (double)rv[k] * (double)rv[k]; });
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        rv[k] = as[k * kSlab + t] - rv[k];
+        as[k * kSlab + t] = rv[k];
+      }
+      sum_rows(1, [&](int k) { return (double)rv[k] * (double)rv[k]; });
+    }
+    return meet(2, true);
+  };
+  if (!residual()) return;
+  double nb = sqrt(total(0)), nr0 = sqrt(total(1));
+  int m = 0;
   const int relat = nb < 1.0 ? 0 : 1;
   if (nb < 1.0) nb = 1.0;
   double prec = nr0 / nb;
   int products = 0;
   bool updated = false;
-  // the stop tests (gmres.f:207, :367)
-  bool stop = m == 0 ? prec <= a.eps : !(prec >= a.eps && m < a.nitmax);
-  const bool ran = !stop;
+  bool stop = prec <= a.eps;  // (gmres.f:207)
   while (!stop) {
     ++m;
     // V_0 = -R0 / ||R0|| (gmres.f:243), halo included
-    if constexpr (kMixed) {
 #pragma unroll
-      for (int k = 0; k < R; ++k) {
-        const int p = rowpos[k * kSlab + t];
-        const T v = p != 0xffff ? (T)(-1.0 / nr0 * a.r0[r0 + p]) : (T)0;
-        ds[k * kSlab + t] = vb[(size_t)k * kSlab] = v;
-      }
-      for (int h = t; h < nh; h += kSlab)
-        dh[h] = vh[h] = (T)(-1.0 / nr0 * a.r0[ra.halo_row[h0 + h]]);
-    } else {
-#pragma unroll
-      for (int k = 0; k < R; ++k)
-        ds[k * kSlab + t] = vb[(size_t)k * kSlab] = (T)(-1.0 / nr0) * rv[k];
-      for (int h = t; h < nh; h += kSlab) dh[h] = vh[h] = (T)(-1.0 / nr0) * ah[h];
+    for (int k = 0; k < R; ++k) {
+      const T r = kMixed ? as[k * kSlab + t] : rv[k];
+      ds[k * kSlab + t] = vb[(size_t)k * kSlab] = (T)(-1.0 / nr0 * (double)r);
     }
+    for (int h = t; h < nh; h += kSlab) dh[h] = vh[h] = (T)(-1.0 / nr0 * (double)ah[h]);
     __syncthreads();
     int kk = a.krylov;
     for (int j = 0; j < kk; ++j) {
@@ -1169,21 +1178,42 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, RowsGmres a, T* basis, T* hb
       stop = true;
       break;
     }
-    // X += sum y_l V_l, R0 += sum y_l A V_l (gmres.f:354-359)
+    // X += sum y_l V_l, R0 += sum y_l A V_l (gmres.f:354-359); mixed: X in FP64,
+    // halo included, and R0 anew
 #pragma unroll
     for (int k = 0; k < R; ++k) {
       const int p = rowpos[k * kSlab + t];
-      double xv = p == 0xffff ? 0.0 : a.first && !updated ? a.x0[r0 + p] : a.x[r0 + p];
+      double xv = 0.0;
+      if constexpr (kMixed)
+        xv = xs[k * kSlab + t];
+      else if (p != 0xffff)
+        xv = updated ? a.x[r0 + p] : a.x0[r0 + p];
 #pragma unroll 2
       for (int l = 0; l < kk; ++l) {
         const double yl = sh.y[l];
         xv += yl * (double)vb[l * vstride + (size_t)k * kSlab];
         if constexpr (!kMixed) rv[k] += yl * avb[l * vstride + (size_t)k * kSlab];
       }
-      if (p != 0xffff) a.x[r0 + p] = xv;
+      if constexpr (kMixed)
+        xs[k * kSlab + t] = xv;
+      else if (p != 0xffff)
+        a.x[r0 + p] = xv;
     }
     updated = true;
-    if constexpr (kMixed) break;
+    if constexpr (kMixed) {
+      for (int h = t; h < nh; h += kSlab) {
+        double xv = xs[R * kSlab + h];
+#pragma unroll 2
+        for (int l = 0; l < kk; ++l) xv += sh.y[l] * (double)vh[l * hstride + h];
+        xs[R * kSlab + h] = xv;
+      }
+      __syncthreads();
+      if (!residual()) return;
+      nr0 = sqrt(total(1));
+      prec = nr0 / nb;
+      stop = !(prec >= a.eps && m < a.nitmax);
+      continue;
+    }
     nr0 = fabs(sh.y[kk]);
     prec = nr0 / nb;
     stop = !(prec >= a.eps && m < a.nitmax);
@@ -1199,17 +1229,20 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, RowsGmres a, T* basis, T* hb
       stop = !(prec >= a.eps);
     }
   }
-  if (lead) {
-    st->prec = prec;
-    st->relat = relat;
-    if (ran || a.first) {
-      store_relaxed(&st->m, m);
-      st->products = (a.first ? 0 : st->products) + products;
-      st->updated = updated || (!a.first && st->updated);
+  if constexpr (kMixed)
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const int p = rowpos[k * kSlab + t];
+      if (p != 0xffff && updated) a.x[r0 + p] = xs[k * kSlab + t];
     }
-    store_relaxed(&st->done, stop ? 1 : 0);
+  if (lead) {
+    a.st->prec = prec;
+    a.st->relat = relat;
+    a.st->m = m;
+    a.st->products = products;
+    a.st->updated = updated;
+    __hip_atomic_store(ra.sy.epoch + 1 - ra.ep, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  leave();
 }
 
 // ---------------------------------------------------------------------------
@@ -1422,7 +1455,6 @@ struct RowsDev {
   int nhalo = 0;
   Buf<unsigned char> gm, gmh;
   size_t gm_bytes = 0, gmh_bytes = 0;
-  GmState* gm_state = nullptr;
 };
 
 static size_t cg_lds(const RowsDev& r, int bytes) {
@@ -1463,8 +1495,9 @@ static hipError_t cg_fits(const RowsDev& r, int lds_max, bool* fits) {
 }
 
 static size_t gm_lds(const RowsDev& r, int bytes) {
-  // V_j and A V_j of own rows and of the halo
-  return (size_t)2 * (r.group * kSlab + r.max_halo) * bytes;
+  // V_j and A V_j of own rows and of the halo; mixed: X of both in FP64
+  return (size_t)2 * (r.group * kSlab + r.max_halo) * bytes +
+         (bytes == 4 ? ((size_t)r.group * kSlab + r.max_halo + 1) * sizeof(double) : 0);
 }
 
 template <typename T, typename F>
@@ -1561,7 +1594,7 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
   const bool gm = r->gm_fits[0] || r->gm_fits[1];
   const size_t nexp = R.exp_loc.size();
   const size_t nepoch = (2 * (size_t)nsys + 1) / 2 + 1;  // in 64-bit words
-  const size_t tail = 4 * nexp + nepoch + 2 + (sizeof(GmState) + 7) / 8;
+  const size_t tail = 4 * nexp + nepoch + 2;
   const size_t nslot[3] = {(size_t)2 * kReplicas * kSums * R.nwg * 2,
                            (size_t)2 * kReplicas * kSums * R.nwg * 2,
                            gm ? (size_t)2 * kReplicas * kGmSums * R.nwg * 2 : 0};
@@ -1579,11 +1612,6 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
     s.abort = reinterpret_cast<int*>(p += 1);
     s.ticks = ticks;
     p += 1;
-    if (k == 2) {
-      r->gm_state = reinterpret_cast<GmState*>(p);
-      s.abort = &r->gm_state->gave_up;
-    }
-    p += (sizeof(GmState) + 7) / 8;
   }
   hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, stream, r->words.p, (long)nwords);
   if (!ok(hipGetLastError()) || !ok(hipStreamSynchronize(stream))) return nullptr;
@@ -1721,17 +1749,14 @@ hipError_t rows_gmres(RowsDev* r, const RowsGmres& a, hipStream_t stream) {
   else
     val = r->v32.p;
   return with_gm_kernel<T>(r->group, [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(r->nwg), dim3(kSlab), gm_lds(*r, sizeof(T)), stream, ra, val, a,
-                       reinterpret_cast<T*>(r->gm.p), reinterpret_cast<T*>(r->gmh.p),
-                       r->gm_state);
+    hipLaunchKernelGGL(kern, dim3(r->nwg), dim3(kSlab), gm_lds(*r, sizeof(T)), stream, ra, val,
+                       r->v64.p, a, reinterpret_cast<T*>(r->gm.p),
+                       reinterpret_cast<T*>(r->gmh.p));
     return hipGetLastError();
   });
 }
 template hipError_t rows_gmres<double>(RowsDev*, const RowsGmres&, hipStream_t);
 template hipError_t rows_gmres<float>(RowsDev*, const RowsGmres&, hipStream_t);
 
-hipError_t rows_gmres_state(const RowsDev* r, GmState* host, hipStream_t stream) {
-  return hipMemcpyAsync(host, r->gm_state, sizeof(GmState), hipMemcpyDeviceToHost, stream);
-}
 
 }  // namespace bhip

@@ -68,32 +68,26 @@ struct RowsCg {
 };
 hipError_t rows_cg(RowsDev* r, bool mixed, RowsCg a, hipStream_t stream);
 
-// Restarted GMRES (gmres.f:171-372) of a context of one system: FP64, the
-// whole solve in one launch; FP32, one cycle of the mixed solve from the FP64
-// residual r0 (nothing where the stop test on it ends the solve). Vectors in
-// internal node order.
-struct GmState {  // on the device, written by a launch
+// Restarted GMRES (gmres.f:171-372) of a context of one system, a whole solve
+// in one launch: FP64, or mixed (FP32 cycles, FP64 residuals; the rows in both
+// precisions). Vectors in internal node order.
+struct GmState {
   double prec;    // ||R0|| / max(||B||, 1)
-  int m, products, done, relat;
+  int m, products, relat;
   int updated;    // x has been written
-  int gave_up;    // a launch gave up waiting for its workgroups (never reset)
+  int gave_up;    // only ever set
 };
 struct RowsGmres {
-  const double* x0;  // initial solution
-  double* x;         // solution, if updated (not x0: see RowsCg)
+  const double* x0;    // initial solution
+  double* x;           // solution, if updated (not x0: see RowsCg)
   const double* diag;  // diagonal, or nullptr for a unit diagonal
-  const double* b;     // FP64
-  const double* r0;    // FP32: A x - b, and the partial sums of r0.r0 and b.b
-  const double* part_rr;
-  const double* part_bb;
-  int npart_rr, npart_bb;
+  const double* b;
   double eps;
   int nitmax, krylov;
-  int first;           // first launch of the solve
+  GmState* st;         // the outcome; host memory will do
 };
 bool rows_gmres_fits(const RowsDev* r, int bytes);
 template <typename T>
 hipError_t rows_gmres(RowsDev* r, const RowsGmres& a, hipStream_t stream);
-hipError_t rows_gmres_state(const RowsDev* r, GmState* host, hipStream_t stream);
 
 }  // namespace bhip
