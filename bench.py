@@ -23,7 +23,8 @@ storage (telemac2d's default MATRIX STORAGE = 3), the 2M SUPG tracer system by
 GMRES(5) (FP64 and mixed), the 500k-node adjoint (gradient/forward cost,
 finite-difference and tangent-linear checks), the 256-member ensemble
 (systems/s, per-system latency) and the 5M-node prism systems; each with
-the roofline figure of its dominant kernel.
+the roofline figure of its element-by-element product (the CG direction kernel;
+systems of up to 2,097,152 rows are solved on assembled rows instead).
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload all|...]
 """
@@ -327,8 +328,9 @@ def bench_estuary(args, dev, m, sysd):
     rel_mixed_vs_fp64 = float(np.linalg.norm(sols["mixed"] - sols["fp64"])
                               / np.linalg.norm(sols["fp64"]))
 
-    # algorithmic bytes per launch of the dominant kernels (int32
-    # connectivity, 3 coefficients per element, node vectors):
+    # algorithmic bytes per launch of the element-by-element CG kernels (int32
+    # connectivity, 3 coefficients per element, node vectors), which larger
+    # systems run on (this one is solved in one launch on assembled rows):
     #  * FP64 CG direction + EBE mat-vec + D.AD: R, D_old read; D, AD written
     #  * mixed inner CG: the same kernel in FP32
     bytes_f64 = ne * (3 * 8 + 12) + nprime * 4 * 8
@@ -709,7 +711,7 @@ def bench_adjoint(args, npoin=500_000, nsteps=50, checkpoint=10, n_fd=20):
         jd = tl_model.run(fwAD.make_dual(k, dk), fwAD.make_dual(zb, dz), nsteps, gauges, obs)
         tl = float(fwAD.unpack_dual(jd).tangent)
     adj = float((gk * dk).sum() + (gz * dz).sum())
-    # the dominant kernel: the inner CG's direction + EBE product (FP32)
+    # the element-by-element CG's direction + product (FP32)
     ms_dir, _ = model.ctx.time_cg_kernels(bief.PREC_MIXED, reps=50)
     roof = _roof(m.nelem * (3 * 4 + 12) + m.npoin * 4 * 4, ms_dir)
     roof["kernel"] = "k_ebe<float,...,STAGE_CGDIR,EPI_CGAD,FIN_CG> (mixed inner CG direction)"

@@ -13,7 +13,7 @@
 // the k-th rows of its lanes) have nearly the same number of entries. Each
 // half of a slab is sorted by it; rank g * 64 + v becomes leaf 8 v + j(g), j =
 // 0, 4, 1, 5, 2, 6, 3, 7: groups of 8 take one run of 64 ranks per slice,
-// groups of 4 two neighbouring ones. (Groups of 1 and 2 keep their rows'
+// groups of 4 two neighbouring ones. (Groups of up to 4 keep their rows'
 // first entries in registers, where padding costs nothing.)
 //
 // A slice stores its coefficients entry by entry, 64 lanes wide (coalesced):
