@@ -970,7 +970,8 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ v
   }
   __syncthreads();
   // R0 = A X - B with its norm, and ||B||^2 (gmres.f:188-207), as the sums 0 and
-  // 1 of a meeting that brings the halo of R0; mixed: in FP64, FP32 in rv
+  // 1 of a meeting that brings the halo of R0; mixed: in FP64, times `sc` in FP32
+  double sc = 1.0;
   auto residual = [&]() -> bool {
     if constexpr (kMixed) {
       int tt = t;
@@ -992,7 +993,7 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ v
         }
         bb += b * b;
         rr += q * q;
-        as[k * kSlab + tt] = (T)q;
+        as[k * kSlab + tt] = (T)(q * sc);
       }
       bb = sum64(bb);
       rr = sum64(rr);
@@ -1023,13 +1024,21 @@ k_gmres_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ v
   bool stop = prec <= a.eps;  // (gmres.f:207)
   while (!stop) {
     ++m;
+    if constexpr (kMixed)
+      if (!(nr0 > 1e-25 && nr0 < 1e25) && nr0 > 0.0 && nr0 < 1e300) {
+        // R0 again, scaled into FP32's range
+        sc = 1.0 / nr0;
+        if (!residual()) return;
+      }
     // V_0 = -R0 / ||R0|| (gmres.f:243), halo included
+    const double r1 = -1.0 / (nr0 * sc);
+    sc = 1.0;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
       const T r = kMixed ? as[k * kSlab + t] : rv[k];
-      ds[k * kSlab + t] = vb[(size_t)k * kSlab] = (T)(-1.0 / nr0 * (double)r);
+      ds[k * kSlab + t] = vb[(size_t)k * kSlab] = (T)(r1 * (double)r);
     }
-    for (int h = t; h < nh; h += kSlab) dh[h] = vh[h] = (T)(-1.0 / nr0 * (double)ah[h]);
+    for (int h = t; h < nh; h += kSlab) dh[h] = vh[h] = (T)(r1 * (double)ah[h]);
     __syncthreads();
     int kk = a.krylov;
     for (int j = 0; j < kk; ++j) {

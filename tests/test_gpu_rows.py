@@ -255,3 +255,22 @@ def test_a_gmres_launch_that_gives_up_falls_back(gpu, monkeypatch):
     monkeypatch.setenv("BHIP_ROWS_WAIT", "0")
     m = M.channel_mesh(120, 90, 1200.0, 900.0)
     _check_gmres(m, _system(m), 5)
+
+
+def test_mixed_gmres_of_residuals_beyond_float(gpu):
+    """A right-hand side of 2^130 times another's: all operations scale by a
+    power of two, so only FP32's range could tell the two apart. (1e-6: the
+    scaled residual rounds elsewhere in FP32, both solves stop at 1e-9.)"""
+    m = M.channel_mesh(120, 90, 1200.0, 900.0)
+    sysd = _system(m)
+    b = 1.0 + np.random.default_rng(3).random(m.npoin)
+    out = []
+    for scale in (1.0, 2.0 ** 130):
+        ctx = bief.Context(m)
+        ctx.set_matrix("Q", "S", sysd["da"], sysd["xa"])
+        x, info = ctx.solve(np.zeros(m.npoin), b * scale, slv=7, precon=2, eps=1e-9, nitmax=100,
+                            krylov=5, precision=bief.PREC_MIXED)
+        assert info["converged"], info
+        out.append(x / scale)
+        ctx.close()
+    assert np.linalg.norm(out[1] - out[0]) <= 1e-6 * np.linalg.norm(out[0])
