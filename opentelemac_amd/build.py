@@ -97,7 +97,7 @@ def build_dropin():
     os.makedirs(mod, exist_ok=True)
     srcs = [os.path.join(FSRC, "bief_hip_capi.f90"), os.path.join(FSRC, "bief_hip_shim.F90"),
             os.path.join(ROOT, "oracle", "ref_driver.f90")]
-    _run([_fc(), "-O2", "-cpp", "-ffixed-line-length-132", "-fPIC",
+    _run([_fc(), "-O2", "-cpp", "-ffixed-line-length-132", "-fPIC", "-shared",
           "-I", os.path.join(ref, "mod"), "-module-dir", mod, *srcs,
           os.path.join(ref, "libbief_ref.a"), "-L", HERE, "-lbiefhip",
           "-Wl,-rpath,$ORIGIN/../../opentelemac_amd", "-o", out])
