@@ -19,7 +19,8 @@
 // A slice stores its coefficients entry by entry, 64 lanes wide (coalesced):
 // entry j of lane l of slice q is (slice_off[q] + j) * 64 + l. Its column ids
 // are stored two entries to a 32-bit word: ids[((pair_off[q] + j / 2) * 64 + l) * 2
-// + (j & 1)]. Slice k * kSlices + w of workgroup g is q = g * group * kSlices + that.
+// + (j & 1)], at least one word per lane (zeros where the slice is empty). Slice
+// k * kSlices + w of workgroup g is q = g * group * kSlices + that.
 //
 // A workgroup holds the multiplied vector of its own rows and of its halo (rows
 // of other workgroups that its entries name) in LDS; ids[] are indices into that

@@ -305,7 +305,8 @@ __device__ inline T slice_dot(const T* __restrict__ v, const unsigned* __restric
 }
 
 // The first F entries of one row, kept in registers for a whole solve.
-// Slices with fewer read their last one again and multiply it by zero.
+// Slices with fewer read their last one again and multiply it by zero; empty
+// ones read an id word of their own and the coefficients behind them.
 template <typename T, int F>
 struct RowFront {
   T c[F];
@@ -1550,8 +1551,6 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
     return nullptr;
   RowLayout R;
   if (!build_rows(L, nsys, node_off, ncu, R)) return nullptr;
-  // the kernels may read one entry column past the last slice (load_front)
-  R.ids.resize(R.ids.size() + 128, 0);
   std::unique_ptr<RowsDev> r(new RowsDev());
   r->nslice = R.nslice;
   r->group = R.group;
@@ -1561,7 +1560,7 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
   r->by_block = R.by_block;
   r->max_slots = R.max_slots;
   r->lds_max = lds_max;
-  r->nent = R.nent + 64;
+  r->nent = R.nent + 64;  // load_front reads one entry column of an empty slice too
   r->ncu = ncu;
   r->nexp = (int)R.exp_loc.size();
   lds_max -= 2048;  // the kernels' static LDS: their sums

@@ -241,7 +241,9 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
       }
       R.ref_off[i + 1] = (int32_t)runits;
       R.slice_off[i + 1] = (int32_t)units;
-      R.pair_off[i + 1] = R.pair_off[i] + (out[g].width[q] + 1) / 2;
+      // (an id word per lane for an empty slice too: load_front reads one, and
+      // the next slice's would name another workgroup's halo)
+      R.pair_off[i + 1] = R.pair_off[i] + std::max((out[g].width[q] + 1) / 2, 1);
     }
   bool fits = true;
   for (const auto& o : out) fits = fits && wrows + o.halo.size() <= 65535;

@@ -1,0 +1,30 @@
+"""Assembled row storage on the host: built from the sources, no GPU."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "opentelemac_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("rows") / "check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC,
+                    os.path.join(HERE, "rows_layout_check.cpp"),
+                    os.path.join(CSRC, "layout.cpp"), os.path.join(CSRC, "rows_layout.cpp"),
+                    "-lpthread", "-o", exe], check=True)
+    return exe
+
+
+# (max workgroups, block nodes, systems): ragged members before one whose rows
+# have only entries of another workgroup's columns; 1, 2, 4 and 8 slabs
+@pytest.mark.parametrize("args", [
+    (256, 64, "100", "far2048"), (256, 1024, "100", "far2048"), (256, 64, "700", "far4096", "3"),
+    (4, 64, "1300", "far4096"), (2, 1024, "100", "far4096"), (2, 64, "9000", "far8192"),
+    (256, 1024, "1024"), (256, 1024, "1025"),
+])
+def test_ids_stay_within_their_workgroup(check, args):
+    out = subprocess.run([check, *map(str, args)], capture_output=True, text=True)
+    assert out.stdout == "ok\n", (out.stdout, out.returncode)
