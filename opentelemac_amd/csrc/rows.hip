@@ -335,7 +335,10 @@ __device__ inline T front_dot(const RowFront<T, F>& f, const T* ys) {
 
 // as = A ds of the workgroup's rows, without the diagonal: thread t's k-th row
 // at k * kSlab + t. The coefficients of small partitions stay in registers
-// for the whole solve.
+// for the whole solve. Whatever the registers hold, a row's terms are added in
+// one order, so its sum is the same to the bit in every partition: a chain of
+// 8, and to it the sum of the others' chains of 4. (Up to 12 that is what
+// slice_dot<8> does, with more loads in flight.)
 template <typename T, int R>
 struct RowProduct {
   static constexpr bool kKeep = R * sizeof(T) <= 16 || R == 4;
@@ -372,7 +375,6 @@ struct RowProduct {
           const T* v;
           const unsigned* id;
           const int w = slice(ra, val, wg, k, v, id);
-          // (a row's first 8 terms are one chain whatever the registers hold)
           if constexpr (kFront == 4) {
             const T* v4 = v + 4 * 64;
             const unsigned* id4 = id + 2 * 64;
@@ -395,7 +397,9 @@ struct RowProduct {
         const T* v;
         const unsigned* id;
         const int w = slice(ra, val, wg, k, v, id);
-        as[k * kSlab + t] = slice_dot<8>(v, id, lane, 0, w, ds);
+        as[k * kSlab + t] = w <= 12 ? slice_dot<8>(v, id, lane, 0, w, ds)
+                                    : row_dot<T, 8>(v, id, lane, ds) +
+                                          slice_dot<4>(v, id, lane, 8, w, ds);
       }
     }
   }
