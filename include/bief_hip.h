@@ -107,6 +107,12 @@ void* bhip_ctx_stream(bhip_ctx* ctx);
  * context has queued. Safe from several threads. */
 int bhip_ctx_after_stream(bhip_ctx* ctx, void* stream);
 int bhip_stream_after_ctx(bhip_ctx* ctx, void* stream);
+/* The assembled rows that SOLVE's CG and GMRES run on where a context has them:
+ * the device memory they hold (0: there are none; BHIP_ROWS_BYTES in the
+ * environment at bhip_ctx_create is the most they may take), and what the last
+ * SOLVE ran on: 1 the rows, 0 element by element, -1 none yet. A context or a
+ * solve without memory for its rows does without them. Either may be NULL. */
+int bhip_ctx_rows(const bhip_ctx* ctx, int64_t* bytes, int* last_solve);
 /* layout statistics: nblocks, max colours per block, element instances
  * (duplicated halo elements included), halo node count */
 int bhip_ctx_stats(const bhip_ctx* ctx, int* nblocks, int* max_colors,

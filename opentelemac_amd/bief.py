@@ -84,6 +84,7 @@ def lib():
         L.bhip_ctx_destroy.argtypes = [_P]
         L.bhip_ctx_stream.argtypes = [_P]
         L.bhip_ctx_stream.restype = _P
+        L.bhip_ctx_rows.argtypes = [_P, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(_I)]
         L.bhip_ctx_after_stream.argtypes = [_P, _P]
         L.bhip_stream_after_ctx.argtypes = [_P, _P]
         L.bhip_ctx_stats.argtypes = [_P, ctypes.POINTER(_I), ctypes.POINTER(_I),
@@ -252,6 +253,13 @@ class Context:
     def torch_stream(self):
         import torch
         return torch.cuda.ExternalStream(self.stream_ptr())
+
+    def rows(self):
+        """Device memory of the assembled rows (0: none) and whether the last
+        SOLVE ran on them (None: no solve yet)."""
+        n, last = ctypes.c_int64(), _I()
+        _check(lib().bhip_ctx_rows(self._h, ctypes.byref(n), ctypes.byref(last)), "bhip_ctx_rows")
+        return {"bytes": n.value, "last_solve": None if last.value < 0 else bool(last.value)}
 
     def stats(self):
         nb, mc = _I(), _I()

@@ -1062,6 +1062,7 @@ struct bhip_ctx {
   bool use_graphs = true;
   bhip::RowsDev* rows = nullptr;  // assembled rows for the persistent CG, or none
   bool rows_off = false;          // it gave up once: the two-kernel CG from then on
+  int solved_on = -1;             // bhip_ctx_rows: what the last SOLVE ran on
   int prefetch_j = 0;  // register prefetch depth of the element kernels
   int iter_hint[4] = {0, 0, 0, 0};  // FP64 CG, inner CG, inner solves, CGSTAB
   int inner_hint[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // iterations of inner solve k (mixed CG)
@@ -1452,6 +1453,13 @@ int bhip_ctx_destroy(bhip_ctx* c) {
 }
 
 void* bhip_ctx_stream(bhip_ctx* c) { return c ? (void*)c->stream : nullptr; }
+
+int bhip_ctx_rows(const bhip_ctx* c, int64_t* bytes, int* last_solve) {
+  if (!c) return BHIP_EBADARG;
+  if (bytes) *bytes = c->rows ? (int64_t)rows_bytes(c->rows) : 0;
+  if (last_solve) *last_solve = c->solved_on;
+  return BHIP_OK;
+}
 
 // `second` after what `first` holds now. One event of the context serves all
 // such calls (a wait keeps the recording it was given); streams of another
@@ -2227,7 +2235,8 @@ static int cg_mixed(bhip_ctx* c, double* x, const double* b, double eps, int nit
 // ---------------------------------------------------------------------------
 // CG on assembled rows: one persistent launch per (inner) solve
 // ---------------------------------------------------------------------------
-constexpr int kGaveUp = -1;  // the launch gave up: use the two-kernel CG
+constexpr int kGaveUp = -1;    // the launch gave up: use the solver without rows
+constexpr int kNoMemory = -2;  // no memory for the launch: likewise
 
 // At most one persistent launch per GPU at a time: its workgroups wait for
 // each other, so two launches that share the CUs could each hold what the
@@ -2337,11 +2346,17 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   if (diag && td == 'I') td = 'Q';
   if (diag && precon % 2 == 0) td = 'I';
   const int row_bytes = mixed ? 4 : 8, npair = L.ndp * (L.ndp - 1) / 2;
-  const bool use_rows = c->rows && !c->rows_off && td != '0' &&
-                        (cfg->slv == 1 || (cfg->slv == 7 && rows_gmres_fits(c->rows, row_bytes)));
+  bool use_rows = c->rows && !c->rows_off && td != '0' &&
+                  (cfg->slv == 1 || (cfg->slv == 7 && rows_gmres_fits(c->rows, row_bytes)));
+  if (use_rows) {
+    const hipError_t e = rows_reserve(c->rows, row_bytes);
+    if (e == hipErrorOutOfMemory)
+      use_rows = false;
+    else
+      HIP_OK(e);
+  }
   const bool by_block = use_rows && rows_by_block(c->rows);
   const bool both = mixed;  // the FP64 residuals are taken from rows too
-  if (use_rows) HIP_OK(rows_reserve(c->rows, row_bytes));
   if (diag) {
     // PRECD1 (precd1.f:90-149), X and B taken from the caller's vectors
     hipLaunchKernelGGL(k_precd1_nodes, dim3(g), dim3(kThreads), 0, c->stream, c->vx.p, c->vb.p,
@@ -2366,6 +2381,7 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
                          c->typext == 'Q', c->stream));
   }
   int rc;
+  c->solved_on = 0;
   double* xsrc = c->vx.p;  // where the solution is left
   bool written = false;    // it is in x_dev already
   // X <- X*D (solve.f:637-641), back to the caller's order or copied as it is
@@ -2401,7 +2417,7 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
     q.inner_nitmax = std::max(inner_nitmax, 1);
     q.reliable = c->reliable ? 1 : 0;
     const int r = cg_rows(c, mixed, q, info);
-    written = r != kGaveUp;
+    c->solved_on = written = r != kGaveUp;
     if (r == kGaveUp) c->rows_off = true;
     return r;
   };
@@ -2417,7 +2433,9 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
                                       cfg->nitmax, cfg->krylov, info);
       if (moved) xsrc = c->vd1.p;
       if (rc == kGaveUp) c->rows_off = true;
+      c->solved_on = rc != kGaveUp && rc != kNoMemory;
     }
+    if (rc == kNoMemory) rc = kGaveUp;
     if (rc == kGaveUp && mixed)
       rc = bhip::gmres_mixed(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, cfg->krylov, xa32_ready,
                              info);

@@ -626,7 +626,9 @@ static int gmres_rows(bhip_ctx* c, double* x, double* xout, bool* moved, const d
   q.nitmax = nitmax;
   q.krylov = krylov;
   q.st = reinterpret_cast<GmState*>(c->st_host_dev);
-  HIP_OK(rows_gmres<T>(c->rows, q, c->stream));
+  const hipError_t e = rows_gmres<T>(c->rows, q, c->stream);
+  if (e == hipErrorOutOfMemory) return kNoMemory;
+  HIP_OK(e);
   HIP_OK(hipStreamSynchronize(c->stream));
   if (s->gave_up) return kGaveUp;
   *moved = s->updated != 0;

@@ -1430,17 +1430,42 @@ __global__ void k_zero_words(u64* p, long n) {
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+// device memory of one context's rows; BHIP_ROWS_BYTES limits it
+struct RowsMem {
+  size_t used = 0, limit = SIZE_MAX;
+};
 template <typename T>
 struct Buf {
   T* p = nullptr;
-  ~Buf() {
-    if (p) (void)hipFree(p);
+  size_t bytes = 0;
+  RowsMem* mem = nullptr;
+  ~Buf() { (void)release(); }
+  // (a failure for want of memory is not left as HIP's last error: the caller
+  // has another way)
+  hipError_t alloc(size_t n, RowsMem& m) {
+    const size_t want = std::max<size_t>(n, 1) * sizeof(T);
+    if (want > m.limit - m.used) return hipErrorOutOfMemory;
+    const hipError_t e = hipMalloc((void**)&p, want);
+    if (e != hipSuccess) {
+      if (e == hipErrorOutOfMemory) (void)hipGetLastError();
+      p = nullptr;
+      return e;
+    }
+    m.used += want;
+    bytes = want;
+    mem = &m;
+    return e;
   }
-  hipError_t alloc(size_t n) {
-    return hipMalloc((void**)&p, std::max<size_t>(n, 1) * sizeof(T));
+  hipError_t release() {
+    if (!p) return hipSuccess;
+    const hipError_t e = hipFree(p);
+    mem->used -= bytes;
+    p = nullptr;
+    bytes = 0;
+    return e;
   }
-  hipError_t put(const std::vector<T>& v, hipStream_t s) {
-    hipError_t e = alloc(v.size());
+  hipError_t put(const std::vector<T>& v, RowsMem& m, hipStream_t s) {
+    hipError_t e = alloc(v.size(), m);
     if (e == hipSuccess && !v.empty())
       e = hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s);
     return e;
@@ -1448,6 +1473,7 @@ struct Buf {
 };
 
 struct RowsDev {
+  RowsMem mem;
   int nslice = 0, group = 1, nwg = 0, nsys = 1, max_halo = 0;
   int64_t nent = 0;
   int ncu = 0, nexp = 0;
@@ -1468,7 +1494,6 @@ struct RowsDev {
   bool gm_fits[2] = {false, false};
   int nhalo = 0;
   Buf<unsigned char> gm, gmh;
-  size_t gm_bytes = 0, gmh_bytes = 0;
 };
 
 static size_t cg_lds(const RowsDev& r, int bytes) {
@@ -1577,9 +1602,13 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
   if ((*err = gm_fits<double>(*r, r->lds_max, &r->gm_fits[0])) != hipSuccess) return nullptr;
   if ((*err = gm_fits<float>(*r, r->lds_max, &r->gm_fits[1])) != hipSuccess) return nullptr;
   r->nhalo = (int)R.halo_row.size();
+  if (const char* ev = getenv("BHIP_ROWS_BYTES")) r->mem.limit = strtoull(ev, nullptr, 10);
+  // without memory for them there are no rows, and SOLVE runs element by element
   auto ok = [&](hipError_t e) {
-    if (e != hipSuccess) *err = e;
-    return e == hipSuccess;
+    if (e == hipSuccess) return true;
+    if (e != hipErrorOutOfMemory) *err = e;
+    (void)hipStreamSynchronize(stream);  // (copies of the host arrays are under way)
+    return false;
   };
   std::vector<int32_t> slab_slice;
   if (R.by_block)
@@ -1590,16 +1619,16 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
                           R.wg_row0.begin()) - 1;
       slab_slice.push_back(g * R.group * kSlices + (row - R.wg_row0[g]) / kSlab * (kSlices / R.group));
     }
-  if (!ok(r->wg_row0.put(R.wg_row0, stream)) || !ok(r->refs16.put(R.refs16, stream)) ||
-      !ok(r->slab_slice.put(slab_slice, stream)) || !ok(r->slice_off.put(R.slice_off, stream)) ||
-      !ok(r->pair_off.put(R.pair_off, stream)) ||
-      !ok(r->refs.put(R.refs, stream)) ||
-      !ok(r->wg_sys.put(R.wg_sys, stream)) || !ok(r->sys_wg.put(R.sys_wg, stream)) ||
-      !ok(r->halo_off.put(R.halo_off, stream)) || !ok(r->halo_row.put(R.halo_row, stream)) ||
-      !ok(r->halo_src.put(R.halo_src, stream)) || !ok(r->exp_off.put(R.exp_off, stream)) ||
-      !ok(r->rowpos.put(R.rowpos, stream)) || !ok(r->ids.put(R.ids, stream)) ||
-      !ok(r->exp_loc.put(R.exp_loc, stream)) || !ok(r->ref_end.put(R.ref_end, stream)) ||
-      !ok(r->ref_off.put(R.ref_off, stream)) || !ok(r->v64.alloc(r->nent)))
+  if (!ok(r->wg_row0.put(R.wg_row0, r->mem, stream)) || !ok(r->refs16.put(R.refs16, r->mem, stream)) ||
+      !ok(r->slab_slice.put(slab_slice, r->mem, stream)) || !ok(r->slice_off.put(R.slice_off, r->mem, stream)) ||
+      !ok(r->pair_off.put(R.pair_off, r->mem, stream)) ||
+      !ok(r->refs.put(R.refs, r->mem, stream)) ||
+      !ok(r->wg_sys.put(R.wg_sys, r->mem, stream)) || !ok(r->sys_wg.put(R.sys_wg, r->mem, stream)) ||
+      !ok(r->halo_off.put(R.halo_off, r->mem, stream)) || !ok(r->halo_row.put(R.halo_row, r->mem, stream)) ||
+      !ok(r->halo_src.put(R.halo_src, r->mem, stream)) || !ok(r->exp_off.put(R.exp_off, r->mem, stream)) ||
+      !ok(r->rowpos.put(R.rowpos, r->mem, stream)) || !ok(r->ids.put(R.ids, r->mem, stream)) ||
+      !ok(r->exp_loc.put(R.exp_loc, r->mem, stream)) || !ok(r->ref_end.put(R.ref_end, r->mem, stream)) ||
+      !ok(r->ref_off.put(R.ref_off, r->mem, stream)) || !ok(r->v64.alloc(r->nent, r->mem)))
     return nullptr;
   // sync words of CG in both precisions and of GMRES: sums, exchange, then
   // the counters
@@ -1611,7 +1640,7 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
                            (size_t)2 * kReplicas * kSums * R.nwg * 2,
                            gm ? (size_t)2 * kReplicas * kGmSums * R.nwg * 2 : 0};
   const size_t nwords = nslot[0] + nslot[1] + nslot[2] + 3 * tail;
-  if (!ok(r->words.alloc(nwords))) return nullptr;
+  if (!ok(r->words.alloc(nwords, r->mem))) return nullptr;
   u64 ticks = kWaitTicks;
   if (const char* ev = getenv("BHIP_ROWS_WAIT")) ticks = strtoull(ev, nullptr, 10);
   u64* p = r->words.p;
@@ -1632,13 +1661,16 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
 
 void rows_destroy(RowsDev* r) { delete r; }
 
+size_t rows_bytes(const RowsDev* r) { return r->mem.used; }
+
 hipError_t rows_reserve(RowsDev* r, int bytes) {
-  if (bytes == 8) return r->v64.p ? hipSuccess : r->v64.alloc(r->nent);
-  if (!r->res.p) {
-    const hipError_t e = r->res.alloc((size_t)r->nwg * r->group * kSlab);
-    if (e != hipSuccess) return e;
+  if (bytes == 8 || r->v32.p) return hipSuccess;
+  hipError_t e = r->res.alloc((size_t)r->nwg * r->group * kSlab, r->mem);
+  if (e == hipSuccess) {
+    e = r->v32.alloc(r->nent, r->mem);
+    if (e != hipSuccess) (void)r->res.release();
   }
-  return r->v32.p ? hipSuccess : r->v32.alloc(r->nent);
+  return e;
 }
 
 hipError_t rows_assemble(RowsDev* r, int bytes, bool both, const double* xa, int nslot_pad,
@@ -1738,20 +1770,13 @@ hipError_t rows_gmres(RowsDev* r, const RowsGmres& a, hipStream_t stream) {
   const size_t own = (size_t)r->nwg * r->group * kSlab * sizeof(T) *
                      ((sizeof(T) == 8 ? 2 : 1) * a.krylov + 1);
   const size_t halo = (size_t)std::max(r->nhalo, 1) * sizeof(T) * a.krylov;
-  auto grow = [&](Buf<unsigned char>& b, size_t& have, size_t want) -> hipError_t {
-    if (have >= want) return hipSuccess;
-    if (b.p) {
-      const hipError_t e = hipFree(b.p);
-      b.p = nullptr;
-      have = 0;
-      if (e != hipSuccess) return e;
-    }
-    const hipError_t e = b.alloc(want);
-    if (e == hipSuccess) have = want;
-    return e;
+  auto grow = [&](Buf<unsigned char>& b, size_t want) -> hipError_t {
+    if (b.bytes >= want) return hipSuccess;
+    const hipError_t e = b.release();
+    return e == hipSuccess ? b.alloc(want, r->mem) : e;
   };
-  hipError_t e = grow(r->gm, r->gm_bytes, own);
-  if (e == hipSuccess) e = grow(r->gmh, r->gmh_bytes, halo);
+  hipError_t e = grow(r->gm, own);
+  if (e == hipSuccess) e = grow(r->gmh, halo);
   if (e != hipSuccess) return e;
   const RowArgs ra = row_args(r, 2);
   r->ep[2] ^= 1;

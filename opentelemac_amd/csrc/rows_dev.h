@@ -10,14 +10,18 @@ namespace bhip {
 struct RowsDev;
 
 // The rows of a layout on the current device, or nullptr when they cannot be
-// used (build_rows; *err stays hipSuccess then). Work is queued on stream;
+// used (build_rows, or no memory for them; *err stays hipSuccess then). Work is queued on stream;
 // the host arrays are read before it returns.
 RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStream_t stream,
                      hipError_t* err);
 void rows_destroy(RowsDev* r);
 
-// Row values of precision 8 or 4 bytes: allocated here when first asked for.
+// Row values of precision 8 or 4 bytes: those of 4 are allocated here when first
+// asked for. hipErrorOutOfMemory: solve without the rows.
 hipError_t rows_reserve(RowsDev* r, int bytes);
+
+// device memory that the rows hold
+size_t rows_bytes(const RowsDev* r);
 
 // Assembles the rows of the precision from the slot coefficients xa (upper
 // npair columns, and the lower ones when nonsym), nslot_pad apart. both: in
@@ -87,6 +91,8 @@ struct RowsGmres {
   GmState* st;         // the outcome; host memory will do
 };
 bool rows_gmres_fits(const RowsDev* r, int bytes);
+// (allocates the basis when a larger K is first asked for; hipErrorOutOfMemory
+// as of rows_reserve)
 template <typename T>
 hipError_t rows_gmres(RowsDev* r, const RowsGmres& a, hipStream_t stream);
 
