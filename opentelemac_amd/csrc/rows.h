@@ -83,6 +83,7 @@ struct RowLayout {
 // Rows of the layout's matrix for nsys systems of node_off[nsys + 1] nodes.
 // max_wg: workgroups that can be resident at once. Returns false (and leaves R
 // empty) when a system needs more workgroups than that, or more than kMaxGang.
+// Throws std::bad_alloc.
 bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, RowLayout& R);
 
 }  // namespace bhip

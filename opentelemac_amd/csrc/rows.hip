@@ -51,6 +51,7 @@
 #include <cstdlib>
 #include <type_traits>
 #include <memory>
+#include <new>
 #include <vector>
 
 namespace bhip {
@@ -1567,8 +1568,8 @@ static hipError_t gm_fits(const RowsDev& r, int lds_max, bool* fits) {
   });
 }
 
-RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStream_t stream,
-                     hipError_t* err) {
+static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
+                           hipStream_t stream, hipError_t* err) {
   *err = hipSuccess;
   int dev = 0, ncu = 0, lds_max = 0;
   if ((*err = hipGetDevice(&dev)) != hipSuccess) return nullptr;
@@ -1657,6 +1658,15 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
   hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, stream, r->words.p, (long)nwords);
   if (!ok(hipGetLastError()) || !ok(hipStreamSynchronize(stream))) return nullptr;
   return r.release();
+}
+
+RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStream_t stream,
+                     hipError_t* err) {
+  try {
+    return rows_build(L, nsys, node_off, stream, err);
+  } catch (const std::bad_alloc&) {  // no host memory for them: no rows either
+    return nullptr;
+  }
 }
 
 void rows_destroy(RowsDev* r) { delete r; }

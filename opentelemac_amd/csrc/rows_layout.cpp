@@ -3,6 +3,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <exception>
+#include <mutex>
 #include <thread>
 
 namespace bhip {
@@ -10,20 +12,33 @@ namespace bhip {
 namespace {
 
 // f(i) for i in [0, n) on a few host threads, each with its own scratch from
-// make()
+// make(). An exception of any of them is thrown here, once all have ended; where
+// no (more) threads can be started, those that are there do the work.
 template <typename Make, typename F>
 void parallel_for(int n, Make make, F f) {
   const int hw = (int)std::thread::hardware_concurrency();
   const int nt = std::max(1, std::min({hw, 8, n / 16}));
   std::atomic<int> next{0};
+  std::exception_ptr failed;
+  std::mutex mu;
   auto work = [&]() {
-    auto scratch = make();
-    for (int i; (i = next.fetch_add(1)) < n;) f(i, scratch);
+    try {
+      auto scratch = make();
+      for (int i; (i = next.fetch_add(1)) < n;) f(i, scratch);
+    } catch (...) {
+      std::lock_guard<std::mutex> one(mu);
+      failed = std::current_exception();
+      next = n;
+    }
   };
   std::vector<std::thread> pool;
-  for (int t = 1; t < nt; ++t) pool.emplace_back(work);
+  try {
+    for (int t = 1; t < nt; ++t) pool.emplace_back(work);
+  } catch (...) {
+  }
   work();
   for (auto& t : pool) t.join();
+  if (failed) std::rethrow_exception(failed);
 }
 
 struct Contribution {

@@ -1,14 +1,39 @@
 // Host-side check of the assembled row storage: prints "ok" or what is wrong.
-// Arguments: nsys, then per system the nodes (in segment storage, a chain of
-// neighbours, or `far`: two halves joined only with each other).
+// Arguments: workgroups that fit, nodes per block, then per system its nodes (in
+// segment storage, a chain of neighbours, or `far`: two halves joined only with
+// each other). CHECK_FAIL in the environment: "threads", no thread can be
+// started; "memory=<n>", the n-th allocation of build_rows fails (and "bad_alloc"
+// is printed).
 #include "rows.h"
 
+#include <dlfcn.h>
+#include <errno.h>
+#include <pthread.h>
+
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <random>
 
 using namespace bhip;
+
+static bool no_threads = false;
+static std::atomic<long> allocations_left{-1};  // negative: no limit
+
+extern "C" int pthread_create(pthread_t* t, const pthread_attr_t* a, void* (*f)(void*), void* p) {
+  typedef int (*Real)(pthread_t*, const pthread_attr_t*, void* (*)(void*), void*);
+  static const Real real = (Real)dlsym(RTLD_NEXT, "pthread_create");
+  return no_threads ? EAGAIN : real(t, a, f, p);
+}
+void* operator new(size_t n) {
+  if (allocations_left >= 0 && allocations_left-- == 0) throw std::bad_alloc();
+  if (void* p = malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
 
 static int wrong(const char* what, int at) {
   printf("%s (%d)\n", what, at);
@@ -54,6 +79,21 @@ int main(int argc, char** argv) {
   std::vector<int64_t> off(1, 0);
   for (int n : np) off.push_back(off.back() + n);
   RowLayout R;
+  if (const char* f = getenv("CHECK_FAIL")) {
+    no_threads = strcmp(f, "threads") == 0;
+    if (strncmp(f, "memory=", 7) == 0) {
+      allocations_left = atol(f + 7);
+      try {
+        const bool built = build_rows(L, nsys, off.data(), max_wg, R);
+        allocations_left = -1;
+        printf("%s\n", built ? "built" : "no rows");
+      } catch (const std::bad_alloc&) {
+        allocations_left = -1;
+        printf("bad_alloc\n");
+      }
+      return 0;
+    }
+  }
   if (!build_rows(L, nsys, off.data(), max_wg, R)) return wrong("no rows", 0);
   const int wrows = R.group * kSlab;
   // every id that the kernels read, a slice's and those load_front reads of a

@@ -14,7 +14,7 @@ def check(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", CSRC,
                     os.path.join(HERE, "rows_layout_check.cpp"),
                     os.path.join(CSRC, "layout.cpp"), os.path.join(CSRC, "rows_layout.cpp"),
-                    "-lpthread", "-o", exe], check=True)
+                    "-rdynamic", "-lpthread", "-ldl", "-o", exe], check=True)
     return exe
 
 
@@ -28,3 +28,24 @@ def check(tmp_path_factory):
 def test_ids_stay_within_their_workgroup(check, args):
     out = subprocess.run([check, *map(str, args)], capture_output=True, text=True)
     assert out.stdout == "ok\n", (out.stdout, out.returncode)
+
+
+def _run(check, fail, *args):
+    out = subprocess.run([check, *args], capture_output=True, text=True,
+                         env=dict(os.environ, CHECK_FAIL=fail))
+    assert out.returncode == 0, (out.returncode, out.stdout, out.stderr)
+    return out.stdout
+
+
+MANY = ("256", "64", "60000", "far40960")  # enough workgroups for several threads
+
+
+def test_rows_are_built_without_threads(check):
+    assert _run(check, "threads", *MANY) == "ok\n"
+
+
+def test_a_failed_allocation_reaches_the_caller(check):
+    """In the caller's thread or in another, first and last ones among them."""
+    got = [_run(check, f"memory={n}", *MANY) for n in (0, 1, 5, 20, 60, 200, 1000, 5000, 20000)]
+    assert set(got) <= {"bad_alloc\n", "built\n"} and got[0] == "bad_alloc\n"
+    assert got.count("bad_alloc\n") >= 6
