@@ -1061,7 +1061,8 @@ struct bhip_ctx {
   std::vector<SolveGraph> solve_graphs;
   bool use_graphs = true;
   bhip::RowsDev* rows = nullptr;  // assembled rows for the persistent CG, or none
-  bool rows_off = false;          // it gave up once: the two-kernel CG from then on
+  // a launch gave up: so many solves without rows, twice as many after the next
+  int rows_pause = 0, rows_next_pause = 64;
   int solved_on = -1;             // bhip_ctx_rows: what the last SOLVE ran on
   int prefetch_j = 0;  // register prefetch depth of the element kernels
   int iter_hint[4] = {0, 0, 0, 0};  // FP64 CG, inner CG, inner solves, CGSTAB
@@ -2238,12 +2239,25 @@ static int cg_mixed(bhip_ctx* c, double* x, const double* b, double eps, int nit
 constexpr int kGaveUp = -1;    // the launch gave up: use the solver without rows
 constexpr int kNoMemory = -2;  // no memory for the launch: likewise
 
-// At most one persistent launch per GPU at a time: its workgroups wait for
-// each other, so two launches that share the CUs could each hold what the
-// other needs.
+// At most one persistent launch of this process per GPU at a time: its
+// workgroups wait for each other, so two launches that share the CUs could each
+// hold what the other needs. (Two processes can: a launch then gives up after its
+// limit.)
 static std::mutex& rows_mutex(int dev) {
   static std::mutex mu[64];
   return mu[dev & 63];
+}
+
+// Solves without rows follow, more each time: a launch that gives up has waited
+// 4 s, so the waits stay few however long the GPU is shared.
+static void rows_gave_up(bhip_ctx* c) {
+  c->rows_pause = c->rows_next_pause;
+  if (c->rows_next_pause < (1 << 24)) c->rows_next_pause *= 2;
+  fprintf(stderr,
+          "libbiefhip: the workgroups of a solve did not run at the same time (does another "
+          "process use the GPU, or a CU mask apply?); this and the next %d solves of the "
+          "context run element by element\n",
+          c->rows_pause);
 }
 
 // CG as in cg_fp64 or cg_mixed; the solution goes to q.x, X = 0 of a zero
@@ -2258,6 +2272,7 @@ static int cg_rows(bhip_ctx* c, bool mixed, RowsCg q, bhip_solve_info* info) {
   HIP_OK(hipStreamSynchronize(c->stream));
   for (int sy = 0; sy < c->nsys; ++sy)
     if (c->st_host[sy].gave_up) return kGaveUp;
+  rows_ended(c->rows, mixed ? kRowsCgMixed : kRowsCg);
   return collect_infos(c, nullptr, mixed, info);
 }
 
@@ -2346,8 +2361,12 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
   if (diag && td == 'I') td = 'Q';
   if (diag && precon % 2 == 0) td = 'I';
   const int row_bytes = mixed ? 4 : 8, npair = L.ndp * (L.ndp - 1) / 2;
-  bool use_rows = c->rows && !c->rows_off && td != '0' &&
+  bool use_rows = c->rows && td != '0' &&
                   (cfg->slv == 1 || (cfg->slv == 7 && rows_gmres_fits(c->rows, row_bytes)));
+  if (use_rows && c->rows_pause > 0) {
+    --c->rows_pause;
+    use_rows = false;
+  }
   if (use_rows) {
     const hipError_t e = rows_reserve(c->rows, row_bytes);
     if (e == hipErrorOutOfMemory)
@@ -2418,7 +2437,7 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
     q.reliable = c->reliable ? 1 : 0;
     const int r = cg_rows(c, mixed, q, info);
     c->solved_on = written = r != kGaveUp;
-    if (r == kGaveUp) c->rows_off = true;
+    if (r == kGaveUp) rows_gave_up(c);
     return r;
   };
   if (cfg->slv == 6) {
@@ -2432,7 +2451,7 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
                  : gmres_rows<double>(c, c->vx.p, c->vd1.p, &moved, c->vb.p, cfg->eps,
                                       cfg->nitmax, cfg->krylov, info);
       if (moved) xsrc = c->vd1.p;
-      if (rc == kGaveUp) c->rows_off = true;
+      if (rc == kGaveUp) rows_gave_up(c);
       c->solved_on = rc != kGaveUp && rc != kNoMemory;
     }
     if (rc == kNoMemory) rc = kGaveUp;

@@ -631,6 +631,7 @@ static int gmres_rows(bhip_ctx* c, double* x, double* xout, bool* moved, const d
   HIP_OK(e);
   HIP_OK(hipStreamSynchronize(c->stream));
   if (s->gave_up) return kGaveUp;
+  rows_ended(c->rows, kRowsGmres);
   *moved = s->updated != 0;
   info->niter = s->m;
   info->relat = s->relat;

@@ -38,13 +38,15 @@
 //
 // Every wait ends: on the number it waits for, or after kWaitTicks of the
 // device clock, when the launch gives up (abort in the sync words), leaves the
-// initial solution as it was and the host falls back to the two-kernel CG
-// (BHIP_ROWS_WAIT=<ticks> changes the limit; 0 gives up at the first word that
-// is not there yet, which the tests use).
-// All workgroups of a system must be resident at once: the host launches at
-// most one such kernel per GPU at a time. When a launch has more workgroups
-// than fit the GPU, they take their numbers in the order in which they start,
-// so the system with the lowest numbers always has all of its own running.
+// initial solution as it was and the host solves element by element, this time
+// and the next ones (BHIP_ROWS_WAIT=<ticks> changes the limit; 0 gives up at the
+// first word that is not there yet, which the tests use).
+// All workgroups of a system must be resident at once: a process launches at
+// most one such kernel per GPU at a time. Another process that does so too, or a
+// mask on the CUs, can keep some from starting: the limit is for them. When a
+// launch has more workgroups than fit the GPU, they take their numbers in the
+// order in which they start, so the system with the lowest numbers always has
+// all of its own running.
 #include "rows_dev.h"
 
 #include <algorithm>
@@ -119,7 +121,7 @@ struct SyncWords {
   u64* xch;         // [2][2][exported rows], by parity of the meeting (a float has one
                     // word only)
   unsigned* epoch;  // [2][nsys] number of the last meeting, by parity of the launch
-  int* abort;       // a launch has given up
+  int* abort;       // the launch has given up
   unsigned* ticket; // workgroups started (launches larger than the GPU)
   u64 ticks;        // longest wait
 };
@@ -1491,6 +1493,10 @@ struct RowsDev {
   Buf<u64> words;
   SyncWords sy[3];  // CG FP64, CG FP32, GMRES
   int ep[3] = {0, 0, 0};
+  size_t sy_words[3] = {0, 0, 0};
+  // a launch that is not known to have ended well (rows_ended) may have left
+  // any meeting's number in the words: they are cleared before the next one
+  bool open[3] = {false, false, false};
   // GMRES: fits (FP64, FP32), scratch for a basis of gm_k vectors
   bool gm_fits[2] = {false, false};
   int nhalo = 0;
@@ -1568,6 +1574,11 @@ static hipError_t gm_fits(const RowsDev& r, int lds_max, bool* fits) {
   });
 }
 
+static u64 wait_ticks() {
+  const char* ev = getenv("BHIP_ROWS_WAIT");
+  return ev ? strtoull(ev, nullptr, 10) : kWaitTicks;
+}
+
 static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
                            hipStream_t stream, hipError_t* err) {
   *err = hipSuccess;
@@ -1642,8 +1653,6 @@ static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
                            gm ? (size_t)2 * kReplicas * kGmSums * R.nwg * 2 : 0};
   const size_t nwords = nslot[0] + nslot[1] + nslot[2] + 3 * tail;
   if (!ok(r->words.alloc(nwords, r->mem))) return nullptr;
-  u64 ticks = kWaitTicks;
-  if (const char* ev = getenv("BHIP_ROWS_WAIT")) ticks = strtoull(ev, nullptr, 10);
   u64* p = r->words.p;
   for (int k = 0; k < 3; ++k) {
     SyncWords& s = r->sy[k];
@@ -1652,8 +1661,9 @@ static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
     s.epoch = reinterpret_cast<unsigned*>(p += 4 * nexp);
     s.ticket = reinterpret_cast<unsigned*>(p += nepoch);
     s.abort = reinterpret_cast<int*>(p += 1);
-    s.ticks = ticks;
+    s.ticks = wait_ticks();
     p += 1;
+    r->sy_words[k] = p - s.slots;
   }
   hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, stream, r->words.p, (long)nwords);
   if (!ok(hipGetLastError()) || !ok(hipStreamSynchronize(stream))) return nullptr;
@@ -1726,7 +1736,15 @@ hipError_t rows_dmd(RowsDev* r, int bytes, bool both, const RowsDmd& a, hipStrea
 #undef BHIP_DMD_ROWS
 }
 
-static RowArgs row_args(const RowsDev* r, int k) {
+// for a launch of kind k, which counts as open from here on
+static RowArgs row_args(RowsDev* r, int k, hipStream_t stream) {
+  if (r->open[k]) {
+    hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, stream, r->sy[k].slots,
+                       (long)r->sy_words[k]);
+    r->ep[k] = 0;
+    r->sy[k].ticks = wait_ticks();
+  }
+  r->open[k] = true;
   RowArgs a;
   a.slice_off = r->slice_off.p;
   a.pair_off = r->pair_off.p;
@@ -1746,14 +1764,16 @@ static RowArgs row_args(const RowsDev* r, int k) {
   a.nhalo = r->nhalo;
   a.sy = r->sy[k];
   a.ep = r->ep[k];
+  r->ep[k] ^= 1;
   a.ticketed = r->nwg > r->ncu;
   return a;
 }
 
+void rows_ended(RowsDev* r, RowsKind k) { r->open[k] = false; }
+
 hipError_t rows_cg(RowsDev* r, bool mixed, RowsCg a, hipStream_t stream) {
   a.res = r->res.p;
-  const RowArgs ra = row_args(r, mixed);
-  r->ep[mixed] ^= 1;
+  const RowArgs ra = row_args(r, mixed ? kRowsCgMixed : kRowsCg, stream);
   if (ra.ticketed) {
     hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, stream,
                        reinterpret_cast<u64*>(ra.sy.ticket), 1L);
@@ -1788,8 +1808,7 @@ hipError_t rows_gmres(RowsDev* r, const RowsGmres& a, hipStream_t stream) {
   hipError_t e = grow(r->gm, own);
   if (e == hipSuccess) e = grow(r->gmh, halo);
   if (e != hipSuccess) return e;
-  const RowArgs ra = row_args(r, 2);
-  r->ep[2] ^= 1;
+  const RowArgs ra = row_args(r, kRowsGmres, stream);
   const T* val;
   if constexpr (sizeof(T) == 8)
     val = r->v64.p;

@@ -47,6 +47,12 @@ struct RowsDmd {
 };
 hipError_t rows_dmd(RowsDev* r, int bytes, bool both, const RowsDmd& a, hipStream_t stream);
 
+// Kinds of launches, each with its own words in device memory for what its
+// workgroups tell each other. After a launch that ended without giving up the
+// caller says so; any other clears the words at the next launch of the kind.
+enum RowsKind { kRowsCg, kRowsCgMixed, kRowsGmres };
+void rows_ended(RowsDev* r, RowsKind k);
+
 constexpr int kMaxOuter = 100;  // refinement sweeps of one mixed solve
 
 // SOLVE's CG, one per system of the context, in one launch: from the initial

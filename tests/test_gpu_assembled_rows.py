@@ -189,3 +189,39 @@ def test_memory_that_runs_out_after_the_set_up(gpu, monkeypatch):
             assert ctx.rows()["last_solve"] is on, (slv, prec, limit)
             assert ctx.rows()["bytes"] == (enough if rows else 0)
         ctx.close()
+
+
+@pytest.mark.parametrize("slv", [CG, GMRES])
+@pytest.mark.parametrize("prec", [bief.PREC_FP64, bief.PREC_MIXED])
+def test_rows_are_tried_again_after_a_launch_gave_up(gpu, monkeypatch, capfd, slv, prec):
+    """The solve that a launch gave up and the next 64 run element by element, with
+    one line about it; then the rows serve again, to the same bits as ever."""
+    m, sd = _case(70, 61)
+    eps = 1e-10 if prec == bief.PREC_FP64 else 1e-9
+
+    def solve(ctx):
+        ctx.set_matrix("Q", "S", sd["da"], sd["xa"])
+        x, info = ctx.solve(sd["x0"].copy(), sd["b"].copy(), slv=slv, precon=2, eps=eps,
+                            nitmax=2000, krylov=6, precision=prec)
+        assert info["converged"]
+        return x, info["niter"], ctx.rows()["last_solve"]
+
+    ctx = bief.Context(m)
+    want = solve(ctx)
+    assert want[2] is True
+    ctx.close()
+    monkeypatch.setenv("BHIP_ROWS_WAIT", "0")
+    ctx = bief.Context(m)
+    capfd.readouterr()
+    first = solve(ctx)
+    assert first[2] is False
+    assert np.linalg.norm(first[0] - want[0]) <= TOL[slv, prec] * np.linalg.norm(want[0])
+    assert capfd.readouterr().err.count("the next 64 solves") == 1
+    for _ in range(64):
+        assert solve(ctx)[2] is False
+    monkeypatch.delenv("BHIP_ROWS_WAIT")
+    for _ in range(3):
+        x, niter, on = solve(ctx)
+        assert on is True and niter == want[1] and np.array_equal(x, want[0])
+    assert "solves" not in capfd.readouterr().err
+    ctx.close()
