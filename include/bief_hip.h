@@ -145,8 +145,9 @@ int bhip_batch_create(int nsys, const int* npoin, const int* nelem, int ndp,
                       int block_nodes, bhip_ctx** out);
 int bhip_batch_info(const bhip_ctx* ctx, int nsys, bhip_solve_info* infos);
 /* Per-mesh completion time of the last CG solve of an ensemble (ms, device
- * clock): from the solve's set-up kernel to the kernel that stopped that
- * mesh (converged, NITMAX, or a zero right-hand side: 0). */
+ * clock): from the start of the CG (the launch on assembled rows, or the
+ * set-up kernel), the same for all meshes, to when that mesh stopped
+ * (converged, NITMAX, or a zero right-hand side: 0). */
 int bhip_batch_latency(const bhip_ctx* ctx, int nsys, double* ms);
 
 /* ---- matrix ------------------------------------------------------------ */

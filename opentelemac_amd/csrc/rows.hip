@@ -123,6 +123,7 @@ struct SyncWords {
   unsigned* epoch;  // [2][nsys] number of the last meeting, by parity of the launch
   int* abort;       // the launch has given up
   unsigned* ticket; // workgroups started (launches larger than the GPU)
+  u64* start;       // and the clock before the first of them
   u64 ticks;        // longest wait
 };
 
@@ -432,7 +433,7 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ val6
   unsigned e = __hip_atomic_load(ra.sy.epoch + ra.ep * ra.nsys + sys, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
   constexpr bool kMixed = sizeof(T) == 4;
-  const u64 t_start = wall_clock64();
+  const u64 t_start = ra.ticketed ? ld_word(ra.sy.start) : wall_clock64();
   if (load_relaxed(ra.sy.abort)) {
     store_relaxed(&st->gave_up, 1);
     if (lead)
@@ -769,7 +770,7 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ val6
       st->final_m = zero ? 0 : m;
       st->final_rr = zero ? 0.0 : rr;
     }
-    st->t_done = wall_clock64();
+    st->t_done = zero ? t_start : wall_clock64();
     st->done = status;
     __hip_atomic_store(ra.sy.epoch + (1 - ra.ep) * ra.nsys + sys, e, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
@@ -1424,6 +1425,12 @@ k_rows_assemble(T* __restrict__ val, double* __restrict__ val64, const double* _
   }
 }
 
+// before a launch whose workgroups take numbers as they start
+__global__ void k_rows_start(SyncWords sy) {
+  *sy.ticket = 0;
+  *sy.start = wall_clock64();
+}
+
 __global__ void k_zero_words(u64* p, long n) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n;
        i += (long)gridDim.x * blockDim.x)
@@ -1647,7 +1654,7 @@ static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
   const bool gm = r->gm_fits[0] || r->gm_fits[1];
   const size_t nexp = R.exp_loc.size();
   const size_t nepoch = (2 * (size_t)nsys + 1) / 2 + 1;  // in 64-bit words
-  const size_t tail = 4 * nexp + nepoch + 2;
+  const size_t tail = 4 * nexp + nepoch + 3;
   const size_t nslot[3] = {(size_t)2 * kReplicas * kSums * R.nwg * 2,
                            (size_t)2 * kReplicas * kSums * R.nwg * 2,
                            gm ? (size_t)2 * kReplicas * kGmSums * R.nwg * 2 : 0};
@@ -1660,6 +1667,7 @@ static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
     s.xch = (p += nslot[k]);
     s.epoch = reinterpret_cast<unsigned*>(p += 4 * nexp);
     s.ticket = reinterpret_cast<unsigned*>(p += nepoch);
+    s.start = p += 1;
     s.abort = reinterpret_cast<int*>(p += 1);
     s.ticks = wait_ticks();
     p += 1;
@@ -1774,10 +1782,7 @@ void rows_ended(RowsDev* r, RowsKind k) { r->open[k] = false; }
 hipError_t rows_cg(RowsDev* r, bool mixed, RowsCg a, hipStream_t stream) {
   a.res = r->res.p;
   const RowArgs ra = row_args(r, mixed ? kRowsCgMixed : kRowsCg, stream);
-  if (ra.ticketed) {
-    hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, stream,
-                       reinterpret_cast<u64*>(ra.sy.ticket), 1L);
-  }
+  if (ra.ticketed) hipLaunchKernelGGL(k_rows_start, dim3(1), dim3(1), 0, stream, ra.sy);
   const dim3 grid(r->nwg), block(kSlab);
   const size_t lds = cg_lds(*r, mixed ? 4 : 8);
   if (mixed)

@@ -225,3 +225,24 @@ def test_rows_are_tried_again_after_a_launch_gave_up(gpu, monkeypatch, capfd, sl
         assert on is True and niter == want[1] and np.array_equal(x, want[0])
     assert "solves" not in capfd.readouterr().err
     ctx.close()
+
+
+@pytest.mark.parametrize("prec", [bief.PREC_FP64, bief.PREC_MIXED])
+def test_latencies_count_from_the_start_of_the_solve(gpu, prec):
+    """1024 equal systems on 256 CUs, a workgroup each: the ones that wait for a CU
+    are told by their latencies. A zero right-hand side takes no time."""
+    m, sd = _case(29, 31)
+    n = 1024
+    ens = bief.Ensemble([m] * n)
+    rep = lambda a: np.concatenate([a] * n, axis=-1)  # noqa: E731
+    b = np.tile(sd["b"], (n, 1))
+    b[5] = 0.0
+    ens.set_matrix("Q", "S", rep(sd["da"]), rep(sd["xa"]))
+    _, info = ens.solve(rep(sd["x0"]), b.ravel(), slv=CG, precon=2, eps=1e-9, nitmax=500,
+                        precision=prec)
+    assert info["converged"] and ens.rows()["last_solve"] is True
+    ms = np.array(ens.latencies_ms())
+    assert ms[5] == 0.0
+    ms = np.delete(ms, 5)
+    assert ms.min() > 0.0 and ms.max() >= 2.0 * ms.min()
+    ens.close()
