@@ -36,6 +36,8 @@
 #include "layout.h"
 #include "rows_dev.h"
 
+#include "order.inl"
+
 namespace bhip {
 
 // ---------------------------------------------------------------------------
@@ -999,8 +1001,7 @@ struct bhip_ctx {
   bhip::Layout L;
   hipStream_t stream = nullptr;
   int device = 0;
-  std::mutex order_mu;
-  hipEvent_t order_ev = nullptr;  // order_streams
+  bhip::StreamOrder order;
   int grid_nodes = 0;  // grid of the node-wise kernels that leave a partial sum per block
   int grid_wide = 0;   // of the others
   // layout on device
@@ -1447,7 +1448,7 @@ int bhip_ctx_destroy(bhip_ctx* c) {
     if (sg.exec) (void)hipGraphExecDestroy(sg.exec);
   if (c->rows) rows_destroy(c->rows);
   if (c->st_host) (void)hipHostFree(c->st_host);
-  if (c->order_ev) (void)hipEventDestroy(c->order_ev);
+  if (c->order.ev) (void)hipEventDestroy(c->order.ev);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return BHIP_OK;
@@ -1462,37 +1463,19 @@ int bhip_ctx_rows(const bhip_ctx* c, int64_t* bytes, int* last_solve) {
   return BHIP_OK;
 }
 
-// `second` after what `first` holds now. One event of the context serves all
-// such calls (a wait keeps the recording it was given); streams of another
-// device than the context's take one of their own.
-static int order_streams(bhip_ctx* c, hipStream_t first, hipStream_t second) {
-  if (first == second) return BHIP_OK;
-  int dev = 0;
-  HIP_OK(hipGetDevice(&dev));
-  if (dev != c->device) {
-    hipEvent_t ev;
-    HIP_OK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    hipError_t e = hipEventRecord(ev, first);
-    if (e == hipSuccess) e = hipStreamWaitEvent(second, ev, 0);
-    (void)hipEventDestroy(ev);
-    HIP_OK(e);
-    return BHIP_OK;
-  }
-  std::lock_guard<std::mutex> one(c->order_mu);
-  if (!c->order_ev) HIP_OK(hipEventCreateWithFlags(&c->order_ev, hipEventDisableTiming));
-  HIP_OK(hipEventRecord(c->order_ev, first));
-  HIP_OK(hipStreamWaitEvent(second, c->order_ev, 0));
-  return BHIP_OK;
-}
-
 int bhip_ctx_after_stream(bhip_ctx* c, void* stream) {
   if (!c) return BHIP_EBADARG;
-  return order_streams(c, (hipStream_t)stream, c->stream);
+  hipStream_t s = (hipStream_t)stream;
+  int dev = c->device;
+  if (s != c->stream) HIP_OK(StreamOrder::device_of(s, &dev));
+  HIP_OK(c->order.after(c->device, s, dev, c->stream));
+  return BHIP_OK;
 }
 
 int bhip_stream_after_ctx(bhip_ctx* c, void* stream) {
   if (!c) return BHIP_EBADARG;
-  return order_streams(c, c->stream, (hipStream_t)stream);
+  HIP_OK(c->order.after(c->device, c->stream, c->device, (hipStream_t)stream));
+  return BHIP_OK;
 }
 
 int bhip_layout_check(int npoin, int nelem, int ndp, const int32_t* ikle, const double* x,
