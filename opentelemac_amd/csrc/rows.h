@@ -43,6 +43,7 @@ constexpr int kRefChunk = 4;
 constexpr size_t kSlabLds = 152 << 10;  // LDS of the fused D A D and assembly (by_block)
 constexpr int kMaxGroup = 8;         // slabs of one workgroup
 constexpr int kMaxGang = 256;        // workgroups of one system
+constexpr int kXcds = 8;             // dies that a launch's workgroups go to in turn
 
 struct RowLayout {
   int group = 1, nwg = 0, nslice = 0;
@@ -73,6 +74,13 @@ struct RowLayout {
   // workgroups
   std::vector<int32_t> wg_sys;       // [nwg]
   std::vector<int32_t> sys_wg;       // [nsys + 1]
+  // launches of one solve: first workgroup of each, and nwg. A launch of more
+  // than the GPU holds numbers its workgroups as they start, so that the lowest
+  // unfinished system has all of its own started, or none but its own starting
+  // next. They go to the XCDs in turn, whoever is ahead, so at the end those left
+  // may all wait for one XCD: a system must fit on one, else there are several
+  // launches, each of whole systems that the GPU holds at once.
+  std::vector<int32_t> launch;
   std::vector<int32_t> halo_off;     // [nwg + 1]
   std::vector<int32_t> halo_row;     // internal node id
   std::vector<int32_t> halo_src;     // index into the exported values

@@ -46,7 +46,7 @@
 // mask on the CUs, can keep some from starting: the limit is for them. When a
 // launch has more workgroups than fit the GPU, they take their numbers in the
 // order in which they start, so the system with the lowest numbers always has
-// all of its own running.
+// all of its own running (RowLayout::launch).
 #include "rows_dev.h"
 
 #include <algorithm>
@@ -120,10 +120,10 @@ struct SyncWords {
   u64* slots;       // [2][kReplicas][kSums][nwg][2] sums, by parity of the meeting
   u64* xch;         // [2][2][exported rows], by parity of the meeting (a float has one
                     // word only)
-  unsigned* epoch;  // [2][nsys] number of the last meeting, by parity of the launch
+  unsigned* epoch;  // [2][nsys] number of the last meeting, by parity of the solve
   int* abort;       // the launch has given up
   unsigned* ticket; // workgroups started (launches larger than the GPU)
-  u64* start;       // and the clock before the first of them
+  u64* start;       // the clock before the first of several rounds or launches
   u64 ticks;        // longest wait
 };
 
@@ -142,8 +142,10 @@ struct RowArgs {
   const uint16_t* exp_loc;
   int nwg, nsys, nexp, nhalo;
   SyncWords sy;
-  int ep;        // parity of the launch
+  int ep;        // parity of the solve
+  int first;     // first workgroup of the launch
   int ticketed;  // workgroup numbers by order of start
+  int rounds;    // not all workgroups run from the start
 };
 
 // ---------------------------------------------------------------------------
@@ -422,7 +424,7 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ val6
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   if (t == 0) {
     sh_bad = 0;
-    sh_wg = ra.ticketed ? (int)(atomicAdd(ra.sy.ticket, 1u) % (unsigned)ra.nwg) : blockIdx.x;
+    sh_wg = ra.ticketed ? (int)(atomicAdd(ra.sy.ticket, 1u) % (unsigned)ra.nwg) : ra.first + blockIdx.x;
   }
   __syncthreads();
   const int wg = __builtin_amdgcn_readfirstlane(sh_wg);
@@ -433,7 +435,7 @@ k_cg_rows(RowArgs ra, const T* __restrict__ val, const double* __restrict__ val6
   unsigned e = __hip_atomic_load(ra.sy.epoch + ra.ep * ra.nsys + sys, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
   constexpr bool kMixed = sizeof(T) == 4;
-  const u64 t_start = ra.ticketed ? ld_word(ra.sy.start) : wall_clock64();
+  const u64 t_start = ra.rounds ? ld_word(ra.sy.start) : wall_clock64();
   if (load_relaxed(ra.sy.abort)) {
     store_relaxed(&st->gave_up, 1);
     if (lead)
@@ -1425,7 +1427,7 @@ k_rows_assemble(T* __restrict__ val, double* __restrict__ val64, const double* _
   }
 }
 
-// before a launch whose workgroups take numbers as they start
+// before the launches of a solve whose workgroups do not all run from the start
 __global__ void k_rows_start(SyncWords sy) {
   *sy.ticket = 0;
   *sy.start = wall_clock64();
@@ -1487,6 +1489,7 @@ struct RowsDev {
   int nslice = 0, group = 1, nwg = 0, nsys = 1, max_halo = 0;
   int64_t nent = 0;
   int ncu = 0, nexp = 0;
+  std::vector<int32_t> launch;
   Buf<int32_t> wg_row0, slice_off, pair_off, ref_off, refs, wg_sys, sys_wg, halo_off, halo_row, halo_src,
       exp_off;
   Buf<uint16_t> rowpos, ids, exp_loc, refs16;
@@ -1611,6 +1614,7 @@ static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
   r->nent = R.nent + 64;  // load_front reads one entry column of an empty slice too
   r->ncu = ncu;
   r->nexp = (int)R.exp_loc.size();
+  r->launch = R.launch;
   lds_max -= 2048;  // the kernels' static LDS: their sums
   if (cg_lds(*r, sizeof(double)) > (size_t)lds_max || cg_lds(*r, sizeof(float)) > (size_t)lds_max)
     return nullptr;
@@ -1773,7 +1777,9 @@ static RowArgs row_args(RowsDev* r, int k, hipStream_t stream) {
   a.sy = r->sy[k];
   a.ep = r->ep[k];
   r->ep[k] ^= 1;
-  a.ticketed = r->nwg > r->ncu;
+  a.first = 0;
+  a.rounds = r->nwg > r->ncu;
+  a.ticketed = a.rounds && r->launch.size() == 2;
   return a;
 }
 
@@ -1781,19 +1787,24 @@ void rows_ended(RowsDev* r, RowsKind k) { r->open[k] = false; }
 
 hipError_t rows_cg(RowsDev* r, bool mixed, RowsCg a, hipStream_t stream) {
   a.res = r->res.p;
-  const RowArgs ra = row_args(r, mixed ? kRowsCgMixed : kRowsCg, stream);
-  if (ra.ticketed) hipLaunchKernelGGL(k_rows_start, dim3(1), dim3(1), 0, stream, ra.sy);
-  const dim3 grid(r->nwg), block(kSlab);
+  RowArgs ra = row_args(r, mixed ? kRowsCgMixed : kRowsCg, stream);
+  if (ra.rounds) hipLaunchKernelGGL(k_rows_start, dim3(1), dim3(1), 0, stream, ra.sy);
   const size_t lds = cg_lds(*r, mixed ? 4 : 8);
+  auto go = [&](auto kern, auto* val) -> hipError_t {
+    for (size_t i = 0; i + 1 < r->launch.size(); ++i) {
+      ra.first = r->launch[i];
+      hipLaunchKernelGGL(kern, dim3(r->launch[i + 1] - ra.first), dim3(kSlab), lds, stream, ra,
+                         val, r->v64.p, a);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  };
   if (mixed)
-    return with_cg_kernel<float>(r->group, a.diag != nullptr, [&](auto kern) {
-      hipLaunchKernelGGL(kern, grid, block, lds, stream, ra, r->v32.p, r->v64.p, a);
-      return hipGetLastError();
-    });
-  return with_cg_kernel<double>(r->group, a.diag != nullptr, [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, block, lds, stream, ra, r->v64.p, r->v64.p, a);
-    return hipGetLastError();
-  });
+    return with_cg_kernel<float>(r->group, a.diag != nullptr,
+                                 [&](auto kern) { return go(kern, r->v32.p); });
+  return with_cg_kernel<double>(r->group, a.diag != nullptr,
+                                [&](auto kern) { return go(kern, r->v64.p); });
 }
 
 bool rows_gmres_fits(const RowsDev* r, int bytes) { return r->gm_fits[bytes == 4]; }

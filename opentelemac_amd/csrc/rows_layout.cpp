@@ -112,6 +112,11 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
     R.max_gang = std::max(R.max_gang, R.sys_wg[s + 1] - R.sys_wg[s]);
   }
   R.nwg = (int)R.wg_sys.size();
+  R.launch.assign(1, 0);
+  if (R.nwg > max_wg && R.max_gang > max_wg / kXcds)
+    for (int s = 0; s < nsys; ++s)
+      if (R.sys_wg[s + 1] - R.launch.back() > max_wg) R.launch.push_back(R.sys_wg[s]);
+  R.launch.push_back(R.nwg);
   const int wslices = G * kSlices;  // slices of a workgroup
   R.nslice = R.nwg * wslices;
 

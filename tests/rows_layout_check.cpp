@@ -95,6 +95,17 @@ int main(int argc, char** argv) {
     }
   }
   if (!build_rows(L, nsys, off.data(), max_wg, R)) return wrong("no rows", 0);
+  // launches: whole systems; one of more workgroups than fit has systems of at
+  // most an XCD's share (an eighth)
+  if (R.launch.front() != 0 || R.launch.back() != R.nwg) return wrong("launches", 0);
+  for (size_t i = 0; i + 1 < R.launch.size(); ++i) {
+    const int a = R.launch[i], b = R.launch[i + 1];
+    if (a >= b) return wrong("empty launch", (int)i);
+    if (a > 0 && R.wg_sys[a] == R.wg_sys[a - 1]) return wrong("system cut", (int)i);
+    for (int g = a; b - a > max_wg && g < b; ++g)
+      if (R.sys_wg[R.wg_sys[g] + 1] - R.sys_wg[R.wg_sys[g]] > max_wg / 8)
+        return wrong("system wider than an XCD's share", R.wg_sys[g]);
+  }
   const int wrows = R.group * kSlab;
   // every id that the kernels read, a slice's and those load_front reads of a
   // short or empty one, names D of the workgroup's own rows or halo

@@ -246,3 +246,29 @@ def test_latencies_count_from_the_start_of_the_solve(gpu, prec):
     ms = np.delete(ms, 5)
     assert ms.min() > 0.0 and ms.max() >= 2.0 * ms.min()
     ens.close()
+
+
+def test_wide_systems_beyond_the_gpu(gpu):
+    """Ten systems of 37 workgroups of 8 slabs each: more than the GPU holds, and
+    each wider than an XCD. Whole systems per launch; the bits of each alone."""
+    m = M.channel_mesh(600, 498, 12000.0, 9960.0)
+    sd = S.wave_system(m, 2.0 + m.x / m.x.max(), dt=1.0)
+    rng = np.random.default_rng(3)
+    n = 10
+    b = sd["b"] + 1e-2 * rng.normal(size=(n, m.npoin))
+    rep = lambda a: np.concatenate([a] * n, axis=-1)  # noqa: E731
+    ens, one = bief.Ensemble([m] * n), bief.Context(m)
+    for prec in (bief.PREC_FP64, bief.PREC_MIXED):
+        kw = dict(slv=CG, precon=2, eps=1e-9, nitmax=500, precision=prec)
+        ens.set_matrix("Q", "S", rep(sd["da"]), rep(sd["xa"]))
+        x, info = ens.solve(rep(sd["x0"]), b.flatten(), **kw)
+        assert info["converged"] and ens.rows()["last_solve"] is True
+        ms = np.array(ens.latencies_ms())
+        assert ms.min() > 0.0 and ms[-1] > ms[0]
+        for k in (0, 5, 6, 9):
+            one.set_matrix("Q", "S", sd["da"], sd["xa"])
+            xa, ia = one.solve(sd["x0"].copy(), b[k].copy(), **kw)
+            assert one.rows()["last_solve"] is True and ens.infos()[k]["niter"] == ia["niter"]
+            assert np.array_equal(ens.split(x)[k], xa)
+    ens.close()
+    one.close()

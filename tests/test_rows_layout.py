@@ -24,6 +24,9 @@ def check(tmp_path_factory):
     (256, 64, "100", "far2048"), (256, 1024, "100", "far2048"), (256, 64, "700", "far4096", "3"),
     (4, 64, "1300", "far4096"), (2, 1024, "100", "far4096"), (2, 64, "9000", "far8192"),
     (256, 1024, "1024"), (256, 1024, "1025"),
+    # more workgroups than fit: narrow systems, wide ones, both
+    (16, 64, *["9000"] * 20), (16, 64, *["30000"] * 9), (16, 64, "100", "80000", *["9000"] * 20),
+    (16, 64, *["9000"] * 17, "131072", "100"),
 ])
 def test_ids_stay_within_their_workgroup(check, args):
     out = subprocess.run([check, *map(str, args)], capture_output=True, text=True)
