@@ -76,17 +76,27 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
     slabs[s] = (node_off[s + 1] - node_off[s] + kSlab - 1) / kSlab;
     if (slabs[s] > (int64_t)cap * kMaxGroup) return false;
   }
-  // slabs per workgroup: the fewest that let every system be resident at
-  // once, or (many systems) as many as a workgroup can hold. Two instead of one
-  // already past half of the workgroups: a meeting of 256 workgroups takes 1 us
-  // longer than one of 128, a second slab kept in registers less
+  // slabs per workgroup: the fewest that let every system be resident at once,
+  // or (many systems) more while that saves a fifth of the workgroups: one with
+  // empty slabs costs a round on its CU like any other, and more of a thread's
+  // rows mean fewer coefficients in its registers. us per solve, FP64 / mixed,
+  // with 1, 2, 4, 8 slabs: 2,000 systems of 500 nodes 326/423, 383/519, 606/823,
+  // 868/1336; 300 of 2,000 nodes 212/254, 140/183, 201/241, 289/334; 256 of 5k to
+  // 200k nodes -, 3936/5246, 3835/4056, 3665/3925. Two instead of one already
+  // past half of the workgroups: a meeting of 256 workgroups takes 1 us longer
+  // than one of 128, a second slab kept in registers less
   auto wgs = [&](int g) {
     int64_t t = 0;
     for (int s = 0; s < nsys; ++s) t += (slabs[s] + g - 1) / g;
     return t;
   };
-  R.group = wgs(1) <= cap / 2 ? 1 : 2;
-  while (R.group < kMaxGroup && wgs(R.group) > cap) R.group *= 2;
+  const int64_t widest = *std::max_element(slabs.begin(), slabs.end());
+  auto wants_more = [&](int g) {
+    if (widest > (int64_t)cap * g) return true;
+    return wgs(g) > (g == 1 ? cap / 2 : cap) && 5 * wgs(2 * g) <= 4 * wgs(g);
+  };
+  R.group = 1;
+  while (R.group < kMaxGroup && wants_more(R.group)) R.group *= 2;
   const int G = R.group, wrows = G * kSlab;
   // slabs and node blocks are the same rows when both start anew with each
   // system and hold kSlab of them

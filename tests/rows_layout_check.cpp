@@ -3,7 +3,7 @@
 // segment storage, a chain of neighbours, or `far`: two halves joined only with
 // each other). CHECK_FAIL in the environment: "threads", no thread can be
 // started; "memory=<n>", the n-th allocation of build_rows fails (and "bad_alloc"
-// is printed).
+// is printed). CHECK_PRINT: the slabs per workgroup are printed, nothing else.
 #include "rows.h"
 
 #include <dlfcn.h>
@@ -32,6 +32,9 @@ void* operator new(size_t n) {
   if (void* p = malloc(n ? n : 1)) return p;
   throw std::bad_alloc();
 }
+// (std::stable_sort does without its buffer)
+void* operator new(size_t n, const std::nothrow_t&) noexcept { return malloc(n ? n : 1); }
+void operator delete(void* p, const std::nothrow_t&) noexcept { free(p); }
 void operator delete(void* p) noexcept { free(p); }
 void operator delete(void* p, size_t) noexcept { free(p); }
 
@@ -95,6 +98,7 @@ int main(int argc, char** argv) {
     }
   }
   if (!build_rows(L, nsys, off.data(), max_wg, R)) return wrong("no rows", 0);
+  if (getenv("CHECK_PRINT")) return printf("%d\n", R.group) < 0;
   // launches: whole systems; one of more workgroups than fit has systems of at
   // most an XCD's share (an eighth)
   if (R.launch.front() != 0 || R.launch.back() != R.nwg) return wrong("launches", 0);

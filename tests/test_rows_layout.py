@@ -52,3 +52,17 @@ def test_a_failed_allocation_reaches_the_caller(check):
     got = [_run(check, f"memory={n}", *MANY) for n in (0, 1, 5, 20, 60, 200, 1000, 5000, 20000)]
     assert set(got) <= {"bad_alloc\n", "built\n"} and got[0] == "bad_alloc\n"
     assert got.count("bad_alloc\n") >= 6
+
+
+@pytest.mark.parametrize("systems,group", [
+    (["1024"] * 128, 1), (["131072"], 1), (["131073"], 2), (["262145"], 2), (["530000"], 4),
+    # many small ones: no empty slabs for fewer workgroups, or hardly fewer
+    (["100"] * 300, 1), (["1500"] * 300, 2), (["3000"] * 300, 4), (["9000"] * 60, 4),
+    (["100"] * 300 + ["20000"] * 2, 1),
+    # a system that needs them sets the group of all
+    (["100"] * 300 + ["1050000"], 8),
+])
+def test_slabs_per_workgroup(check, systems, group):
+    out = subprocess.run([check, "256", "1024", *systems], capture_output=True, text=True,
+                         env=dict(os.environ, CHECK_PRINT="1"))
+    assert out.stdout == f"{group}\n"
