@@ -88,10 +88,18 @@ struct RowLayout {
   std::vector<uint16_t> exp_loc;     // LDS index of the exported row
 };
 
+// LDS of the CG kernel for `bytes` (8 or 4) per value: D and A D of own rows; D,
+// A D and R of the halo; mixed: X of both in FP64
+inline size_t cg_lds(int group, size_t max_halo, int bytes) {
+  return ((size_t)2 * group * kSlab + 3 * max_halo) * bytes +
+         (bytes == 4 ? ((size_t)group * kSlab + max_halo + 1) * sizeof(double) : 0);
+}
+
 // Rows of the layout's matrix for nsys systems of node_off[nsys + 1] nodes.
-// max_wg: workgroups that can be resident at once. Returns false (and leaves R
-// empty) when a system needs more workgroups than that, or more than kMaxGang.
-// Throws std::bad_alloc.
-bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, RowLayout& R);
+// max_wg: workgroups that can be resident at once; max_lds: of one. Returns false
+// (and leaves R empty) when a system needs more workgroups than that, or more than
+// kMaxGang, or a workgroup's halo more LDS. Throws std::bad_alloc.
+bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, size_t max_lds,
+                RowLayout& R);
 
 }  // namespace bhip

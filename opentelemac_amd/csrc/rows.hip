@@ -1513,12 +1513,6 @@ struct RowsDev {
   Buf<unsigned char> gm, gmh;
 };
 
-static size_t cg_lds(const RowsDev& r, int bytes) {
-  // D and A D of own rows; D, A D and R of the halo; mixed: X of both in FP64
-  return ((size_t)2 * r.group * kSlab + (size_t)3 * r.max_halo) * bytes +
-         (bytes == 4 ? ((size_t)r.group * kSlab + r.max_halo + 1) * sizeof(double) : 0);
-}
-
 template <typename T, typename F>
 static hipError_t with_cg_kernel(int group, bool dq, F&& f) {
 #define BHIP_CG(R) (dq ? f(&k_cg_rows<T, R, true>) : f(&k_cg_rows<T, R, false>))
@@ -1533,7 +1527,7 @@ static hipError_t with_cg_kernel(int group, bool dq, F&& f) {
 
 template <typename T>
 static hipError_t cg_fits(const RowsDev& r, int lds_max, bool* fits) {
-  const size_t lds = cg_lds(r, sizeof(T));
+  const size_t lds = cg_lds(r.group, r.max_halo, sizeof(T));
   for (int dq = 0; dq < 2; ++dq) {
     const hipError_t e = with_cg_kernel<T>(r.group, dq, [&](auto kern) {
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -1600,8 +1594,12 @@ static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
   if ((*err = hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev)) !=
       hipSuccess)
     return nullptr;
+  lds_max -= 2048;  // the CG kernels' static LDS: their sums
+  size_t limit = SIZE_MAX;
+  if (const char* ev = getenv("BHIP_ROWS_BYTES")) limit = strtoull(ev, nullptr, 10);
   RowLayout R;
-  if (!build_rows(L, nsys, node_off, ncu, R)) return nullptr;
+  if (limit == 0 || lds_max <= 0 || !build_rows(L, nsys, node_off, ncu, lds_max, R))
+    return nullptr;
   std::unique_ptr<RowsDev> r(new RowsDev());
   r->nslice = R.nslice;
   r->group = R.group;
@@ -1610,14 +1608,12 @@ static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
   r->max_halo = R.max_halo;
   r->by_block = R.by_block;
   r->max_slots = R.max_slots;
-  r->lds_max = lds_max;
+  r->lds_max = lds_max + 2048;
+  r->mem.limit = limit;
   r->nent = R.nent + 64;  // load_front reads one entry column of an empty slice too
   r->ncu = ncu;
   r->nexp = (int)R.exp_loc.size();
   r->launch = R.launch;
-  lds_max -= 2048;  // the kernels' static LDS: their sums
-  if (cg_lds(*r, sizeof(double)) > (size_t)lds_max || cg_lds(*r, sizeof(float)) > (size_t)lds_max)
-    return nullptr;
   bool fits = true;
   if ((*err = cg_fits<double>(*r, lds_max, &fits)) != hipSuccess) return nullptr;
   if ((*err = cg_fits<float>(*r, lds_max, &fits)) != hipSuccess) return nullptr;
@@ -1625,7 +1621,6 @@ static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
   if ((*err = gm_fits<double>(*r, r->lds_max, &r->gm_fits[0])) != hipSuccess) return nullptr;
   if ((*err = gm_fits<float>(*r, r->lds_max, &r->gm_fits[1])) != hipSuccess) return nullptr;
   r->nhalo = (int)R.halo_row.size();
-  if (const char* ev = getenv("BHIP_ROWS_BYTES")) r->mem.limit = strtoull(ev, nullptr, 10);
   // without memory for them there are no rows, and SOLVE runs element by element
   auto ok = [&](hipError_t e) {
     if (e == hipSuccess) return true;
@@ -1789,7 +1784,7 @@ hipError_t rows_cg(RowsDev* r, bool mixed, RowsCg a, hipStream_t stream) {
   a.res = r->res.p;
   RowArgs ra = row_args(r, mixed ? kRowsCgMixed : kRowsCg, stream);
   if (ra.rounds) hipLaunchKernelGGL(k_rows_start, dim3(1), dim3(1), 0, stream, ra.sy);
-  const size_t lds = cg_lds(*r, mixed ? 4 : 8);
+  const size_t lds = cg_lds(r->group, r->max_halo, mixed ? 4 : 8);
   auto go = [&](auto kern, auto* val) -> hipError_t {
     for (size_t i = 0; i + 1 < r->launch.size(); ++i) {
       ra.first = r->launch[i];

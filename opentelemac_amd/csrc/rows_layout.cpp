@@ -17,7 +17,7 @@ namespace {
 template <typename Make, typename F>
 void parallel_for(int n, Make make, F f) {
   const int hw = (int)std::thread::hardware_concurrency();
-  const int nt = std::max(1, std::min({hw, 8, n / 16}));
+  const int nt = std::max(1, std::min({hw, 8, n / 2}));
   std::atomic<int> next{0};
   std::exception_ptr failed;
   std::mutex mu;
@@ -64,7 +64,8 @@ struct WgOut {
 
 }  // namespace
 
-bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, RowLayout& R) {
+bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, size_t max_lds,
+                RowLayout& R) {
   R = RowLayout();
   const int ndp = L.ndp;
   const int cap = std::min(max_wg, kMaxGang);
@@ -137,7 +138,12 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
   int pair_idx[6][6];
   for (int i = 0, q = 0; i < ndp; ++i)
     for (int j = i + 1; j < ndp; ++j, ++q) pair_idx[i][j] = pair_idx[j][i] = q;
+  auto fits = [&](size_t nh) {
+    return wrows + nh <= 65535 && cg_lds(G, nh, 8) <= max_lds && cg_lds(G, nh, 4) <= max_lds;
+  };
+  std::atomic<bool> refused{false};  // by one of them: the others are not wanted
   parallel_for(R.nwg, [] { return Scratch(); }, [&](int wg, Scratch& w) {
+    if (refused) return;
     const int r0 = R.wg_row0[wg], nr = nrows[wg], r1 = r0 + nr;
     const int b0 = (int)(std::upper_bound(L.node_start.begin(), L.node_start.end(), r0) -
                          L.node_start.begin()) - 1;
@@ -254,7 +260,13 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
         o.halo.push_back(c);
       }
     std::sort(o.halo.begin(), o.halo.end());
+    if (!fits(o.halo.size())) refused = true;
   });
+  if (refused) {
+    R = RowLayout();
+    return false;
+  }
+  for (const auto& o : out) R.max_halo = std::max(R.max_halo, (int)o.halo.size());
   // ---- joined --------------------------------------------------------------
   R.slice_off.assign(R.nslice + 1, 0);
   R.pair_off.assign(R.nslice + 1, 0);
@@ -275,12 +287,6 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
       // the next slice's would name another workgroup's halo)
       R.pair_off[i + 1] = R.pair_off[i] + std::max((out[g].width[q] + 1) / 2, 1);
     }
-  bool fits = true;
-  for (const auto& o : out) fits = fits && wrows + o.halo.size() <= 65535;
-  if (!fits) {
-    R = RowLayout();
-    return false;
-  }
   R.nent = units * 64;
   R.nref = runits * 64;
   R.ids.assign((size_t)R.pair_off.back() * 128, 0);
@@ -351,7 +357,6 @@ bool build_rows(const Layout& L, int nsys, const int64_t* node_off, int max_wg, 
       R.halo_src.push_back(rank[c]);
     }
     R.halo_off.push_back((int32_t)R.halo_row.size());
-    R.max_halo = std::max(R.max_halo, (int)halo[g].size());
   }
   return true;
 }

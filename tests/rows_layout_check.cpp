@@ -44,6 +44,7 @@ static int wrong(const char* what, int at) {
 }
 
 int main(int argc, char** argv) {
+  const size_t max_lds = 158 << 10;
   const int max_wg = atoi(argv[1]), block_nodes = atoi(argv[2]);
   std::vector<int> np, ne;
   std::vector<int32_t> ikle;
@@ -87,7 +88,7 @@ int main(int argc, char** argv) {
     if (strncmp(f, "memory=", 7) == 0) {
       allocations_left = atol(f + 7);
       try {
-        const bool built = build_rows(L, nsys, off.data(), max_wg, R);
+        const bool built = build_rows(L, nsys, off.data(), max_wg, max_lds, R);
         allocations_left = -1;
         printf("%s\n", built ? "built" : "no rows");
       } catch (const std::bad_alloc&) {
@@ -97,7 +98,9 @@ int main(int argc, char** argv) {
       return 0;
     }
   }
-  if (!build_rows(L, nsys, off.data(), max_wg, R)) return wrong("no rows", 0);
+  if (!build_rows(L, nsys, off.data(), max_wg, max_lds, R)) return wrong("no rows", 0);
+  if (cg_lds(R.group, R.max_halo, 8) > max_lds || cg_lds(R.group, R.max_halo, 4) > max_lds)
+    return wrong("more LDS than there is", R.max_halo);
   if (getenv("CHECK_PRINT")) return printf("%d\n", R.group) < 0;
   // launches: whole systems; one of more workgroups than fit has systems of at
   // most an XCD's share (an eighth)

@@ -66,3 +66,9 @@ def test_slabs_per_workgroup(check, systems, group):
     out = subprocess.run([check, "256", "1024", *systems], capture_output=True, text=True,
                          env=dict(os.environ, CHECK_PRINT="1"))
     assert out.stdout == f"{group}\n"
+
+
+def test_halos_beyond_the_lds_are_refused(check):
+    """Joined halves of 2 slabs need a halo of 2 slabs each; of 4, too much."""
+    for n, want in (("far4096", "ok\n"), ("far8192", "no rows (0)\n")):
+        assert subprocess.run([check, "2", "64", n], capture_output=True, text=True).stdout == want
