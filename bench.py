@@ -22,9 +22,10 @@ channel against the reference's CPU SOLVE, the headline system in segment
 storage (telemac2d's default MATRIX STORAGE = 3), the 2M SUPG tracer system by
 GMRES(5) (FP64 and mixed), the 500k-node adjoint (gradient/forward cost,
 finite-difference and tangent-linear checks), the 256-member ensemble
-(systems/s, per-system latency) and the 5M-node prism systems; each with
-the roofline figure of its element-by-element product (the CG direction kernel;
-systems of up to 2,097,152 rows are solved on assembled rows instead).
+(systems/s, per-system latency) and the 5M-node prism systems. The headline's
+roofline is that of the launch its steps spend their time in, the whole CG on
+assembled rows. The others give their element-by-element product's, the kernel of
+larger systems; `in_timed_steps` says whether the timed steps run it.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload all|...]
 """
@@ -222,7 +223,7 @@ def bench_estuary(args, dev, m, sysd):
     """The headline line: the 2M-node estuary wave-equation CG, FP64 and
     mixed, its roofline and the CPU baseline."""
     import torch
-    from opentelemac_amd import bief
+    from opentelemac_amd import bief, system as S
     t = time.time()
     ctx = bief.Context(m, block_nodes=args.block_nodes)
     st = ctx.stats()
@@ -279,13 +280,16 @@ def bench_estuary(args, dev, m, sysd):
         # per-solve latency: each solve on its own, synchronised (an idle gap
         # of 2 ms before each, so that every solve stands apart on a kernel
         # trace of this run)
-        lat = []
+        lat, cg_ms = [], []
         for _ in range(10):
             time.sleep(0.002)
             t1 = time.perf_counter()
             step(prec)
             torch.cuda.synchronize()
             lat.append(time.perf_counter() - t1)
+            cg_ms.append(_cg_ms(ctx))
+        results[name]["ms_cg_launch"] = float(np.median(cg_ms))
+        results[name]["on_rows"] = ctx.rows()["last_solve"]
         results[name]["ms_per_solve_median"] = 1e3 * float(np.median(lat))
         results[name]["ms_per_solve_max"] = 1e3 * float(np.max(lat))
         log(name, json.dumps(results[name]))
@@ -328,43 +332,65 @@ def bench_estuary(args, dev, m, sysd):
     rel_mixed_vs_fp64 = float(np.linalg.norm(sols["mixed"] - sols["fp64"])
                               / np.linalg.norm(sols["fp64"]))
 
-    # algorithmic bytes per launch of the element-by-element CG kernels (int32
-    # connectivity, 3 coefficients per element, node vectors), which larger
-    # systems run on (this one is solved in one launch on assembled rows):
+    # algorithmic bytes of the CG launch on assembled rows: per product a
+    # coefficient and a 16-bit column id for each off-diagonal entry (two per edge
+    # of the mesh), and X0, B, the scale and X once. A mixed solve reads the FP32
+    # rows in each inner iteration and the FP64 rows for each residual.
+    nent = 3 * ne + S.boundary_nodes(m).size
+    vec = 4 * 8 * nprime
+    its = {k: results[k]["iterations"] for k in results}
+    rows_bytes = {"fp64": (its["fp64"] + 1) * nent * 10 + vec,
+                  "mixed": its["mixed"] * nent * 6 +
+                  (results["mixed"]["outer"] + 1) * nent * 10 + vec}
+    tpath = os.path.join(ROOT, "profiles", "traffic_cg_rows_estuary2m.json")
+    traffic = {}
+    if os.path.exists(tpath):
+        with open(tpath) as fh:
+            traffic = json.load(fh)
+
+    # ... and per launch of the element-by-element CG kernels, which larger
+    # systems run on (int32 connectivity, 3 coefficients per element, node
+    # vectors):
     #  * FP64 CG direction + EBE mat-vec + D.AD: R, D_old read; D, AD written
     #  * mixed inner CG: the same kernel in FP32
+    # In the CG loop the FP32 kernel's ~110 MB per launch fits the 256 MB
+    # last-level cache, so part of its traffic is served from there; the
+    # cold-cache launches bound what DRAM alone sustains.
     bytes_f64 = ne * (3 * 8 + 12) + nprime * 4 * 8
     bytes_f32 = ne * (3 * 4 + 12) + nprime * 4 * 4
-    ach32 = bytes_f32 / (results["mixed"]["ms_dir_kernel"] * 1e-3) / 1e9
-    ach64 = bytes_f64 / (results["fp64"]["ms_dir_kernel"] * 1e-3) / 1e9
-    traffic = None
+    elements = _roof(bytes_f32, results["mixed"]["ms_dir_kernel"])
+    elements["kernel"] = "k_ebe<float,...,STAGE_CGDIR,EPI_CGAD,FIN_CG> (mixed inner CG direction)"
+    elements["in_timed_steps"] = not results["mixed"]["on_rows"]
+    elements["traffic"] = None
     tpath = os.path.join(ROOT, "profiles", "traffic_cg_dir_estuary2m.json")
     if os.path.exists(tpath):
         with open(tpath) as fh:
-            tj = json.load(fh)
-        traffic = tj.get("mixed_bytes_per_launch")
-    kname = "k_ebe<float,...,STAGE_CGDIR,EPI_CGAD,FIN_CG> (mixed inner CG direction)"
-    # In the CG loop the FP32 kernel's ~110 MB per launch fits the 256 MB
-    # last-level cache, so part of its traffic is served from there; the
-    # cold-cache launches below bound what DRAM alone sustains.
-    cold32 = _roof(bytes_f32, results["mixed"]["ms_dir_kernel_cold"])
-    cold64 = _roof(bytes_f64, results["fp64"]["ms_dir_kernel_cold"])
-    roofline = {"bound": "hbm", "achieved": round(ach32, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(ach32 / HBM_PEAK_GBS, 4), "traffic": traffic,
-                "kernel": kname,
-                "algorithmic_bytes_per_launch": bytes_f32,
-                "avg_launch_ms": results["mixed"]["ms_dir_kernel"],
-                "fp64_kernel": {"achieved": round(ach64, 1), "frac": round(ach64 / HBM_PEAK_GBS, 4),
-                                "algorithmic_bytes_per_launch": bytes_f64,
-                                "avg_launch_ms": results["fp64"]["ms_dir_kernel"]},
-                "cold_cache": {"note": "each launch after a 512 MiB read pass (last-level "
-                                       "cache evicted); only the kernel is timed",
-                               "fp32": {k: cold32[k] for k in ("avg_launch_ms", "achieved",
-                                                                "frac")},
-                               "fp64": {k: cold64[k] for k in ("avg_launch_ms", "achieved",
-                                                                "frac")}},
-                "copy_same_bytes": _copy_rate(dev, bytes_f32),
-                "copy_1gib": _copy_rate(dev, 1 << 30, reps=10)}
+            elements["traffic"] = json.load(fh).get("mixed_bytes_per_launch")
+    short = ("achieved", "frac", "algorithmic_bytes_per_launch", "avg_launch_ms")
+    elements["fp64_kernel"] = {k: v for k, v in
+                               _roof(bytes_f64, results["fp64"]["ms_dir_kernel"]).items()
+                               if k in short}
+    elements["cold_cache"] = {
+        "note": "each launch after a 512 MiB read pass (last-level cache evicted); only the "
+                "kernel is timed",
+        "fp32": {k: v for k, v in _roof(bytes_f32, results["mixed"]["ms_dir_kernel_cold"]).items()
+                 if k in short[:2] + short[3:]},
+        "fp64": {k: v for k, v in _roof(bytes_f64, results["fp64"]["ms_dir_kernel_cold"]).items()
+                 if k in short[:2] + short[3:]}}
+    roofline = dict(elements)
+    if results["mixed"]["on_rows"]:
+        roofline = _roof(rows_bytes["mixed"], results["mixed"]["ms_cg_launch"])
+        roofline["kernel"] = "k_cg_rows<float, ...> (the whole mixed CG, one launch)"
+        roofline["in_timed_steps"] = True
+        roofline["traffic"] = traffic.get("mixed_bytes_per_launch")
+        roofline["fp64_kernel"] = {k: v for k, v in _roof(rows_bytes["fp64"],
+                                                          results["fp64"]["ms_cg_launch"]).items()
+                                   if k in short}
+        roofline["fp64_kernel"]["traffic"] = traffic.get("fp64_bytes_per_launch")
+        roofline["elements"] = elements
+    roofline.update({
+        "copy_same_bytes": _copy_rate(dev, bytes_f32),
+        "copy_1gib": _copy_rate(dev, 1 << 30, reps=10)})
 
     cpu = None
     if not args.no_cpu_baseline:
@@ -412,6 +438,15 @@ def bench_estuary(args, dev, m, sysd):
     return line
 
 
+
+
+def _cg_ms(ctx):
+    """Device clock of the last CG solve (one system), without its preconditioning."""
+    from opentelemac_amd import bief
+    ms = np.zeros(1)
+    bief._check(bief.lib().bhip_batch_latency(ctx.handle, 1, ms.ctypes.data),
+                "bhip_batch_latency")
+    return float(ms[0])
 
 
 def _copy_rate(dev, nbytes, reps=50):
@@ -583,6 +618,7 @@ def bench_prisms(args):
         res["fp64_kernel_GBps"] = round(b64 / (res["fp64"]["ms_dir_kernel"] * 1e-3) / 1e9, 1)
         res["roofline"] = _roof(b32, res["mixed"]["ms_dir_kernel"])
         res["roofline"]["kernel"] = "k_ebe<float,...,6,...,STAGE_CGDIR,EPI_CGAD,FIN_CG>"
+        res["roofline"]["in_timed_steps"] = not ctx.rows()["last_solve"]
         res["roofline_fp64"] = _roof(b64, res["fp64"]["ms_dir_kernel"])
         res["roofline"]["cold_cache_frac"] = _roof(b32, res["mixed"]["ms_dir_kernel_cold"])["frac"]
         res["roofline_fp64"]["cold_cache_frac"] = _roof(b64,
@@ -715,6 +751,7 @@ def bench_adjoint(args, npoin=500_000, nsteps=50, checkpoint=10, n_fd=20):
     ms_dir, _ = model.ctx.time_cg_kernels(bief.PREC_MIXED, reps=50)
     roof = _roof(m.nelem * (3 * 4 + 12) + m.npoin * 4 * 4, ms_dir)
     roof["kernel"] = "k_ebe<float,...,STAGE_CGDIR,EPI_CGAD,FIN_CG> (mixed inner CG direction)"
+    roof["in_timed_steps"] = not model.ctx.rows()["last_solve"]
     return {"roofline": roof, "block_nodes": bn, "autotune_ms_per_iteration": table,
             "workload": "wave-equation adjoint, 500k nodes, 50 steps, checkpoints every 10",
             "npoin": m.npoin, "nelem": m.nelem, "steps": nsteps, "cost": j0,
@@ -819,6 +856,7 @@ def bench_supg(args, dt=10.0, nu=0.1, mesh=None):
     ne, npo = m.nelem, m.npoin
     out["roofline"] = _roof(ne * (6 * 4 + 12) + npo * 2 * 4, out["mixed"]["ms_ebe_product"])
     out["roofline"]["kernel"] = "k_ebe<float,...,SYMQ=false,...,STAGE_PLAIN,EPI_OP> (FP32 'Q')"
+    out["roofline"]["in_timed_steps"] = not ctx.rows()["last_solve"]
     out["roofline_fp64"] = _roof(ne * (6 * 8 + 12) + npo * 2 * 8, out["fp64"]["ms_ebe_product"])
     ctx.close()
     return out
@@ -834,8 +872,8 @@ def bench_ensemble(args, nsys=256):
     by CG + PRECON 2 to 1e-8, mixed precision (the configuration) and FP64,
     the node-block size chosen by the autotuner on the first 32 members. A
     step restores the assembled matrices and solves all members. Reported:
-    systems/s, and per-system completion latency (device clock from the
-    solve's set-up kernel to the kernel that stopped the system) p50/p99 over
+    systems/s, and per-system completion latency (device clock from the start
+    of the CG, the same for all, to when the system stopped) p50/p99 over
     all members of the timed steps. Beside it: the same meshes one context
     each, solved one after the other."""
     import torch
@@ -900,6 +938,7 @@ def bench_ensemble(args, nsys=256):
         roof = _roof(ne * (3 * sv + 12) + total * 4 * sv, ms_dir)
         roof["kernel"] = ("k_ebe<%s,...,STAGE_CGDIR,EPI_CGAD,FIN_CG> over all members"
                           % ("float" if sv == 4 else "double"))
+        roof["in_timed_steps"] = not ens.rows()["last_solve"]
         out[name] = {"ms_per_ensemble_step_median": float(np.median(st_ms)),
                      "systems_per_s": float(nsys * 1e3 / st_ms.mean()),
                      "per_system_latency_ms_p50": float(np.percentile(lat_sys, 50)),
@@ -979,7 +1018,8 @@ def bench_segments(args, m, sysd):
                      "iterations": infos[-1]["niter"], "outer": infos[-1]["outer_iters"],
                      "relres": infos[-1]["relres"], "converged": bool(infos[-1]["converged"]),
                      "ms_dir_kernel": ms_dir, "ms_upd_kernel": ms_upd,
-                     "roofline": _roof(alg[name], ms_dir)}
+                     "roofline": dict(_roof(alg[name], ms_dir),
+                                      in_timed_steps=not ctx.rows()["last_solve"])}
         log("segments", name, json.dumps(out[name]))
     out["mixed_speedup_vs_fp64"] = round(out["fp64"]["ms_per_solve"] /
                                          out["mixed"]["ms_per_solve"], 3)

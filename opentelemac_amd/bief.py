@@ -775,7 +775,7 @@ class Ensemble(Context):
 
     def latencies_ms(self):
         """Completion time of each mesh in the last solve (ms of device
-        clock from the solve's set-up kernel to the kernel that stopped it)."""
+        clock from the start of the CG, the same for all, to when it stopped)."""
         out = np.zeros(self.nsys)
         _check(lib().bhip_batch_latency(self._h, self.nsys, out.ctypes.data),
                "bhip_batch_latency")
