@@ -7,7 +7,7 @@
 // residual and the (inner) solution of its rows in registers, `group` rows per
 // thread, and D and A D in LDS; the first coefficients of each row stay in
 // registers too where they fit (RowProduct). Larger groups read the matrix again
-// each iteration, out of the last-level cache (120 MB for 2M rows in FP64).
+// each iteration, out of the last-level cache (143 MB for 2M rows in FP64).
 //
 // Workgroups meet once per iteration: D.AD, AD.AD, R.AD and R.R together, with
 // the exchange of A D of the halo rows. RO is R.R / D.AD; the next ||R||^2 is
@@ -28,9 +28,11 @@
 // at 1M. Beside the iterations a solve takes 75 to 130 us up to 500k nodes (PRECD1,
 // the rows, this launch's start, the state back on the host) and 310 / 380 at 2M.
 // What bounds it: below 500k the meeting (two trips through memory, 1.7 us for 20
-// workgroups, 3.5 for 245), then the matrix (8.0 TB/s in FP64 at 2M rows) and, in
-// FP32 at 2M, registers (33 spilled: with one launch per inner solve 16.7, but the
-// launches take what that gains).
+// workgroups, 3.5 for 245), then the matrix. At 2M rows in FP64 the counters see
+// 143 MB per iteration (the entries are 120) at 5.9 TB/s, from the last-level
+// cache: a copy of as much reaches 6.9, one of 1 GiB 5.2. Each wave has one slice's
+// loads in flight; more of them spill. In FP32 at 2M also registers (33 spilled:
+// with one launch per inner solve 16.7, but the launches take what that gains).
 //
 // Sums are binary trees over the rows' leaf numbers (rows.h) and do not depend
 // on how many rows a workgroup holds: a system gives the same bits alone and
