@@ -37,6 +37,7 @@
 #include "rows_dev.h"
 
 #include "order.inl"
+#include "turn.inl"
 
 namespace bhip {
 
@@ -2221,15 +2222,50 @@ static int cg_mixed(bhip_ctx* c, double* x, const double* b, double eps, int nit
 // ---------------------------------------------------------------------------
 constexpr int kGaveUp = -1;    // the launch gave up: use the solver without rows
 constexpr int kNoMemory = -2;  // no memory for the launch: likewise
+constexpr int kBusy = -3;      // other processes keep the GPU: likewise
 
-// At most one persistent launch of this process per GPU at a time: its
-// workgroups wait for each other, so two launches that share the CUs could each
-// hold what the other needs. (Two processes can: a launch then gives up after its
-// limit.)
-static std::mutex& rows_mutex(int dev) {
-  static std::mutex mu[64];
-  return mu[dev & 63];
-}
+// A launch whose workgroups wait for each other has the GPU to itself among such
+// launches: two that share the CUs could each hold what the other needs. Threads
+// take turns by a mutex per device, processes by a file per GPU (turn.inl).
+// Systems of one workgroup each wait for nothing and take no turn. ok: false when
+// another process has kept the GPU for kTurnSeconds.
+constexpr double kTurnSeconds = 2.0;
+class RowsTurn {
+ public:
+  explicit RowsTurn(bhip_ctx* c) {
+    if (!rows_meet(c->rows)) return;
+    static std::mutex mu[64];
+    static int file[64];  // its descriptor + 1, once opened; -1: none
+    const int d = c->device & 63;
+    one_ = std::unique_lock<std::mutex>(mu[d]);
+    if (file[d] == 0) {
+      static const char* const dirs[] = {"/dev/shm", "/tmp"};
+      hipUUID id;
+      std::string name = "bhip-gpu-";
+      const bool named = hipDeviceGetUuid(&id, c->device) == hipSuccess;
+      for (const char b : id.bytes) {
+        char hex[3];
+        snprintf(hex, sizeof hex, "%02x", (unsigned)(unsigned char)b);
+        name += hex;
+      }
+      const int fd = named ? turn_open(dirs, 2, name) : -1;
+      file[d] = fd < 0 ? -1 : fd + 1;
+    }
+    fd_ = file[d] - 1;
+    ok_ = turn_take(fd_, kTurnSeconds);
+  }
+  ~RowsTurn() {
+    if (ok_) turn_give(fd_);
+  }
+  RowsTurn(const RowsTurn&) = delete;
+  RowsTurn& operator=(const RowsTurn&) = delete;
+  bool ok() const { return ok_; }
+
+ private:
+  std::unique_lock<std::mutex> one_;
+  int fd_ = -1;
+  bool ok_ = true;
+};
 
 // Solves without rows follow, more each time: a launch that gives up has waited
 // 4 s, so the waits stay few however long the GPU is shared.
@@ -2237,8 +2273,8 @@ static void rows_gave_up(bhip_ctx* c) {
   c->rows_pause = c->rows_next_pause;
   if (c->rows_next_pause < (1 << 24)) c->rows_next_pause *= 2;
   fprintf(stderr,
-          "libbiefhip: the workgroups of a solve did not run at the same time (does another "
-          "process use the GPU, or a CU mask apply?); this and the next %d solves of the "
+          "libbiefhip: the workgroups of a solve did not run at the same time (does a process of "
+          "another container use the GPU, or a CU mask apply?); this and the next %d solves of the "
           "context run element by element\n",
           c->rows_pause);
 }
@@ -2246,7 +2282,8 @@ static void rows_gave_up(bhip_ctx* c) {
 // CG as in cg_fp64 or cg_mixed; the solution goes to q.x, X = 0 of a zero
 // right-hand side included
 static int cg_rows(bhip_ctx* c, bool mixed, RowsCg q, bhip_solve_info* info) {
-  std::lock_guard<std::mutex> one(rows_mutex(c->device));
+  RowsTurn turn(c);
+  if (!turn.ok()) return kBusy;
   // the launch writes the states into the pinned host copies (a copy on the
   // stream after it takes 4 us and a gap before it)
   for (int sy = 0; sy < c->nsys; ++sy) c->st_host[sy].gave_up = 0;
@@ -2419,9 +2456,9 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
     q.inner_nitmax = std::max(inner_nitmax, 1);
     q.reliable = c->reliable ? 1 : 0;
     const int r = cg_rows(c, mixed, q, info);
-    c->solved_on = written = r != kGaveUp;
     if (r == kGaveUp) rows_gave_up(c);
-    return r;
+    c->solved_on = written = r != kGaveUp && r != kBusy;
+    return written ? r : kGaveUp;
   };
   if (cfg->slv == 6) {
     rc = bhip::cgstab_fp64(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, info);
@@ -2435,9 +2472,9 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
                                       cfg->nitmax, cfg->krylov, info);
       if (moved) xsrc = c->vd1.p;
       if (rc == kGaveUp) rows_gave_up(c);
-      c->solved_on = rc != kGaveUp && rc != kNoMemory;
+      c->solved_on = rc != kGaveUp && rc != kNoMemory && rc != kBusy;
+      if (!c->solved_on) rc = kGaveUp;
     }
-    if (rc == kNoMemory) rc = kGaveUp;
     if (rc == kGaveUp && mixed)
       rc = bhip::gmres_mixed(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, cfg->krylov, xa32_ready,
                              info);

@@ -612,7 +612,8 @@ static int gmres_mixed(bhip_ctx* c, double* x, const double* b, double eps, int 
 template <typename T>
 static int gmres_rows(bhip_ctx* c, double* x, double* xout, bool* moved, const double* b,
                       double eps, int nitmax, int krylov, bhip_solve_info* info) {
-  std::lock_guard<std::mutex> one(rows_mutex(c->device));
+  RowsTurn turn(c);
+  if (!turn.ok()) return kBusy;
   // the state lies in the pinned memory of the solver states
   static_assert(sizeof(GmState) <= sizeof(SolveState), "one fits");
   GmState* s = reinterpret_cast<GmState*>(c->st_host);

@@ -43,8 +43,8 @@
 // initial solution as it was and the host solves element by element, this time
 // and the next ones (BHIP_ROWS_WAIT=<ticks> changes the limit; 0 gives up at the
 // first word that is not there yet, which the tests use).
-// All workgroups of a system must be resident at once: a process launches at
-// most one such kernel per GPU at a time. Another process that does so too, or a
+// All workgroups of a system must be resident at once: threads and processes
+// take turns on a GPU. A process that sees none of the others' files, or a
 // mask on the CUs, can keep some from starting: the limit is for them. When a
 // launch has more workgroups than fit the GPU, they take their numbers in the
 // order in which they start, so the system with the lowest numbers always has
@@ -1490,7 +1490,7 @@ struct RowsDev {
   RowsMem mem;
   int nslice = 0, group = 1, nwg = 0, nsys = 1, max_halo = 0;
   int64_t nent = 0;
-  int ncu = 0, nexp = 0;
+  int ncu = 0, nexp = 0, max_gang = 1;
   std::vector<int32_t> launch;
   Buf<int32_t> wg_row0, slice_off, pair_off, ref_off, refs, wg_sys, sys_wg, halo_off, halo_row, halo_src,
       exp_off;
@@ -1616,6 +1616,7 @@ static RowsDev* rows_build(const Layout& L, int nsys, const int64_t* node_off,
   r->ncu = ncu;
   r->nexp = (int)R.exp_loc.size();
   r->launch = R.launch;
+  r->max_gang = R.max_gang;
   bool fits = true;
   if ((*err = cg_fits<double>(*r, lds_max, &fits)) != hipSuccess) return nullptr;
   if ((*err = cg_fits<float>(*r, lds_max, &fits)) != hipSuccess) return nullptr;
@@ -1689,6 +1690,8 @@ RowsDev* rows_create(const Layout& L, int nsys, const int64_t* node_off, hipStre
 }
 
 void rows_destroy(RowsDev* r) { delete r; }
+
+bool rows_meet(const RowsDev* r) { return r->max_gang > 1; }
 
 size_t rows_bytes(const RowsDev* r) { return r->mem.used; }
 

@@ -20,6 +20,10 @@ void rows_destroy(RowsDev* r);
 // asked for. hipErrorOutOfMemory: solve without the rows.
 hipError_t rows_reserve(RowsDev* r, int bytes);
 
+// whether a launch has workgroups that wait for each other: it must not share the
+// GPU with another such launch
+bool rows_meet(const RowsDev* r);
+
 // device memory that the rows hold
 size_t rows_bytes(const RowsDev* r);
 
