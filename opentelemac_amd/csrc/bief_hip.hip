@@ -1063,7 +1063,8 @@ struct bhip_ctx {
   std::vector<SolveGraph> solve_graphs;
   bool use_graphs = true;
   bhip::RowsDev* rows = nullptr;  // assembled rows for the persistent CG, or none
-  // a launch gave up: so many solves without rows, twice as many after the next
+  // a launch gave up, or had no turn: so many solves without rows, twice as many
+  // after the next
   int rows_pause = 0, rows_next_pause = 64;
   int solved_on = -1;             // bhip_ctx_rows: what the last SOLVE ran on
   int prefetch_j = 0;  // register prefetch depth of the element kernels
@@ -2267,15 +2268,16 @@ class RowsTurn {
   bool ok_ = true;
 };
 
-// Solves without rows follow, more each time: a launch that gives up has waited
-// 4 s, so the waits stay few however long the GPU is shared.
-static void rows_gave_up(bhip_ctx* c) {
+// Solves without rows follow, more each time: what led here has taken seconds (a
+// launch's limit, or a turn's), so these stay few however long the GPU is shared.
+static void rows_gave_up(bhip_ctx* c, int why) {
   c->rows_pause = c->rows_next_pause;
   if (c->rows_next_pause < (1 << 24)) c->rows_next_pause *= 2;
   fprintf(stderr,
-          "libbiefhip: the workgroups of a solve did not run at the same time (does a process of "
-          "another container use the GPU, or a CU mask apply?); this and the next %d solves of the "
-          "context run element by element\n",
+          "libbiefhip: %s; this and the next %d solves of the context run element by element\n",
+          why == kBusy ? "another process has kept the GPU"
+                       : "the workgroups of a solve did not run at the same time (does a process "
+                         "of another container use the GPU, or a CU mask apply?)",
           c->rows_pause);
 }
 
@@ -2456,9 +2458,10 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
     q.inner_nitmax = std::max(inner_nitmax, 1);
     q.reliable = c->reliable ? 1 : 0;
     const int r = cg_rows(c, mixed, q, info);
-    if (r == kGaveUp) rows_gave_up(c);
     c->solved_on = written = r != kGaveUp && r != kBusy;
-    return written ? r : kGaveUp;
+    if (written) return r;
+    rows_gave_up(c, r);
+    return kGaveUp;
   };
   if (cfg->slv == 6) {
     rc = bhip::cgstab_fp64(c, c->vx.p, c->vb.p, cfg->eps, cfg->nitmax, info);
@@ -2471,7 +2474,7 @@ static int solve_dev(bhip_ctx* c, const bhip_solver_cfg* cfg, double* x_dev, dou
                  : gmres_rows<double>(c, c->vx.p, c->vd1.p, &moved, c->vb.p, cfg->eps,
                                       cfg->nitmax, cfg->krylov, info);
       if (moved) xsrc = c->vd1.p;
-      if (rc == kGaveUp) rows_gave_up(c);
+      if (rc == kGaveUp || rc == kBusy) rows_gave_up(c, rc);
       c->solved_on = rc != kGaveUp && rc != kNoMemory && rc != kBusy;
       if (!c->solved_on) rc = kGaveUp;
     }

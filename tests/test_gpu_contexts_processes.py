@@ -5,6 +5,7 @@ import os
 import subprocess
 import sys
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -74,12 +75,14 @@ def _context(nx, ny):
     return ctx, solve
 
 
-def test_a_gpu_that_another_process_keeps(gpu):
+@pytest.mark.parametrize("slv", [1, 7])
+def test_a_gpu_that_another_process_keeps(gpu, capfd, slv):
     """While its file is locked elsewhere, a solve waits its time and runs element
-    by element; a system of one workgroup needs no turn. Then the rows serve again."""
+    by element, and so do the next 64, at once and with one line about it; a system
+    of one workgroup needs no turn. Then the rows serve again."""
     ctx, solve = _context(70, 61)
     one, solve_one = _context(20, 21)
-    want = solve()
+    want = solve(slv)
     assert want[1] is True
     held = []
     for path in glob.glob("/dev/shm/bhip-gpu-*") + glob.glob("/tmp/bhip-gpu-*"):
@@ -87,15 +90,19 @@ def test_a_gpu_that_another_process_keeps(gpu):
         fcntl.flock(fd, fcntl.LOCK_EX | fcntl.LOCK_NB)
         held.append(fd)
     assert held
-    for slv in (1, 7):
+    capfd.readouterr()
+    t = time.perf_counter()
+    for _ in range(65):
         x, on = solve(slv)
         assert on is False
         # both stop at eps 1e-10; the scaled system's condition number is below 100
         assert np.linalg.norm(x - want[0]) <= 2e-8 * np.linalg.norm(want[0])
+    assert 2.0 <= time.perf_counter() - t <= 4.0
+    assert capfd.readouterr().err.count("another process") == 1
     assert solve_one()[1] is True
     for fd in held:
         os.close(fd)
-    x, on = solve()
+    x, on = solve(slv)
     assert on is True and np.array_equal(x, want[0])
     ctx.close()
     one.close()
